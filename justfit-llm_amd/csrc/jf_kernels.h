@@ -19,7 +19,9 @@ struct RowParams {
   uint32_t top_k;             // effective: the vocabulary when disabled
   float inv_t;                // 1 / temperature
   float top_p;
-  float minp_offset;          // temperature * log(min_p)
+  float minp_offset;          // temperature * log(min_p); without min-p, how far
+                              // below the maximum a top-p or top-k row's
+                              // boundary bins need to reach (below zero)
   float repetition;
   float repetition_inverse;   // min(1 / repetition, FLT_MAX)
   float presence;
@@ -53,40 +55,44 @@ enum RowFlags : uint32_t {
 // One block's summary of its chunk of a row.
 struct BlockHeader {
   float maximum;       // sampled: largest admitted logit (-FLT_MAX if none)
-  uint32_t count;      // sampled: candidates written
+  uint32_t count;      // sampled: candidates written (wide_row: lanes that
+                       // admit a token)
   uint32_t admitted;   // sampled: 1 when the chunk admits a non-NaN token
   uint32_t overflow;   // sampled: candidates did not fit
   float best_value;    // greedy
   uint32_t best_id;    // greedy
   uint32_t floor_key;  // sampled: the row's K-th key is at least this
+                       // (wide_row: `count` tokens of the chunk reach it)
   uint32_t reserved;
 };
 static_assert(sizeof(BlockHeader) == 32, "block headers are 32 bytes");
 
-// A row the single pass could not finish: the multi-pass stages carry it.
+// A row of the cut passes (cut_hist_kernel and the launches after it).
 struct RowState {
-  uint32_t stage;
+  uint32_t stage;     // RowStage
   float maximum;
-  uint32_t thr_key;      // min-p floor key, 0 without min-p
-  uint32_t bkey;         // kept set boundary in (key desc, id asc) order
+  uint32_t thr_key;   // min-p floor key, 0 without min-p
+  float scale;        // bins per unit below the maximum
+  uint32_t b0, b1;    // the bins that hold the kept set's end (kCutBins: no cut)
+  uint32_t bk;        // the bin of the top-k boundary (kCutBins: top-k cuts nothing)
+  uint32_t need_k;    // tokens of bin bk that top-k keeps
+  uint64_t mass_b0;   // mass of the bins before b0, before bk, of all
+  uint64_t mass_bk;
+  uint64_t total;
+  uint32_t topp;      // top-p closes the kept set in [b0, b1]
+  uint32_t bkey;      // the kept set's last token in (key desc, id asc) order
   uint32_t bid;
-  uint32_t prefix;       // radix descent
-  uint32_t pmask;
-  uint32_t chunk;        // the chunk a locate or walk stage works in
-  uint64_t remaining;    // radix descent: count or mass still to place
-  uint64_t n1;           // tokens at or above the min-p floor
-  uint64_t mass2;
-  uint64_t nucleus;
-  uint64_t mass3;
-  uint64_t target;
-  uint64_t within;       // target or rank inside `chunk`
-  uint32_t tie_key;
-  uint32_t residual;
-  float draft_w;
-  uint32_t drafted;
-  uint64_t reserved[3];
+  uint32_t kept;      // its size, where kept outputs are asked for
+  uint64_t mass3;     // its mass
+  uint64_t reserved[6];
 };
 static_assert(sizeof(RowState) == 128, "row states are 128 bytes");
+enum RowStage : uint32_t {
+  kRowDone = 0,
+  kRowWide = 1,    // the merge's min-p row with more candidates than its lists
+  kRowGather = 2,  // cut_hist_kernel found its boundary bins
+  kRowEmit = 3,    // cut_draw_kernel found its kept set; outputs or a draft's draw remain
+};
 
 struct StagePartial {
   uint64_t v[256];
@@ -98,9 +104,22 @@ constexpr int kWaves = 4;
 constexpr int kBlockCandidates = 1024;
 constexpr int kMergeCapacity = 2048;
 constexpr int kPenaltyWordsLds = 2048;
+// A sampled row with no min-p floor whose top-k is off or past this takes the
+// cut passes; up to it, the candidate lists and the merge.
+constexpr uint32_t kListTopK = 1024;
+constexpr uint32_t kCutBins = 512;    // bins of a row's values below its maximum
+constexpr uint32_t kCutRoom = 1008;   // boundary tokens a chunk can list
+constexpr uint32_t kCutItems = 3072;  // boundary tokens of a row resolved in LDS
 constexpr int kMaxExtra = 16;
 constexpr uint32_t kChunkF32 = 8192;
 constexpr uint32_t kChunkBF16 = 8192;
+
+// A sampled row of the cut passes by its policy alone (a min-p row past the
+// lists joins them too).
+__host__ __device__ constexpr bool wide_row(uint32_t flags, uint32_t top_k) {
+  return (flags & kRowSampled) && !(flags & kRowMinP) && (flags & (kRowTopP | kRowTopK)) &&
+         top_k > kListTopK;
+}
 
 struct SampleLaunch {
   const void *logits;
@@ -113,7 +132,6 @@ struct SampleLaunch {
   uint32_t rows;
   uint32_t stop0;
   uint32_t stop1;
-  uint32_t stage;
   uint32_t aligned;       // rows start on 16-byte boundaries: vector loads
   uint32_t finish_greedy; // no merge runs: uncut_kernel finishes the greedy
                           // rows
@@ -207,54 +225,6 @@ struct NoFinish {};
 struct UncutFinish {};
 struct StoreWeights {};
 constexpr uint32_t kExtraOffsetMask = (1u << 27) - 1u;
-
-// Multi-pass stages, in launch order.
-enum Stage : uint32_t {
-  kStageDone = 0,
-  kStageCount1 = 1,
-  kStageTopK3 = 2,
-  kStageTopK0 = 5,
-  kStageTopKTie = 6,
-  kStageTopKLocate = 7,
-  kStageMass2 = 8,
-  kStageTopP3 = 9,
-  kStageTopP0 = 12,
-  kStageTopPTie = 13,
-  kStageTopPLocate = 14,
-  kStageMass3 = 15,     // picks the draw's chunk for a row without a draft
-  kStageDraw = 16,      // drafted rows: residual masses, the draw's chunk
-  kStageWalk = 17,      // one block per row: the draw inside its chunk
-  kStageKeptCount = 18,
-  kStageKeptWrite = 19,
-  kStageLast = 19,
-};
-
-// Classes of stages that share code (one stage-kernel build each).
-enum StageClass : int {
-  kClsCount = 0,     // kStageCount1
-  kClsDigits = 1,    // radix digits of the k-th key and of the nucleus
-  kClsTie = 2,       // ties at the boundary key
-  kClsLocate = 3,    // the boundary token inside one chunk
-  kClsMass = 4,      // kStageMass2, kStageMass3, kStageKeptCount
-  kClsDraw = 5,
-  kClsKeptWrite = 6,
-  kClsWalk = 7,      // walk_kernel, not a stage_kernel build
-  kClsNone = 8,
-};
-__host__ __device__ constexpr int stage_class(uint32_t stage) {
-  return stage == kStageCount1 ? kClsCount
-         : (stage >= kStageTopK3 && stage <= kStageTopK0) ||
-                   (stage >= kStageTopP3 && stage <= kStageTopP0)
-             ? kClsDigits
-         : stage == kStageTopKTie || stage == kStageTopPTie       ? kClsTie
-         : stage == kStageTopKLocate || stage == kStageTopPLocate ? kClsLocate
-         : stage == kStageMass2 || stage == kStageMass3 || stage == kStageKeptCount
-             ? kClsMass
-         : stage == kStageDraw      ? kClsDraw
-         : stage == kStageKeptWrite ? kClsKeptWrite
-         : stage == kStageWalk      ? kClsWalk
-                                    : kClsNone;
-}
 
 struct AcceptChainLane {
   uint32_t remaining;
@@ -436,7 +406,9 @@ struct LeanLaunch {
   uint32_t row_of[kKernargRows];
 };
 int launch_residual(const LeanLaunch &l, uint32_t dtype, void *stream);
-int launch_stage(const SampleLaunch &a, uint32_t dtype, void *stream);
+// The cut passes over the rows that take them: cut_hist_kernel, cut_draw_kernel
+// and, with `emit` (kept outputs or drafted rows), cut_emit_kernel.
+int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream);
 int launch_accept_chain(const AcceptChainLaunch &a, void *stream);
 int launch_accept_tree(const AcceptTreeLaunch &a, void *stream);
 // jf_draft.hip; the events, when set, bracket the top-16 kernel.

@@ -648,6 +648,14 @@ __device__ __forceinline__ bool uncut_row(const RowParams &rp) {
   return (rp.flags & kRowSampled) && !(rp.flags & (kRowMinP | kRowTopK | kRowTopP));
 }
 
+// Whether cut_hist_kernel and the launches after it may have the row: always
+// (wide_row), or when the merge finds its min-p candidates past the lists.
+__device__ __forceinline__ bool cut_pass_row(const RowParams &rp) {
+  return wide_row(rp.flags, rp.top_k) ||
+         ((rp.flags & kRowSampled) && (rp.flags & kRowMinP) &&
+          rp.top_k > (uint32_t)kBlockCandidates);
+}
+
 template <class L>
 __device__ __forceinline__ float draft_q(const SampleLaunch &a, const RowParams &rp,
                                          uint32_t token, const L &s) {
@@ -1451,28 +1459,6 @@ __device__ __forceinline__ uint32_t reselect_chunk(const SampleLaunch &a,
   return n;
 }
 
-// Starts the multi-pass stages of a row the merge cannot finish.
-__device__ __forceinline__ void begin_stages(const SampleLaunch &a, const RowParams &rp,
-                             uint32_t row, float maximum) {
-  RowState st = {};
-  st.maximum = maximum;
-  st.bkey = 0;
-  st.bid = 0;
-  // The members' count decides whether top-k cuts; a row with neither
-  // min-p nor top-k keeps every admitted token.
-  if (rp.flags & (kRowMinP | kRowTopK)) {
-    st.thr_key = (rp.flags & kRowMinP)
-                     ? logit_key(__builtin_fminf(maximum + rp.minp_offset, maximum))
-                     : 0u;
-    st.stage = kStageCount1;
-  } else {
-    st.thr_key = 0;
-    st.stage = (rp.flags & kRowTopP) ? kStageMass2 : kStageMass3;
-  }
-  st.drafted = row_draft(a, rp) != kNoToken ? 1u : 0u;
-  a.states[row] = st;
-}
-
 template <int DT>
 __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowParams &rp,
                               uint32_t row, Lds &s) {
@@ -1544,7 +1530,7 @@ __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowPa
   if (admitted == 0 || maximum == __builtin_inff()) {
     if (tid == 0) {
       write_result(a, row, kNoToken, 0.0f, 0);
-      a.states[row].stage = kStageDone;
+      a.states[row].stage = kRowDone;
     }
     return;
   }
@@ -1584,10 +1570,11 @@ __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowPa
   const bool fits = n_all <= (uint32_t)kMergeCapacity;
   if ((overflow && K > (uint32_t)kBlockCandidates) ||
       (!fits && K > (uint32_t)kMergeCapacity)) {
-    if (tid == 0) begin_stages(a, rp, row, maximum);
+    // A min-p floor that leaves more tokens than the lists hold.
+    if (tid == 0) a.states[row].stage = kRowWide;
     return;
   }
-  if (tid == 0) a.states[row].stage = kStageDone;
+  if (tid == 0) a.states[row].stage = kRowDone;
   MergeLds &m = s.merge;
   uint32_t n;
   if (spec && !overflow && s.row_maxcount <= P && thr > kLowestKey) {
@@ -1773,11 +1760,8 @@ __device__ __forceinline__ void merge_row(const SampleLaunch &a,
                                           const RowParams &rp, uint32_t row,
                                           Lds &s) {
   const uint32_t S = a.chunks, tid = threadIdx.x;
-  if (uncut_row(rp)) {
-    // The uncut kernel draws it; no stage may pick it up.
-    if (tid == 0) a.states[row].stage = kStageDone;
-    return;
-  }
+  // The uncut kernel draws it, or cut_hist_kernel and the launches after it.
+  if (uncut_row(rp) || wide_row(rp.flags, rp.top_k)) return;
   if (!(rp.flags & kRowSampled)) {
     if (tid < 64) {
       float bv = -__builtin_inff();
@@ -1792,10 +1776,7 @@ __device__ __forceinline__ void merge_row(const SampleLaunch &a,
         }
       }
       wave_argmax(bv, bi);
-      if (tid == 0) {
-        write_result(a, row, bi, 0.0f, 0);
-        a.states[row].stage = kStageDone;
-      }
+      if (tid == 0) write_result(a, row, bi, 0.0f, 0);
     }
     return;
   }
@@ -1971,10 +1952,14 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
     const uint32_t K = rp.top_k;
     const uint32_t kw = (K + kWaves - 1) / kWaves;
     const bool bound = (rp.flags & kRowTopK) && kw <= 64;
+    const bool wide = wide_row(rp.flags, K);
     uint32_t wth = 0;
-    if (bound) wth = wave_kth_largest(any ? logit_key(mx) : 0u, kw);
+    if (wide)
+      wth = wave_min_u32(any ? logit_key(mx) : 0xffffffffu);
+    else if (bound)
+      wth = wave_kth_largest(any ? logit_key(mx) : 0u, kw);
     const float wmax = wave_max_f32(mx);
-    const uint32_t wany = ballot(any) != 0 ? 1u : 0u;
+    const uint32_t wany = (uint32_t)__popcll(ballot(any));
     if (lane == 0) {
       s.wf[w] = wmax;
       s.wu[w] = wany;
@@ -1993,7 +1978,19 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
       return;
     }
     const uint32_t tk =
-        bound ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
+        bound || wide ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
+    if (wide) {
+      // No candidates: every lane that admits a token holds one at or above
+      // the least of the lanes' maxima.
+      if (tid == 0) {
+        hdr->maximum = bmax;
+        hdr->count = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
+        hdr->admitted = badm;
+        hdr->overflow = 0;
+        hdr->floor_key = tk;
+      }
+      return;
+    }
     uint32_t thr = tk;
     if (rp.flags & kRowMinP)
       thr = max(thr, logit_key(__builtin_fminf(bmax + rp.minp_offset, bmax)));
@@ -3073,10 +3070,14 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
   const uint32_t K = rp.top_k;
   const uint32_t kw = (K + kWaves - 1) / kWaves;
   const bool bound = (flags & kRowTopK) && kw <= 64;
+  const bool wide = wide_row(flags, K);
   uint32_t wth = 0;
-  if (bound) wth = wave_kth_bound16(any ? logit_key(mx) : 0u, kw);
+  if (wide)
+    wth = wave_min_u32(any ? logit_key(mx) : 0xffffffffu);
+  else if (bound)
+    wth = wave_kth_bound16(any ? logit_key(mx) : 0u, kw);
   const float wmax = wave_max_f32(mx);
-  const uint32_t wany = ballot(any) != 0 ? 1u : 0u;
+  const uint32_t wany = (uint32_t)__popcll(ballot(any));
   if (lane == 0) {
     s.wf[w] = wmax;
     s.wu[w] = wany;
@@ -3090,7 +3091,19 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
       -3.402823466e38f);
   const uint32_t badm = s.wu[0] | s.wu[1] | s.wu[2] | s.wu[3];
   const uint32_t tk =
-      bound ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
+      bound || wide ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
+  if (wide) {
+    // No candidates: every lane that admits a token holds one at or above the
+    // least of the lanes' maxima.
+    if (tid == 0) {
+      hdr->maximum = bmax;
+      hdr->count = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
+      hdr->admitted = badm;
+      hdr->overflow = 0;
+      hdr->floor_key = tk;
+    }
+    return;
+  }
   if (uncut) {
     // The row keeps every admitted token: the uncut kernel's chunk summary,
     // or (FUSE) the row finished here.
@@ -3466,11 +3479,10 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
       cpr = a.cand_probs[(uint64_t)rp.cand_index * 16 + tid];
     }
   }
-  if (uncut_row(rp)) {
-    // The uncut kernel draws it.
-    if (tid == 0) a.states[row].stage = kStageDone;
-    return;
-  }
+  // The uncut kernel draws it, or cut_hist_kernel and the launches after it.
+  if (uncut_row(rp) || wide_row(rp.flags, rp.top_k)) return;
+  // The general path may hand a min-p row on to cut_hist_kernel.
+  if (tid == 0 && cut_pass_row(rp)) a.states[row].stage = kRowDone;
 
   if (!(rp.flags & kRowSampled)) {
     // Greedy: the largest chunk best, the lowest id among equals.
@@ -3584,7 +3596,7 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
 }
 #endif
 
-// ---- multi-pass stages ---------------------------------------------------
+// ---- reading a chunk again -------------------------------------------------
 
 // A drafted row's dense q over this thread's tokens of a chunk, in the
 // order of the chunk's logits; 16-byte loads when the rows are aligned.
@@ -3699,451 +3711,711 @@ __device__ __forceinline__ uint32_t walk_chunk(const SampleLaunch &a, const RowP
   return s.hit;
 }
 
-// The stage kernel is compiled once per class of stages, so each launch
-// carries only its stage's code and registers.
+// ---- rows whose cut the candidate lists cannot hold -------------------------
+//
+// A sampled row that keeps many tokens (no top-k, or one past kListTopK, with
+// no min-p floor; or a min-p floor whose candidates overflowed their lists)
+// finds its kept set's boundary from a histogram of its values, in two passes
+// over the logits after the select's:
+//  - cut_hist_kernel: every chunk bins its members by their distance below the
+//    row maximum (kCutBins equal steps over the range that can hold the
+//    boundary, cut_range) and sums each bin's exact mass (and count, where
+//    top-k or the kept outputs need it). The row's last chunk to arrive adds
+//    the chunks' bins up and finds the bins that hold the top-k and top-p
+//    boundaries.
+//  - cut_draw_kernel: every chunk lists its tokens in those bins and sums its
+//    mass before them; the row's last chunk to arrive finds the exact boundary
+//    among the listed tokens, each chunk's kept mass, and draws: the chunk,
+//    then the walk inside it.
+//  - cut_emit_kernel, only for kept outputs and drafted rows: writes the kept
+//    tokens, sums the residual masses, and draws a drafted row.
+// The bins are equal for equal keys and fall with the key, so they only
+// bracket the boundary: every decision is made on exact counts and masses,
+// and a row whose boundary bins hold more tokens than the lists (ties, a
+// range far off) is resolved by the same steps over its logits instead
+// (cut_rescan).
+struct __align__(16) CutHistLds {
+  PrepLds prep;
+  uint64_t mass[kCutBins];
+  uint32_t count[kCutBins];
+  uint64_t wl[kWaves];
+  uint32_t last;
+  uint32_t sel[3];  // b0, b1, bk
+  uint32_t need_k;
+  uint64_t base[2];  // mass before b0, before bk
+  uint64_t bin_mass;
+};
+
+struct __align__(16) CutLds {
+  union {
+    PrepLds prep;
+    uint64_t items[kCutItems];
+  };
+  uint64_t hist[256];
+  uint32_t hcount[256];
+  uint64_t small[64];
+  uint64_t sorted[64];
+  uint64_t cmass[kMaxChunks];
+  uint32_t ccount[kMaxChunks];
+  uint32_t coff[kMaxChunks + 1];
+  uint64_t wj[kWaves][8];
+  uint64_t wl[kWaves];
+  uint64_t wl2[kWaves];
+  uint32_t cids[16];
+  float cprobs[16];
+  uint32_t last;
+  uint32_t hit;
+  uint32_t n;
+  uint32_t sel_bin;
+  uint32_t sel_chunk;
+  uint64_t sel_excl;
+  uint64_t u64a;
+  uint64_t bound;  // the kept set's last token, as cut_item
+};
+
+// A (row, chunk)'s part of the candidate area during these passes, in 64-bit
+// words: the bins' masses [0, kCutBins) and counts (two a word) from
+// kCutBins, overwritten by the listed tokens [0, kCutRoom) once this chunk's
+// bins are summed; the last words hold the chunk's sums.
+constexpr uint32_t kCutMassWord = kBlockCandidates - 8;   // mass before b0
+constexpr uint32_t kCutCountWord = kBlockCandidates - 7;  // tokens before b0 | listed << 32
+constexpr uint32_t kCutKeptWord = kBlockCandidates - 6;   // kept tokens of the chunks before
+constexpr uint32_t kCutResidualWord = kBlockCandidates - 5;
+constexpr uint32_t kCutDraftWord = kBlockCandidates - 4;  // draft token's weight bits | 1 << 32
+static_assert(kCutBins + kCutBins / 2 <= kCutRoom && kCutRoom <= kCutMassWord);
+
+__device__ __forceinline__ uint64_t *cut_area(const SampleLaunch &a, uint32_t row, uint32_t chunk) {
+  return a.cands + ((uint64_t)row * a.chunks + chunk) * kBlockCandidates;
+}
+// The bin of a member: its distance below the maximum in steps of 1 / scale,
+// the last bin open-ended. Falls monotonically with the key (each operation
+// rounds monotonically; fmin also takes the NaN of inf * 0 to the last bin).
+__device__ __forceinline__ uint32_t cut_bin(float v, float maximum, float scale) {
+  return (uint32_t)__builtin_fminf((maximum - v) * scale, (float)(kCutBins - 1));
+}
+// A token as one word that orders as (key, lower id first): ids are below 2^19.
+__device__ __forceinline__ uint64_t cut_item(uint32_t key, uint32_t id) {
+  return ((uint64_t)key << 19) | (0x7ffffu - id);
+}
+__device__ __forceinline__ uint32_t cut_key(uint64_t item) { return (uint32_t)(item >> 19); }
+__device__ __forceinline__ uint32_t cut_id(uint64_t item) { return 0x7ffffu - ((uint32_t)item & 0x7ffffu); }
+
+
+// Bound: HBM or the Infinity Cache, then the weights (about 30 VALU
+// instructions a token). LDS atomics only for the tokens inside the bins'
+// range: for top-p alone the range leaves out every token that together
+// cannot hold the boundary (cut_range), which in a language model's row is
+// most of them; they add to the mass from registers.
 #if JF_IN(3)
-template <int DT, int CLS>
-__global__ __launch_bounds__(kThreads) void stage_kernel(SampleLaunch a) {
-  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
-                LOADS = Geo<DT>::LOADS;
-  constexpr uint32_t CHUNK = Geo<DT>::CHUNK;
-  constexpr uint32_t VMASK = (1u << VEC) - 1u;
-  __shared__ Lds s;
+template <int DT>
+__global__ __launch_bounds__(kThreads) void cut_hist_kernel(SampleLaunch a) {
+  constexpr int TPL = Geo<DT>::TPL;
+  __shared__ CutHistLds s;
   const uint32_t S = a.chunks;
   const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
-  const uint32_t tid = threadIdx.x;
-  const uint32_t stage = a.stage;
-  if (stage_class(stage) != CLS) return;
-  // The row's parameters are requested with its state, in one round trip.
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
   const RowParams rp = a.params[row];
-  RowState st = a.states[row];
-  if (st.stage != stage) return;
-  const bool single = stage == kStageTopKLocate || stage == kStageTopPLocate;
-  if (single && chunk != st.chunk) return;
-  // The draw stage's dense q is requested ahead of the chunk's logits.
-  float qv[CLS == kClsDraw ? TPL : 1];
-  if constexpr (CLS == kClsDraw)
-    if (a.dense_q) load_dense_q<DT>(a, rp, chunk, qv);
+  if (!cut_pass_row(rp)) return;
+  if (!wide_row(rp.flags, rp.top_k) && a.states[row].stage != kRowWide) return;
+  // The row's chunk summaries, one a lane in every wave (S <= 64).
+  const BlockHeader *hb = a.headers + (uint64_t)row * S;
+  const BlockHeader h = hb[min(lane, S - 1)];
   float xs[TPL];
   load_chunk<DT>(a, rp, row, chunk, s, xs);
-  stage_candidates(a, rp, s);
-  const uint32_t lane_base = chunk * CHUNK + tid * VEC;
-  const float M = st.maximum, inv_t = rp.inv_t;
-  // Members: admitted (non-NaN), at or above the min-p floor, at or before
-  // the kept boundary.
-  uint64_t mem = 0;
+  for (uint32_t b = tid; b < kCutBins; b += kThreads) {
+    s.mass[b] = 0;
+    s.count[b] = 0;
+  }
+  const float M = wave_max_f32(h.maximum);
+  const uint32_t admitted = wave_max_u32(h.admitted);
+  if (!admitted || M == __builtin_inff()) {
+    if (chunk == 0 && tid == 0) {
+      write_result(a, row, kNoToken, 0.0f, 0);
+      a.states[row].stage = kRowDone;
+    }
+    return;
+  }
+  const float inv_t = rp.inv_t;
+  const bool minp = (rp.flags & kRowMinP) != 0, topk = (rp.flags & kRowTopK) != 0;
+  const uint32_t thr_key = minp ? logit_key(__builtin_fminf(M + rp.minp_offset, M)) : 0u;
+  // The bins' range below the maximum.
+  float range = -rp.minp_offset;
+  if (topk && !minp) {
+    // Each chunk's floor_key: a key that `count` of its tokens reach.
+    const bool in = lane < S && h.count;
+    const uint32_t floor_key = wave_min_u32(in ? h.floor_key : 0xffffffffu);
+    const uint32_t reach = wave_sum_u32(in ? h.count : 0u);
+    const float r = M - key_logit(floor_key);
+    if (rp.top_k <= reach && r < 1.0e30f) range = r;
+  }
+  const float scale = __builtin_fminf((float)(kCutBins - 1) / range, 3.0e38f);
+  const bool counts = topk || a.out_kept_ids;
+  __syncthreads();
+  uint64_t tail = 0;
+  uint32_t tail_n = 0;
 #pragma unroll
   for (int i = 0; i < TPL; ++i) {
     const float v = xs[i];
-    if (v != v) continue;
-    const uint32_t k = logit_key(v);
-    const uint32_t t = lane_base + (i / VEC) * SLAB + (i % VEC);
-    if (k >= st.thr_key && at_or_before(k, t, st.bkey, st.bid)) mem |= 1ull << i;
+    const bool member = v == v && (!minp || logit_key(v) >= thr_key);
+    const uint64_t wq = member ? quantized_weight(v, M, inv_t) : 0ull;
+    const uint32_t b = cut_bin(v, M, scale);
+    if (member && b < kCutBins - 1) {
+      atomicAdd((unsigned long long *)&s.mass[b], (unsigned long long)wq);
+      if (counts) atomicAdd(&s.count[b], 1u);
+    } else {
+      tail += wq;
+      tail_n += member ? 1u : 0u;
+    }
   }
-  StagePartial *part = a.partials + (uint64_t)row * S + chunk;
-  const uint32_t draft = row_draft(a, rp);
-
-  auto wq_of = [&](int i) -> uint64_t {
-    return quantize(weight_of(xs[i], M, inv_t));
-  };
-  auto tok_of = [&](int i) -> uint32_t {
-    return lane_base + (i / VEC) * SLAB + (i % VEC);
-  };
-  // The `within`-th (0-based) token with a set bit, in id order; returns
-  // its token in every thread.
-  auto locate = [&](uint64_t bits, uint64_t within) -> uint32_t {
-    if (tid == 0) s.hit = kNoToken;
-    uint32_t nb[LOADS], off[LOADS];
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j) nb[j] = __popc((uint32_t)(bits >> (j * VEC)) & VMASK);
-    order_offsets<LOADS>(nb, off, s);
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j) {
-      uint64_t idx = off[j];
-#pragma unroll
-      for (int e = 0; e < VEC; ++e)
-        if ((bits >> (j * VEC + e)) & 1u) {
-          if (idx == within) s.hit = tok_of(j * VEC + e);
-          ++idx;
-        }
-    }
-    __syncthreads();
-    return s.hit;
-  };
-
-  switch (stage) {
-    case kStageCount1: {
-      if constexpr (CLS == kClsCount) {
-      const uint32_t c = block_sum_u32(__popcll(mem), s);
-      if (tid == 0) st_dev(&part->v[0], (uint64_t)c);
-      }
-      break;
-    }
-    case kStageTopK3: case kStageTopK3 + 1: case kStageTopK3 + 2: case kStageTopK0:
-    case kStageTopP3: case kStageTopP3 + 1: case kStageTopP3 + 2: case kStageTopP0: {
-      if constexpr (CLS == kClsDigits) {
-      const bool by_mass = stage >= kStageTopP3;
-      const int d = by_mass ? (int)(kStageTopP0 - stage) : (int)(kStageTopK0 - stage);
-      s.hist[tid] = 0;
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < TPL; ++i) {
-        if (!((mem >> i) & 1)) continue;
-        const uint32_t k = logit_key(xs[i]);
-        if ((k & st.pmask) != st.prefix) continue;
-        const uint64_t v = by_mass ? wq_of(i) : 1ull;
-        if (v) atomicAdd((unsigned long long *)&s.hist[(k >> (8 * d)) & 255u],
-                         (unsigned long long)v);
-      }
-      __syncthreads();
-      st_dev(&part->v[tid], s.hist[tid]);
-      }
-      break;
-    }
-    case kStageTopKTie:
-    case kStageTopPTie: {
-      if constexpr (CLS == kClsTie) {
-      uint32_t c = 0;
-#pragma unroll
-      for (int i = 0; i < TPL; ++i)
-        c += ((mem >> i) & 1) && logit_key(xs[i]) == st.tie_key;
-      c = block_sum_u32(c, s);
-      if (tid == 0) st_dev(&part->v[0], (uint64_t)c);
-      }
-      break;
-    }
-    case kStageTopKLocate:
-    case kStageTopPLocate:
-      break;
-    case kStageMass2:
-    case kStageMass3:
-    case kStageKeptCount: {
-      if constexpr (CLS == kClsMass) {
-      uint64_t sum = 0;
-      uint32_t c = 0;
-      if (tid == 0) {
-        s.found_w = 0.0f;
-        s.u32a = 0;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < TPL; ++i)
-        if ((mem >> i) & 1) {
-          sum += wq_of(i);
-          ++c;
-        }
-      if (stage == kStageMass3 && draft != kNoToken) {
-#pragma unroll
-        for (int i = 0; i < TPL; ++i)
-          if (((mem >> i) & 1) && tok_of(i) == draft) {
-            s.found_w = weight_of(xs[i], M, inv_t);
-            s.u32a = 1;
-          }
-      }
-      sum = block_sum_u64(sum, s);
-      c = block_sum_u32(c, s);
-      if (tid == 0) {
-        st_dev(&part->v[0], stage == kStageKeptCount ? (uint64_t)c : sum);
-        st_dev(&part->v[1], (uint64_t)s.u32a);
-        st_dev(&part->v[2], (uint64_t)__float_as_uint(s.found_w));
-      }
-      }
-      break;
-    }
-    case kStageDraw: {
-      if constexpr (CLS == kClsDraw) {
-      uint64_t dsum = 0, wsum = 0;
-      uint32_t any = 0;
-#pragma unroll
-      for (int i = 0; i < TPL; ++i)
-        if ((mem >> i) & 1) {
-          const uint64_t wq = wq_of(i);
-          wsum += wq;
-          if (st.drafted) {
-            const float q = a.dense_q ? qv[i] : draft_q(a, rp, tok_of(i), s);
-            const uint64_t d = residual_of(wq, st.mass3, q);
-            dsum += d;
-            any |= d > 0;
-          }
-        }
-      dsum = block_sum_u64(dsum, s);
-      wsum = block_sum_u64(wsum, s);
-      any = block_max_u32(any, s);
-      if (tid == 0) {
-        st_dev(&part->v[0], dsum);
-        st_dev(&part->v[1], wsum);
-        st_dev(&part->v[2], (uint64_t)any);
-      }
-      }
-      break;
-    }
-    case kStageKeptWrite: {
-      if constexpr (CLS == kClsKeptWrite) {
-      // Offset of this chunk: the kept counts of the chunks before it.
-      uint64_t off = 0;
-      for (uint32_t c = 0; c < chunk; ++c) off += a.partials[(uint64_t)row * S + c].v[0];
-      const double scale = (double)st.mass3 * 0x1p-44;
-      uint32_t nb[LOADS], offs[LOADS];
-#pragma unroll
-      for (int j = 0; j < LOADS; ++j) nb[j] = __popc((uint32_t)(mem >> (j * VEC)) & VMASK);
-      order_offsets<LOADS>(nb, offs, s);
-#pragma unroll
-      for (int j = 0; j < LOADS; ++j) {
-        uint64_t idx = off + offs[j];
-#pragma unroll
-        for (int e = 0; e < VEC; ++e)
-          if ((mem >> (j * VEC + e)) & 1u) {
-            if (idx < a.kept_cap) {
-              const int i = j * VEC + e;
-              a.out_kept_ids[(uint64_t)row * a.kept_cap + idx] = tok_of(i);
-              a.out_kept_probs[(uint64_t)row * a.kept_cap + idx] =
-                  st.mass3 ? (float)((double)weight_of(xs[i], M, inv_t) / scale)
-                           : 0.0f;
-            }
-            ++idx;
-          }
-      }
-      }
-      break;
-    }
-    default:
-      break;
+  tail = wave_sum_u64(tail);
+  tail_n = wave_sum_u32(tail_n);
+  if (lane == 0) {
+    atomicAdd((unsigned long long *)&s.mass[kCutBins - 1], (unsigned long long)tail);
+    atomicAdd(&s.count[kCutBins - 1], tail_n);
   }
-
-  if constexpr (CLS == kClsLocate) {
-  if (stage == kStageTopKLocate || stage == kStageTopPLocate) {
-    // The within-th tie of this chunk closes the kept set.
-    uint64_t ties = 0;
-#pragma unroll
-    for (int i = 0; i < TPL; ++i)
-      if (((mem >> i) & 1) && logit_key(xs[i]) == st.tie_key) ties |= 1ull << i;
-    const uint32_t id = locate(ties, st.within);
-    if (tid == 0) {
-      RowState &ns = a.states[row];
-      ns.bkey = st.tie_key;
-      ns.bid = id;
-      ns.prefix = 0;
-      ns.pmask = 0;
-      if (stage == kStageTopKLocate && (rp.flags & kRowTopP))
-        ns.stage = kStageMass2;
-      else
-        ns.stage = kStageMass3;
-    }
-    return;
-  }
-  }
+  __syncthreads();
+  uint64_t *area = cut_area(a, row, chunk);
+  st_dev(area + 2 * tid, s.mass[2 * tid]);
+  st_dev(area + 2 * tid + 1, s.mass[2 * tid + 1]);
+  if (counts)
+    st_dev(area + kCutBins + tid,
+           (uint64_t)s.count[2 * tid] | ((uint64_t)s.count[2 * tid + 1] << 32));
   if (!arrive_last(a.counters + row, S, s)) return;
 
-  // Finalize the stage for this row. The chunks' partials are read with
-  // every load in flight at once: a runtime loop of device-coherent loads
-  // would wait a round trip per chunk.
-  const StagePartial *parts = a.partials + (uint64_t)row * S;
-  if constexpr (CLS == kClsDigits) {
-  if ((stage >= kStageTopK3 && stage <= kStageTopK0) ||
-      (stage >= kStageTopP3 && stage <= kStageTopP0)) {
-    uint64_t h = 0;
-    for (uint32_t c0 = 0; c0 < S; c0 += 8) {
-      uint64_t t[8];
+  // The row's bins: thread t sums bins 2t and 2t + 1 over the chunks.
+  uint64_t m0 = 0, m1 = 0;
+  uint32_t n0 = 0, n1 = 0;
+  const uint64_t *rows = cut_area(a, row, 0);
+  constexpr int B = 16;
+  for (uint32_t c0 = 0; c0 < S; c0 += B) {
+    uint64_t t0[B], t1[B];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) t[k] = ld_dev(&parts[min(c0 + k, S - 1)].v[tid]);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) h += c0 + k < S ? t[k] : 0ull;
+    for (int k = 0; k < B; ++k) {
+      const uint64_t *p = rows + (uint64_t)min(c0 + k, S - 1) * kBlockCandidates;
+      t0[k] = ld_dev(p + 2 * tid);
+      t1[k] = ld_dev(p + 2 * tid + 1);
     }
-    s.hist[tid] = h;
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      m0 += c0 + k < S ? t0[k] : 0ull;
+      m1 += c0 + k < S ? t1[k] : 0ull;
+    }
+  }
+  if (counts)
+    for (uint32_t c0 = 0; c0 < S; c0 += B) {
+      uint64_t t[B];
+#pragma unroll
+      for (int k = 0; k < B; ++k)
+        t[k] = ld_dev(rows + (uint64_t)min(c0 + k, S - 1) * kBlockCandidates + kCutBins + tid);
+#pragma unroll
+      for (int k = 0; k < B; ++k) {
+        n0 += c0 + k < S ? (uint32_t)t[k] : 0u;
+        n1 += c0 + k < S ? (uint32_t)(t[k] >> 32) : 0u;
+      }
+    }
+  if (tid == 0) {
+    s.sel[0] = s.sel[1] = s.sel[2] = kCutBins;
+    s.need_k = 0;
+    s.base[0] = s.base[1] = s.bin_mass = 0;
+  }
+  uint64_t total, members = 0;
+  const uint64_t me = block_excl_scan_u64(m0 + m1, s, &total);
+  if (topk) {
+    const uint32_t ce = (uint32_t)block_excl_scan_u64(n0 + n1, s, &members);
+    const uint32_t K = rp.top_k;
+    if (K < members) {
+      // The bin of the K-th member.
+      const bool lo = ce < K && ce + n0 >= K, hi = ce + n0 < K && ce + n0 + n1 >= K;
+      if (lo || hi) {
+        s.sel[2] = 2 * tid + (hi ? 1u : 0u);
+        s.need_k = K - ce - (hi ? n0 : 0u);
+        s.base[1] = me + (hi ? m0 : 0ull);
+        s.bin_mass = hi ? m1 : m0;
+      }
+    }
     __syncthreads();
-    crossing_bin(s, st.remaining);
-    if (tid == 0) {
-      const bool by_mass = stage >= kStageTopP3;
-      const int d = by_mass ? (int)(kStageTopP0 - stage) : (int)(kStageTopK0 - stage);
-      RowState &ns = a.states[row];
-      ns.remaining = st.remaining - s.sel_excl;
-      ns.prefix = st.prefix | (s.sel_bin << (8 * d));
-      ns.pmask = st.pmask | (255u << (8 * d));
-      if (d > 0) {
-        ns.stage = stage + 1;
-      } else {
-        ns.tie_key = ns.prefix;
-        if (by_mass) {
-          // Tied tokens weigh the same; keep as many as reach the mass.
-          const uint64_t wk = quantize(weight_of(key_logit(ns.prefix), M, inv_t));
-          ns.remaining = (ns.remaining + wk - 1) / wk;
-          ns.stage = kStageTopPTie;
-        } else {
-          ns.stage = kStageTopKTie;
-        }
-      }
-    }
-    return;
   }
+  // The top-p boundary's bin, for the least and the largest mass the top-k set
+  // can have (its last bin's tokens are not ranked yet).
+  const bool cut_k = s.need_k != 0;
+  const uint64_t least = cut_k ? s.base[1] : total, most = cut_k ? least + s.bin_mass : total;
+  const bool topp = (rp.flags & kRowTopP) && most != 0;
+  if (topp) {
+    const uint64_t t0 = floor_mul(least, rp.top_p) + 1, t1 = floor_mul(most, rp.top_p) + 1;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint64_t e = k ? me + m0 : me, i = e + (k ? m1 : m0);
+      if (e < t0 && i >= t0) {
+        s.sel[0] = 2 * tid + k;
+        s.base[0] = e;
+      }
+      if (e < t1 && i >= t1) s.sel[1] = 2 * tid + k;
+    }
+  } else if (cut_k && tid == 0) {
+    s.sel[0] = s.sel[1] = s.sel[2];
+    s.base[0] = s.base[1];
   }
-  // The other stages: wave 0, one lane per chunk (S <= 64).
-  if (tid >= 64) return;
-  const bool in = tid < S;
-  const StagePartial *pl = parts + min(tid, S - 1);
-  auto lane_v = [&](int f) -> uint64_t {
-    const uint64_t v = ld_dev(&pl->v[f]);
-    return in ? v : 0ull;
-  };
-  // The first chunk whose running total passes `target` (strictly when
-  // `strict`), and the total before it; the last chunk and the whole total
-  // when none does.
-  auto pick = [&](uint64_t v, uint64_t target, bool strict, uint32_t &chunk_out,
-                  uint64_t &before) {
-    const uint64_t incl = wave_incl_scan_u64(v);
-    const uint64_t m = ballot(in && (strict ? incl > target : incl >= target));
-    if (m) {
-      const int c = (int)__builtin_ctzll(m);
-      chunk_out = (uint32_t)c;
-      before = readlane_u64(incl - v, c);
-    } else {
-      chunk_out = S - 1;
-      before = readlane_u64(incl, 63);
-    }
-  };
-  RowState &ns = a.states[row];
-  const bool lead = tid == 0;
-  switch (stage) {
-    case kStageCount1: {
-      if constexpr (CLS == kClsCount) {
-      const uint64_t n1 = wave_sum_u64(lane_v(0));
-      if (lead) {
-        ns.n1 = n1;
-        if (rp.top_k < n1) {
-          ns.stage = kStageTopK3;
-          ns.remaining = rp.top_k;
-        } else {
-          ns.stage = (rp.flags & kRowTopP) ? kStageMass2 : kStageMass3;
-        }
-      }
-      }
-      break;
-    }
-    case kStageTopKTie:
-    case kStageTopPTie: {
-      if constexpr (CLS == kClsTie) {
-      uint32_t c;
-      uint64_t cum;
-      pick(lane_v(0), st.remaining, false, c, cum);
-      if (lead) {
-        ns.chunk = c;
-        ns.within = st.remaining - cum - 1;
-        ns.stage = stage == kStageTopKTie ? kStageTopKLocate : kStageTopPLocate;
-      }
-      }
-      break;
-    }
-    case kStageMass2: {
-      if constexpr (CLS == kClsMass) {
-      const uint64_t mass = wave_sum_u64(lane_v(0));
-      if (lead) {
-        ns.mass2 = mass;
-        if (mass == 0) {
-          ns.stage = kStageMass3;
-        } else {
-          ns.nucleus = floor_mul(mass, rp.top_p);
-          ns.remaining = ns.nucleus + 1;
-          ns.prefix = 0;
-          ns.pmask = 0;
-          ns.stage = kStageTopP3;
-        }
-      }
-      }
-      break;
-    }
-    case kStageMass3: {
-      if constexpr (CLS == kClsMass) {
-      const uint64_t v0 = lane_v(0), v1 = lane_v(1), v2 = lane_v(2);
-      const uint64_t mass = wave_sum_u64(v0);
-      // The chunk holding the draft token reports its weight.
-      const uint64_t fm = ballot(v1 != 0);
-      const uint32_t fw = fm ? (uint32_t)readlane_u64(v2, 63 - __builtin_clzll(fm)) : 0u;
-      uint32_t c = 0;
-      uint64_t cum = 0, target = 0;
-      const bool walk = mass != 0 && !st.drafted;
-      if (walk) {
-        // Without a draft the chunk masses already place the draw.
-        target = floor_mul(mass, row_uniform(a, row));
-        if (target >= mass) target = mass - 1;
-        pick(v0, target, true, c, cum);
-      }
-      if (lead) {
-        if (fm) ns.draft_w = __uint_as_float(fw);
-        ns.mass3 = mass;
-        if (mass == 0) {
-          write_result(a, row, kNoToken, 0.0f, 0);
-          ns.stage = a.out_kept_ids ? kStageKeptCount : kStageDone;
-        } else if (st.drafted) {
-          ns.stage = kStageDraw;
-        } else {
-          ns.residual = 0;
-          ns.chunk = c;
-          ns.within = target - cum;
-          ns.target = target;
-          ns.stage = kStageWalk;
-        }
-      }
-      }
-      break;
-    }
-    case kStageDraw: {
-      if constexpr (CLS == kClsDraw) {
-      const uint64_t v0 = lane_v(0), v1 = lane_v(1), v2 = lane_v(2);
-      const bool residual = st.drafted && ballot(v2 != 0) != 0;
-      const uint64_t v = residual ? v0 : v1;
-      const uint64_t total = wave_sum_u64(v);
-      uint64_t target = floor_mul(total, row_uniform(a, row));
-      if (target >= total) target = total - 1;
-      uint32_t c;
-      uint64_t cum;
-      pick(v, target, true, c, cum);
-      if (lead) {
-        ns.residual = residual ? 1u : 0u;
-        ns.chunk = c;
-        ns.within = target - cum;
-        ns.target = target;
-        ns.stage = kStageWalk;
-      }
-      }
-      break;
-    }
-    case kStageKeptCount: {
-      if constexpr (CLS == kClsMass) {
-      const uint64_t kept = wave_sum_u64(lane_v(0));
-      if (lead) {
-        if (a.out_kept_counts) a.out_kept_counts[row] = (uint32_t)kept;
-        ns.stage = kStageKeptWrite;
-      }
-      }
-      break;
-    }
-    case kStageKeptWrite:
-      if (lead) ns.stage = kStageDone;
-      break;
-    default:
-      break;
+  __syncthreads();
+  if (tid == 0) {
+    RowState st = {};
+    st.stage = kRowGather;
+    st.maximum = M;
+    st.thr_key = thr_key;
+    st.scale = scale;
+    st.b0 = s.sel[0];
+    st.b1 = s.sel[1];
+    st.bk = s.sel[2];
+    st.need_k = s.need_k;
+    st.topp = topp ? 1u : 0u;
+    st.mass_b0 = topp || cut_k ? s.base[0] : total;
+    st.mass_bk = s.base[1];
+    st.total = total;
+    a.states[row] = st;
   }
 }
 #endif
 
-// The draw inside the chunk the row's last stage chose: one block per row.
-#if JF_IN(3)
-template <int DT>
-__global__ __launch_bounds__(kThreads) void walk_kernel(SampleLaunch a) {
-  __shared__ Lds s;
-  const uint32_t row = blockIdx.x;
-  const RowParams rp = a.params[row];
-  const RowState st = a.states[row];
-  if (st.stage != kStageWalk) return;
-  stage_candidates(a, rp, s);
-  const uint32_t hit = walk_chunk<DT>(a, rp, row, st.chunk, st.maximum, st.thr_key,
-                                      st.bkey, st.bid, st.residual != 0, st.mass3,
-                                      st.within, s);
-  if (threadIdx.x == 0) {
-    const double scale = (double)st.mass3 * 0x1p-44;
-    write_result(a, row, hit,
-                 st.drafted ? (float)((double)st.draft_w / scale) : 0.0f, 0);
-    a.states[row].stage = a.out_kept_ids ? kStageKeptCount : kStageDone;
+// Wave 0 finds the highest of s.hist's (s.hcount's) 256 bins whose suffix sum
+// reaches T (the total does): s.sel_bin, and s.sel_excl the sum above it.
+__device__ __forceinline__ void cut_crossing_bin(CutLds &s, uint64_t T, bool by_mass) {
+  if (threadIdx.x < 64) {
+    const uint32_t l = threadIdx.x;
+    uint64_t h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = by_mass ? s.hist[4 * l + k] : s.hcount[4 * l + k];
+    const uint64_t own = h[0] + h[1] + h[2] + h[3];
+    const uint64_t incl = wave_incl_scan_u64(own);
+    const uint64_t suf = readlane_u64(incl, 63) - (incl - own);
+    const uint64_t m = ballot(suf >= T);
+    const int L = m ? 63 - (int)__builtin_clzll(m) : 0;
+    if ((int)l == L) {
+      uint64_t acc = suf - own;
+      uint32_t k = 3;
+      while (k > 0 && acc + h[k] < T) acc += h[k--];
+      s.sel_bin = 4 * l + k;
+      s.sel_excl = acc;
+    }
   }
+  __syncthreads();
+}
+
+// The item at which the running count (or exact mass) of the items that `in`
+// takes, largest first, reaches `target` (which it does): a radix descent by
+// up to 8 bits a pass from the highest bit in which they differ, until the
+// bin holds at most a wave's worth, which one wave ranks. `each(f)` calls
+// f(item) for every item, each thread its own.
+template <class Each, class In>
+__device__ __forceinline__ uint64_t cut_crossing(Each each, In in, bool by_mass, uint64_t target,
+                                                 float M, float inv_t, CutLds &s) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  uint64_t any1 = 0, any0 = 0;  // bits set in some item, clear in some item
+  each([&](uint64_t c) {
+    if (in(c)) {
+      any1 |= c;
+      any0 |= ~c;
+    }
+  });
+  auto wave_or = [](uint64_t v) {
+    v |= xor_u64<1>(v);
+    v |= xor_u64<2>(v);
+    v |= xor_u64<4>(v);
+    v |= xor_u64<8>(v);
+    v |= xor_u64<16>(v);
+    v |= xor_u64<32>(v);
+    return v;
+  };
+  any1 = wave_or(any1);
+  any0 = wave_or(any0);
+  __syncthreads();
+  if (lane == 0) {
+    s.wl[w] = any1;
+    s.wl2[w] = any0;
+  }
+  __syncthreads();
+  any1 = s.wl[0] | s.wl[1] | s.wl[2] | s.wl[3];
+  any0 = s.wl2[0] | s.wl2[1] | s.wl2[2] | s.wl2[3];
+  const uint64_t differ = any1 & any0;
+  const int bits = differ ? 64 - (int)__builtin_clzll(differ) : 1;  // low bits not yet fixed
+  int width = min(bits, 8), shift = bits - width;
+  uint64_t prefix = any1 >> bits;  // the bits above agree
+  for (;;) {
+    const uint32_t mask = (1u << width) - 1u;
+    s.hist[tid] = 0;
+    s.hcount[tid] = 0;
+    __syncthreads();
+    each([&](uint64_t c) {
+      if (in(c) && (c >> (shift + width)) == prefix) {
+        const uint32_t d = (uint32_t)(c >> shift) & mask;
+        atomicAdd(&s.hcount[d], 1u);
+        if (by_mass)
+          atomicAdd((unsigned long long *)&s.hist[d],
+                    (unsigned long long)quantized_weight(key_logit(cut_key(c)), M, inv_t));
+      }
+    });
+    __syncthreads();
+    cut_crossing_bin(s, target, by_mass);
+    target -= s.sel_excl;
+    prefix = (prefix << width) | s.sel_bin;
+    const uint32_t n = s.hcount[s.sel_bin];
+    if (n <= 64u || shift == 0) break;
+    width = min(shift, 8);
+    shift -= width;
+    __syncthreads();
+  }
+  __syncthreads();
+  if (tid == 0) s.n = 0;
+  __syncthreads();
+  each([&](uint64_t c) {
+    if (in(c) && (c >> shift) == prefix) s.small[atomicAdd(&s.n, 1u) & 63u] = c;
+  });
+  __syncthreads();
+  if (w == 0) {
+    const uint32_t n = min(s.n, 64u);
+    const uint64_t c = lane < n ? s.small[lane] : 0ull;
+    uint32_t rank = 0;
+    for (uint32_t j = 0; j < n; ++j) rank += s.small[j] > c ? 1u : 0u;
+    if (lane < n) s.sorted[rank] = c;
+    wave_lds_sync();
+    const uint64_t o = lane < n ? s.sorted[lane] : 0ull;
+    const uint64_t v = lane >= n ? 0ull
+                       : by_mass ? quantized_weight(key_logit(cut_key(o)), M, inv_t)
+                                 : 1ull;
+    const uint64_t reached = ballot(lane < n && wave_incl_scan_u64(v) >= target);
+    if ((int)lane == (reached ? (int)__builtin_ctzll(reached) : (int)n - 1)) s.u64a = o;
+  }
+  __syncthreads();
+  return s.u64a;
+}
+
+// The kept set of a row from the tokens of its boundary bins (`each`): its
+// last token into s.bound, and what those tokens add to each chunk's kept
+// mass and count (s.cmass, s.ccount: the bins before them on entry).
+template <class Each>
+__device__ __forceinline__ void cut_resolve(const RowParams &rp, const RowState &st, Each each,
+                                            bool counts, CutLds &s) {
+  const float M = st.maximum, inv_t = rp.inv_t;
+  auto bin = [&](uint64_t c) { return cut_bin(key_logit(cut_key(c)), M, st.scale); };
+  uint64_t bound = 0, mass2 = st.total;
+  if (st.need_k) {
+    bound = cut_crossing(each, [&](uint64_t c) { return bin(c) == st.bk; }, false, st.need_k, M,
+                         inv_t, s);
+    if (st.topp) {
+      uint64_t m = 0;
+      each([&](uint64_t c) {
+        if (bin(c) == st.bk && c >= bound) m += quantized_weight(key_logit(cut_key(c)), M, inv_t);
+      });
+      mass2 = st.mass_bk + block_sum_u64(m, s);
+    }
+  }
+  if (st.topp && mass2) {
+    const uint64_t kth = bound;
+    bound = cut_crossing(
+        each,
+        [&](uint64_t c) {
+          const uint32_t b = bin(c);
+          return c >= kth && b >= st.b0 && b <= st.b1;
+        },
+        true, floor_mul(mass2, rp.top_p) + 1 - st.mass_b0, M, inv_t, s);
+  }
+  each([&](uint64_t c) {
+    if (c >= bound && bin(c) >= st.b0) {
+      const uint32_t k = cut_id(c) / kChunkF32;
+      atomicAdd((unsigned long long *)&s.cmass[k],
+                (unsigned long long)quantized_weight(key_logit(cut_key(c)), M, inv_t));
+      if (counts) atomicAdd(&s.ccount[k], 1u);
+    }
+  });
+  if (threadIdx.x == 0) s.bound = bound;
+  __syncthreads();
+}
+
+#if JF_IN(3)
+__shared__ CutLds g_cut_lds;
+__shared__ SampleLaunch g_cut_launch;
+
+// cut_resolve over the row's logits, for a row whose boundary bins hold more
+// tokens than the lists: each step reads the row's chunks again. Out of line
+// (with the launch record copied to LDS, since a called function cannot reach
+// the kernel's arguments), so its registers stay out of the common path.
+template <int DT>
+__device__ __noinline__ void cut_rescan(uint32_t row) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
+  const RowParams rp = g_cut_launch.params[row];
+  const RowState st = g_cut_launch.states[row];
+  auto each = [&](auto f) {
+#pragma unroll 1
+    for (uint32_t c = 0; c < g_cut_launch.chunks; ++c) {
+      float xs[TPL];
+      load_chunk<DT>(g_cut_launch, rp, row, c, g_cut_lds, xs);
+      const uint32_t lane_base = c * kChunkF32 + threadIdx.x * VEC;
+#pragma unroll
+      for (int i = 0; i < TPL; ++i) {
+        const float v = xs[i];
+        const uint32_t k = logit_key(v), b = cut_bin(v, st.maximum, st.scale);
+        if (v == v && k >= st.thr_key && ((b >= st.b0 && b <= st.b1) || b == st.bk))
+          f(cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC)));
+      }
+    }
+  };
+  cut_resolve(rp, st, each, g_cut_launch.out_kept_ids != nullptr, g_cut_lds);
+}
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void cut_draw_kernel(SampleLaunch a) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
+  CutLds &s = g_cut_lds;
+  const uint32_t S = a.chunks;
+  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const RowParams rp = a.params[row];
+  if (!cut_pass_row(rp)) return;
+  const RowState st = a.states[row];
+  if (st.stage != kRowGather) return;
+  const bool counts = a.out_kept_ids != nullptr;
+  uint64_t *area = cut_area(a, row, chunk);
+  // This chunk's bins before b0: thread t holds bins 2t and 2t + 1.
+  uint64_t before = (2 * tid < st.b0 ? area[2 * tid] : 0ull) +
+                    (2 * tid + 1 < st.b0 ? area[2 * tid + 1] : 0ull);
+  uint32_t before_n = 0;
+  if (counts) {
+    const uint64_t n = area[kCutBins + tid];
+    before_n = (2 * tid < st.b0 ? (uint32_t)n : 0u) + (2 * tid + 1 < st.b0 ? (uint32_t)(n >> 32) : 0u);
+  }
+  const bool listing = st.b0 < kCutBins;
+  float xs[TPL];
+  if (listing) load_chunk<DT>(a, rp, row, chunk, s, xs);
+  before = block_sum_u64(before, s);
+  if (counts) before_n = (uint32_t)block_sum_u64(before_n, s);
+  uint32_t listed = 0;
+  if (listing) {
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+    const uint32_t lane_base = chunk * kChunkF32 + tid * VEC;
+#pragma unroll
+    for (int i = 0; i < TPL; ++i) {
+      const float v = xs[i];
+      const uint32_t k = logit_key(v), b = cut_bin(v, st.maximum, st.scale);
+      if (v == v && k >= st.thr_key && ((b >= st.b0 && b <= st.b1) || b == st.bk)) {
+        const uint32_t slot = atomicAdd(&s.n, 1u);
+        if (slot < kCutRoom)
+          st_dev(area + slot, cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC)));
+      }
+    }
+    __syncthreads();
+    listed = s.n;
+  }
+  if (tid == 0) {
+    st_dev(area + kCutMassWord, before);
+    st_dev(area + kCutCountWord, (uint64_t)before_n | ((uint64_t)listed << 32));
+  }
+  if (!arrive_last(a.counters + row, S, s)) return;
+
+  const uint64_t *rows = cut_area(a, row, 0);
+  if (tid < 64) {
+    const uint64_t *p = rows + (uint64_t)min(lane, S - 1) * kBlockCandidates;
+    const uint64_t cm = ld_dev(p + kCutMassWord), cn = ld_dev(p + kCutCountWord);
+    const bool in = lane < S;
+    const uint32_t n = in ? (uint32_t)(cn >> 32) : 0u;
+    const uint32_t incl = wave_incl_scan_u32(n);
+    const uint64_t over = ballot(n > kCutRoom);
+    s.cmass[lane] = in ? cm : 0ull;
+    s.ccount[lane] = in ? (uint32_t)cn : 0u;
+    s.coff[lane + 1] = incl;
+    if (lane == 0) {
+      s.coff[0] = 0;
+      s.bound = 0;
+    }
+    const uint32_t all = readlane_u32(incl, 63);
+    if (lane == 0) s.n = over || all > kCutItems ? 0xffffffffu : all;
+  }
+  __syncthreads();
+  const uint32_t n = s.n;
+  if (n == 0xffffffffu) {
+    const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(&g_cut_launch);
+    for (uint32_t k = tid; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
+    __syncthreads();
+    cut_rescan<DT>(row);
+  } else if (listing) {
+    // The lists, compact, into LDS: item i's chunk by a binary search.
+    for (uint32_t i = tid; i < n; i += kThreads) {
+      uint32_t c = 0;
+      for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
+        if (c + step < S && s.coff[c + step] <= i) c += step;
+      s.items[i] = ld_dev(rows + (uint64_t)c * kBlockCandidates + (i - s.coff[c]));
+    }
+    __syncthreads();
+    auto each = [&](auto f) {
+      for (uint32_t i = tid; i < n; i += kThreads) f(g_cut_lds.items[i]);
+    };
+    cut_resolve(rp, st, each, counts, s);
+  }
+  // The kept mass, the kept tokens before each chunk, and the draw's chunk.
+  const uint32_t draft = row_draft(a, rp);
+  const bool drafted = draft != kNoToken;
+  if (tid < 64) {
+    const uint64_t m = lane < S ? s.cmass[lane] : 0ull;
+    const uint64_t incl = wave_incl_scan_u64(m);
+    const uint64_t mass3 = readlane_u64(incl, 63);
+    uint64_t target = 0;
+    if (mass3 && !drafted) {
+      target = floor_mul(mass3, row_uniform(a, row));
+      if (target >= mass3) target = mass3 - 1;
+    }
+    const uint64_t hm = ballot(lane < S && incl > target);
+    const int c = hm ? (int)__builtin_ctzll(hm) : 0;
+    const uint64_t excl = readlane_u64(incl - m, c);
+    uint32_t kept = 0;
+    if (counts) {
+      const uint32_t kn = lane < S ? s.ccount[lane] : 0u;
+      const uint32_t ki = wave_incl_scan_u32(kn);
+      kept = readlane_u32(ki, 63);
+      if (lane < S) cut_area(a, row, lane)[kCutKeptWord] = ki - kn;
+    }
+    if (drafted) {
+      // For cut_emit_kernel: the chunks' kept masses, no draft weight yet.
+      if (lane < S) cut_area(a, row, lane)[kCutMassWord] = m;
+      if (lane == 0 && draft < a.vocabulary)
+        cut_area(a, row, draft / kChunkF32)[kCutDraftWord] = 0;
+    }
+    if (lane == 0) {
+      s.u64a = mass3;
+      s.sel_chunk = (uint32_t)c;
+      s.sel_excl = target - excl;
+      s.n = kept;
+      RowState &ns = a.states[row];
+      ns.bkey = cut_key(s.bound);
+      ns.bid = s.bound ? cut_id(s.bound) : 0u;
+      ns.mass3 = mass3;
+      ns.kept = kept;
+      ns.stage = counts || (drafted && mass3) ? kRowEmit : kRowDone;
+    }
+  }
+  __syncthreads();
+  const uint64_t mass3 = s.u64a;
+  if (mass3 == 0) {
+    if (tid == 0) write_result(a, row, kNoToken, 0.0f, s.n);
+    return;
+  }
+  if (drafted) return;
+  const uint64_t bound = s.bound;
+  const uint32_t kept = s.n, c = s.sel_chunk;
+  const uint64_t within = s.sel_excl;
+  __syncthreads();  // the items' area becomes the walk's
+  const uint32_t hit = walk_chunk<DT>(a, rp, row, c, st.maximum, st.thr_key, cut_key(bound),
+                                      bound ? cut_id(bound) : 0u, false, mass3, within, s);
+  if (tid == 0) write_result(a, row, hit, 0.0f, kept);
+}
+
+// Kept outputs, and drafted rows: the residual masses per chunk, and in the
+// row's last chunk to arrive the draw.
+template <int DT>
+__global__ __launch_bounds__(kThreads) void cut_emit_kernel(SampleLaunch a) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
+                LOADS = Geo<DT>::LOADS;
+  constexpr uint32_t VMASK = (1u << VEC) - 1u;
+  __shared__ DrawLds s;
+  const uint32_t S = a.chunks;
+  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  const uint32_t tid = threadIdx.x;
+  const RowParams rp = a.params[row];
+  if (!cut_pass_row(rp)) return;
+  const RowState st = a.states[row];
+  if (st.stage != kRowEmit) return;
+  const uint32_t draft = row_draft(a, rp);
+  const bool drafted = draft != kNoToken && st.mass3 != 0;
+  uint64_t *area = cut_area(a, row, chunk);
+  const uint64_t kept_before = a.out_kept_ids ? area[kCutKeptWord] : 0ull;
+  if (!drafted && kept_before >= a.kept_cap) return;
+  float qv[TPL];
+  if (drafted && a.dense_q) load_dense_q<DT>(a, rp, chunk, qv);
+  float xs[TPL];
+  load_chunk<DT>(a, rp, row, chunk, s, xs);
+  stage_candidates(a, rp, s);
+  const uint32_t lane_base = chunk * kChunkF32 + tid * VEC;
+  const float M = st.maximum, inv_t = rp.inv_t;
+  auto tok_of = [&](int i) -> uint32_t { return lane_base + (i / VEC) * SLAB + (i % VEC); };
+  uint32_t mem = 0;
+#pragma unroll
+  for (int i = 0; i < TPL; ++i) {
+    const float v = xs[i];
+    const uint32_t k = logit_key(v);
+    if (v == v && k >= st.thr_key && at_or_before(k, tok_of(i), st.bkey, st.bid)) mem |= 1u << i;
+  }
+  const double scale = (double)st.mass3 * 0x1p-44;
+  if (a.out_kept_ids) {
+    uint32_t nb[LOADS], offs[LOADS];
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) nb[j] = __popc((mem >> (j * VEC)) & VMASK);
+    order_offsets<LOADS>(nb, offs, s);
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      uint64_t idx = kept_before + offs[j];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e)
+        if ((mem >> (j * VEC + e)) & 1u) {
+          if (idx < a.kept_cap) {
+            const int i = j * VEC + e;
+            a.out_kept_ids[(uint64_t)row * a.kept_cap + idx] = tok_of(i);
+            a.out_kept_probs[(uint64_t)row * a.kept_cap + idx] =
+                st.mass3 ? (float)((double)weight_of(xs[i], M, inv_t) / scale) : 0.0f;
+          }
+          ++idx;
+        }
+    }
+  }
+  if (!drafted) return;
+  uint64_t dsum = 0, held = 0;
+#pragma unroll
+  for (int i = 0; i < TPL; ++i)
+    if ((mem >> i) & 1u) {
+      const uint64_t wq = quantized_weight(xs[i], M, inv_t);
+      dsum += residual_of(wq, st.mass3, a.dense_q ? qv[i] : draft_q(a, rp, tok_of(i), s));
+      if (tok_of(i) == draft) held = (uint64_t)f2u(weight_of(xs[i], M, inv_t)) | (1ull << 32);
+    }
+  if (held) st_dev(area + kCutDraftWord, held);
+  dsum = block_sum_u64(dsum, s);
+  if (tid == 0) {
+    st_dev(area + kCutResidualWord, dsum);
+    s.sel_excl = 0;
+  }
+  if (!arrive_last(a.counters + row, S, s)) return;
+  if (tid < 64) {
+    const uint32_t lane = tid;
+    const bool in = lane < S;
+    const uint64_t *p = cut_area(a, row, min(lane, S - 1));
+    const uint64_t d = in ? ld_dev(p + kCutResidualWord) : 0ull;
+    // No residual mass: the plain draw, over the chunks' kept masses.
+    const bool residual = ballot(d != 0) != 0;
+    const uint64_t v = residual ? d : in ? ld_dev(p + kCutMassWord) : 0ull;
+    const uint64_t incl = wave_incl_scan_u64(v), total = readlane_u64(incl, 63);
+    uint64_t target = floor_mul(total, row_uniform(a, row));
+    if (target >= total) target = total - 1;
+    const uint64_t hm = ballot(in && incl > target);
+    const int c = hm ? (int)__builtin_ctzll(hm) : 0;
+    const uint64_t excl = readlane_u64(incl - v, c);
+    // The draft token's weight, from its chunk when that keeps it.
+    const uint64_t dw = draft < a.vocabulary
+                            ? ld_dev(cut_area(a, row, draft / kChunkF32) + kCutDraftWord)
+                            : 0ull;
+    if (lane == 0) {
+      s.slice = (uint32_t)c;
+      s.slice_within = target - excl;
+      s.hit = residual ? 1u : 0u;
+      s.u64a = dw;
+      a.states[row].stage = kRowDone;
+    }
+  }
+  __syncthreads();
+  const uint64_t dw = s.u64a, within = s.slice_within;
+  const uint32_t c = s.slice;
+  const bool residual = s.hit != 0;
+  __syncthreads();
+  const uint32_t hit = walk_chunk<DT>(a, rp, row, c, M, st.thr_key, st.bkey, st.bid, residual,
+                                      st.mass3, within, s);
+  if (tid == 0)
+    write_result(a, row, hit, dw >> 32 ? (float)((double)u2f((uint32_t)dw) / scale) : 0.0f,
+                 st.kept);
 }
 #endif
 
@@ -5182,38 +5454,17 @@ int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, void *s
 #endif
 
 #if JF_IN(3)
-int launch_stage(const SampleLaunch &a, uint32_t dtype, void *stream) {
+int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream) {
   const dim3 grid(a.rows * a.chunks), block(kThreads);
   const hipStream_t st = (hipStream_t)stream;
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, a); };
-  const int cls = stage_class(a.stage);
-  if (cls == kClsWalk) {
-    if (dtype == 0)
-      hipLaunchKernelGGL(walk_kernel<0>, dim3(a.rows), block, 0, st, a);
-    else
-      hipLaunchKernelGGL(walk_kernel<1>, dim3(a.rows), block, 0, st, a);
-    return (int)hipGetLastError();
-  }
-#define JF_STAGE_CASE(C)                              \
-  case C:                                             \
-    if (dtype == 0)                                   \
-      go(stage_kernel<0, C>);                         \
-    else                                              \
-      go(stage_kernel<1, C>);                         \
-    break;
-  switch (cls) {
-    JF_STAGE_CASE(kClsCount)
-    JF_STAGE_CASE(kClsDigits)
-    JF_STAGE_CASE(kClsTie)
-    JF_STAGE_CASE(kClsLocate)
-    JF_STAGE_CASE(kClsMass)
-    JF_STAGE_CASE(kClsDraw)
-    JF_STAGE_CASE(kClsKeptWrite)
-    default:
-      return (int)hipErrorInvalidValue;
-  }
-#undef JF_STAGE_CASE
-  return (int)hipGetLastError();
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, a);
+    return hipGetLastError();
+  };
+  hipError_t e = dtype == 0 ? go(cut_hist_kernel<0>) : go(cut_hist_kernel<1>);
+  if (e == hipSuccess) e = dtype == 0 ? go(cut_draw_kernel<0>) : go(cut_draw_kernel<1>);
+  if (e == hipSuccess && emit) e = dtype == 0 ? go(cut_emit_kernel<0>) : go(cut_emit_kernel<1>);
+  return (int)e;
 }
 #endif
 

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(kParamsPerLaunch * 16) void store_params_kernel(
   if (t < b.n * 16u) params[t] = ((const uint32_t *)b.p)[t];
   if (t < b.n) {
     ((uint32_t *)(base + kCountersOff))[b.first + t] = 0u;
-    ((jf::RowState *)(base + kStatesOff))[b.first + t].stage = jf::kStageDone;
+    ((jf::RowState *)(base + kStatesOff))[b.first + t].stage = jf::kRowDone;
   }
 }
 

@@ -659,9 +659,8 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     return fail(JF_ERR_INVALID_ARGUMENT,
                 "kept outputs need ids, probabilities, counts and a capacity");
   const uint32_t W = (V + 31) / 32;
-  bool any_constrained = false, any_sampled = false, staged = false, any_drafted = false;
+  bool any_constrained = false, any_sampled = false, any_drafted = false;
   const bool row_indexed = a->draft_token_index || a->draft_cand_index;
-  bool need_count1 = false, need_topk = false, need_topp = false;
   for (uint32_t r = 0; r < rows; ++r) {
     const jf_policy &p = a->policies[r];
     rc = jf_policy_validate(&p);
@@ -678,14 +677,17 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
       if (p.min_p > 0.0f) {
         rp.flags |= jf::kRowMinP;
         rp.minp_offset = p.temperature * std::log(p.min_p);
+      } else if (jf::wide_row(rp.flags, rp.top_k)) {
+        // Weights below e^-30.5 of the maximum's are zero in 44 bits. With
+        // top-p alone, all tokens below (1 - top_p) / (2 V) of it together
+        // hold less than half of the 1 - top_p that closes the nucleus, so
+        // its last token lies above that.
+        double reach = 31.0;
+        if (!(rp.flags & jf::kRowTopK))
+          reach = std::min(reach, 1.001 * std::log(2.0 * V / (1.0 - (double)p.top_p)));
+        rp.minp_offset = -(float)(p.temperature * reach);
       }
       any_sampled = true;
-      if (rp.top_k > (uint32_t)jf::kBlockCandidates) {
-        staged = true;
-        need_count1 |= (rp.flags & (jf::kRowMinP | jf::kRowTopK)) != 0;
-        need_topk |= (rp.flags & jf::kRowTopK) != 0;
-        need_topp |= (rp.flags & jf::kRowTopP) != 0;
-      }
     }
     if (p.flags & JF_POLICY_CONSTRAINED) {
       rp.flags |= jf::kRowConstrained;
@@ -850,7 +852,9 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   // uncut_drafted: drafted uncut rows whose residual pass stays in
   // uncut_kernel (not kRowLean).
   bool any_uncut = false, any_cut = false, any_greedy = false, uncut_drafted = false;
-  staged = need_count1 = need_topk = need_topp = false;
+  // any_listed: cut rows of the merge; passes: rows that take the cut passes,
+  // or may (min-p rows whose candidates may outgrow the lists).
+  bool any_listed = false, passes = false;
   for (uint32_t r = 0; r < rows; ++r) {
     const jf::RowParams &rp = params[r];
     if (!(rp.flags & jf::kRowSampled)) {
@@ -860,12 +864,9 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
       if (rp.draft_index != JF_NO_TOKEN && !(rp.flags & jf::kRowLean)) uncut_drafted = true;
     } else {
       any_cut = true;
-      if (rp.top_k > (uint32_t)jf::kBlockCandidates) {
-        staged = true;
-        need_count1 |= (rp.flags & (jf::kRowMinP | jf::kRowTopK)) != 0;
-        need_topk |= (rp.flags & jf::kRowTopK) != 0;
-        need_topp |= (rp.flags & jf::kRowTopP) != 0;
-      }
+      const bool wide = jf::wide_row(rp.flags, rp.top_k);
+      any_listed |= !wide;
+      passes |= wide || rp.top_k > (uint32_t)jf::kBlockCandidates;
     }
   }
   // A fast launch of rows that all keep every admitted token, with no draft,
@@ -874,10 +875,10 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   bool fuse_uncut = fast && any_uncut && !any_cut && !any_greedy && !any_drafted && !kept;
   for (uint32_t r = 0; fuse_uncut && r < rows; ++r)
     fuse_uncut = !(params[r].flags & jf::kRowPenalized) && !params[r].extra_count;
-  // The merge finishes the cut rows, and the greedy rows unless the launch
-  // is all greedy and fast (fused) or has uncut rows and no cut ones (then
-  // uncut_kernel takes them).
-  const bool need_merge = !fused && (any_cut || (any_greedy && !any_uncut));
+  // The merge finishes the cut rows with candidate lists, and the greedy rows
+  // unless the launch is all greedy and fast (fused) or has uncut rows and no
+  // listed ones (then uncut_kernel takes them).
+  const bool need_merge = !fused && (any_listed || (any_greedy && !any_uncut));
   L.finish_greedy = any_greedy && !need_merge && !fused ? 1u : 0u;
   if (!fast) {
     e = jf::launch_select(L, a->dtype, stream, a->select_start_event,
@@ -952,11 +953,12 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   // by their top-k, or have a min-p floor (which usually leaves few: rows
   // whose floor leaves more than 64 take its general path), and read sparse
   // draft probabilities (or none).
-  bool small = !staged && !a->draft_q && a->uniform_offset <= 0xffffffffull &&
+  bool small = !a->draft_q && a->uniform_offset <= 0xffffffffull &&
                a->uniform_stride <= 0xffffffffull;
   bool wide = false;
   for (uint32_t r = 0; small && r < rows; ++r) {
     const jf::RowParams &rp = params[r];
+    if (jf::wide_row(rp.flags, rp.top_k)) continue;
     if ((rp.flags & jf::kRowSampled) && (rp.flags & kCuts) &&
         !((rp.flags & jf::kRowTopK) && rp.top_k <= 64u) && !(rp.flags & jf::kRowMinP))
       small = false;
@@ -967,17 +969,9 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
               : jf::launch_merge(L, a->dtype, stream);
     if (e != hipSuccess) return hip_fail((hipError_t)e, "merge launch");
   }
-  if (staged) {
-    for (uint32_t stage = jf::kStageCount1; stage <= jf::kStageLast; ++stage) {
-      if (stage == jf::kStageCount1 && !need_count1) continue;
-      if (stage >= jf::kStageTopK3 && stage <= jf::kStageTopKLocate && !need_topk) continue;
-      if (stage >= jf::kStageMass2 && stage <= jf::kStageTopPLocate && !need_topp) continue;
-      if (stage == jf::kStageDraw && !L.drafted_rows) continue;
-      if (stage >= jf::kStageKeptCount && !kept) continue;
-      L.stage = stage;
-      e = jf::launch_stage(L, a->dtype, stream);
-      if (e != hipSuccess) return hip_fail((hipError_t)e, "stage launch");
-    }
+  if (passes) {
+    e = jf::launch_cut(L, a->dtype, kept || any_drafted, stream);
+    if (e != hipSuccess) return hip_fail((hipError_t)e, "cut pass launch");
   }
   if (any_uncut && !fuse_uncut) {
     // residual_kernel over the kRowLean rows, then uncut_kernel: one block
