@@ -90,7 +90,7 @@ static_assert(sizeof(RowState) == 128, "row states are 128 bytes");
 enum RowStage : uint32_t {
   kRowDone = 0,
   kRowWide = 1,    // the merge's min-p row with more candidates than its lists
-  kRowGather = 2,  // cut_hist_kernel found its boundary bins
+  kRowGather = 2,  // cut_list_kernel found and listed its boundary bins
   kRowEmit = 3,    // cut_draw_kernel found its kept set; outputs or a draft's draw remain
 };
 
@@ -108,8 +108,7 @@ constexpr int kPenaltyWordsLds = 2048;
 // cut passes; up to it, the candidate lists and the merge.
 constexpr uint32_t kListTopK = 1024;
 constexpr uint32_t kCutBins = 512;    // bins of a row's values below its maximum
-constexpr uint32_t kCutRoom = 1008;   // boundary tokens a chunk can list
-constexpr uint32_t kCutItems = 3072;  // boundary tokens of a row resolved in LDS
+constexpr uint32_t kCutItems = 6144;  // boundary tokens of a row resolved in LDS
 constexpr int kMaxExtra = 16;
 constexpr uint32_t kChunkF32 = 8192;
 constexpr uint32_t kChunkBF16 = 8192;
@@ -406,8 +405,8 @@ struct LeanLaunch {
   uint32_t row_of[kKernargRows];
 };
 int launch_residual(const LeanLaunch &l, uint32_t dtype, void *stream);
-// The cut passes over the rows that take them: cut_hist_kernel, cut_draw_kernel
-// and, with `emit` (kept outputs or drafted rows), cut_emit_kernel.
+// The cut passes over the rows that take them: cut_hist_kernel, cut_list_kernel,
+// cut_draw_kernel and, with `emit` (kept outputs or drafted rows), cut_emit_kernel.
 int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream);
 int launch_accept_chain(const AcceptChainLaunch &a, void *stream);
 int launch_accept_tree(const AcceptTreeLaunch &a, void *stream);

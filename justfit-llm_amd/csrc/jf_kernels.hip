@@ -3070,7 +3070,8 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
   const uint32_t K = rp.top_k;
   const uint32_t kw = (K + kWaves - 1) / kWaves;
   const bool bound = (flags & kRowTopK) && kw <= 64;
-  const bool wide = wide_row(flags, K);
+  // (A launch that finishes its rows here has no wide row.)
+  const bool wide = !FUSE && !ACCEPT && wide_row(flags, K);
   uint32_t wth = 0;
   if (wide)
     wth = wave_min_u32(any ? logit_key(mx) : 0xffffffffu);
@@ -3092,18 +3093,6 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
   const uint32_t badm = s.wu[0] | s.wu[1] | s.wu[2] | s.wu[3];
   const uint32_t tk =
       bound || wide ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
-  if (wide) {
-    // No candidates: every lane that admits a token holds one at or above the
-    // least of the lanes' maxima.
-    if (tid == 0) {
-      hdr->maximum = bmax;
-      hdr->count = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
-      hdr->admitted = badm;
-      hdr->overflow = 0;
-      hdr->floor_key = tk;
-    }
-    return;
-  }
   if (uncut) {
     // The row keeps every admitted token: the uncut kernel's chunk summary,
     // or (FUSE) the row finished here.
@@ -3120,50 +3109,57 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
     }
     return;
   }
-  uint32_t thr = tk;
-  if (flags & kRowMinP)
-    thr = max(thr, logit_key(__builtin_fminf(bmax + rp.minp_offset, bmax)));
-  const float tv = thr <= kLowestKey ? -__builtin_inff() : key_logit(thr);
-  uint64_t *stage = s.stage[w];
-  uint32_t run = 0;
-  auto emit = [&](float x, uint32_t token) {
-    const bool hit = x >= tv;
-    const uint64_t m = ballot(hit);
-    if (m) {
-      // Hits past the wave's list land on its last entry: the wave's count
-      // then exceeds the list and the chunk is flagged as overflowed, so
-      // its staged list is never copied out.
-      const uint32_t slot_i = min(__builtin_amdgcn_mbcnt_hi(
-                                      (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, run)),
-                                  (uint32_t)kWaveCandidates - 1u);
-      if (hit) stage[slot_i] = (uint64_t)f2u(x) | ((uint64_t)token << 32);
-      run += (uint32_t)__popcll(m);
+  uint32_t c;
+  if (wide) {
+    // No candidates: every lane that admits a token holds one at or above the
+    // least of the lanes' maxima (the summary's count and floor).
+    c = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
+  } else {
+    uint32_t thr = tk;
+    if (flags & kRowMinP)
+      thr = max(thr, logit_key(__builtin_fminf(bmax + rp.minp_offset, bmax)));
+    const float tv = thr <= kLowestKey ? -__builtin_inff() : key_logit(thr);
+    uint64_t *stage = s.stage[w];
+    uint32_t run = 0;
+    auto emit = [&](float x, uint32_t token) {
+      const bool hit = x >= tv;
+      const uint64_t m = ballot(hit);
+      if (m) {
+        // Hits past the wave's list land on its last entry: the wave's count
+        // then exceeds the list and the chunk is flagged as overflowed, so
+        // its staged list is never copied out.
+        const uint32_t slot_i = min(__builtin_amdgcn_mbcnt_hi(
+                                        (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, run)),
+                                    (uint32_t)kWaveCandidates - 1u);
+        if (hit) stage[slot_i] = (uint64_t)f2u(x) | ((uint64_t)token << 32);
+        run += (uint32_t)__popcll(m);
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) emit(xs[j * VEC + e], lane_base + j * SLAB + e);
+#pragma unroll
+    for (int k = 0; k < SPT; ++k) emit(side.val[k], side.tok[k]);
+    if (lane == 0) s.wcount[w] = run;
+    __syncthreads();
+    uint32_t off[kWaves + 1], over = 0;
+    off[0] = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+      const uint32_t n = s.wcount[k];
+      over |= n > kWaveCandidates;
+      off[k + 1] = off[k] + min(n, kWaveCandidates);
     }
-  };
-#pragma unroll
-  for (int j = 0; j < LOADS; ++j)
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) emit(xs[j * VEC + e], lane_base + j * SLAB + e);
-#pragma unroll
-  for (int k = 0; k < SPT; ++k) emit(side.val[k], side.tok[k]);
-  if (lane == 0) s.wcount[w] = run;
-  __syncthreads();
-  uint32_t off[kWaves + 1], over = 0;
-  off[0] = 0;
-#pragma unroll
-  for (int k = 0; k < kWaves; ++k) {
-    const uint32_t n = s.wcount[k];
-    over |= n > kWaveCandidates;
-    off[k + 1] = off[k] + min(n, kWaveCandidates);
+    uint64_t *dst = a.cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
+    if (!over)
+      for (uint32_t i = tid; i < off[kWaves]; i += kThreads) {
+        const uint32_t k = (i >= off[1]) + (i >= off[2]) + (i >= off[3]);
+        const uint64_t e = s.stage[k][i - off[k]];
+        dst[i] = (uint64_t)logit_key(u2f((uint32_t)e)) | (e & 0xffffffff00000000ull);
+      }
+    c = over ? kBlockCandidates + 1 : off[kWaves];
   }
-  uint64_t *dst = a.cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
-  if (!over)
-    for (uint32_t i = tid; i < off[kWaves]; i += kThreads) {
-      const uint32_t k = (i >= off[1]) + (i >= off[2]) + (i >= off[3]);
-      const uint64_t e = s.stage[k][i - off[k]];
-      dst[i] = (uint64_t)logit_key(u2f((uint32_t)e)) | (e & 0xffffffff00000000ull);
-    }
-  const uint32_t c = over ? kBlockCandidates + 1 : off[kWaves];
   if (tid == 0) {
     hdr->maximum = bmax;
     hdr->count = min(c, (uint32_t)kBlockCandidates);
@@ -3719,33 +3715,36 @@ __device__ __forceinline__ uint32_t walk_chunk(const SampleLaunch &a, const RowP
 // over the logits after the select's:
 //  - cut_hist_kernel: every chunk bins its members by their distance below the
 //    row maximum (kCutBins equal steps over the range that can hold the
-//    boundary, cut_range) and sums each bin's exact mass (and count, where
-//    top-k or the kept outputs need it). The row's last chunk to arrive adds
-//    the chunks' bins up and finds the bins that hold the top-k and top-p
-//    boundaries.
-//  - cut_draw_kernel: every chunk lists its tokens in those bins and sums its
-//    mass before them; the row's last chunk to arrive finds the exact boundary
-//    among the listed tokens, each chunk's kept mass, and draws: the chunk,
-//    then the walk inside it.
+//    boundary) and sums each bin's exact mass (and count, where top-k or the
+//    kept outputs need it), with the sums of each kCutGroup bins.
+//  - cut_list_kernel: every chunk finds the bins that hold the row's top-k and
+//    top-p boundaries from the chunks' group sums and then the bins of the
+//    group or two that matter (while its logits arrive), lists its tokens in
+//    those bins and sums its mass before them.
+//  - cut_draw_kernel, a block a row: the exact boundary among the listed
+//    tokens, each chunk's kept mass, and the draw: the chunk, then the walk
+//    inside it.
 //  - cut_emit_kernel, only for kept outputs and drafted rows: writes the kept
 //    tokens, sums the residual masses, and draws a drafted row.
-// The bins are equal for equal keys and fall with the key, so they only
-// bracket the boundary: every decision is made on exact counts and masses,
-// and a row whose boundary bins hold more tokens than the lists (ties, a
-// range far off) is resolved by the same steps over its logits instead
-// (cut_rescan).
+// A bin falls with the key and is the same for equal keys, so the bins only
+// bracket the boundary: every decision is made on exact counts and masses, and
+// a row whose boundary bins hold more tokens than the lists (ties, a range far
+// off) is resolved by the same steps over its logits instead (cut_rescan).
+constexpr uint32_t kCutGroup = 16, kCutGroups = kCutBins / kCutGroup;
+static_assert(kCutGroups == 32 && kCutBins == 2 * kThreads);
+
 struct __align__(16) CutHistLds {
   PrepLds prep;
   uint64_t mass[kCutBins];
   uint32_t count[kCutBins];
-  uint64_t wl[kWaves];
-  uint32_t last;
-  uint32_t sel[3];  // b0, b1, bk
-  uint32_t need_k;
-  uint64_t base[2];  // mass before b0, before bk
-  uint64_t bin_mass;
 };
-
+struct __align__(16) CutListLds {
+  PrepLds prep;
+  uint64_t part[kThreads];
+  uint32_t part_n[kThreads];
+  uint64_t wl[kWaves];
+  uint32_t n;
+};
 struct __align__(16) CutLds {
   union {
     PrepLds prep;
@@ -3763,7 +3762,6 @@ struct __align__(16) CutLds {
   uint64_t wl2[kWaves];
   uint32_t cids[16];
   float cprobs[16];
-  uint32_t last;
   uint32_t hit;
   uint32_t n;
   uint32_t sel_bin;
@@ -3774,18 +3772,30 @@ struct __align__(16) CutLds {
 };
 
 // A (row, chunk)'s part of the candidate area during these passes, in 64-bit
-// words: the bins' masses [0, kCutBins) and counts (two a word) from
-// kCutBins, overwritten by the listed tokens [0, kCutRoom) once this chunk's
-// bins are summed; the last words hold the chunk's sums.
+// words: the bins' masses, the groups' masses and, where counts are kept, the
+// bins' counts (two a word) and the groups' (two a word); then the listed
+// tokens; the last words hold the chunk's sums.
+constexpr uint32_t kCutGroupWord = kCutBins;
+constexpr uint32_t kCutBinCountWord = kCutGroupWord + kCutGroups;
+constexpr uint32_t kCutGroupCountWord = kCutBinCountWord + kCutBins / 2;
 constexpr uint32_t kCutMassWord = kBlockCandidates - 8;   // mass before b0
-constexpr uint32_t kCutCountWord = kBlockCandidates - 7;  // tokens before b0 | listed << 32
-constexpr uint32_t kCutKeptWord = kBlockCandidates - 6;   // kept tokens of the chunks before
-constexpr uint32_t kCutResidualWord = kBlockCandidates - 5;
-constexpr uint32_t kCutDraftWord = kBlockCandidates - 4;  // draft token's weight bits | 1 << 32
-static_assert(kCutBins + kCutBins / 2 <= kCutRoom && kCutRoom <= kCutMassWord);
+constexpr uint32_t kCutCountWord = kCutMassWord + 1;      // tokens before b0 | listed << 32
+constexpr uint32_t kCutKeptWord = kCutMassWord + 2;       // kept tokens of the chunks before
+constexpr uint32_t kCutResidualWord = kCutMassWord + 3;
+constexpr uint32_t kCutDraftWord = kCutMassWord + 4;  // draft token's weight bits | 1 << 32
+__device__ __forceinline__ uint32_t cut_list_word(bool counts) {
+  return counts ? kCutGroupCountWord + kCutGroups / 2 : kCutBinCountWord;
+}
+__device__ __forceinline__ uint32_t cut_list_room(bool counts) {
+  return kCutMassWord - cut_list_word(counts);
+}
 
 __device__ __forceinline__ uint64_t *cut_area(const SampleLaunch &a, uint32_t row, uint32_t chunk) {
   return a.cands + ((uint64_t)row * a.chunks + chunk) * kBlockCandidates;
+}
+// Whether the row's bins are counted.
+__device__ __forceinline__ bool cut_counts(const SampleLaunch &a, const RowParams &rp) {
+  return (rp.flags & kRowTopK) || a.out_kept_ids;
 }
 // The bin of a member: its distance below the maximum in steps of 1 / scale,
 // the last bin open-ended. Falls monotonically with the key (each operation
@@ -3800,11 +3810,39 @@ __device__ __forceinline__ uint64_t cut_item(uint32_t key, uint32_t id) {
 __device__ __forceinline__ uint32_t cut_key(uint64_t item) { return (uint32_t)(item >> 19); }
 __device__ __forceinline__ uint32_t cut_id(uint64_t item) { return 0x7ffffu - ((uint32_t)item & 0x7ffffu); }
 
+// What every block of a row derives from its chunk summaries, one a lane (S <=
+// 64; each wave for itself).
+struct CutRow {
+  float maximum;
+  float scale;
+  uint32_t thr_key;
+  bool none;  // nothing admitted, or a maximum of +inf: the sentinel
+};
+__device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader &h, uint32_t S) {
+  CutRow r;
+  const uint32_t lane = lane_id();
+  r.maximum = wave_max_f32(h.maximum);
+  r.none = !wave_max_u32(h.admitted) || r.maximum == __builtin_inff();
+  const bool minp = (rp.flags & kRowMinP) != 0;
+  r.thr_key = minp ? logit_key(__builtin_fminf(r.maximum + rp.minp_offset, r.maximum)) : 0u;
+  // The bins' range below the maximum.
+  float range = -rp.minp_offset;
+  if (!minp && (rp.flags & kRowTopK)) {
+    // Each chunk's floor_key: a key that `count` of its tokens reach.
+    const bool in = lane < S && h.count;
+    const uint32_t floor_key = wave_min_u32(in ? h.floor_key : 0xffffffffu);
+    const uint32_t reach = wave_sum_u32(in ? h.count : 0u);
+    const float d = r.maximum - key_logit(floor_key);
+    if (rp.top_k <= reach && d < 1.0e30f) range = d;
+  }
+  r.scale = __builtin_fminf((float)(kCutBins - 1) / range, 3.0e38f);
+  return r;
+}
 
-// Bound: HBM or the Infinity Cache, then the weights (about 30 VALU
-// instructions a token). LDS atomics only for the tokens inside the bins'
-// range: for top-p alone the range leaves out every token that together
-// cannot hold the boundary (cut_range), which in a language model's row is
+// Bound by the weights' arithmetic (about 30 VALU instructions a token) and
+// the Infinity Cache's reads. LDS atomics only for the tokens inside the bins'
+// range: for top-p alone the range leaves out every token that all together
+// cannot hold the boundary (minp_offset), which in a language model's row is
 // most of them; they add to the mass from registers.
 #if JF_IN(3)
 template <int DT>
@@ -3817,48 +3855,30 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(SampleLaunch a) {
   const RowParams rp = a.params[row];
   if (!cut_pass_row(rp)) return;
   if (!wide_row(rp.flags, rp.top_k) && a.states[row].stage != kRowWide) return;
-  // The row's chunk summaries, one a lane in every wave (S <= 64).
-  const BlockHeader *hb = a.headers + (uint64_t)row * S;
-  const BlockHeader h = hb[min(lane, S - 1)];
+  const BlockHeader h = a.headers[(uint64_t)row * S + min(lane, S - 1)];
   float xs[TPL];
   load_chunk<DT>(a, rp, row, chunk, s, xs);
-  for (uint32_t b = tid; b < kCutBins; b += kThreads) {
-    s.mass[b] = 0;
-    s.count[b] = 0;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    s.mass[tid + k * kThreads] = 0;
+    s.count[tid + k * kThreads] = 0;
   }
-  const float M = wave_max_f32(h.maximum);
-  const uint32_t admitted = wave_max_u32(h.admitted);
-  if (!admitted || M == __builtin_inff()) {
-    if (chunk == 0 && tid == 0) {
-      write_result(a, row, kNoToken, 0.0f, 0);
-      a.states[row].stage = kRowDone;
-    }
+  const CutRow r = cut_row(rp, h, S);
+  if (r.none) {
+    if (chunk == 0 && tid == 0) write_result(a, row, kNoToken, 0.0f, 0);
     return;
   }
-  const float inv_t = rp.inv_t;
-  const bool minp = (rp.flags & kRowMinP) != 0, topk = (rp.flags & kRowTopK) != 0;
-  const uint32_t thr_key = minp ? logit_key(__builtin_fminf(M + rp.minp_offset, M)) : 0u;
-  // The bins' range below the maximum.
-  float range = -rp.minp_offset;
-  if (topk && !minp) {
-    // Each chunk's floor_key: a key that `count` of its tokens reach.
-    const bool in = lane < S && h.count;
-    const uint32_t floor_key = wave_min_u32(in ? h.floor_key : 0xffffffffu);
-    const uint32_t reach = wave_sum_u32(in ? h.count : 0u);
-    const float r = M - key_logit(floor_key);
-    if (rp.top_k <= reach && r < 1.0e30f) range = r;
-  }
-  const float scale = __builtin_fminf((float)(kCutBins - 1) / range, 3.0e38f);
-  const bool counts = topk || a.out_kept_ids;
+  const float M = r.maximum, inv_t = rp.inv_t;
+  const bool counts = cut_counts(a, rp), minp = r.thr_key != 0;
   __syncthreads();
   uint64_t tail = 0;
   uint32_t tail_n = 0;
 #pragma unroll
   for (int i = 0; i < TPL; ++i) {
     const float v = xs[i];
-    const bool member = v == v && (!minp || logit_key(v) >= thr_key);
+    const bool member = v == v && (!minp || logit_key(v) >= r.thr_key);
     const uint64_t wq = member ? quantized_weight(v, M, inv_t) : 0ull;
-    const uint32_t b = cut_bin(v, M, scale);
+    const uint32_t b = cut_bin(v, M, r.scale);
     if (member && b < kCutBins - 1) {
       atomicAdd((unsigned long long *)&s.mass[b], (unsigned long long)wq);
       if (counts) atomicAdd(&s.count[b], 1u);
@@ -3874,103 +3894,194 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(SampleLaunch a) {
     atomicAdd(&s.count[kCutBins - 1], tail_n);
   }
   __syncthreads();
+  // Thread t: bins 2t and 2t + 1; the eight threads of a group of 16 add up.
   uint64_t *area = cut_area(a, row, chunk);
-  st_dev(area + 2 * tid, s.mass[2 * tid]);
-  st_dev(area + 2 * tid + 1, s.mass[2 * tid + 1]);
-  if (counts)
-    st_dev(area + kCutBins + tid,
-           (uint64_t)s.count[2 * tid] | ((uint64_t)s.count[2 * tid + 1] << 32));
-  if (!arrive_last(a.counters + row, S, s)) return;
+  const ulonglong2 m = *(const ulonglong2 *)&s.mass[2 * tid];
+  *(ulonglong2 *)(area + 2 * tid) = m;
+  uint64_t g = m.x + m.y;
+  g += xor_u64<1>(g);
+  g += xor_u64<2>(g);
+  g += xor_u64<4>(g);
+  if (tid % 8 == 0) area[kCutGroupWord + tid / 8] = g;
+  if (counts) {
+    const uint2 n = *(const uint2 *)&s.count[2 * tid];
+    ((uint2 *)(area + kCutBinCountWord))[tid] = n;
+    uint32_t gn = n.x + n.y;
+    gn += xor_u32<1>(gn);
+    gn += xor_u32<2>(gn);
+    gn += xor_u32<4>(gn);
+    if (tid % 8 == 0) ((uint32_t *)(area + kCutGroupCountWord))[tid / 8] = gn;
+  }
+}
 
-  // The row's bins: thread t sums bins 2t and 2t + 1 over the chunks.
-  uint64_t m0 = 0, m1 = 0;
-  uint32_t n0 = 0, n1 = 0;
-  const uint64_t *rows = cut_area(a, row, 0);
-  constexpr int B = 16;
-  for (uint32_t c0 = 0; c0 < S; c0 += B) {
-    uint64_t t0[B], t1[B];
+// The sums over the row's chunks of `n` (16 or 32) words (counts) from word
+// `word` of each chunk's area on: lane l < n of every wave gets sum l. Every
+// thread of the block calls it.
+template <int N>
+__device__ __forceinline__ void cut_sums(const SampleLaunch &a, uint32_t row, uint32_t word,
+                                         uint32_t count_word, uint32_t at, bool counts,
+                                         CutListLds &s, uint64_t &sum, uint32_t &sum_n) {
+  constexpr uint32_t SUB = kThreads / N;
+  const uint32_t tid = threadIdx.x, l = tid % N, sub = tid / N, S = a.chunks;
+  const uint64_t *p = cut_area(a, row, 0) + word + at + l;
+  const uint32_t *q = (const uint32_t *)(cut_area(a, row, 0) + count_word) + at + l;
+  uint64_t m = 0;
+  uint32_t n = 0;
+  constexpr uint32_t B = 4;
+  for (uint32_t c0 = sub; c0 < S; c0 += SUB * B) {
+    uint64_t t[B];
+    uint32_t u[B];
 #pragma unroll
-    for (int k = 0; k < B; ++k) {
-      const uint64_t *p = rows + (uint64_t)min(c0 + k, S - 1) * kBlockCandidates;
-      t0[k] = ld_dev(p + 2 * tid);
-      t1[k] = ld_dev(p + 2 * tid + 1);
+    for (uint32_t k = 0; k < B; ++k) {
+      const uint32_t c = min(c0 + k * SUB, S - 1);
+      t[k] = p[(uint64_t)c * kBlockCandidates];
+      u[k] = counts ? q[(uint64_t)c * (2 * kBlockCandidates)] : 0u;
     }
 #pragma unroll
-    for (int k = 0; k < B; ++k) {
-      m0 += c0 + k < S ? t0[k] : 0ull;
-      m1 += c0 + k < S ? t1[k] : 0ull;
+    for (uint32_t k = 0; k < B; ++k) {
+      m += c0 + k * SUB < S ? t[k] : 0ull;
+      n += c0 + k * SUB < S ? u[k] : 0u;
     }
   }
+  __syncthreads();
+  s.part[tid] = m;
+  s.part_n[tid] = n;
+  __syncthreads();
+  const uint32_t lane = tid & 63;
+  m = 0;
+  n = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < SUB; ++k) {
+    m += s.part[k * N + (lane % N)];
+    n += s.part_n[k * N + (lane % N)];
+  }
+  sum = lane < (uint32_t)N ? m : 0ull;
+  sum_n = lane < (uint32_t)N ? n : 0u;
+}
+
+// Bound by the reads of the logits from L2 and the Infinity Cache; the two
+// round trips for the group and bin sums overlap them.
+template <int DT>
+__global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
+  __shared__ CutListLds s;
+  const uint32_t S = a.chunks;
+  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const RowParams rp = a.params[row];
+  if (!cut_pass_row(rp)) return;
+  if (!wide_row(rp.flags, rp.top_k)) {
+    // (The row's first block marks it kRowGather while others still start.)
+    const uint32_t stage = a.states[row].stage;
+    if (stage != kRowWide && stage != kRowGather) return;
+  }
+  const bool counts = cut_counts(a, rp);
+  uint64_t *area = cut_area(a, row, chunk);
+  const BlockHeader h = a.headers[(uint64_t)row * S + min(lane, S - 1)];
+  const ulonglong2 own = *(const ulonglong2 *)(area + 2 * tid);
+  uint2 own_n = make_uint2(0u, 0u);
+  if (counts) own_n = ((const uint2 *)(area + kCutBinCountWord))[tid];
+  float xs[TPL];
+  load_chunk<DT>(a, rp, row, chunk, s, xs);
+  const CutRow r = cut_row(rp, h, S);
+  if (r.none) {
+    if (chunk == 0 && tid == 0) a.states[row].stage = kRowDone;
+    return;
+  }
+  // The row's groups, one a lane, then the bins of those that hold a boundary.
+  uint64_t gm;
+  uint32_t gn;
+  cut_sums<kCutGroups>(a, row, kCutGroupWord, kCutGroupCountWord, 0, counts, s, gm, gn);
+  const uint64_t gi = wave_incl_scan_u64(gm), total = readlane_u64(gi, 63);
+  uint32_t b0 = kCutBins, b1 = kCutBins, bk = kCutBins, need_k = 0;
+  uint64_t mass_b0 = total, mass_bk = 0, bin_mass = 0;
+  if (rp.flags & kRowTopK) {
+    const uint32_t ni = wave_incl_scan_u32(gn), K = rp.top_k;
+    const uint64_t at = ballot(ni >= K);
+    if (K < readlane_u32(ni, 63)) {
+      const int g = (int)__builtin_ctzll(at);
+      uint64_t fm;
+      uint32_t fn;
+      cut_sums<kCutGroup>(a, row, 0, kCutBinCountWord, g * kCutGroup, true, s, fm, fn);
+      const uint64_t fi = wave_incl_scan_u64(fm);
+      const uint32_t fni = wave_incl_scan_u32(fn);
+      const uint32_t before = readlane_u32(ni - gn, g);
+      const int b = (int)__builtin_ctzll(ballot(before + fni >= K));
+      bk = g * kCutGroup + b;
+      need_k = K - before - readlane_u32(fni - fn, b);
+      mass_bk = readlane_u64(gi - gm, g) + readlane_u64(fi - fm, b);
+      bin_mass = readlane_u64(fm, b);
+      b0 = b1 = bk;
+      mass_b0 = mass_bk;
+    }
+  }
+  // The top-p boundary's bin, for the least and the largest mass the top-k
+  // set can have (its last bin's tokens are not ranked yet).
+  const uint64_t least = need_k ? mass_bk : total, most = need_k ? mass_bk + bin_mass : total;
+  const bool topp = (rp.flags & kRowTopP) && most != 0;
+  if (topp) {
+    auto bin_at = [&](uint64_t t, uint64_t &before) -> uint32_t {
+      const int g = (int)__builtin_ctzll(ballot(gi >= t));
+      uint64_t fm;
+      uint32_t fn;
+      cut_sums<kCutGroup>(a, row, 0, kCutBinCountWord, g * kCutGroup, false, s, fm, fn);
+      const uint64_t fi = wave_incl_scan_u64(fm), base = readlane_u64(gi - gm, g);
+      const int b = (int)__builtin_ctzll(ballot(base + fi >= t));
+      before = base + readlane_u64(fi - fm, b);
+      return g * kCutGroup + b;
+    };
+    b0 = b1 = bin_at(floor_mul(least, rp.top_p) + 1, mass_b0);
+    uint64_t unused;
+    if (need_k) b1 = bin_at(floor_mul(most, rp.top_p) + 1, unused);
+  }
+  // This chunk's mass (and tokens) before b0: thread t holds bins 2t, 2t + 1.
+  const uint64_t before =
+      block_sum_u64((2 * tid < b0 ? own.x : 0ull) + (2 * tid + 1 < b0 ? own.y : 0ull), s);
+  uint32_t before_n = 0;
   if (counts)
-    for (uint32_t c0 = 0; c0 < S; c0 += B) {
-      uint64_t t[B];
+    before_n = (uint32_t)block_sum_u64(
+        (2 * tid < b0 ? own_n.x : 0u) + (2 * tid + 1 < b0 ? own_n.y : 0u), s);
+  uint32_t listed = 0;
+  if (b0 < kCutBins) {
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+    uint64_t *list = area + cut_list_word(counts);
+    const uint32_t room = cut_list_room(counts);
+    const uint32_t lane_base = chunk * kChunkF32 + tid * VEC;
 #pragma unroll
-      for (int k = 0; k < B; ++k)
-        t[k] = ld_dev(rows + (uint64_t)min(c0 + k, S - 1) * kBlockCandidates + kCutBins + tid);
-#pragma unroll
-      for (int k = 0; k < B; ++k) {
-        n0 += c0 + k < S ? (uint32_t)t[k] : 0u;
-        n1 += c0 + k < S ? (uint32_t)(t[k] >> 32) : 0u;
-      }
-    }
-  if (tid == 0) {
-    s.sel[0] = s.sel[1] = s.sel[2] = kCutBins;
-    s.need_k = 0;
-    s.base[0] = s.base[1] = s.bin_mass = 0;
-  }
-  uint64_t total, members = 0;
-  const uint64_t me = block_excl_scan_u64(m0 + m1, s, &total);
-  if (topk) {
-    const uint32_t ce = (uint32_t)block_excl_scan_u64(n0 + n1, s, &members);
-    const uint32_t K = rp.top_k;
-    if (K < members) {
-      // The bin of the K-th member.
-      const bool lo = ce < K && ce + n0 >= K, hi = ce + n0 < K && ce + n0 + n1 >= K;
-      if (lo || hi) {
-        s.sel[2] = 2 * tid + (hi ? 1u : 0u);
-        s.need_k = K - ce - (hi ? n0 : 0u);
-        s.base[1] = me + (hi ? m0 : 0ull);
-        s.bin_mass = hi ? m1 : m0;
+    for (int i = 0; i < TPL; ++i) {
+      const float v = xs[i];
+      const uint32_t b = cut_bin(v, r.maximum, r.scale);
+      if ((b >= b0 && b <= b1) || b == bk) {
+        const uint32_t k = logit_key(v);
+        if (v == v && k >= r.thr_key) {
+          const uint32_t slot = atomicAdd(&s.n, 1u);
+          if (slot < room) list[slot] = cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC));
+        }
       }
     }
     __syncthreads();
+    listed = s.n;
   }
-  // The top-p boundary's bin, for the least and the largest mass the top-k set
-  // can have (its last bin's tokens are not ranked yet).
-  const bool cut_k = s.need_k != 0;
-  const uint64_t least = cut_k ? s.base[1] : total, most = cut_k ? least + s.bin_mass : total;
-  const bool topp = (rp.flags & kRowTopP) && most != 0;
-  if (topp) {
-    const uint64_t t0 = floor_mul(least, rp.top_p) + 1, t1 = floor_mul(most, rp.top_p) + 1;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const uint64_t e = k ? me + m0 : me, i = e + (k ? m1 : m0);
-      if (e < t0 && i >= t0) {
-        s.sel[0] = 2 * tid + k;
-        s.base[0] = e;
-      }
-      if (e < t1 && i >= t1) s.sel[1] = 2 * tid + k;
-    }
-  } else if (cut_k && tid == 0) {
-    s.sel[0] = s.sel[1] = s.sel[2];
-    s.base[0] = s.base[1];
-  }
-  __syncthreads();
   if (tid == 0) {
-    RowState st = {};
-    st.stage = kRowGather;
-    st.maximum = M;
-    st.thr_key = thr_key;
-    st.scale = scale;
-    st.b0 = s.sel[0];
-    st.b1 = s.sel[1];
-    st.bk = s.sel[2];
-    st.need_k = s.need_k;
-    st.topp = topp ? 1u : 0u;
-    st.mass_b0 = topp || cut_k ? s.base[0] : total;
-    st.mass_bk = s.base[1];
-    st.total = total;
-    a.states[row] = st;
+    area[kCutMassWord] = before;
+    area[kCutCountWord] = (uint64_t)before_n | ((uint64_t)listed << 32);
+    if (chunk == 0) {
+      RowState st = {};
+      st.stage = kRowGather;
+      st.maximum = r.maximum;
+      st.thr_key = r.thr_key;
+      st.scale = r.scale;
+      st.b0 = b0;
+      st.b1 = b1;
+      st.bk = bk;
+      st.need_k = need_k;
+      st.topp = topp ? 1u : 0u;
+      st.mass_b0 = mass_b0;
+      st.mass_bk = mass_bk;
+      st.total = total;
+      a.states[row] = st;
+    }
   }
 }
 #endif
@@ -4160,73 +4271,39 @@ __device__ __noinline__ void cut_rescan(uint32_t row) {
   cut_resolve(rp, st, each, g_cut_launch.out_kept_ids != nullptr, g_cut_lds);
 }
 
+// Latency-bound: a block a row. Its registers (the rescan's) cost nothing
+// here, where a chunk-parallel kernel would run two waves a SIMD for them.
 template <int DT>
 __global__ __launch_bounds__(kThreads) void cut_draw_kernel(SampleLaunch a) {
-  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
   CutLds &s = g_cut_lds;
-  const uint32_t S = a.chunks;
-  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  const uint32_t S = a.chunks, row = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const RowParams rp = a.params[row];
   if (!cut_pass_row(rp)) return;
   const RowState st = a.states[row];
   if (st.stage != kRowGather) return;
   const bool counts = a.out_kept_ids != nullptr;
-  uint64_t *area = cut_area(a, row, chunk);
-  // This chunk's bins before b0: thread t holds bins 2t and 2t + 1.
-  uint64_t before = (2 * tid < st.b0 ? area[2 * tid] : 0ull) +
-                    (2 * tid + 1 < st.b0 ? area[2 * tid + 1] : 0ull);
-  uint32_t before_n = 0;
-  if (counts) {
-    const uint64_t n = area[kCutBins + tid];
-    before_n = (2 * tid < st.b0 ? (uint32_t)n : 0u) + (2 * tid + 1 < st.b0 ? (uint32_t)(n >> 32) : 0u);
-  }
-  const bool listing = st.b0 < kCutBins;
-  float xs[TPL];
-  if (listing) load_chunk<DT>(a, rp, row, chunk, s, xs);
-  before = block_sum_u64(before, s);
-  if (counts) before_n = (uint32_t)block_sum_u64(before_n, s);
-  uint32_t listed = 0;
-  if (listing) {
-    if (tid == 0) s.n = 0;
-    __syncthreads();
-    const uint32_t lane_base = chunk * kChunkF32 + tid * VEC;
-#pragma unroll
-    for (int i = 0; i < TPL; ++i) {
-      const float v = xs[i];
-      const uint32_t k = logit_key(v), b = cut_bin(v, st.maximum, st.scale);
-      if (v == v && k >= st.thr_key && ((b >= st.b0 && b <= st.b1) || b == st.bk)) {
-        const uint32_t slot = atomicAdd(&s.n, 1u);
-        if (slot < kCutRoom)
-          st_dev(area + slot, cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC)));
-      }
-    }
-    __syncthreads();
-    listed = s.n;
-  }
-  if (tid == 0) {
-    st_dev(area + kCutMassWord, before);
-    st_dev(area + kCutCountWord, (uint64_t)before_n | ((uint64_t)listed << 32));
-  }
-  if (!arrive_last(a.counters + row, S, s)) return;
-
+  const uint32_t draft = row_draft(a, rp);
+  const bool drafted = draft != kNoToken;
+  const float u = row_uniform(a, row);
   const uint64_t *rows = cut_area(a, row, 0);
+  const uint32_t room = cut_list_room(cut_counts(a, rp));
   if (tid < 64) {
     const uint64_t *p = rows + (uint64_t)min(lane, S - 1) * kBlockCandidates;
-    const uint64_t cm = ld_dev(p + kCutMassWord), cn = ld_dev(p + kCutCountWord);
+    const uint64_t cm = p[kCutMassWord], cn = p[kCutCountWord];
     const bool in = lane < S;
     const uint32_t n = in ? (uint32_t)(cn >> 32) : 0u;
     const uint32_t incl = wave_incl_scan_u32(n);
-    const uint64_t over = ballot(n > kCutRoom);
+    const uint64_t over = ballot(n > room);
     s.cmass[lane] = in ? cm : 0ull;
     s.ccount[lane] = in ? (uint32_t)cn : 0u;
     s.coff[lane + 1] = incl;
+    const uint32_t all = readlane_u32(incl, 63);
     if (lane == 0) {
       s.coff[0] = 0;
       s.bound = 0;
+      s.n = over || all > kCutItems ? 0xffffffffu : all;
     }
-    const uint32_t all = readlane_u32(incl, 63);
-    if (lane == 0) s.n = over || all > kCutItems ? 0xffffffffu : all;
   }
   __syncthreads();
   const uint32_t n = s.n;
@@ -4236,13 +4313,14 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(SampleLaunch a) {
     for (uint32_t k = tid; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
     __syncthreads();
     cut_rescan<DT>(row);
-  } else if (listing) {
+  } else if (st.b0 < kCutBins) {
     // The lists, compact, into LDS: item i's chunk by a binary search.
+    const uint64_t *list = rows + cut_list_word(cut_counts(a, rp));
     for (uint32_t i = tid; i < n; i += kThreads) {
       uint32_t c = 0;
       for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
         if (c + step < S && s.coff[c + step] <= i) c += step;
-      s.items[i] = ld_dev(rows + (uint64_t)c * kBlockCandidates + (i - s.coff[c]));
+      s.items[i] = list[(uint64_t)c * kBlockCandidates + (i - s.coff[c])];
     }
     __syncthreads();
     auto each = [&](auto f) {
@@ -4251,15 +4329,13 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(SampleLaunch a) {
     cut_resolve(rp, st, each, counts, s);
   }
   // The kept mass, the kept tokens before each chunk, and the draw's chunk.
-  const uint32_t draft = row_draft(a, rp);
-  const bool drafted = draft != kNoToken;
   if (tid < 64) {
     const uint64_t m = lane < S ? s.cmass[lane] : 0ull;
     const uint64_t incl = wave_incl_scan_u64(m);
     const uint64_t mass3 = readlane_u64(incl, 63);
     uint64_t target = 0;
     if (mass3 && !drafted) {
-      target = floor_mul(mass3, row_uniform(a, row));
+      target = floor_mul(mass3, u);
       if (target >= mass3) target = mass3 - 1;
     }
     const uint64_t hm = ballot(lane < S && incl > target);
@@ -5457,13 +5533,16 @@ int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, void *s
 int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream) {
   const dim3 grid(a.rows * a.chunks), block(kThreads);
   const hipStream_t st = (hipStream_t)stream;
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, st, a);
+  auto go = [&](auto kernel, dim3 blocks) {
+    hipLaunchKernelGGL(kernel, blocks, block, 0, st, a);
     return hipGetLastError();
   };
-  hipError_t e = dtype == 0 ? go(cut_hist_kernel<0>) : go(cut_hist_kernel<1>);
-  if (e == hipSuccess) e = dtype == 0 ? go(cut_draw_kernel<0>) : go(cut_draw_kernel<1>);
-  if (e == hipSuccess && emit) e = dtype == 0 ? go(cut_emit_kernel<0>) : go(cut_emit_kernel<1>);
+  hipError_t e = dtype == 0 ? go(cut_hist_kernel<0>, grid) : go(cut_hist_kernel<1>, grid);
+  if (e == hipSuccess) e = dtype == 0 ? go(cut_list_kernel<0>, grid) : go(cut_list_kernel<1>, grid);
+  const dim3 rows(a.rows);
+  if (e == hipSuccess) e = dtype == 0 ? go(cut_draw_kernel<0>, rows) : go(cut_draw_kernel<1>, rows);
+  if (e == hipSuccess && emit)
+    e = dtype == 0 ? go(cut_emit_kernel<0>, grid) : go(cut_emit_kernel<1>, grid);
   return (int)e;
 }
 #endif
