@@ -182,7 +182,7 @@ void jf_stage_sampling_cycle(uint64_t seed, uint64_t *counter,
  * then each greedy row's argmax or each sampled row's min-p/top-k/top-p draw
  * — generalized from <= 4 lanes x 8/16 rows to `rows` independent rows with
  * explicit strides. Row r reads:
- *   logits  + r * logits_stride   (elements of dtype; 16-byte aligned rows)
+ *   logits  + r * logits_stride   (elements of dtype)
  *   masks   + r * mask_stride     (uint32 words; constrained rows only)
  *   uniforms[uniform_index ? uniform_index[r]
  *            : uniform_offset + r * uniform_stride]   (sampled rows; a

@@ -41,6 +41,8 @@ constexpr uint32_t kRank = 256;
 constexpr uint32_t kPad = kRank + 4;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// A row of draft logits starts at any float: one 16-byte load all the same.
+typedef f32x4 RowF32x4 __attribute__((aligned(4)));
 
 __device__ __forceinline__ float bf16f(uint32_t b) { return u2f(b << 16); }
 __device__ __forceinline__ float readlane_f32(float v, int l) {
@@ -142,7 +144,6 @@ struct __align__(16) DraftTopLds {
 // wave sorts the 64 wave leaders to find it. The tokens at or above the bound
 // are compacted by a prefix sum and ranked by counting. A chunk with more
 // than 256 of them (ties) takes its top 16 by 16 rounds of block maxima.
-template <bool ALIGNED>
 __global__ __launch_bounds__(kThreads) void draft_top16_kernel(DraftLaunch d) {
   __shared__ DraftTopLds s;
   const uint32_t chunk = blockIdx.x, row = blockIdx.y;
@@ -154,10 +155,10 @@ __global__ __launch_bounds__(kThreads) void draft_top16_kernel(DraftLaunch d) {
   auto token_of = [&](int i) -> uint32_t { return lane_base + (i >> 2) * 1024 + (i & 3); };
 
   float x[kDraftTokens];
-  if (ALIGNED && base + kDraftChunk <= V) {
+  if (base + kDraftChunk <= V) {
 #pragma unroll
     for (int j = 0; j < kDraftLoads; ++j) {
-      const f32x4 v = *(const f32x4 *)(rowp + lane_base + j * 1024);
+      const f32x4 v = *(const RowF32x4 *)(rowp + lane_base + j * 1024);
       x[j * 4 + 0] = v.x;
       x[j * 4 + 1] = v.y;
       x[j * 4 + 2] = v.z;
@@ -672,16 +673,12 @@ __global__ __launch_bounds__(kThreads) void draft_edges_kernel(DraftLaunch d) {
   }
 }
 
-int launch_draft_select(const DraftLaunch &d, bool aligned, void *stream,
+int launch_draft_select(const DraftLaunch &d, void *stream,
                         void *start_event, void *stop_event) {
   const hipStream_t st = (hipStream_t)stream;
   const dim3 g1(d.chunks, d.lanes * kDraftPositions), block(kThreads);
-  if (aligned)
-    hipExtLaunchKernelGGL(draft_top16_kernel<true>, g1, block, 0, st, (hipEvent_t)start_event,
-                          (hipEvent_t)stop_event, 0, d);
-  else
-    hipExtLaunchKernelGGL(draft_top16_kernel<false>, g1, block, 0, st, (hipEvent_t)start_event,
-                          (hipEvent_t)stop_event, 0, d);
+  hipExtLaunchKernelGGL(draft_top16_kernel, g1, block, 0, st, (hipEvent_t)start_event,
+                        (hipEvent_t)stop_event, 0, d);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(draft_edges_kernel, dim3(kDraftPositions, d.lanes), block, 0, st, d);

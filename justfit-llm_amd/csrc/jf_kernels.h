@@ -131,7 +131,6 @@ struct SampleLaunch {
   uint32_t rows;
   uint32_t stop0;
   uint32_t stop1;
-  uint32_t aligned;       // rows start on 16-byte boundaries: vector loads
   uint32_t finish_greedy; // no merge runs: uncut_kernel finishes the greedy
                           // rows
   uint32_t row_indexed;   // drafts are addressed through RowParams'
@@ -411,7 +410,7 @@ int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream);
 int launch_accept_chain(const AcceptChainLaunch &a, void *stream);
 int launch_accept_tree(const AcceptTreeLaunch &a, void *stream);
 // jf_draft.hip; the events, when set, bracket the top-16 kernel.
-int launch_draft_select(const DraftLaunch &d, bool aligned, void *stream,
+int launch_draft_select(const DraftLaunch &d, void *stream,
                         void *start_event = nullptr, void *stop_event = nullptr);
 // jf_gather.hip; vec8: 8 columns per thread with 16-byte accesses.
 int launch_tree_gather(const GatherLaunch &g, bool vec8, void *stream,

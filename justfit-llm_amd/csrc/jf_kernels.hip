@@ -269,8 +269,21 @@ __device__ __forceinline__ uint32_t scalar_load_u32(const uint32_t *p) {
                : "memory");
   return v;
 }
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// A 16-byte load of logits (or a draft's q) at any element's alignment: one
+// global_load_dwordx4, which the hardware splits where it crosses a line. Rows
+// that start past a 16-byte boundary (an odd vocabulary, a view into a padded
+// buffer) read 16 bytes a lane like the others; element-sized loads of them
+// cost the select pass 17.5 us against 12.6 (64 x 151,936 fp32).
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+template <int DT>
+__device__ __forceinline__ u32x4 row_load(const void *p) {
+  if constexpr (DT == 0)
+    return *(const u32x4_at4 *)p;
+  else
+    return *(const u32x4_at2 *)p;
+}
 
 // The select kernel's first round of a chunk's penalized tokens, held by
 // the threads of their table entries: token id and penalized value (NaN when
@@ -311,12 +324,12 @@ __device__ __forceinline__ void load_chunk(const SampleLaunch &a,
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
       const uint32_t t0 = lane_base + j * SLAB;
-      if (t0 + VEC <= V && a.aligned) {
-        const f32x4 v = *(const f32x4 *)(rowp + t0);
-        xs[j * 4 + 0] = v.x;
-        xs[j * 4 + 1] = v.y;
-        xs[j * 4 + 2] = v.z;
-        xs[j * 4 + 3] = v.w;
+      if (t0 + VEC <= V) {
+        const u32x4 v = row_load<DT>(rowp + t0);
+        xs[j * 4 + 0] = u2f(v.x);
+        xs[j * 4 + 1] = u2f(v.y);
+        xs[j * 4 + 2] = u2f(v.z);
+        xs[j * 4 + 3] = u2f(v.w);
       } else {
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
@@ -329,8 +342,8 @@ __device__ __forceinline__ void load_chunk(const SampleLaunch &a,
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
       const uint32_t t0 = lane_base + j * SLAB;
-      if (t0 + VEC <= V && a.aligned) {
-        const u32x4 v = *(const u32x4 *)(rowp + t0);
+      if (t0 + VEC <= V) {
+        const u32x4 v = row_load<DT>(rowp + t0);
         xs[j * 8 + 0] = u2f(v.x << 16);
         xs[j * 8 + 1] = u2f(v.x & 0xffff0000u);
         xs[j * 8 + 2] = u2f(v.y << 16);
@@ -2106,11 +2119,11 @@ __device__ __forceinline__ void draw_in_slice(const SampleLaunch &a, uint32_t ro
   if constexpr (DT == 0) {
     const float *rowp = (const float *)a.logits + (uint64_t)row * a.stride;
     if (t0 + VEC <= V) {
-      const f32x4 v = *(const f32x4 *)(rowp + t0);
-      x[0] = v.x;
-      x[1] = v.y;
-      x[2] = v.z;
-      x[3] = v.w;
+      const u32x4 v = row_load<DT>(rowp + t0);
+      x[0] = u2f(v.x);
+      x[1] = u2f(v.y);
+      x[2] = u2f(v.z);
+      x[3] = u2f(v.w);
     } else {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) x[e] = t0 + e < V ? rowp[t0 + e] : kNotAdmitted;
@@ -2118,7 +2131,7 @@ __device__ __forceinline__ void draw_in_slice(const SampleLaunch &a, uint32_t ro
   } else {
     const uint16_t *rowp = (const uint16_t *)a.logits + (uint64_t)row * a.stride;
     if (t0 + VEC <= V) {
-      const u32x4 v = *(const u32x4 *)(rowp + t0);
+      const u32x4 v = row_load<DT>(rowp + t0);
       const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -2251,8 +2264,8 @@ __device__ __forceinline__ void finish_tree_lane(const AcceptTreeLaunch &a, uint
 
 // ---- the fast selection kernel ---------------------------------------------
 //
-// select_kernel's results for the rows the host admits (16-byte aligned rows,
-// every penalty chunk within its fixed slots, no extra verify tokens), with a
+// select_kernel's results for the rows the host admits (every penalty chunk
+// within its fixed slots), with a
 // load phase that requests everything before it waits on anything:
 //   1. the chunk's penalty slots (their address needs only the kernel
 //      arguments), then the logits with 16-byte loads, then a constrained
@@ -2358,7 +2371,7 @@ __device__ __forceinline__ void fast_load(const void *logits, uint64_t stride,
   for (int j = 0; j < LOADS; ++j) {
     const uint32_t t0 = lane_base + j * SLAB;
     const uint32_t tl = full || t0 + VEC <= vfull ? t0 : vfull - VEC;
-    v[j] = *(const u32x4 *)(rowp + tl);
+    v[j] = row_load<DT>(rowp + tl);
   }
   tail_j = 0xffu;
   if (!full) {
@@ -3595,7 +3608,7 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
 // ---- reading a chunk again -------------------------------------------------
 
 // A drafted row's dense q over this thread's tokens of a chunk, in the
-// order of the chunk's logits; 16-byte loads when the rows are aligned.
+// order of the chunk's logits.
 template <int DT>
 __device__ __forceinline__ void load_dense_q(const SampleLaunch &a, const RowParams &rp,
                                              uint32_t chunk,
@@ -3604,16 +3617,16 @@ __device__ __forceinline__ void load_dense_q(const SampleLaunch &a, const RowPar
   constexpr uint32_t CHUNK = Geo<DT>::CHUNK;
   const uint32_t lane_base = chunk * CHUNK + threadIdx.x * VEC;
   const float *q = a.dense_q + (uint64_t)rp.cand_index * a.q_stride;
-  if (a.q_aligned && chunk * CHUNK + CHUNK <= a.vocabulary) {
+  if (chunk * CHUNK + CHUNK <= a.vocabulary) {
 #pragma unroll
     for (int j = 0; j < LOADS; ++j)
 #pragma unroll
       for (int h = 0; h < VEC / 4; ++h) {
-        const float4 f = *reinterpret_cast<const float4 *>(q + lane_base + j * SLAB + 4 * h);
-        qv[j * VEC + 4 * h + 0] = f.x;
-        qv[j * VEC + 4 * h + 1] = f.y;
-        qv[j * VEC + 4 * h + 2] = f.z;
-        qv[j * VEC + 4 * h + 3] = f.w;
+        const u32x4 f = row_load<0>(q + lane_base + j * SLAB + 4 * h);
+        qv[j * VEC + 4 * h + 0] = u2f(f.x);
+        qv[j * VEC + 4 * h + 1] = u2f(f.y);
+        qv[j * VEC + 4 * h + 2] = u2f(f.z);
+        qv[j * VEC + 4 * h + 3] = u2f(f.w);
       }
   } else {
 #pragma unroll
@@ -4849,7 +4862,9 @@ __global__ __launch_bounds__(kThreads) void residual_kernel(LeanLaunch l) {
   const uint32_t V = a.vocabulary, base = chunk * CHUNK;
   const uint32_t lane_base = base + tid * VEC;
   const bool full = base + CHUNK <= V;
-  const bool vec_x = full && a.aligned, vec_q = full && a.q_aligned;
+  // (q by an unaligned 16-byte load under `full` alone: 30.1 us against 28.5
+  // at 256 rows x 151,936, the compiler then waits between the loads.)
+  const bool vec_q = full && a.q_aligned;
   const float *qrow = DENSE ? a.dense_q + (uint64_t)rp.cand_index * a.q_stride : nullptr;
   const bool stops = (rp.flags & kRowExcludeStop) &&
                      ((a.stop0 >= base && a.stop0 < base + CHUNK) ||
@@ -4878,12 +4893,12 @@ __global__ __launch_bounds__(kThreads) void residual_kernel(LeanLaunch l) {
         pv[jj * 4 + 3] = v.w;
       } else if constexpr (DT == 0) {
         const float *rowp = (const float *)a.logits + (uint64_t)row * a.stride;
-        if (vec_x) {
-          const f32x4 v = *(const f32x4 *)(rowp + t0);
-          xv[jj * 4 + 0] = v.x;
-          xv[jj * 4 + 1] = v.y;
-          xv[jj * 4 + 2] = v.z;
-          xv[jj * 4 + 3] = v.w;
+        if (full) {
+          const u32x4 v = row_load<DT>(rowp + t0);
+          xv[jj * 4 + 0] = u2f(v.x);
+          xv[jj * 4 + 1] = u2f(v.y);
+          xv[jj * 4 + 2] = u2f(v.z);
+          xv[jj * 4 + 3] = u2f(v.w);
         } else {
 #pragma unroll
           for (int e = 0; e < VEC; ++e)
@@ -4891,8 +4906,8 @@ __global__ __launch_bounds__(kThreads) void residual_kernel(LeanLaunch l) {
         }
       } else {
         const uint16_t *rowp = (const uint16_t *)a.logits + (uint64_t)row * a.stride;
-        if (vec_x) {
-          const u32x4 v = *(const u32x4 *)(rowp + t0);
+        if (full) {
+          const u32x4 v = row_load<DT>(rowp + t0);
           const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
           for (int k = 0; k < 4; ++k) {

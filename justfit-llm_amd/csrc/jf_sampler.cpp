@@ -651,8 +651,6 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     return fail(JF_ERR_INVALID_ARGUMENT, "logits row stride is below the vocabulary");
   if ((uintptr_t)a->logits % esize)
     return fail(JF_ERR_INVALID_ARGUMENT, "logits are not aligned to their element size");
-  const bool aligned =
-      (uintptr_t)a->logits % 16 == 0 && (rows == 1 || (a->logits_stride * esize) % 16 == 0);
   const bool kept = a->out_kept_ids || a->out_kept_probs || a->out_kept_counts;
   if (kept && (!a->out_kept_ids || !a->out_kept_probs || !a->out_kept_counts ||
                !a->kept_capacity))
@@ -738,14 +736,14 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   if (any_drafted && !a->draft_q && (!a->draft_cand_ids || !a->draft_cand_probs))
     return fail(JF_ERR_INVALID_ARGUMENT, "drafted rows need draft probabilities");
 
-  // The rows the fast selection kernel takes: in a launch of 16-byte-aligned
-  // rows (and a vocabulary of at least one vector), each row whose penalty
+  // The rows the fast selection kernel takes: in a launch whose vocabulary
+  // holds at least one vector, each row whose penalty
   // row fits its fixed slots and whose extra verify tokens (if any) start
   // below 2^27 (their offset travels in 27 bits of a kernel argument). When
   // only some rows qualify the launch is split: the fast kernel selects
   // those, and select_kernel the others (it skips rows marked fast_row).
   const uint64_t stride_el = rows > 1 ? a->logits_stride : V;
-  const bool launch_fast = aligned && V >= 8 && stride_el <= 0xffffffffull &&
+  const bool launch_fast = V >= 8 && stride_el <= 0xffffffffull &&
                            !(a->mask_rows && any_constrained);
   uint32_t n_fast = 0;
   for (uint32_t r = 0; r < rows; ++r) {
@@ -788,7 +786,6 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   L.rows = rows;
   L.stop0 = a->stop_token_0;
   L.stop1 = a->stop_token_1;
-  L.aligned = aligned ? 1u : 0u;
   if (a->penalties) {
     L.pen_entries = a->penalties->entries;
     L.pen_offsets = a->penalties->offsets;
@@ -1456,8 +1453,7 @@ int jf_draft_select(jf_draft_selector *d, const jf_draft_select_args *a, void *s
   L.choices = d->choices;
   L.choice_q = d->choice_q;
   L.counters = d->counters;
-  const bool aligned = (uintptr_t)a->logits % 16 == 0 && a->logits_stride % 4 == 0;
-  const int e = jf::launch_draft_select(L, aligned, stream, a->select_start_event,
+  const int e = jf::launch_draft_select(L, stream, a->select_start_event,
                                         a->select_done_event);
   if (e != hipSuccess) return hip_fail((hipError_t)e, "draft selector launch");
   return JF_OK;
