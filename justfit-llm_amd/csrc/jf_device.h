@@ -75,16 +75,17 @@ __device__ __forceinline__ uint64_t quantize(float w) {
 // result is y * 2^n exactly (y in [0.70, 1.42], n in [-124, 0], a normal
 // float), so floor(y * 2^(n + 44)) is the integer Y = y * 2^30 (exact: y
 // has 24 mantissa bits and exponent -1 or 0) shifted by n + 14, here
-// (Y << 32) >> (18 - n); a shift of 63 gives zero, below -86 or for NaN.
-// Checked equal to quantize(exp_weight(x)) for every float x in [-90, 0]
-// and NaN. weight_yk returns Y and that shift k = min(18 - n, 63).
+// (Y << 32) >> (18 - n); a shift of 63 gives zero. Below -86, where
+// exp_weight is zero, and for NaN (which the maximum takes to -87), n is at
+// most -124 and the shift is 63 by itself: no range test. Checked equal to
+// quantize(exp_weight(x)) for every float x from -infinity to 0 and quiet NaN.
+// weight_yk returns Y and that shift k = min(18 - n, 63).
 struct WeightYK {
   uint32_t Y;
   int k;
 };
-__device__ __forceinline__ WeightYK weight_yk(float value, float maximum, float inv_t) {
-  const float x_in = (value - maximum) * inv_t;
-  const float x = __builtin_fminf(__builtin_fmaxf(x_in, -87.0f), 88.0f);
+__device__ __forceinline__ WeightYK weight_yk_at(float x_in) {
+  const float x = __builtin_fmaxf(x_in, -87.0f);
   const float n = __builtin_rintf(x * 1.44269504088896341f);
   float r = __builtin_fmaf(n, -0.693359375f, x);
   r = __builtin_fmaf(n, 2.12194440e-4f, r);
@@ -96,10 +97,10 @@ __device__ __forceinline__ WeightYK weight_yk(float value, float maximum, float 
   p = __builtin_fmaf(p, r, 5.0000001201e-1f);
   const float r2 = r * r;
   const float y = __builtin_fmaf(p, r2, r) + 1.0f;
-  WeightYK w;
-  w.Y = (uint32_t)(y * 0x1p30f);
-  w.k = x_in >= -86.0f ? min(18 - (int)n, 63) : 63;
-  return w;
+  return {(uint32_t)(y * 0x1p30f), min(18 - (int)n, 63)};
+}
+__device__ __forceinline__ WeightYK weight_yk(float value, float maximum, float inv_t) {
+  return weight_yk_at((value - maximum) * inv_t);
 }
 __device__ __forceinline__ uint64_t quantized_weight(float value, float maximum,
                                                      float inv_t) {

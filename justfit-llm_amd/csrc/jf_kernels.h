@@ -405,8 +405,13 @@ struct LeanLaunch {
 };
 int launch_residual(const LeanLaunch &l, uint32_t dtype, void *stream);
 // The cut passes over the rows that take them: cut_hist_kernel, cut_list_kernel,
-// cut_draw_kernel and, with `emit` (kept outputs or drafted rows), cut_emit_kernel.
-int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream);
+// cut_draw_kernel and, for kept outputs or drafted rows, cut_emit_kernel.
+struct CutLaunch {
+  bool all;      // every row takes them by its policy (wide_row)
+  bool plain;    // no row is penalized
+  bool drafted;  // some row is drafted
+};
+int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *stream);
 int launch_accept_chain(const AcceptChainLaunch &a, void *stream);
 int launch_accept_tree(const AcceptTreeLaunch &a, void *stream);
 // jf_draft.hip; the events, when set, bracket the top-16 kernel.

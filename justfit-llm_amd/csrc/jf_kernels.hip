@@ -2321,19 +2321,21 @@ __device__ __forceinline__ uint32_t wave_kth_bound16(uint32_t v, uint32_t k) {
 // compiler places between such a load and its wait, such as register copies,
 // would read registers the load has not yet written.)
 typedef const __attribute__((address_space(4))) uint32_t *ConstWords;
-__device__ __forceinline__ RowParams load_row_policy(const RowParams *p) {
+template <class T>
+__device__ __forceinline__ T load_const(const T *p) {
   const uint64_t addr = (uint64_t)p;
   const uint64_t u =
       ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(addr >> 32)) << 32) |
       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)addr);
   const ConstWords w = (ConstWords)u;
-  uint32_t v[sizeof(RowParams) / 4];
+  uint32_t v[sizeof(T) / 4];
 #pragma unroll
-  for (int i = 0; i < (int)(sizeof(RowParams) / 4); ++i) v[i] = w[i];
-  RowParams rp;
-  __builtin_memcpy(&rp, v, sizeof(rp));
-  return rp;
+  for (int i = 0; i < (int)(sizeof(T) / 4); ++i) v[i] = w[i];
+  T t;
+  __builtin_memcpy(&t, v, sizeof(t));
+  return t;
 }
+__device__ __forceinline__ RowParams load_row_policy(const RowParams *p) { return load_const(p); }
 
 // Register i of a thread and the thread that loads chunk offset o.
 template <int DT>
@@ -3732,8 +3734,8 @@ __device__ __forceinline__ uint32_t walk_chunk(const SampleLaunch &a, const RowP
 //    kept outputs need it), with the sums of each kCutGroup bins.
 //  - cut_list_kernel: every chunk finds the bins that hold the row's top-k and
 //    top-p boundaries from the chunks' group sums and then the bins of the
-//    group or two that matter (while its logits arrive), lists its tokens in
-//    those bins and sums its mass before them.
+//    group or two that matter, lists its tokens in those bins and sums its
+//    mass before them.
 //  - cut_draw_kernel, a block a row: the exact boundary among the listed
 //    tokens, each chunk's kept mass, and the draw: the chunk, then the walk
 //    inside it.
@@ -3745,6 +3747,13 @@ __device__ __forceinline__ uint32_t walk_chunk(const SampleLaunch &a, const RowP
 // off) is resolved by the same steps over its logits instead (cut_rescan).
 constexpr uint32_t kCutGroup = 16, kCutGroups = kCutBins / kCutGroup;
 static_assert(kCutGroups == 32 && kCutBins == 2 * kThreads);
+
+// The launch facts its blocks need before their first load, as leading
+// arguments (preloaded into scalar registers): 5 pointers, the row stride, the
+// vocabulary and `bits`: the chunks per row, and these.
+constexpr uint32_t kCutAll = 0x100u;    // every row takes the passes by its policy
+constexpr uint32_t kCutPlain = 0x200u;  // no row is penalized, the vocabulary holds a vector
+constexpr uint32_t kCutKept = 0x400u;   // kept outputs are asked for
 
 struct __align__(16) CutHistLds {
   PrepLds prep;
@@ -3770,13 +3779,12 @@ struct __align__(16) CutLds {
   uint64_t cmass[kMaxChunks];
   uint32_t ccount[kMaxChunks];
   uint32_t coff[kMaxChunks + 1];
-  uint64_t wj[kWaves][8];
+  uint64_t slices[kWaves * 8];
   uint64_t wl[kWaves];
   uint64_t wl2[kWaves];
-  uint32_t cids[16];
-  float cprobs[16];
-  uint32_t hit;
+  uint32_t kept;
   uint32_t n;
+  uint32_t small_n;
   uint32_t sel_bin;
   uint32_t sel_chunk;
   uint64_t sel_excl;
@@ -3807,14 +3815,17 @@ __device__ __forceinline__ uint64_t *cut_area(const SampleLaunch &a, uint32_t ro
   return a.cands + ((uint64_t)row * a.chunks + chunk) * kBlockCandidates;
 }
 // Whether the row's bins are counted.
-__device__ __forceinline__ bool cut_counts(const SampleLaunch &a, const RowParams &rp) {
-  return (rp.flags & kRowTopK) || a.out_kept_ids;
+__device__ __forceinline__ bool cut_counts(const RowParams &rp, uint32_t bits) {
+  return (rp.flags & kRowTopK) || (bits & kCutKept);
 }
 // The bin of a member: its distance below the maximum in steps of 1 / scale,
 // the last bin open-ended. Falls monotonically with the key (each operation
 // rounds monotonically; fmin also takes the NaN of inf * 0 to the last bin).
+__device__ __forceinline__ uint32_t cut_bin_at(float below, float scale) {
+  return (uint32_t)__builtin_fminf(below * scale, (float)(kCutBins - 1));
+}
 __device__ __forceinline__ uint32_t cut_bin(float v, float maximum, float scale) {
-  return (uint32_t)__builtin_fminf((maximum - v) * scale, (float)(kCutBins - 1));
+  return cut_bin_at(maximum - v, scale);
 }
 // A token as one word that orders as (key, lower id first): ids are below 2^19.
 __device__ __forceinline__ uint64_t cut_item(uint32_t key, uint32_t id) {
@@ -3823,12 +3834,70 @@ __device__ __forceinline__ uint64_t cut_item(uint32_t key, uint32_t id) {
 __device__ __forceinline__ uint32_t cut_key(uint64_t item) { return (uint32_t)(item >> 19); }
 __device__ __forceinline__ uint32_t cut_id(uint64_t item) { return 0x7ffffu - ((uint32_t)item & 0x7ffffu); }
 
+// A chunk of a row of these passes: xs[i] as load_chunk leaves it. A row with
+// no penalty requests its logits first thing (fast_load), before its record
+// has arrived; a penalized one takes load_chunk.
+template <int DT, class L>
+__device__ __forceinline__ void cut_load(const SampleLaunch &a, const void *logits, uint64_t stride,
+                                         uint32_t V, uint32_t row, uint32_t chunk, bool plain,
+                                         const RowParams &rp, L &s, float (&xs)[Geo<DT>::TPL]) {
+  constexpr int VEC = Geo<DT>::VEC, LOADS = Geo<DT>::LOADS, SLAB = Geo<DT>::SLAB,
+                TPL = Geo<DT>::TPL;
+  constexpr uint32_t VMASK = (1u << VEC) - 1u;
+  if (!plain && ((rp.flags & kRowPenalized) || V < 8)) {
+    load_chunk<DT>(a, rp, row, chunk, s, xs);
+    return;
+  }
+  const uint32_t base = chunk * kChunkF32, lane_base = base + threadIdx.x * VEC;
+  const bool full = base + kChunkF32 <= V;
+  std::conditional_t<DT == 0, float, uint32_t> tail[VEC];
+  uint32_t tail_j;
+  fast_load<DT>(logits, stride, V, row, base, full, xs, tail, tail_j);
+  uint32_t drop = 0;
+  if (rp.flags & kRowConstrained) {
+    const uint32_t *mrow = a.masks + (uint64_t)rp.mask_row * a.mask_stride;
+    uint32_t mw[LOADS];
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const uint32_t t0 = lane_base + j * SLAB;
+      mw[j] = t0 < V ? mrow[t0 >> 5] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j)
+      drop |= (~(mw[j] >> ((lane_base + j * SLAB) & 31)) & VMASK) << (j * VEC);
+  }
+  if (rp.flags & kRowExcludeStop) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t o = (k ? a.stop1 : a.stop0) - base;
+      if (o < kChunkF32 && owner_of<DT>(o) == threadIdx.x) drop |= 1u << register_of<DT>(o);
+    }
+  }
+  if (!full) {
+    drop |= past_end_bits<DT>(V, base);
+    if (tail_j != 0xffu)
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          xs[j * VEC + e] = (uint32_t)j == tail_j ? (DT == 0 ? (float)tail[e] : bf16_to_float((uint32_t)tail[e]))
+                                                  : xs[j * VEC + e];
+  }
+  if ((rp.flags & (kRowConstrained | kRowExcludeStop)) || !full) {
+#pragma unroll
+    for (int i = 0; i < TPL; ++i) {
+      const uint32_t m = (uint32_t)((int32_t)(drop << (31 - i)) >> 31);
+      xs[i] = u2f(f2u(xs[i]) | (m & 0x7fc00000u));
+    }
+  }
+}
+
 // What every block of a row derives from its chunk summaries, one a lane (S <=
 // 64; each wave for itself).
 struct CutRow {
   float maximum;
   float scale;
-  uint32_t thr_key;
+  float floor;  // members are at or above it (-inf without min-p)
   bool none;  // nothing admitted, or a maximum of +inf: the sentinel
 };
 __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader &h, uint32_t S) {
@@ -3837,7 +3906,7 @@ __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader
   r.maximum = wave_max_f32(h.maximum);
   r.none = !wave_max_u32(h.admitted) || r.maximum == __builtin_inff();
   const bool minp = (rp.flags & kRowMinP) != 0;
-  r.thr_key = minp ? logit_key(__builtin_fminf(r.maximum + rp.minp_offset, r.maximum)) : 0u;
+  r.floor = minp ? __builtin_fminf(r.maximum + rp.minp_offset, r.maximum) : -__builtin_inff();
   // The bins' range below the maximum.
   float range = -rp.minp_offset;
   if (!minp && (rp.flags & kRowTopK)) {
@@ -3859,18 +3928,21 @@ __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader
 // most of them; they add to the mass from registers.
 #if JF_IN(3)
 template <int DT>
-__global__ __launch_bounds__(kThreads) void cut_hist_kernel(SampleLaunch a) {
+__global__ __launch_bounds__(kThreads) void cut_hist_kernel(
+    const void *logits, const RowParams *params, const BlockHeader *headers, uint64_t *cands,
+    RowState *states, uint64_t stride, uint32_t V, uint32_t bits, SampleLaunch a) {
   constexpr int TPL = Geo<DT>::TPL;
   __shared__ CutHistLds s;
-  const uint32_t S = a.chunks;
-  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  const uint32_t S = bits & 0xffu, row = blockIdx.y, chunk = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const RowParams rp = a.params[row];
-  if (!cut_pass_row(rp)) return;
-  if (!wide_row(rp.flags, rp.top_k) && a.states[row].stage != kRowWide) return;
-  const BlockHeader h = a.headers[(uint64_t)row * S + min(lane, S - 1)];
+  const BlockHeader h = headers[(uint64_t)row * S + min(lane, S - 1)];
+  const RowParams rp = load_row_policy(params + row);
+  if (!(bits & kCutAll)) {
+    if (!cut_pass_row(rp)) return;
+    if (!wide_row(rp.flags, rp.top_k) && states[row].stage != kRowWide) return;
+  }
   float xs[TPL];
-  load_chunk<DT>(a, rp, row, chunk, s, xs);
+  cut_load<DT>(a, logits, stride, V, row, chunk, (bits & kCutPlain) != 0, rp, s, xs);
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     s.mass[tid + k * kThreads] = 0;
@@ -3882,33 +3954,38 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(SampleLaunch a) {
     return;
   }
   const float M = r.maximum, inv_t = rp.inv_t;
-  const bool counts = cut_counts(a, rp), minp = r.thr_key != 0;
+  const bool counts = cut_counts(rp, bits);
   __syncthreads();
-  uint64_t tail = 0;
+  if (rp.flags & kRowMinP)  // members are the tokens at or above the floor
+#pragma unroll
+    for (int i = 0; i < TPL; ++i) xs[i] = xs[i] >= r.floor ? xs[i] : kNotAdmitted;
+  uint64_t all = 0, inside = 0;  // the mass of all members, of those below the last bin
   uint32_t tail_n = 0;
 #pragma unroll
   for (int i = 0; i < TPL; ++i) {
-    const float v = xs[i];
-    const bool member = v == v && (!minp || logit_key(v) >= r.thr_key);
-    const uint64_t wq = member ? quantized_weight(v, M, inv_t) : 0ull;
-    const uint32_t b = cut_bin(v, M, r.scale);
-    if (member && b < kCutBins - 1) {
+    const float d = xs[i] - M;
+    const WeightYK y = weight_yk_at(d * inv_t);
+    const uint64_t wq = ((uint64_t)y.Y << 32) >> y.k;
+    all += wq;
+    const uint32_t b = cut_bin_at(-d, r.scale);  // (NaN, not admitted: the last bin)
+    if (b < kCutBins - 1) {
+      inside += wq;
       atomicAdd((unsigned long long *)&s.mass[b], (unsigned long long)wq);
       if (counts) atomicAdd(&s.count[b], 1u);
-    } else {
-      tail += wq;
-      tail_n += member ? 1u : 0u;
+    } else if (counts) {
+      tail_n += d == d ? 1u : 0u;
     }
   }
-  tail = wave_sum_u64(tail);
-  tail_n = wave_sum_u32(tail_n);
-  if (lane == 0) {
+  const uint64_t tail = wave_sum_u64(all - inside);
+  if (lane == 0)
     atomicAdd((unsigned long long *)&s.mass[kCutBins - 1], (unsigned long long)tail);
-    atomicAdd(&s.count[kCutBins - 1], tail_n);
+  if (counts) {
+    tail_n = wave_sum_u32(tail_n);
+    if (lane == 0) atomicAdd(&s.count[kCutBins - 1], tail_n);
   }
   __syncthreads();
   // Thread t: bins 2t and 2t + 1; the eight threads of a group of 16 add up.
-  uint64_t *area = cut_area(a, row, chunk);
+  uint64_t *area = cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
   const ulonglong2 m = *(const ulonglong2 *)&s.mass[2 * tid];
   *(ulonglong2 *)(area + 2 * tid) = m;
   uint64_t g = m.x + m.y;
@@ -3931,13 +4008,13 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(SampleLaunch a) {
 // `word` of each chunk's area on: lane l < n of every wave gets sum l. Every
 // thread of the block calls it.
 template <int N>
-__device__ __forceinline__ void cut_sums(const SampleLaunch &a, uint32_t row, uint32_t word,
+__device__ __forceinline__ void cut_sums(const uint64_t *area, uint32_t S, uint32_t word,
                                          uint32_t count_word, uint32_t at, bool counts,
                                          CutListLds &s, uint64_t &sum, uint32_t &sum_n) {
   constexpr uint32_t SUB = kThreads / N;
-  const uint32_t tid = threadIdx.x, l = tid % N, sub = tid / N, S = a.chunks;
-  const uint64_t *p = cut_area(a, row, 0) + word + at + l;
-  const uint32_t *q = (const uint32_t *)(cut_area(a, row, 0) + count_word) + at + l;
+  const uint32_t tid = threadIdx.x, l = tid % N, sub = tid / N;
+  const uint64_t *p = area + word + at + l;
+  const uint32_t *q = (const uint32_t *)(area + count_word) + at + l;
   uint64_t m = 0;
   uint32_t n = 0;
   constexpr uint32_t B = 4;
@@ -3972,39 +4049,44 @@ __device__ __forceinline__ void cut_sums(const SampleLaunch &a, uint32_t row, ui
   sum_n = lane < (uint32_t)N ? n : 0u;
 }
 
-// Bound by the reads of the logits from L2 and the Infinity Cache; the two
-// round trips for the group and bin sums overlap them.
+// Latency-bound: the round trips for the row's summaries, the group sums and
+// the bin sums, then the logits of the chunks that hold boundary tokens, from
+// L2 or the Infinity Cache. With every chunk's logits requested first it took
+// 12.7 us against 9.1 (64 x 151,936 fp32, top-p 0.95), and 0.3 us less where
+// every chunk holds some.
 template <int DT>
-__global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
+__global__ __launch_bounds__(kThreads) void cut_list_kernel(
+    const void *logits, const RowParams *params, const BlockHeader *headers, uint64_t *cands,
+    RowState *states, uint64_t stride, uint32_t V, uint32_t bits, SampleLaunch a) {
   constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
   __shared__ CutListLds s;
-  const uint32_t S = a.chunks;
-  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  const uint32_t S = bits & 0xffu, row = blockIdx.y, chunk = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const RowParams rp = a.params[row];
-  if (!cut_pass_row(rp)) return;
-  if (!wide_row(rp.flags, rp.top_k)) {
-    // (The row's first block marks it kRowGather while others still start.)
-    const uint32_t stage = a.states[row].stage;
-    if (stage != kRowWide && stage != kRowGather) return;
-  }
-  const bool counts = cut_counts(a, rp);
-  uint64_t *area = cut_area(a, row, chunk);
-  const BlockHeader h = a.headers[(uint64_t)row * S + min(lane, S - 1)];
+  uint64_t *rows = cands + (uint64_t)row * S * kBlockCandidates;
+  uint64_t *area = rows + (uint64_t)chunk * kBlockCandidates;
+  const BlockHeader h = headers[(uint64_t)row * S + min(lane, S - 1)];
   const ulonglong2 own = *(const ulonglong2 *)(area + 2 * tid);
+  const RowParams rp = load_row_policy(params + row);
+  if (!(bits & kCutAll)) {
+    if (!cut_pass_row(rp)) return;
+    if (!wide_row(rp.flags, rp.top_k)) {
+      // (The row's first block marks it kRowGather while others still start.)
+      const uint32_t stage = states[row].stage;
+      if (stage != kRowWide && stage != kRowGather) return;
+    }
+  }
+  const bool counts = cut_counts(rp, bits);
   uint2 own_n = make_uint2(0u, 0u);
   if (counts) own_n = ((const uint2 *)(area + kCutBinCountWord))[tid];
-  float xs[TPL];
-  load_chunk<DT>(a, rp, row, chunk, s, xs);
   const CutRow r = cut_row(rp, h, S);
   if (r.none) {
-    if (chunk == 0 && tid == 0) a.states[row].stage = kRowDone;
+    if (chunk == 0 && tid == 0) states[row].stage = kRowDone;
     return;
   }
   // The row's groups, one a lane, then the bins of those that hold a boundary.
   uint64_t gm;
   uint32_t gn;
-  cut_sums<kCutGroups>(a, row, kCutGroupWord, kCutGroupCountWord, 0, counts, s, gm, gn);
+  cut_sums<kCutGroups>(rows, S, kCutGroupWord, kCutGroupCountWord, 0, counts, s, gm, gn);
   const uint64_t gi = wave_incl_scan_u64(gm), total = readlane_u64(gi, 63);
   uint32_t b0 = kCutBins, b1 = kCutBins, bk = kCutBins, need_k = 0;
   uint64_t mass_b0 = total, mass_bk = 0, bin_mass = 0;
@@ -4015,7 +4097,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
       const int g = (int)__builtin_ctzll(at);
       uint64_t fm;
       uint32_t fn;
-      cut_sums<kCutGroup>(a, row, 0, kCutBinCountWord, g * kCutGroup, true, s, fm, fn);
+      cut_sums<kCutGroup>(rows, S, 0, kCutBinCountWord, g * kCutGroup, true, s, fm, fn);
       const uint64_t fi = wave_incl_scan_u64(fm);
       const uint32_t fni = wave_incl_scan_u32(fn);
       const uint32_t before = readlane_u32(ni - gn, g);
@@ -4037,7 +4119,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
       const int g = (int)__builtin_ctzll(ballot(gi >= t));
       uint64_t fm;
       uint32_t fn;
-      cut_sums<kCutGroup>(a, row, 0, kCutBinCountWord, g * kCutGroup, false, s, fm, fn);
+      cut_sums<kCutGroup>(rows, S, 0, kCutBinCountWord, g * kCutGroup, false, s, fm, fn);
       const uint64_t fi = wave_incl_scan_u64(fm), base = readlane_u64(gi - gm, g);
       const int b = (int)__builtin_ctzll(ballot(base + fi >= t));
       before = base + readlane_u64(fi - fm, b);
@@ -4054,8 +4136,16 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
   if (counts)
     before_n = (uint32_t)block_sum_u64(
         (2 * tid < b0 ? own_n.x : 0u) + (2 * tid + 1 < b0 ? own_n.y : 0u), s);
+  // The chunk's logits only when one of its tokens lies in those bins: a row
+  // whose distribution is narrow has few tokens there, in few chunks.
+  const uint32_t span = b1 - b0;
+  auto boundary = [&](uint32_t b) { return b - b0 <= span || b == bk; };
+  const bool mine = (boundary(2 * tid) && (counts ? own_n.x != 0 : own.x != 0)) ||
+                    (boundary(2 * tid + 1) && (counts ? own_n.y != 0 : own.y != 0));
   uint32_t listed = 0;
-  if (b0 < kCutBins) {
+  if (b0 < kCutBins && __syncthreads_or(mine)) {
+    float xs[TPL];
+    cut_load<DT>(a, logits, stride, V, row, chunk, (bits & kCutPlain) != 0, rp, s, xs);
     if (tid == 0) s.n = 0;
     __syncthreads();
     uint64_t *list = area + cut_list_word(counts);
@@ -4064,12 +4154,13 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
 #pragma unroll
     for (int i = 0; i < TPL; ++i) {
       const float v = xs[i];
-      const uint32_t b = cut_bin(v, r.maximum, r.scale);
-      if ((b >= b0 && b <= b1) || b == bk) {
-        const uint32_t k = logit_key(v);
-        if (v == v && k >= r.thr_key) {
+      // (One unsigned range test: the two-sided one took the pass from 12.7
+      // to 14.1 us at 64 x 151,936.)
+      if (boundary(cut_bin(v, r.maximum, r.scale))) {
+        if (v >= r.floor) {
           const uint32_t slot = atomicAdd(&s.n, 1u);
-          if (slot < room) list[slot] = cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC));
+          if (slot < room)
+            list[slot] = cut_item(logit_key(v), lane_base + (i / VEC) * SLAB + (i % VEC));
         }
       }
     }
@@ -4083,7 +4174,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
       RowState st = {};
       st.stage = kRowGather;
       st.maximum = r.maximum;
-      st.thr_key = r.thr_key;
+      st.thr_key = rp.flags & kRowMinP ? logit_key(r.floor) : 0u;
       st.scale = r.scale;
       st.b0 = b0;
       st.b1 = b1;
@@ -4093,7 +4184,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(SampleLaunch a) {
       st.mass_b0 = mass_b0;
       st.mass_bk = mass_bk;
       st.total = total;
-      a.states[row] = st;
+      states[row] = st;
     }
   }
 }
@@ -4187,14 +4278,14 @@ __device__ __forceinline__ uint64_t cut_crossing(Each each, In in, bool by_mass,
     __syncthreads();
   }
   __syncthreads();
-  if (tid == 0) s.n = 0;
+  if (tid == 0) s.small_n = 0;
   __syncthreads();
   each([&](uint64_t c) {
-    if (in(c) && (c >> shift) == prefix) s.small[atomicAdd(&s.n, 1u) & 63u] = c;
+    if (in(c) && (c >> shift) == prefix) s.small[atomicAdd(&s.small_n, 1u) & 63u] = c;
   });
   __syncthreads();
   if (w == 0) {
-    const uint32_t n = min(s.n, 64u);
+    const uint32_t n = min(s.small_n, 64u);
     const uint64_t c = lane < n ? s.small[lane] : 0ull;
     uint32_t rank = 0;
     for (uint32_t j = 0; j < n; ++j) rank += s.small[j] > c ? 1u : 0u;
@@ -4257,170 +4348,312 @@ __device__ __forceinline__ void cut_resolve(const RowParams &rp, const RowState 
 __shared__ CutLds g_cut_lds;
 __shared__ SampleLaunch g_cut_launch;
 
+// The tokens of the row's boundary bins in half `h` of chunk `c` (loads h *
+// LOADS / 2 on), into g_cut_lds.items; returns how many.
+template <int DT>
+__device__ __noinline__ uint32_t cut_collect(uint32_t row, uint32_t c, uint32_t h) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
+  const SampleLaunch &a = g_cut_launch;
+  const RowParams rp = a.params[row];
+  const RowState &st = a.states[row];
+  const float M = st.maximum, scale = st.scale;
+  const uint32_t thr_key = st.thr_key, b0 = st.b0, b1 = st.b1, bk = st.bk;
+  float xs[TPL];
+  load_chunk<DT>(a, rp, row, c, g_cut_lds, xs);
+  __syncthreads();  // the prep area becomes the items'
+  if (threadIdx.x == 0) g_cut_lds.n = 0;
+  __syncthreads();
+  const uint32_t lane_base = c * kChunkF32 + threadIdx.x * VEC;
+#pragma unroll
+  for (int i = 0; i < TPL; ++i) {
+    const float v = xs[i];
+    const uint32_t k = logit_key(v), b = cut_bin(v, M, scale);
+    if ((uint32_t)(i / (TPL / 2)) == h && v == v && k >= thr_key &&
+        ((b >= b0 && b <= b1) || b == bk))
+      g_cut_lds.items[atomicAdd(&g_cut_lds.n, 1u)] =
+          cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC));
+  }
+  __syncthreads();
+  return g_cut_lds.n;
+}
+static_assert(kCutItems >= kChunkF32 / 2, "half a chunk's tokens fit the items");
+
 // cut_resolve over the row's logits, for a row whose boundary bins hold more
 // tokens than the lists: each step reads the row's chunks again. Out of line
 // (with the launch record copied to LDS, since a called function cannot reach
 // the kernel's arguments), so its registers stay out of the common path.
 template <int DT>
 __device__ __noinline__ void cut_rescan(uint32_t row) {
-  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
   const RowParams rp = g_cut_launch.params[row];
   const RowState st = g_cut_launch.states[row];
   auto each = [&](auto f) {
-#pragma unroll 1
-    for (uint32_t c = 0; c < g_cut_launch.chunks; ++c) {
-      float xs[TPL];
-      load_chunk<DT>(g_cut_launch, rp, row, c, g_cut_lds, xs);
-      const uint32_t lane_base = c * kChunkF32 + threadIdx.x * VEC;
-#pragma unroll
-      for (int i = 0; i < TPL; ++i) {
-        const float v = xs[i];
-        const uint32_t k = logit_key(v), b = cut_bin(v, st.maximum, st.scale);
-        if (v == v && k >= st.thr_key && ((b >= st.b0 && b <= st.b1) || b == st.bk))
-          f(cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC)));
-      }
+    for (uint32_t p = 0; p < 2 * g_cut_launch.chunks; ++p) {
+      const uint32_t n = cut_collect<DT>(row, p >> 1, p & 1u);
+      for (uint32_t i = threadIdx.x; i < n; i += kThreads) f(g_cut_lds.items[i]);
+      __syncthreads();
     }
   };
   cut_resolve(rp, st, each, g_cut_launch.out_kept_ids != nullptr, g_cut_lds);
 }
 
-// Latency-bound: a block a row. Its registers (the rescan's) cost nothing
-// here, where a chunk-parallel kernel would run two waves a SIMD for them.
+// The draw inside chunk c of a row without a draft: the first kept token, in id
+// order, whose running weight passes `within`; the thread that holds it writes
+// the row's result. Per-slice sums (64 x VEC consecutive tokens), then one
+// wave walks the slice that holds `within`.
 template <int DT>
-__global__ __launch_bounds__(kThreads) void cut_draw_kernel(SampleLaunch a) {
-  CutLds &s = g_cut_lds;
-  const uint32_t S = a.chunks, row = blockIdx.x;
-  const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const RowParams rp = a.params[row];
-  if (!cut_pass_row(rp)) return;
-  const RowState st = a.states[row];
-  if (st.stage != kRowGather) return;
-  const bool counts = a.out_kept_ids != nullptr;
-  const uint32_t draft = row_draft(a, rp);
+__device__ __forceinline__ void cut_walk(const SampleLaunch &a, const RowParams &rp,
+                                         const RowState &st, uint32_t bits, uint32_t row,
+                                         uint32_t c, uint64_t bound, uint64_t within,
+                                         uint32_t kept, CutLds &s) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
+                LOADS = Geo<DT>::LOADS;
+  const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  float xs[TPL];
+  cut_load<DT>(a, a.logits, a.stride, a.vocabulary, row, c, (bits & kCutPlain) != 0, rp, s, xs);
+  const uint32_t lane_base = c * kChunkF32 + tid * VEC;
+  const float M = st.maximum, inv_t = rp.inv_t;
+  // Kept: above the kept set's last value, or equal to it up to its last id;
+  // where nothing cuts, every member.
+  const float bv = bound        ? key_logit(cut_key(bound))
+                   : st.thr_key ? key_logit(st.thr_key)
+                                : -__builtin_inff();
+  const uint32_t bid = bound ? cut_id(bound) : kNoToken;
+  auto weight = [&](float v, uint32_t t) -> uint64_t {
+    uint64_t q = 0;
+    if (v > bv || (v == bv && t <= bid)) q = quantized_weight(v, M, inv_t);
+    return q;
+  };
+#pragma unroll
+  for (int h = 0; h < LOADS / 4; ++h) {
+    uint64_t lv[4];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int j = h * 4 + jj;
+      lv[jj] = 0;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e)
+        lv[jj] += weight(xs[j * VEC + e], lane_base + j * SLAB + e);
+    }
+    // Lane l holds the wave's sum of load h * 4 + l / 16.
+    const uint64_t sl = wave_sums_u64<4>(lv);
+    if (lane % 16 == 0) s.slices[(h * 4 + lane / 16) * kWaves + w] = sl;
+  }
+  __syncthreads();
+  const uint64_t vg = lane < (uint32_t)(LOADS * kWaves) ? s.slices[lane] : 0ull;
+  const uint32_t g = pick_slice(vg, LOADS * kWaves, within), jg = g / kWaves;
+  if (w != g % kWaves) return;
+  const uint32_t t0 = lane_base + jg * SLAB;
+  uint64_t q[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    float x = 0.0f;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) x = (uint32_t)j == jg ? xs[j * VEC + e] : x;
+    q[e] = weight(x, t0 + e);
+  }
+  uint32_t e_hit;
+  if (lane == slice_hit<VEC>(q, within, e_hit)) write_result(a, row, t0 + e_hit, 0.0f, kept);
+}
+
+// cut_resolve by one wave, for at most 64 listed tokens (lane i holds item i):
+// ranked by counting, the cuts by scans over the ranks.
+__device__ __forceinline__ void cut_resolve_wave(const RowParams &rp, const RowState &st,
+                                                 uint64_t item, uint32_t n, bool counts,
+                                                 CutLds &s) {
+  const uint32_t lane = lane_id();
+  const float M = st.maximum, inv_t = rp.inv_t;
+  s.small[lane] = item;
+  wave_lds_sync();
+  uint32_t rank = 0;
+#pragma unroll 4
+  for (uint32_t j = 0; j < n; ++j) rank += s.small[j] > item ? 1u : 0u;
+  if (lane < n) s.sorted[rank] = item;
+  wave_lds_sync();
+  const bool in = lane < n;
+  const uint64_t c = in ? s.sorted[lane] : 0ull;
+  const float v = key_logit(cut_key(c));
+  const uint32_t b = in ? cut_bin(v, M, st.scale) : 0u;
+  const uint64_t wq = in ? quantized_weight(v, M, inv_t) : 0ull;
+  uint64_t bound = 0, mass2 = st.total;
+  if (st.need_k) {
+    const bool at = in && b == st.bk;
+    const uint32_t run = wave_incl_scan_u32(at ? 1u : 0u);
+    const uint64_t hit = ballot(at && run == st.need_k);
+    bound = readlane_u64(c, hit ? (int)__builtin_ctzll(hit) : 63);
+    if (st.topp) mass2 = st.mass_bk + wave_sum_u64(at && c >= bound ? wq : 0ull);
+  }
+  if (st.topp && mass2) {
+    const bool at = in && c >= bound && b >= st.b0 && b <= st.b1;
+    const uint64_t run = wave_incl_scan_u64(at ? wq : 0ull);
+    const uint64_t hit = ballot(at && run >= floor_mul(mass2, rp.top_p) + 1 - st.mass_b0);
+    if (hit) bound = readlane_u64(c, (int)__builtin_ctzll(hit));
+  }
+  if (in && c >= bound && b >= st.b0) {
+    const uint32_t k = cut_id(c) / kChunkF32;
+    atomicAdd((unsigned long long *)&s.cmass[k], (unsigned long long)wq);
+    if (counts) atomicAdd(&s.ccount[k], 1u);
+  }
+  if (lane == 0) s.bound = bound;
+  wave_lds_sync();
+}
+
+// Wave 0: the kept mass, the kept tokens before each chunk, the draw's chunk,
+// and what cut_emit_kernel reads.
+__device__ __forceinline__ void cut_pick(const SampleLaunch &a, uint32_t row, uint32_t S,
+                                         uint32_t draft, float u, bool counts, CutLds &s) {
+  const uint32_t lane = lane_id();
   const bool drafted = draft != kNoToken;
-  const float u = row_uniform(a, row);
-  const uint64_t *rows = cut_area(a, row, 0);
-  const uint32_t room = cut_list_room(cut_counts(a, rp));
+  const uint64_t m = lane < S ? s.cmass[lane] : 0ull;
+  const uint64_t incl = wave_incl_scan_u64(m);
+  const uint64_t mass3 = readlane_u64(incl, 63);
+  uint64_t target = 0;
+  if (mass3 && !drafted) {
+    target = floor_mul(mass3, u);
+    if (target >= mass3) target = mass3 - 1;
+  }
+  const uint64_t hm = ballot(lane < S && incl > target);
+  const int c = hm ? (int)__builtin_ctzll(hm) : 0;
+  const uint64_t excl = readlane_u64(incl - m, c);
+  uint32_t kept = 0;
+  if (counts) {
+    const uint32_t kn = lane < S ? s.ccount[lane] : 0u;
+    const uint32_t ki = wave_incl_scan_u32(kn);
+    kept = readlane_u32(ki, 63);
+    if (lane < S) cut_area(a, row, lane)[kCutKeptWord] = ki - kn;
+  }
+  if (drafted) {
+    // For cut_emit_kernel: the chunks' kept masses, no draft weight yet.
+    if (lane < S) cut_area(a, row, lane)[kCutMassWord] = m;
+    if (lane == 0 && draft < a.vocabulary)
+      cut_area(a, row, draft / kChunkF32)[kCutDraftWord] = 0;
+  }
+  if (lane == 0) {
+    s.u64a = mass3;
+    s.sel_chunk = (uint32_t)c;
+    s.sel_excl = target - excl;
+    s.kept = kept;
+    RowState &ns = a.states[row];
+    ns.bkey = cut_key(s.bound);
+    ns.bid = s.bound ? cut_id(s.bound) : 0u;
+    ns.mass3 = mass3;
+    ns.kept = kept;
+    ns.stage = counts || (drafted && mass3) ? kRowEmit : kRowDone;
+  }
+}
+
+// Latency-bound: a block a row. Its registers (the rescan's) cost nothing
+// here, where a chunk-parallel kernel would run two waves a SIMD for them. The
+// row's record, its boundary bins and its chunks' sums go out together from
+// preloaded arguments; up to 64 listed tokens (most rows) are resolved by one
+// wave without a barrier.
+template <int DT>
+__global__ __launch_bounds__(kThreads) void cut_draw_kernel(
+    const RowParams *params, const RowState *states, const uint64_t *cands,
+    const float *uniforms, const uint32_t *uniform_index, const uint32_t *draft_tokens,
+    uint32_t bits, SampleLaunch a) {
+  CutLds &s = g_cut_lds;
+  const uint32_t S = bits & 0xffu, row = blockIdx.x;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint64_t *rows = cands + (uint64_t)row * S * kBlockCandidates;
+  const ulonglong2 sums =
+      *(const ulonglong2 *)(rows + (uint64_t)min(lane, S - 1) * kBlockCandidates + kCutMassWord);
+  const uint32_t at = uniform_index ? uniform_index[row] : 0u;
+  const RowParams rp = load_row_policy(params + row);
+  const RowState st = load_const(states + row);
+  if (!cut_pass_row(rp) || st.stage != kRowGather) return;
+  const float u =
+      uniforms[uniform_index ? (uint64_t)at : a.uniform_offset + row * a.uniform_stride];
+  const bool counts = (bits & kCutKept) != 0, listed = cut_counts(rp, bits);
+  const uint64_t *list = rows + cut_list_word(listed);
+  const uint32_t draft =
+      draft_tokens && rp.draft_index != kNoToken ? draft_tokens[rp.draft_index] : kNoToken;
+  const bool drafted = draft != kNoToken;
+  // Item i of the row's lists: its chunk by a binary search of the offsets.
+  auto item = [&](uint32_t i) {
+    uint32_t c = 0;
+    for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
+      if (c + step < S && g_cut_lds.coff[c + step] <= i) c += step;
+    return list[(uint64_t)c * kBlockCandidates + (i - g_cut_lds.coff[c])];
+  };
   if (tid < 64) {
-    const uint64_t *p = rows + (uint64_t)min(lane, S - 1) * kBlockCandidates;
-    const uint64_t cm = p[kCutMassWord], cn = p[kCutCountWord];
     const bool in = lane < S;
-    const uint32_t n = in ? (uint32_t)(cn >> 32) : 0u;
-    const uint32_t incl = wave_incl_scan_u32(n);
-    const uint64_t over = ballot(n > room);
-    s.cmass[lane] = in ? cm : 0ull;
-    s.ccount[lane] = in ? (uint32_t)cn : 0u;
+    const uint32_t n = in ? (uint32_t)(sums.y >> 32) : 0u;
+    const uint32_t incl = wave_incl_scan_u32(n), all = readlane_u32(incl, 63);
+    const uint64_t over = ballot(n > cut_list_room(listed));
+    s.cmass[lane] = in ? sums.x : 0ull;
+    s.ccount[lane] = in ? (uint32_t)sums.y : 0u;
     s.coff[lane + 1] = incl;
-    const uint32_t all = readlane_u32(incl, 63);
     if (lane == 0) {
       s.coff[0] = 0;
       s.bound = 0;
       s.n = over || all > kCutItems ? 0xffffffffu : all;
     }
+    wave_lds_sync();
+    if (!over && all <= 64u) {
+      if (st.b0 < kCutBins)
+        cut_resolve_wave(rp, st, lane < all ? item(lane) : 0ull, all, counts, s);
+      cut_pick(a, row, S, draft, u, counts, s);
+    }
   }
   __syncthreads();
   const uint32_t n = s.n;
-  if (n == 0xffffffffu) {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(&g_cut_launch);
-    for (uint32_t k = tid; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
+  if (n > 64u) {
+    if (n == 0xffffffffu) {
+      const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
+      uint32_t *dst = reinterpret_cast<uint32_t *>(&g_cut_launch);
+      for (uint32_t k = tid; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
+      __syncthreads();
+      cut_rescan<DT>(row);
+    } else {
+      for (uint32_t i = tid; i < n; i += kThreads) s.items[i] = item(i);
+      __syncthreads();
+      auto each = [&](auto f) {
+        for (uint32_t i = tid; i < n; i += kThreads) f(g_cut_lds.items[i]);
+      };
+      cut_resolve(rp, st, each, counts, s);
+    }
+    if (tid < 64) cut_pick(a, row, S, draft, u, counts, s);
     __syncthreads();
-    cut_rescan<DT>(row);
-  } else if (st.b0 < kCutBins) {
-    // The lists, compact, into LDS: item i's chunk by a binary search.
-    const uint64_t *list = rows + cut_list_word(cut_counts(a, rp));
-    for (uint32_t i = tid; i < n; i += kThreads) {
-      uint32_t c = 0;
-      for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
-        if (c + step < S && s.coff[c + step] <= i) c += step;
-      s.items[i] = list[(uint64_t)c * kBlockCandidates + (i - s.coff[c])];
-    }
-    __syncthreads();
-    auto each = [&](auto f) {
-      for (uint32_t i = tid; i < n; i += kThreads) f(g_cut_lds.items[i]);
-    };
-    cut_resolve(rp, st, each, counts, s);
   }
-  // The kept mass, the kept tokens before each chunk, and the draw's chunk.
-  if (tid < 64) {
-    const uint64_t m = lane < S ? s.cmass[lane] : 0ull;
-    const uint64_t incl = wave_incl_scan_u64(m);
-    const uint64_t mass3 = readlane_u64(incl, 63);
-    uint64_t target = 0;
-    if (mass3 && !drafted) {
-      target = floor_mul(mass3, u);
-      if (target >= mass3) target = mass3 - 1;
-    }
-    const uint64_t hm = ballot(lane < S && incl > target);
-    const int c = hm ? (int)__builtin_ctzll(hm) : 0;
-    const uint64_t excl = readlane_u64(incl - m, c);
-    uint32_t kept = 0;
-    if (counts) {
-      const uint32_t kn = lane < S ? s.ccount[lane] : 0u;
-      const uint32_t ki = wave_incl_scan_u32(kn);
-      kept = readlane_u32(ki, 63);
-      if (lane < S) cut_area(a, row, lane)[kCutKeptWord] = ki - kn;
-    }
-    if (drafted) {
-      // For cut_emit_kernel: the chunks' kept masses, no draft weight yet.
-      if (lane < S) cut_area(a, row, lane)[kCutMassWord] = m;
-      if (lane == 0 && draft < a.vocabulary)
-        cut_area(a, row, draft / kChunkF32)[kCutDraftWord] = 0;
-    }
-    if (lane == 0) {
-      s.u64a = mass3;
-      s.sel_chunk = (uint32_t)c;
-      s.sel_excl = target - excl;
-      s.n = kept;
-      RowState &ns = a.states[row];
-      ns.bkey = cut_key(s.bound);
-      ns.bid = s.bound ? cut_id(s.bound) : 0u;
-      ns.mass3 = mass3;
-      ns.kept = kept;
-      ns.stage = counts || (drafted && mass3) ? kRowEmit : kRowDone;
-    }
-  }
-  __syncthreads();
   const uint64_t mass3 = s.u64a;
   if (mass3 == 0) {
-    if (tid == 0) write_result(a, row, kNoToken, 0.0f, s.n);
+    if (tid == 0) write_result(a, row, kNoToken, 0.0f, s.kept);
     return;
   }
-  if (drafted) return;
-  const uint64_t bound = s.bound;
-  const uint32_t kept = s.n, c = s.sel_chunk;
-  const uint64_t within = s.sel_excl;
-  __syncthreads();  // the items' area becomes the walk's
-  const uint32_t hit = walk_chunk<DT>(a, rp, row, c, st.maximum, st.thr_key, cut_key(bound),
-                                      bound ? cut_id(bound) : 0u, false, mass3, within, s);
-  if (tid == 0) write_result(a, row, hit, 0.0f, kept);
+  if (!drafted)
+    cut_walk<DT>(a, rp, st, bits, row, s.sel_chunk, s.bound, s.sel_excl, s.kept, s);
 }
 
 // Kept outputs, and drafted rows: the residual masses per chunk, and in the
 // row's last chunk to arrive the draw.
-template <int DT>
-__global__ __launch_bounds__(kThreads) void cut_emit_kernel(SampleLaunch a) {
+// DRAFT: the launch has drafted rows (a separate build: their residual pass
+// takes three times the registers).
+template <int DT, bool DRAFT>
+__global__ __launch_bounds__(kThreads) void cut_emit_kernel(
+    const void *logits, const RowParams *params, const BlockHeader *headers, uint64_t *cands,
+    RowState *states, uint64_t stride, uint32_t V, uint32_t bits, SampleLaunch a) {
   constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
                 LOADS = Geo<DT>::LOADS;
   constexpr uint32_t VMASK = (1u << VEC) - 1u;
   __shared__ DrawLds s;
-  const uint32_t S = a.chunks;
-  const uint32_t row = blockIdx.x / S, chunk = blockIdx.x % S;
+  (void)headers;
+  const uint32_t S = bits & 0xffu, row = blockIdx.y, chunk = blockIdx.x;
   const uint32_t tid = threadIdx.x;
-  const RowParams rp = a.params[row];
-  if (!cut_pass_row(rp)) return;
-  const RowState st = a.states[row];
-  if (st.stage != kRowEmit) return;
-  const uint32_t draft = row_draft(a, rp);
-  const bool drafted = draft != kNoToken && st.mass3 != 0;
-  uint64_t *area = cut_area(a, row, chunk);
+  uint64_t *area = cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
+  const RowParams rp = load_row_policy(params + row);
+  // (A plain load: a drafted row's last block marks it done.)
+  const RowState st = states[row];
+  if (!cut_pass_row(rp) || st.stage != kRowEmit) return;
+  const uint32_t draft = DRAFT ? row_draft(a, rp) : kNoToken;
+  const bool drafted = DRAFT && draft != kNoToken && st.mass3 != 0;
   const uint64_t kept_before = a.out_kept_ids ? area[kCutKeptWord] : 0ull;
   if (!drafted && kept_before >= a.kept_cap) return;
-  float qv[TPL];
-  if (drafted && a.dense_q) load_dense_q<DT>(a, rp, chunk, qv);
+  float qv[DRAFT ? TPL : 1];
+  if constexpr (DRAFT)
+    if (drafted && a.dense_q) load_dense_q<DT>(a, rp, chunk, qv);
   float xs[TPL];
-  load_chunk<DT>(a, rp, row, chunk, s, xs);
-  stage_candidates(a, rp, s);
+  cut_load<DT>(a, logits, stride, V, row, chunk, (bits & kCutPlain) != 0, rp, s, xs);
+  if constexpr (DRAFT) stage_candidates(a, rp, s);
   const uint32_t lane_base = chunk * kChunkF32 + tid * VEC;
   const float M = st.maximum, inv_t = rp.inv_t;
   auto tok_of = [&](int i) -> uint32_t { return lane_base + (i / VEC) * SLAB + (i % VEC); };
@@ -4453,58 +4686,60 @@ __global__ __launch_bounds__(kThreads) void cut_emit_kernel(SampleLaunch a) {
         }
     }
   }
-  if (!drafted) return;
-  uint64_t dsum = 0, held = 0;
+  if constexpr (DRAFT) {
+    if (!drafted) return;
+    uint64_t dsum = 0, held = 0;
 #pragma unroll
-  for (int i = 0; i < TPL; ++i)
-    if ((mem >> i) & 1u) {
-      const uint64_t wq = quantized_weight(xs[i], M, inv_t);
-      dsum += residual_of(wq, st.mass3, a.dense_q ? qv[i] : draft_q(a, rp, tok_of(i), s));
-      if (tok_of(i) == draft) held = (uint64_t)f2u(weight_of(xs[i], M, inv_t)) | (1ull << 32);
+    for (int i = 0; i < TPL; ++i)
+      if ((mem >> i) & 1u) {
+        const uint64_t wq = quantized_weight(xs[i], M, inv_t);
+        dsum += residual_of(wq, st.mass3, a.dense_q ? qv[i] : draft_q(a, rp, tok_of(i), s));
+        if (tok_of(i) == draft) held = (uint64_t)f2u(weight_of(xs[i], M, inv_t)) | (1ull << 32);
+      }
+    if (held) st_dev(area + kCutDraftWord, held);
+    dsum = block_sum_u64(dsum, s);
+    if (tid == 0) {
+      st_dev(area + kCutResidualWord, dsum);
+      s.sel_excl = 0;
     }
-  if (held) st_dev(area + kCutDraftWord, held);
-  dsum = block_sum_u64(dsum, s);
-  if (tid == 0) {
-    st_dev(area + kCutResidualWord, dsum);
-    s.sel_excl = 0;
-  }
-  if (!arrive_last(a.counters + row, S, s)) return;
-  if (tid < 64) {
-    const uint32_t lane = tid;
-    const bool in = lane < S;
-    const uint64_t *p = cut_area(a, row, min(lane, S - 1));
-    const uint64_t d = in ? ld_dev(p + kCutResidualWord) : 0ull;
-    // No residual mass: the plain draw, over the chunks' kept masses.
-    const bool residual = ballot(d != 0) != 0;
-    const uint64_t v = residual ? d : in ? ld_dev(p + kCutMassWord) : 0ull;
-    const uint64_t incl = wave_incl_scan_u64(v), total = readlane_u64(incl, 63);
-    uint64_t target = floor_mul(total, row_uniform(a, row));
-    if (target >= total) target = total - 1;
-    const uint64_t hm = ballot(in && incl > target);
-    const int c = hm ? (int)__builtin_ctzll(hm) : 0;
-    const uint64_t excl = readlane_u64(incl - v, c);
-    // The draft token's weight, from its chunk when that keeps it.
-    const uint64_t dw = draft < a.vocabulary
-                            ? ld_dev(cut_area(a, row, draft / kChunkF32) + kCutDraftWord)
-                            : 0ull;
-    if (lane == 0) {
-      s.slice = (uint32_t)c;
-      s.slice_within = target - excl;
-      s.hit = residual ? 1u : 0u;
-      s.u64a = dw;
-      a.states[row].stage = kRowDone;
+    if (!arrive_last(a.counters + row, S, s)) return;
+    if (tid < 64) {
+      const uint32_t lane = tid;
+      const bool in = lane < S;
+      const uint64_t *p = cut_area(a, row, min(lane, S - 1));
+      const uint64_t d = in ? ld_dev(p + kCutResidualWord) : 0ull;
+      // No residual mass: the plain draw, over the chunks' kept masses.
+      const bool residual = ballot(d != 0) != 0;
+      const uint64_t v = residual ? d : in ? ld_dev(p + kCutMassWord) : 0ull;
+      const uint64_t incl = wave_incl_scan_u64(v), total = readlane_u64(incl, 63);
+      uint64_t target = floor_mul(total, row_uniform(a, row));
+      if (target >= total) target = total - 1;
+      const uint64_t hm = ballot(in && incl > target);
+      const int c = hm ? (int)__builtin_ctzll(hm) : 0;
+      const uint64_t excl = readlane_u64(incl - v, c);
+      // The draft token's weight, from its chunk when that keeps it.
+      const uint64_t dw = draft < a.vocabulary
+                              ? ld_dev(cut_area(a, row, draft / kChunkF32) + kCutDraftWord)
+                              : 0ull;
+      if (lane == 0) {
+        s.slice = (uint32_t)c;
+        s.slice_within = target - excl;
+        s.hit = residual ? 1u : 0u;
+        s.u64a = dw;
+        states[row].stage = kRowDone;
+      }
     }
+    __syncthreads();
+    const uint64_t dw = s.u64a, within = s.slice_within;
+    const uint32_t c = s.slice;
+    const bool residual = s.hit != 0;
+    __syncthreads();
+    const uint32_t hit = walk_chunk<DT>(a, rp, row, c, M, st.thr_key, st.bkey, st.bid, residual,
+                                        st.mass3, within, s);
+    if (tid == 0)
+      write_result(a, row, hit, dw >> 32 ? (float)((double)u2f((uint32_t)dw) / scale) : 0.0f,
+                   st.kept);
   }
-  __syncthreads();
-  const uint64_t dw = s.u64a, within = s.slice_within;
-  const uint32_t c = s.slice;
-  const bool residual = s.hit != 0;
-  __syncthreads();
-  const uint32_t hit = walk_chunk<DT>(a, rp, row, c, M, st.thr_key, st.bkey, st.bid, residual,
-                                      st.mass3, within, s);
-  if (tid == 0)
-    write_result(a, row, hit, dw >> 32 ? (float)((double)u2f((uint32_t)dw) / scale) : 0.0f,
-                 st.kept);
 }
 #endif
 
@@ -5545,19 +5780,31 @@ int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, void *s
 #endif
 
 #if JF_IN(3)
-int launch_cut(const SampleLaunch &a, uint32_t dtype, bool emit, void *stream) {
-  const dim3 grid(a.rows * a.chunks), block(kThreads);
+int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *stream) {
+  const dim3 grid(a.chunks, a.rows), block(kThreads);
   const hipStream_t st = (hipStream_t)stream;
-  auto go = [&](auto kernel, dim3 blocks) {
-    hipLaunchKernelGGL(kernel, blocks, block, 0, st, a);
+  const uint32_t bits = a.chunks | (c.all ? kCutAll : 0u) |
+                        (c.plain && a.vocabulary >= 8 ? kCutPlain : 0u) |
+                        (a.out_kept_ids ? kCutKept : 0u);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, a.logits, a.params,
+                       (const BlockHeader *)a.headers, a.cands, a.states, a.stride, a.vocabulary,
+                       bits, a);
     return hipGetLastError();
   };
-  hipError_t e = dtype == 0 ? go(cut_hist_kernel<0>, grid) : go(cut_hist_kernel<1>, grid);
-  if (e == hipSuccess) e = dtype == 0 ? go(cut_list_kernel<0>, grid) : go(cut_list_kernel<1>, grid);
-  const dim3 rows(a.rows);
-  if (e == hipSuccess) e = dtype == 0 ? go(cut_draw_kernel<0>, rows) : go(cut_draw_kernel<1>, rows);
-  if (e == hipSuccess && emit)
-    e = dtype == 0 ? go(cut_emit_kernel<0>, grid) : go(cut_emit_kernel<1>, grid);
+  auto draw = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.rows), block, 0, st, a.params, (const RowState *)a.states,
+                       (const uint64_t *)a.cands, a.uniforms, a.uniform_index, a.draft_tokens,
+                       bits, a);
+    return hipGetLastError();
+  };
+  hipError_t e = dtype == 0 ? go(cut_hist_kernel<0>) : go(cut_hist_kernel<1>);
+  if (e == hipSuccess) e = dtype == 0 ? go(cut_list_kernel<0>) : go(cut_list_kernel<1>);
+  if (e == hipSuccess) e = dtype == 0 ? draw(cut_draw_kernel<0>) : draw(cut_draw_kernel<1>);
+  if (e == hipSuccess && c.drafted)
+    e = dtype == 0 ? go(cut_emit_kernel<0, true>) : go(cut_emit_kernel<1, true>);
+  else if (e == hipSuccess && a.out_kept_ids)
+    e = dtype == 0 ? go(cut_emit_kernel<0, false>) : go(cut_emit_kernel<1, false>);
   return (int)e;
 }
 #endif

@@ -967,7 +967,12 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     if (e != hipSuccess) return hip_fail((hipError_t)e, "merge launch");
   }
   if (passes) {
-    e = jf::launch_cut(L, a->dtype, kept || any_drafted, stream);
+    jf::CutLaunch c{true, true, any_drafted};
+    for (uint32_t r = 0; r < rows; ++r) {
+      c.all &= jf::wide_row(params[r].flags, params[r].top_k);
+      c.plain &= !(params[r].flags & jf::kRowPenalized);
+    }
+    e = jf::launch_cut(L, a->dtype, c, stream);
     if (e != hipSuccess) return hip_fail((hipError_t)e, "cut pass launch");
   }
   if (any_uncut && !fuse_uncut) {
