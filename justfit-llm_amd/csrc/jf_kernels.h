@@ -59,7 +59,7 @@ struct BlockHeader {
                        // admit a token)
   uint32_t admitted;   // sampled: 1 when the chunk admits a non-NaN token
   uint32_t overflow;   // sampled: candidates did not fit
-  float best_value;    // greedy
+  float best_value;    // greedy (wide_row: the chunk's least value)
   uint32_t best_id;    // greedy
   uint32_t floor_key;  // sampled: the row's K-th key is at least this
                        // (wide_row: `count` tokens of the chunk reach it)
@@ -103,10 +103,16 @@ constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kBlockCandidates = 1024;
 constexpr int kMergeCapacity = 2048;
+constexpr uint32_t kMergeItems = 3072;  // tokens of a row the general merge holds
 constexpr int kPenaltyWordsLds = 2048;
 // A sampled row with no min-p floor whose top-k is off or past this takes the
-// cut passes; up to it, the candidate lists and the merge.
-constexpr uint32_t kListTopK = 1024;
+// cut passes; up to it, the candidate lists and the merge. The select pass
+// bounds a chunk's K-th token by its waves' ceil(K / 4)-th largest lane maxima
+// (64 of them), so the lists grow faster than K: 64 rows x 151,936 fp32 ran
+// 33.0 us at top-k 65, 38.4 at 96, 42.0 at 112, 70 at 128 (lists that overflow)
+// through the lists, and 46.8-47.5 through the cut passes; in bf16 31.3, 37.2,
+// 46.1, 70 against 43.5-44.1.
+constexpr uint32_t kListTopK = 96;
 constexpr uint32_t kCutBins = 512;    // bins of a row's values below its maximum
 constexpr uint32_t kCutItems = 6144;  // boundary tokens of a row resolved in LDS
 constexpr int kMaxExtra = 16;

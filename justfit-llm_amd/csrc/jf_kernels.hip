@@ -67,7 +67,11 @@ struct PrepLds {
 struct MergeLds {
   uint32_t key[kMergeCapacity];
   uint32_t id[kMergeCapacity];
-  uint8_t fl[kMergeCapacity];
+  uint32_t bins[1024];
+};
+struct ItemsLds {
+  uint64_t items[kMergeItems];    // token_item words, any order
+  uint64_t grouped[kMergeItems];  // the kept ones by id range
   uint32_t bins[1024];
 };
 
@@ -75,8 +79,15 @@ struct __align__(16) Lds {
   union {
     PrepLds prep;
     MergeLds merge;
+    ItemsLds general;
   };
   uint64_t hist[256];
+  uint32_t hcount[256];
+  uint64_t small[64];
+  uint64_t sorted[64];
+  uint64_t wl2[kWaves];
+  uint32_t small_n;
+  uint32_t n;
   uint64_t wj[kWaves][8];
   uint64_t wl[kWaves];
   float wf[kWaves];
@@ -116,6 +127,7 @@ struct __align__(16) SelectLds {
   float wf[kWaves];
   uint32_t wu[kWaves];
   uint32_t wu2[kWaves];
+  float wmin[kWaves];
 };
 
 // The mass-and-draw kernel's LDS: the chunk's penalty lookup, the
@@ -196,46 +208,6 @@ __device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, L &s,
   }
   if (total) *total = tot;
   return off + incl - v;
-}
-
-// Wave 0 finds the highest bin b of s.hist whose suffix sum (bins >= b)
-// reaches T; s.sel_bin = b, s.sel_excl = sum of the bins above b. The
-// caller guarantees the total reaches T.
-__device__ __forceinline__ void crossing_bin(Lds &s, uint64_t T) {
-  if (threadIdx.x < 64) {
-    const uint32_t l = threadIdx.x;
-    const uint64_t h0 = s.hist[4 * l], h1 = s.hist[4 * l + 1],
-                   h2 = s.hist[4 * l + 2], h3 = s.hist[4 * l + 3];
-    const uint64_t own = h0 + h1 + h2 + h3;
-    // Suffix sum over lanes: the total less the prefix before this lane.
-    const uint64_t incl = wave_incl_scan_u64(own);
-    const uint64_t suf = readlane_u64(incl, 63) - (incl - own);
-    const uint64_t m = ballot(suf >= T);
-    const int L = m ? (int)__popcll(m) - 1 : 0;
-    const uint64_t above = readlane_u64(suf - own, L);
-    if ((int)l == L) {
-      // Walk this lane's four bins from the top.
-      uint64_t acc = above;
-      uint32_t bin = 4 * l;
-      uint64_t excl = acc;
-      if (acc + h3 >= T) {
-        bin = 4 * l + 3;
-        excl = acc;
-      } else if (acc + h3 + h2 >= T) {
-        bin = 4 * l + 2;
-        excl = acc + h3;
-      } else if (acc + h3 + h2 + h1 >= T) {
-        bin = 4 * l + 1;
-        excl = acc + h3 + h2;
-      } else {
-        bin = 4 * l;
-        excl = acc + h3 + h2 + h1;
-      }
-      s.sel_bin = bin;
-      s.sel_excl = excl;
-    }
-  }
-  __syncthreads();
 }
 
 __device__ __forceinline__ bool at_or_before(uint32_t key, uint32_t token,
@@ -706,282 +678,18 @@ __device__ __forceinline__ uint64_t residual_of(uint64_t wq, uint64_t mass,
   return wq > qm ? wq - qm : 0;
 }
 
-// ---- the merge of a sampled row ------------------------------------------
-
-// Items of the merge live in s.merge (key, id, flag) in id order. Per-thread
-// contiguous ranges give ordered scans.
-struct ItemRange {
-  uint32_t begin, end;
-};
-__device__ __forceinline__ ItemRange my_items(uint32_t n) {
-  const uint32_t per = (n + kThreads - 1) / kThreads;
-  const uint32_t b = min(threadIdx.x * per, n);
-  return {b, min(b + per, n)};
+// ---- a row's tokens as items -----------------------------------------------
+//
+// A token as one word that orders as (key, lower id first): ids are below 2^19.
+__device__ __forceinline__ uint64_t token_item(uint32_t key, uint32_t id) {
+  return ((uint64_t)key << 19) | (0x7ffffu - id);
 }
-
-// Keeps, among flagged items, the first `keep` in (key desc, id asc) order:
-// radix descent over the key bytes, then the lowest ids among the ties.
-__device__ __forceinline__ void lds_topk(Lds &s, uint32_t n, uint32_t keep) {
-  MergeLds &m = s.merge;
-  uint32_t prefix = 0, pmask = 0;
-  uint64_t need = keep;
-  for (int d = 3; d >= 0; --d) {
-    s.hist[threadIdx.x] = 0;
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
-      const uint32_t k = m.key[i];
-      if (m.fl[i] && (k & pmask) == prefix)
-        atomicAdd((unsigned long long *)&s.hist[(k >> (8 * d)) & 255u], 1ull);
-    }
-    __syncthreads();
-    crossing_bin(s, need);
-    need -= s.sel_excl;
-    prefix |= s.sel_bin << (8 * d);
-    pmask |= 255u << (8 * d);
-    __syncthreads();
-  }
-  // need = how many tokens tied at `prefix` stay, lowest ids first.
-  const ItemRange r = my_items(n);
-  uint32_t ties = 0;
-  for (uint32_t i = r.begin; i < r.end; ++i) ties += m.fl[i] && m.key[i] == prefix;
-  uint32_t rank = (uint32_t)block_excl_scan_u64(ties, s, nullptr);
-  for (uint32_t i = r.begin; i < r.end; ++i) {
-    if (!m.fl[i]) continue;
-    const uint32_t k = m.key[i];
-    if (k > prefix) continue;
-    if (k < prefix) {
-      m.fl[i] = 0;
-    } else {
-      m.fl[i] = rank < need ? 1 : 0;
-      ++rank;
-    }
-  }
-  __syncthreads();
+__device__ __forceinline__ uint32_t item_key(uint64_t item) { return (uint32_t)(item >> 19); }
+__device__ __forceinline__ uint32_t item_id(uint64_t item) {
+  return 0x7ffffu - ((uint32_t)item & 0x7ffffu);
 }
-
-// Top-p over the flagged items (sampling.metal:615-641): keep them in order
-// until the running mass exceeds floor(top_p * mass); that token stays.
-__device__ __forceinline__ void lds_topp(Lds &s, uint32_t n, float maximum, float inv_t,
-                         float top_p) {
-  MergeLds &m = s.merge;
-  uint64_t local = 0;
-  for (uint32_t i = threadIdx.x; i < n; i += kThreads)
-    if (m.fl[i]) local += quantize(weight_of(key_logit(m.key[i]), maximum, inv_t));
-  const uint64_t mass = block_sum_u64(local, s);
-  if (mass == 0) return;  // nothing weighs: the nucleus never closes
-  const uint64_t nucleus = floor_mul(mass, top_p);
-  uint64_t need = nucleus + 1;  // the kept prefix's mass must reach this
-  uint32_t prefix = 0, pmask = 0;
-  for (int d = 3; d >= 0; --d) {
-    s.hist[threadIdx.x] = 0;
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
-      const uint32_t k = m.key[i];
-      if (m.fl[i] && (k & pmask) == prefix) {
-        const uint64_t wq = quantize(weight_of(key_logit(k), maximum, inv_t));
-        if (wq) atomicAdd((unsigned long long *)&s.hist[(k >> (8 * d)) & 255u],
-                          (unsigned long long)wq);
-      }
-    }
-    __syncthreads();
-    crossing_bin(s, need);
-    need -= s.sel_excl;
-    prefix |= s.sel_bin << (8 * d);
-    pmask |= 255u << (8 * d);
-    __syncthreads();
-  }
-  const uint64_t wk = quantize(weight_of(key_logit(prefix), maximum, inv_t));
-  const uint64_t ties_kept = (need + wk - 1) / wk;
-  const ItemRange r = my_items(n);
-  uint32_t ties = 0;
-  for (uint32_t i = r.begin; i < r.end; ++i) ties += m.fl[i] && m.key[i] == prefix;
-  uint32_t rank = (uint32_t)block_excl_scan_u64(ties, s, nullptr);
-  for (uint32_t i = r.begin; i < r.end; ++i) {
-    if (!m.fl[i]) continue;
-    const uint32_t k = m.key[i];
-    if (k > prefix) continue;
-    if (k < prefix) {
-      m.fl[i] = 0;
-    } else {
-      m.fl[i] = rank < ties_kept ? 1 : 0;
-      ++rank;
-    }
-  }
-  __syncthreads();
-}
-
-// The draw over the flagged items in id order (sampling.metal:694-829) and
-// the row's outputs.
-__device__ __forceinline__ void lds_draw(const SampleLaunch &a, const RowParams &rp,
-                                         uint32_t row, Lds &s, uint32_t n, float maximum,
-                                         float inv_t) {
-  MergeLds &m = s.merge;
-  const ItemRange r = my_items(n);
-  uint64_t mloc = 0;
-  uint32_t kloc = 0;
-  for (uint32_t i = r.begin; i < r.end; ++i)
-    if (m.fl[i]) {
-      mloc += quantize(weight_of(key_logit(m.key[i]), maximum, inv_t));
-      ++kloc;
-    }
-  uint64_t mass3;
-  (void)block_excl_scan_u64(mloc, s, &mass3);
-  uint64_t kept_total;
-  const uint32_t kept_rank = (uint32_t)block_excl_scan_u64(kloc, s, &kept_total);
-  const double scale = (double)mass3 * 0x1p-44;
-  if (a.out_kept_ids) {
-    uint32_t k = kept_rank;
-    for (uint32_t i = r.begin; i < r.end; ++i) {
-      if (!m.fl[i]) continue;
-      if (k < a.kept_cap) {
-        const float w = weight_of(key_logit(m.key[i]), maximum, inv_t);
-        a.out_kept_ids[(uint64_t)row * a.kept_cap + k] = m.id[i];
-        a.out_kept_probs[(uint64_t)row * a.kept_cap + k] =
-            mass3 ? (float)((double)w / scale) : 0.0f;
-      }
-      ++k;
-    }
-  }
-  if (mass3 == 0) {
-    if (threadIdx.x == 0) write_result(a, row, kNoToken, 0.0f, (uint32_t)kept_total);
-    return;
-  }
-  const uint32_t draft = row_draft(a, rp);
-  const bool drafted = draft != kNoToken;
-  uint64_t dloc = 0;
-  uint32_t any = 0;
-  if (drafted) {
-    for (uint32_t i = r.begin; i < r.end; ++i)
-      if (m.fl[i]) {
-        const uint64_t wq =
-            quantize(weight_of(key_logit(m.key[i]), maximum, inv_t));
-        const uint64_t d = residual_of(wq, mass3, draft_q(a, rp, m.id[i], s));
-        dloc += d;
-        any |= d > 0;
-      }
-  }
-  const bool residual = drafted && block_max_u32(any, s) != 0;
-  if (!residual) dloc = mloc;
-  uint64_t total;
-  const uint64_t excl = block_excl_scan_u64(dloc, s, &total);
-  uint64_t target = floor_mul(total, row_uniform(a, row));
-  if (target >= total) target = total - 1;
-  if (threadIdx.x == 0) {
-    s.hit = kNoToken;
-    s.found_w = 0.0f;
-  }
-  __syncthreads();
-  if (excl <= target && excl + dloc > target) {
-    uint64_t run = excl;
-    for (uint32_t i = r.begin; i < r.end; ++i) {
-      if (!m.fl[i]) continue;
-      const uint64_t wq =
-          quantize(weight_of(key_logit(m.key[i]), maximum, inv_t));
-      run += residual ? residual_of(wq, mass3, draft_q(a, rp, m.id[i], s)) : wq;
-      if (run > target) {
-        s.hit = m.id[i];
-        break;
-      }
-    }
-  }
-  if (drafted)
-    for (uint32_t i = r.begin; i < r.end; ++i)
-      if (m.fl[i] && m.id[i] == draft)
-        s.found_w = weight_of(key_logit(m.key[i]), maximum, inv_t);
-  __syncthreads();
-  if (threadIdx.x == 0)
-    write_result(a, row, s.hit,
-                 drafted ? (float)((double)s.found_w / scale) : 0.0f,
-                 (uint32_t)kept_total);
-}
-
-// The merge of at most kThreads items in s.merge (any order): thread t
-// holds item t and counts its rank in (key desc, id asc) order, which gives
-// the top-k cut and the rank-order walk of top-p; the kept items' ranks by id
-// give the id-order draw.
-__device__ __forceinline__ void small_merge(const SampleLaunch &a,
-                                            const RowParams &rp, uint32_t row,
-                                            Lds &s, uint32_t n, float maximum) {
-  MergeLds &m = s.merge;
-  const uint32_t t = threadIdx.x;
-  const bool have = t < n;
-  const uint32_t key = have ? m.key[t] : 0u;
-  const uint32_t id = have ? m.id[t] : kNoToken;
-  uint32_t rank = 0;
-  if (have)
-    for (uint32_t j = 0; j < n; ++j) {
-      const uint32_t kj = m.key[j];
-      rank += (kj > key) || (kj == key && m.id[j] < id);
-    }
-  const uint32_t n2 = min(rp.top_k, n);
-  const float w = have ? weight_of(key_logit(key), maximum, rp.inv_t) : 0.0f;
-  const uint64_t wq = quantize(w);
-  if (have) m.bins[t] = rank;
-  uint32_t n3 = n2;
-  if (rp.flags & kRowTopP) {
-    // Weights in rank order, their running sum, the first rank past the
-    // nucleus.
-    __syncthreads();
-    if (have && rank < n2) s.hist[rank] = wq;
-    __syncthreads();
-    const uint64_t mine = t < n2 ? s.hist[t] : 0;
-    uint64_t mass2;
-    const uint64_t excl = block_excl_scan_u64(mine, s, &mass2);
-    if (t == 0) s.hit = n2;
-    __syncthreads();
-    if (mass2) {
-      const uint64_t nucleus = floor_mul(mass2, rp.top_p);
-      if (t < n2 && excl <= nucleus && excl + mine > nucleus) s.hit = t + 1;
-    }
-    __syncthreads();
-    n3 = s.hit;
-  }
-  __syncthreads();
-  const bool kept = have && rank < n3;
-  uint32_t irank = 0;  // rank by id among the kept items
-  if (kept)
-    for (uint32_t j = 0; j < n; ++j) irank += m.bins[j] < n3 && m.id[j] < id;
-  uint64_t mass3;
-  (void)block_excl_scan_u64(kept ? wq : 0, s, &mass3);
-  const double scale = (double)mass3 * 0x1p-44;
-  if (a.out_kept_ids && kept && irank < a.kept_cap) {
-    a.out_kept_ids[(uint64_t)row * a.kept_cap + irank] = id;
-    a.out_kept_probs[(uint64_t)row * a.kept_cap + irank] =
-        mass3 ? (float)((double)w / scale) : 0.0f;
-  }
-  if (mass3 == 0) {
-    if (t == 0) write_result(a, row, kNoToken, 0.0f, n3);
-    return;
-  }
-  const uint32_t draft = row_draft(a, rp);
-  const bool drafted = draft != kNoToken;
-  uint64_t d = kept ? wq : 0;
-  if (drafted) {
-    const uint64_t r = kept ? residual_of(wq, mass3, draft_q(a, rp, id, s)) : 0;
-    if (block_max_u32(r > 0 ? 1u : 0u, s)) d = r;
-  }
-  // The draw weights in id order, their running sum, the first past u.
-  __syncthreads();
-  if (kept) {
-    s.hist[irank] = d;
-    m.bins[256 + irank] = id;
-  }
-  if (t == 0) {
-    s.found_w = 0.0f;
-    s.hit = kNoToken;
-  }
-  __syncthreads();
-  const uint64_t dp = t < n3 ? s.hist[t] : 0;
-  uint64_t total;
-  const uint64_t excl = block_excl_scan_u64(dp, s, &total);
-  uint64_t target = floor_mul(total, row_uniform(a, row));
-  if (target >= total) target = total - 1;
-  if (t < n3 && excl <= target && excl + dp > target) s.hit = m.bins[256 + t];
-  if (drafted && kept && id == draft) s.found_w = w;
-  __syncthreads();
-  if (t == 0)
-    write_result(a, row, s.hit, drafted ? (float)((double)s.found_w / scale) : 0.0f,
-                 n3);
+__device__ __forceinline__ uint64_t item_weight(uint64_t item, float maximum, float inv_t) {
+  return quantized_weight(key_logit(item_key(item)), maximum, inv_t);
 }
 
 // Makes one wave's LDS writes visible to its own later LDS reads of other
@@ -992,376 +700,125 @@ __device__ __forceinline__ void wave_lds_sync() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
-// The last steps of a row with at most 64 items left (s.merge.key/id[0, n),
-// any order), run by one wave. Each item counts the items ahead of it in
-// (key desc, id asc) order, which gives the top-k cut and the walk of top-p
-// (sampling.metal:585-650); each kept item counts the kept items of lower
-// id, which gives the draw's order and the kept outputs
-// (sampling.metal:700-829).
-__device__ __forceinline__ void wave_merge(const SampleLaunch &a,
-                                           const RowParams &rp, uint32_t row,
-                                           Lds &s, uint32_t n, float maximum,
-                                           float u, uint32_t draft) {
-  MergeLds &m = s.merge;
-  uint64_t *A = s.hist;        // items as key:~id, arrival order
-  uint64_t *B = s.hist + 64;   // the same in rank order
-  uint64_t *D = s.hist + 128;  // draw weights in id order
-  uint32_t *E = m.bins;        // kept ids in rank order
-  uint32_t *F = m.bins + 128;  // kept ids in id order
-  const uint32_t lane = lane_id();
-  const bool have = lane < n;
-  // (key desc, id asc) is the descending order of key:~id.
-  const uint64_t c = have ? ((uint64_t)m.key[lane] << 32) | (uint32_t)~m.id[lane] : 0ull;
-  A[lane] = c;
-  wave_lds_sync();
-  // Lanes at or past n hold 0, which ranks after every item.
-  uint32_t rank = 0;
+// Wave 0 finds the highest of s.hist's (s.hcount's) 256 bins whose suffix sum
+// reaches T (the total does): s.sel_bin, and s.sel_excl the sum above it.
+template <class L>
+__device__ __forceinline__ void items_crossing_bin(L &s, uint64_t T, bool by_mass) {
+  if (threadIdx.x < 64) {
+    const uint32_t l = threadIdx.x;
+    uint64_t h[4];
 #pragma unroll
-  for (int j = 0; j < 64; j += 2) {
-    const uint64_t c0 = A[j], c1 = A[j + 1];
-    rank += (c0 > c ? 1u : 0u) + (c1 > c ? 1u : 0u);
-  }
-  if (have) B[rank] = c;
-  wave_lds_sync();
-  const uint64_t cr = have ? B[lane] : 0ull;
-  const uint32_t key = (uint32_t)(cr >> 32), id = ~(uint32_t)cr;
-  const uint32_t n2 = min(rp.top_k, n);
-  const bool in2 = lane < n2;
-  const float w = in2 ? weight_of(key_logit(key), maximum, rp.inv_t) : 0.0f;
-  const uint64_t wq = quantize(w);
-  uint32_t n3 = n2;
-  if (rp.flags & kRowTopP) {
-    const uint64_t incl = wave_incl_scan_u64(wq);
-    const uint64_t mass2 = readlane_u64(incl, 63);
-    if (mass2) {
-      const uint64_t nucleus = floor_mul(mass2, rp.top_p);
-      const uint64_t hm = ballot(in2 && incl - wq <= nucleus && incl > nucleus);
-      if (hm) n3 = (uint32_t)__builtin_ctzll(hm) + 1;
-    }
-  }
-  const bool kept = lane < n3;
-  const uint64_t mass3 = wave_sum_u64(kept ? wq : 0);
-  // Id order of the kept items: rank among the kept ids.
-  E[lane] = kept ? id : kNoToken;
-  wave_lds_sync();
-  uint32_t irank = 0;
+    for (int k = 0; k < 4; ++k) h[k] = by_mass ? s.hist[4 * l + k] : s.hcount[4 * l + k];
+    const uint64_t own = h[0] + h[1] + h[2] + h[3];
+    const uint64_t incl = wave_incl_scan_u64(own);
+    const uint64_t suf = readlane_u64(incl, 63) - (incl - own);
+    const uint64_t m = ballot(suf >= T);
+    const int top = m ? 63 - (int)__builtin_clzll(m) : 0;
+    if ((int)l == top) {
+      uint64_t acc = suf - own;
+      uint32_t k = 3;
 #pragma unroll
-  for (int q = 0; q < 64; q += 4) {
-    const uint4 e4 = *(const uint4 *)&E[q];
-    irank += (e4.x < id ? 1u : 0u) + (e4.y < id ? 1u : 0u) + (e4.z < id ? 1u : 0u) +
-             (e4.w < id ? 1u : 0u);
-  }
-  const double scale = (double)mass3 * 0x1p-44;
-  if (a.out_kept_ids && kept && irank < a.kept_cap) {
-    a.out_kept_ids[(uint64_t)row * a.kept_cap + irank] = id;
-    a.out_kept_probs[(uint64_t)row * a.kept_cap + irank] =
-        mass3 ? (float)((double)w / scale) : 0.0f;
-  }
-  if (mass3 == 0) {
-    if (lane == 0) write_result(a, row, kNoToken, 0.0f, n3);
-    return;
-  }
-  const bool drafted = draft != kNoToken;
-  uint64_t d = kept ? wq : 0;
-  if (drafted) {
-    const uint64_t r = kept ? residual_of(wq, mass3, draft_q(a, rp, id, s)) : 0;
-    if (ballot(r > 0)) d = r;
-  }
-  const uint64_t fm = ballot(drafted && kept && id == draft);
-  const float fw = u2f(readlane_u32(f2u(w), fm ? (int)__builtin_ctzll(fm) : 0));
-  if (kept) {
-    D[irank] = d;
-    F[irank] = id;
-  }
-  wave_lds_sync();
-  const uint64_t dd = kept ? D[lane] : 0ull;
-  const uint64_t incl = wave_incl_scan_u64(dd);
-  const uint64_t total = readlane_u64(incl, 63);
-  uint64_t target = floor_mul(total, u);
-  if (target >= total) target = total - 1;
-  const uint64_t hm = ballot(kept && incl - dd <= target && incl > target);
-  const uint32_t token = hm ? F[__builtin_ctzll(hm)] : kNoToken;
-  if (lane == 0)
-    write_result(a, row, token, drafted && fm ? (float)((double)fw / scale) : 0.0f, n3);
-}
-
-// The exact top-K (K <= 64) of the candidates at or above `thr` that the
-// block holds in registers (v[k] = item first + k, key in the low word, id
-// in the high word): a 1024-bin value histogram over [value(thr), maximum]
-// finds the bin where the count from the top reaches K, and that bin's
-// items are ranked exactly. The kept items (all of them when there are at
-// most K) are appended to s.merge.key/id; returns their number, or -1 when
-// the boundary bin holds more than kThreads items or the values do not
-// spread over the bins. The caller zeroed s.merge.bins before a barrier.
-template <int PER>
-__device__ __forceinline__ int fast_select(const uint64_t (&v)[PER],
-                                           uint32_t first, uint32_t n_all,
-                                           uint32_t thr, uint32_t K,
-                                           float maximum, Lds &s) {
-  MergeLds &m = s.merge;
-  const uint32_t tid = threadIdx.x;
-  const float lo = key_logit(thr);
-  const float scale = 1023.0f / (maximum - lo);
-  if (!(scale > 0.0f && scale < 3.0e38f)) return -1;
-  auto bin_of = [&](uint32_t key) -> uint32_t {
-    return min(1023u, (uint32_t)((key_logit(key) - lo) * scale));
-  };
-  if (tid == 0) {
-    s.u32a = 0;
-    s.nbound = 0;
-  }
-#pragma unroll
-  for (int k = 0; k < PER; ++k)
-    if (first + k < n_all && (uint32_t)v[k] >= thr)
-      atomicAdd(&m.bins[bin_of((uint32_t)v[k])], 1u);
-  __syncthreads();
-  uint32_t own = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) own += m.bins[4 * tid + k];
-  uint64_t total;
-  const uint32_t before = (uint32_t)block_excl_scan_u64(own, s, &total);
-  const uint32_t suffix = (uint32_t)total - before;  // bins >= 4 tid
-  const bool all = total <= K;
-  if (!all && suffix >= K && suffix - own < K) {
-    uint32_t acc = suffix - own;
-    uint32_t b = 4 * tid + 3;
-    for (int k = 3; k >= 0; --k) {
-      b = 4 * tid + k;
-      if (acc + m.bins[b] >= K) break;
-      acc += m.bins[b];
-    }
-    s.sel_bin = b;
-    s.sel_excl = acc;
-  }
-  __syncthreads();
-  const uint32_t bstar = all ? 0u : s.sel_bin;
-  const uint32_t need = all ? 0u : K - (uint32_t)s.sel_excl;
-  if (!all && m.bins[bstar] > (uint32_t)kThreads) return -1;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const uint32_t key = (uint32_t)v[k];
-    if (first + k >= n_all || key < thr) continue;
-    const uint32_t b = bin_of(key);
-    if (all || b > bstar) {
-      const uint32_t slot = atomicAdd(&s.u32a, 1u);
-      m.key[slot] = key;
-      m.id[slot] = (uint32_t)(v[k] >> 32);
-    } else if (b == bstar) {
-      s.hist[atomicAdd(&s.nbound, 1u)] = v[k];
-    }
-  }
-  __syncthreads();
-  const uint32_t nb = s.nbound;
-  if (tid < nb) {
-    const uint64_t me = s.hist[tid];
-    const uint32_t key = (uint32_t)me, id = (uint32_t)(me >> 32);
-    uint32_t rank = 0;
-    for (uint32_t j = 0; j < nb; ++j) {
-      const uint64_t o = s.hist[j];
-      const uint32_t ok = (uint32_t)o, oi = (uint32_t)(o >> 32);
-      rank += ok > key || (ok == key && oi < id);
-    }
-    if (rank < need) {
-      const uint32_t slot = atomicAdd(&s.u32a, 1u);
-      m.key[slot] = key;
-      m.id[slot] = id;
-    }
-  }
-  __syncthreads();
-  return (int)s.u32a;
-}
-
-// The exact top-K (K <= 64) candidates of a row held in registers (v[k] =
-// key | id << 32; bit k of `valid` set for a real item at or above the
-// floor): a 1024-bin
-// value histogram over [value(thr), maximum] locates the bin where the
-// count from the top reaches K (wave 0 finds it), and every item of that
-// bin and above goes to s.merge.key/id. Returns their number (then K plus
-// the boundary bin's other items, or all items when there are at most K),
-// or -1 when the values do not spread over the bins. The caller zeroed
-// s.merge.bins before a barrier.
-template <int PER>
-__device__ __forceinline__ int spec_select(const uint64_t (&v)[PER], uint32_t valid,
-                                           uint32_t thr, uint32_t K, float maximum,
-                                           Lds &s) {
-  MergeLds &m = s.merge;
-  const uint32_t tid = threadIdx.x;
-  const float lo = key_logit(thr);
-  const float scale = 1023.0f / (maximum - lo);
-  if (!(scale > 0.0f && scale < 3.0e38f)) return -1;
-  auto bin_of = [&](uint32_t key) -> uint32_t {
-    return min(1023u, (uint32_t)((key_logit(key) - lo) * scale));
-  };
-  if (tid == 0) s.u32a = 0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k)
-    if ((valid >> k) & 1) atomicAdd(&m.bins[bin_of((uint32_t)v[k])], 1u);
-  __syncthreads();
-  if (tid < 64) {
-    // Lane l owns bins 16 l .. 16 l + 15; the suffix count from the top.
-    uint32_t own = 0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) own += m.bins[16 * tid + k];
-    const uint32_t incl = wave_incl_scan_u32(own);
-    const uint32_t total = readlane_u32(incl, 63);
-    const uint32_t suffix = total - (incl - own);  // bins >= 16 l
-    if (total <= K) {
-      if (tid == 0) s.sel_bin = 0;
-    } else if (suffix >= K && suffix - own < K) {
-      uint32_t acc = suffix - own, b = 16 * tid + 15;
-      for (int k = 15; k >= 0; --k) {
-        b = 16 * tid + k;
-        if (acc + m.bins[b] >= K) break;
-        acc += m.bins[b];
-      }
-      s.sel_bin = b;
-    }
-  }
-  __syncthreads();
-  const uint32_t bstar = s.sel_bin;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    if (!((valid >> k) & 1)) continue;
-    const uint32_t key = (uint32_t)v[k];
-    if (bin_of(key) >= bstar) {
-      const uint32_t slot = atomicAdd(&s.u32a, 1u);
-      m.key[slot] = key;
-      m.id[slot] = (uint32_t)(v[k] >> 32);
-    }
-  }
-  __syncthreads();
-  return (int)s.u32a;
-}
-
-// Sorts the n items of s.merge by id (bitonic, padded to a power of two
-// with id kNoToken), so that the radix path sees them in id order.
-__device__ __forceinline__ void lds_sort_by_id(Lds &s, uint32_t n) {
-  MergeLds &m = s.merge;
-  uint32_t P = 1;
-  while (P < n) P <<= 1;
-  for (uint32_t i = n + threadIdx.x; i < P; i += kThreads) {
-    m.key[i] = 0;
-    m.id[i] = kNoToken;
-  }
-  __syncthreads();
-  for (uint32_t size = 2; size <= P; size <<= 1)
-    for (uint32_t stride = size >> 1; stride; stride >>= 1) {
-      for (uint32_t i = threadIdx.x; i < P / 2; i += kThreads) {
-        const uint32_t lo = 2 * stride * (i / stride) + (i % stride);
-        const uint32_t hi = lo + stride;
-        const bool ascending = (lo & size) == 0;
-        const uint32_t a = m.id[lo], b = m.id[hi];
-        if ((a > b) == ascending) {
-          m.id[lo] = b;
-          m.id[hi] = a;
-          const uint32_t k = m.key[lo];
-          m.key[lo] = m.key[hi];
-          m.key[hi] = k;
+      for (int j = 3; j > 0; --j)
+        if ((int)k == j && acc + h[j] < T) {
+          acc += h[j];
+          k = (uint32_t)j - 1u;
         }
-      }
-      __syncthreads();
+      s.sel_bin = 4 * l + k;
+      s.sel_excl = acc;
     }
-  for (uint32_t i = threadIdx.x; i < n; i += kThreads) m.fl[i] = 1;
+  }
   __syncthreads();
 }
 
-// Keeps the first K of the n compacted items (id order in s.merge) in
-// (key desc, id asc) order, compacted in id order, when K <= kThreads: a
-// 1024-bin histogram of the values between the items' least value and the
-// row maximum finds the bin of the K-th item, whose few items are ranked
-// exactly. Returns false, changing nothing, when the values do not spread
-// over the bins (the caller then takes the radix path).
-__device__ __forceinline__ bool hist_select(Lds &s, uint32_t &n, uint32_t K,
-                                            float maximum) {
-  MergeLds &m = s.merge;
-  constexpr int PER = kMergeCapacity / kThreads;
-  const uint32_t tid = threadIdx.x;
-  uint32_t kmin = 0xffffffffu;
-  for (uint32_t i = tid; i < n; i += kThreads) kmin = min(kmin, m.key[i]);
-  kmin = block_min_u32(kmin, s);
-  const float lo = key_logit(kmin);
-  const float scale = 1023.0f / (maximum - lo);
-  if (!(scale > 0.0f && scale < 3.0e38f) || kmin <= kLowestKey) return false;
-  for (uint32_t b = tid; b < 1024; b += kThreads) m.bins[b] = 0;
-  if (tid == 0) s.u32a = 0;
-  __syncthreads();
-  auto bin_of = [&](uint32_t key) -> uint32_t {
-    const float v = (key_logit(key) - lo) * scale;
-    return min(1023u, (uint32_t)v);
+// The order word (`ord(item)`, distinct) at which the running count (or, by
+// mass, the running sum of `val(item)`) of the items that `in` takes, largest
+// order word first, reaches `target` (which it does): a radix descent by up to
+// 8 bits a pass from the highest bit in which they differ, until the bin holds
+// at most a wave's worth, which one wave ranks. `each(f)` calls f(item) for
+// every item, each thread its own. Every thread of the block calls it. About
+// 1.5 us a pass over a few items a thread: two block-wide LDS passes instead
+// of the sort a merge of these items took (45 us at 256 rows, one of them
+// with 300 tokens past its min-p floor).
+template <class Each, class In, class Ord, class Val, class L>
+__device__ __forceinline__ uint64_t items_crossing(Each each, In in, Ord ord, Val val,
+                                                   bool by_mass, uint64_t target, L &s) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  uint64_t any1 = 0, any0 = 0;  // bits set in some word, clear in some word
+  each([&](uint64_t c) {
+    if (in(c)) {
+      any1 |= ord(c);
+      any0 |= ~ord(c);
+    }
+  });
+  auto wave_or = [](uint64_t v) {
+    v |= xor_u64<1>(v);
+    v |= xor_u64<2>(v);
+    v |= xor_u64<4>(v);
+    v |= xor_u64<8>(v);
+    v |= xor_u64<16>(v);
+    v |= xor_u64<32>(v);
+    return v;
   };
-  for (uint32_t i = tid; i < n; i += kThreads) atomicAdd(&m.bins[bin_of(m.key[i])], 1u);
+  any1 = wave_or(any1);
+  any0 = wave_or(any0);
   __syncthreads();
-  // The highest bin whose suffix count reaches K.
-  uint32_t own = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) own += m.bins[4 * tid + k];
-  uint64_t total;
-  const uint32_t before = (uint32_t)block_excl_scan_u64(own, s, &total);
-  const uint32_t suffix = (uint32_t)total - before;  // bins >= 4 tid
-  if (suffix >= K && suffix - own < K) {
-    uint32_t acc = suffix - own;
-    uint32_t b = 4 * tid + 3;
-    for (int k = 3; k >= 0; --k) {
-      b = 4 * tid + k;
-      if (acc + m.bins[b] >= K) break;
-      acc += m.bins[b];
-    }
-    s.sel_bin = b;
-    s.sel_excl = acc;
+  if (lane == 0) {
+    s.wl[w] = any1;
+    s.wl2[w] = any0;
   }
   __syncthreads();
-  const uint32_t bstar = s.sel_bin;
-  const uint32_t need = K - (uint32_t)s.sel_excl;
-  if (m.bins[bstar] > (uint32_t)kThreads) return false;
-  // The items of the boundary bin, ranked exactly.
-  for (uint32_t i = tid; i < n; i += kThreads) {
-    const uint32_t b = bin_of(m.key[i]);
-    m.fl[i] = b > bstar ? 1 : 0;
-    if (b == bstar) {
-      const uint32_t slot = atomicAdd(&s.u32a, 1u);
-      s.hist[slot] = ((uint64_t)m.key[i] << 32) | i;
-    }
+  any1 = s.wl[0] | s.wl[1] | s.wl[2] | s.wl[3];
+  any0 = s.wl2[0] | s.wl2[1] | s.wl2[2] | s.wl2[3];
+  const uint64_t differ = any1 & any0;
+  const int bits = differ ? 64 - (int)__builtin_clzll(differ) : 1;  // low bits not yet fixed
+  int width = min(bits, 8), shift = bits - width;
+  uint64_t prefix = any1 >> bits;  // the bits above agree
+  for (;;) {
+    const uint32_t mask = (1u << width) - 1u;
+    s.hist[tid] = 0;
+    s.hcount[tid] = 0;
+    __syncthreads();
+    each([&](uint64_t c) {
+      if (in(c) && (ord(c) >> (shift + width)) == prefix) {
+        const uint32_t d = (uint32_t)(ord(c) >> shift) & mask;
+        atomicAdd(&s.hcount[d], 1u);
+        if (by_mass) atomicAdd((unsigned long long *)&s.hist[d], (unsigned long long)val(c));
+      }
+    });
+    __syncthreads();
+    items_crossing_bin(s, target, by_mass);
+    target -= s.sel_excl;
+    prefix = (prefix << width) | s.sel_bin;
+    const uint32_t n = s.hcount[s.sel_bin];
+    if (n <= 64u || shift == 0) break;
+    width = min(shift, 8);
+    shift -= width;
+    __syncthreads();
   }
   __syncthreads();
-  const uint32_t nb = s.u32a;
-  if (tid < nb) {
-    const uint64_t me = s.hist[tid];
-    const uint32_t key = (uint32_t)(me >> 32), pos = (uint32_t)me;
+  if (tid == 0) s.small_n = 0;
+  __syncthreads();
+  each([&](uint64_t c) {
+    if (in(c) && (ord(c) >> shift) == prefix) s.small[atomicAdd(&s.small_n, 1u) & 63u] = c;
+  });
+  __syncthreads();
+  if (w == 0) {
+    const uint32_t n = min(s.small_n, 64u);
+    const uint64_t c = lane < n ? s.small[lane] : 0ull;
     uint32_t rank = 0;
-    for (uint32_t j = 0; j < nb; ++j) {
-      const uint64_t o = s.hist[j];
-      const uint32_t ok = (uint32_t)(o >> 32), op = (uint32_t)o;
-      rank += ok > key || (ok == key && m.id[op] < m.id[pos]);
-    }
-    if (rank < need) m.fl[pos] = 1;
+    for (uint32_t j = 0; j < n; ++j) rank += ord(s.small[j]) > ord(c) ? 1u : 0u;
+    if (lane < n) s.sorted[rank] = c;
+    wave_lds_sync();
+    const uint64_t o = lane < n ? s.sorted[lane] : 0ull;
+    const uint64_t v = lane >= n ? 0ull : by_mass ? val(o) : 1ull;
+    const uint64_t reached = ballot(lane < n && wave_incl_scan_u64(v) >= target);
+    if ((int)lane == (reached ? (int)__builtin_ctzll(reached) : (int)n - 1)) s.u64a = ord(o);
   }
   __syncthreads();
-  // Ordered compaction of the kept items.
-  uint32_t kk[PER], ki[PER];
-  uint32_t cnt = 0;
-  const uint32_t first = tid * PER;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const uint32_t i = first + k;
-    const bool keep = i < n && m.fl[i];
-    kk[k] = keep ? m.key[i] : 0u;
-    ki[k] = keep ? m.id[i] : kNoToken;
-    cnt += keep;
-  }
-  uint64_t kept;
-  uint32_t out = (uint32_t)block_excl_scan_u64(cnt, s, &kept);
-#pragma unroll
-  for (int k = 0; k < PER; ++k)
-    if (ki[k] != kNoToken) {
-      m.key[out] = kk[k];
-      m.id[out] = ki[k];
-      m.fl[out] = 1;
-      ++out;
-    }
-  n = (uint32_t)kept;
-  __syncthreads();
-  return true;
+  return s.u64a;
 }
+
+// ---- the merge of a sampled row ------------------------------------------
 
 // A chunk whose candidates overflowed its list, selected again by the
 // merge with the row's threshold `thr`: its tokens at or above it or, when
@@ -1472,89 +929,124 @@ __device__ __forceinline__ uint32_t reselect_chunk(const SampleLaunch &a,
   return n;
 }
 
+// The last steps of a row with at most 64 items left, s.merge.key/id[0, n)
+// in (key desc, id asc) order (rank_select), by one wave in registers. Rank
+// order gives the top-k cut and the walk of top-p (sampling.metal:585-650);
+// sorting the kept items by id gives the draw's order and the kept outputs
+// (sampling.metal:700-829). DENSE: a drafted row may read a dense q.
+template <bool DENSE = false>
+__device__ __forceinline__ void wave_finish(const SampleLaunch &a, const RowParams &rp,
+                                            uint32_t row, const Lds &s, uint32_t n,
+                                            float maximum, float u, uint32_t draft) {
+  const MergeLds &m = s.merge;
+  const uint32_t lane = lane_id();
+  const uint32_t key = lane < n ? m.key[lane] : 0u;
+  const uint32_t id = lane < n ? m.id[lane] : kNoToken;
+  const uint32_t n2 = min(rp.top_k, n);
+  const bool in2 = lane < n2;
+  const float w = in2 ? weight_of(key_logit(key), maximum, rp.inv_t) : 0.0f;
+  const uint64_t wq = quantize(w);
+  uint32_t n3 = n2;
+  if (rp.flags & kRowTopP) {
+    const uint64_t incl = wave_incl_scan_u64(wq);
+    const uint64_t mass2 = readlane_u64(incl, 63);
+    if (mass2) {
+      const uint64_t nucleus = floor_mul(mass2, rp.top_p);
+      const uint64_t hm = ballot(in2 && incl - wq <= nucleus && incl > nucleus);
+      if (hm) n3 = (uint32_t)__builtin_ctzll(hm) + 1;
+    }
+  }
+  const bool kept = lane < n3;
+  const uint64_t mass3 = wave_sum_u64(kept ? wq : 0);
+  const double scale = (double)mass3 * 0x1p-44;
+  const bool drafted = draft != kNoToken;
+  uint64_t d = kept ? wq : 0;
+  if (drafted) {
+    float q = 0.0f;
+    if constexpr (DENSE)
+      q = kept ? draft_q(a, rp, id, s) : 0.0f;
+    else
+      for (int j = 15; j >= 0; --j) q = s.cids[j] == id ? s.cprobs[j] : q;
+    const uint64_t r = kept ? residual_of(wq, mass3, q) : 0;
+    if (ballot(r > 0)) d = r;
+  }
+  const uint64_t fm = ballot(drafted && kept && id == draft);
+  const float fw = u2f(readlane_u32(f2u(w), fm ? (int)__builtin_ctzll(fm) : 0));
+  // Id order of the kept items, each carrying the lane of its rank (ids are
+  // below 2^19, so id and lane share 32 bits).
+  uint32_t e = kept ? (id << 6) | lane : 0xffffffffu;
+  e = wave_sort_asc_u32(e);
+  const uint32_t src = e & 63u, iid = e >> 6;
+  const uint64_t dq = shfl_u64(d, (int)src);
+  const float wi = __shfl(w, (int)src, kWave);
+  if (a.out_kept_ids && kept && lane < a.kept_cap) {
+    a.out_kept_ids[(uint64_t)row * a.kept_cap + lane] = iid;
+    a.out_kept_probs[(uint64_t)row * a.kept_cap + lane] =
+        mass3 ? (float)((double)wi / scale) : 0.0f;
+  }
+  if (mass3 == 0) {
+    if (lane == 0) write_result(a, row, kNoToken, 0.0f, n3);
+    return;
+  }
+  const uint64_t dd = kept ? dq : 0ull;
+  const uint64_t incl = wave_incl_scan_u64(dd);
+  const uint64_t total = readlane_u64(incl, 63);
+  uint64_t target = floor_mul(total, u);
+  if (target >= total) target = total - 1;
+  const uint64_t hm = ballot(kept && incl - dd <= target && incl > target);
+  const uint32_t token = hm ? readlane_u32(iid, (int)__builtin_ctzll(hm)) : kNoToken;
+  if (lane == 0)
+    write_result(a, row, token, drafted && fm ? (float)((double)fw / scale) : 0.0f, n3);
+}
+
+// A sampled row from its candidate lists, whatever they hold: the tokens at or
+// above its threshold as items in LDS, the top-k and top-p boundaries by
+// items_crossing, and the draw by items_crossing over the ids. A min-p row
+// with more such tokens than LDS takes (and a top-k past the lists) goes on to
+// the cut passes.
 template <int DT>
 __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowParams &rp,
                               uint32_t row, Lds &s) {
-  const uint32_t S = a.chunks, tid = threadIdx.x;
+  const uint32_t S = a.chunks, tid = threadIdx.x, lane = tid & 63;
   const BlockHeader *hb = a.headers + (uint64_t)row * S;
-  // Everything the row needs from memory is requested up front: the chunk
-  // summaries (one lane each, S <= 64), the uniform, the draft token and its
-  // sparse candidates. The select kernel's writes are visible here because
-  // it ended before this launch began.
+  const uint64_t *lists = a.cands + (uint64_t)row * S * kBlockCandidates;
   const float u = row_uniform(a, row);
   const uint32_t draft = row_draft(a, rp);
-  // Rows with a small top-k also fetch the first P slots of every chunk's
-  // candidate list now, before the counts are known (S * P <= SPEC items).
-  constexpr int SPEC = 10;
   const uint32_t K = rp.top_k;
-  const uint32_t P = S <= 20 ? 128u : (S <= 40 ? 64u : 32u);
-  const uint32_t pshift = S <= 20 ? 7u : (S <= 40 ? 6u : 5u);
-  const bool spec = (rp.flags & kRowTopK) && K <= 64u;
-  uint64_t sv[SPEC];
-#pragma unroll
-  for (int k = 0; k < SPEC; ++k) {
-    const uint32_t i = tid + k * kThreads, c = i >> pshift;
-    sv[k] = 0;
-    if (spec && c < S)
-      sv[k] = a.cands[((uint64_t)row * S + c) * kBlockCandidates + (i & (P - 1))];
-  }
-  for (uint32_t b = tid; b < 1024; b += kThreads) s.merge.bins[b] = 0;
-  if (tid < 16) {
-    const bool sparse = !a.dense_q && draft != kNoToken;
-    s.cids[tid] = sparse ? a.cand_ids[(uint64_t)rp.cand_index * 16 + tid] : kNoToken;
-    s.cprobs[tid] = sparse ? a.cand_probs[(uint64_t)rp.cand_index * 16 + tid] : 0.0f;
-  }
+  stage_candidates(a, rp, s);
   if (tid < 64) {
-    float hm = -3.402823466e38f;
-    uint32_t hc = 0, ha = 0, ho = 0, hf = 0;
-    if (tid < S) {
-      const BlockHeader h = hb[tid];
-      hm = h.maximum;
-      hc = h.count;
-      ha = h.admitted;
-      ho = h.overflow;
-      hf = h.floor_key;
+    const bool in = lane < S;
+    const BlockHeader h = hb[min(lane, S - 1)];
+    const float mx = wave_max_f32(in ? h.maximum : -3.402823466e38f);
+    const uint32_t adm = wave_max_u32(in ? h.admitted : 0u),
+                   flr = wave_max_u32(in ? h.floor_key : 0u);
+    const uint64_t omask = ballot(in && h.overflow != 0);
+    if (in) {
+      s.hcnt[lane] = h.count;
+      s.hmax[lane] = h.maximum;
     }
-    const float mx = wave_max_f32(hm);
-    const uint32_t adm = wave_sum_u32(ha), ovf = wave_max_u32(ho),
-                   flr = wave_max_u32(hf), hcmax = wave_max_u32(hc);
-    const uint32_t incl = wave_incl_scan_u32(hc);
-    const uint64_t omask = ballot(ho != 0);
-    if (tid < S) {
-      s.hoff[tid + 1] = incl;
-      s.hcnt[tid] = hc;
-      s.hmax[tid] = hm;
-    }
-    if (tid == 0) {
+    if (lane == 0) {
       s.u64a = omask;
-      s.hoff[0] = 0;
       s.row_max = mx;
       s.row_admitted = adm;
-      s.row_overflow = ovf;
       s.row_floor = flr;
-      s.row_maxcount = hcmax;
     }
   }
   __syncthreads();
-  const float maximum = s.row_max;
-  const uint32_t admitted = s.row_admitted, overflow = s.row_overflow;
-  // The K-th key of the row is at least every block's floor.
-  const uint32_t floor_key = s.row_floor;
-  if (admitted == 0 || maximum == __builtin_inff()) {
-    if (tid == 0) {
-      write_result(a, row, kNoToken, 0.0f, 0);
-      a.states[row].stage = kRowDone;
-    }
+  const float M = s.row_max, inv_t = rp.inv_t;
+  if (s.row_admitted == 0 || M == __builtin_inff()) {
+    if (tid == 0) write_result(a, row, kNoToken, 0.0f, 0);
     return;
   }
-  uint32_t thr = (rp.flags & kRowMinP)
-                     ? logit_key(__builtin_fminf(maximum + rp.minp_offset, maximum))
-                     : 0u;
-  if (rp.flags & kRowTopK) thr = max(thr, floor_key);
+  // The K-th key of the row is at least every chunk's floor.
+  uint32_t thr =
+      (rp.flags & kRowMinP) ? logit_key(__builtin_fminf(M + rp.minp_offset, M)) : 0u;
+  if (rp.flags & kRowTopK) thr = max(thr, s.row_floor);
+  uint64_t om = s.u64a;
+  const bool overflow = om != 0;
   if (overflow && K <= (uint32_t)kBlockCandidates) {
-    // Chunks with more candidates than their lists hold (rare: flat or
-    // tied values): select each again, then recount.
-    uint64_t om = s.u64a;
+    // Chunks with more candidates than their lists hold (flat or tied
+    // values): select each again.
     while (om) {
       const uint32_t c = (uint32_t)__builtin_ctzll(om);
       om &= om - 1;
@@ -1562,191 +1054,188 @@ __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowPa
       if (tid == 0) s.hcnt[c] = n;
     }
     __syncthreads();
-    if (tid < 64) {
-      const uint32_t incl = wave_incl_scan_u32(tid < S ? s.hcnt[tid] : 0u);
-      if (tid < S) s.hoff[tid + 1] = incl;
-    }
-    for (uint32_t b = tid; b < 1024; b += kThreads) s.merge.bins[b] = 0;
-    __syncthreads();
   }
-  // A chunk whose maximum is below the threshold holds no item at or above
-  // it: the offsets skip its list (every use below wants only such items).
-  if (thr > kLowestKey) {
-    if (tid < 64) {
-      const bool use = tid < S && logit_key(s.hmax[tid]) >= thr;
-      const uint32_t incl = wave_incl_scan_u32(use ? s.hcnt[tid] : 0u);
-      if (tid < S) s.hoff[tid + 1] = incl;
+  // The lists of the chunks whose maximum reaches the threshold, end to end.
+  if (tid < 64) {
+    const bool use = lane < S && logit_key(s.hmax[lane]) >= thr;
+    const uint32_t incl = wave_incl_scan_u32(use ? s.hcnt[lane] : 0u);
+    if (lane < S) s.hoff[lane + 1] = incl;
+    if (lane == 0) {
+      s.hoff[0] = 0;
+      s.n = 0;
     }
-    __syncthreads();
   }
+  __syncthreads();
   const uint32_t n_all = s.hoff[S];
-  const bool fits = n_all <= (uint32_t)kMergeCapacity;
-  if ((overflow && K > (uint32_t)kBlockCandidates) ||
-      (!fits && K > (uint32_t)kMergeCapacity)) {
-    // A min-p floor that leaves more tokens than the lists hold.
+  if (K > (uint32_t)kBlockCandidates && (overflow || n_all > kMergeItems)) {
     if (tid == 0) a.states[row].stage = kRowWide;
     return;
   }
-  if (tid == 0) a.states[row].stage = kRowDone;
-  MergeLds &m = s.merge;
-  uint32_t n;
-  if (spec && !overflow && s.row_maxcount <= P && thr > kLowestKey) {
-    // Every list fits in the slots fetched up front: the items at or above
-    // the floor, selected straight from registers.
-    uint32_t valid = 0;
-#pragma unroll
-    for (int k = 0; k < SPEC; ++k) {
-      const uint32_t i = tid + k * kThreads, c = i >> pshift;
-      if (c < S && (i & (P - 1)) < s.hcnt[c] && (uint32_t)sv[k] >= thr) valid |= 1u << k;
-    }
-    const int got = spec_select(sv, valid, thr, K, maximum, s);
-    if (got >= 0) {
-      // At most K items and the boundary bin's: usually 64 or fewer.
-      n = (uint32_t)got;
-      if (n > 64u && !hist_select(s, n, K, maximum)) {
-        lds_sort_by_id(s, n);
-        lds_topk(s, n, K);
-        if (rp.flags & kRowTopP) lds_topp(s, n, maximum, rp.inv_t, rp.top_p);
-        lds_draw(a, rp, row, s, n, maximum, rp.inv_t);
-        return;
-      }
-      if (tid < 64) wave_merge(a, rp, row, s, n, maximum, u, draft);
-      return;
-    }
-  }
-  if (fits) {
-    // Candidates at or above the floor into LDS: every load issued first,
-    // contiguous items per thread, then a compaction.
-    constexpr int PER = kMergeCapacity / kThreads;
-    uint64_t v[PER];
-    const uint32_t first = tid * PER;
+  // (A lambda's own copy of what it reads: a captured reference to LDS would
+  // go through memory.)
+  ItemsLds &g = s.general;
+  auto listed = [&](uint32_t i) -> uint64_t {
     uint32_t c = 0;
     for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
-      if (c + step < S && s.hoff[c + step] <= first) c += step;
-    uint32_t cnt = 0;
+      if (c + step < S && s.hoff[c + step] <= i) c += step;
+    return lists[(uint64_t)c * kBlockCandidates + (i - s.hoff[c])];
+  };
+  // The items at or above `thr` whose word reaches `from`, into LDS; those
+  // past its room are counted only.
+  auto gather = [&](uint64_t from) {
+    constexpr uint32_t B = 4;
+    for (uint32_t i0 = tid; i0 < n_all; i0 += B * kThreads) {
+      uint64_t v[B];
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const uint32_t i = first + k;
-      v[k] = 0;
-      if (i < n_all) {
-        while (s.hoff[c + 1] <= i) ++c;
-        v[k] = a.cands[((uint64_t)row * S + c) * kBlockCandidates + (i - s.hoff[c])];
+      for (uint32_t k = 0; k < B; ++k)
+        v[k] = i0 + k * kThreads < n_all ? listed(i0 + k * kThreads) : 0ull;
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k) {
+        const uint64_t c = token_item((uint32_t)v[k], (uint32_t)(v[k] >> 32));
+        if (i0 + k * kThreads < n_all && (uint32_t)v[k] >= thr && c >= from) {
+          const uint32_t at = atomicAdd(&s.n, 1u);
+          if (at < kMergeItems) g.items[at] = c;
+        }
       }
     }
-    if (K <= 64u && thr > kLowestKey) {
-      const int kept = fast_select(v, first, n_all, thr, K, maximum, s);
-      if (kept >= 0) {
-        if (tid < 64) wave_merge(a, rp, row, s, (uint32_t)kept, maximum, u, draft);
-        return;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < PER; ++k)
-      cnt += (first + k < n_all) && (uint32_t)v[k] >= thr;
-    uint64_t total;
-    uint32_t out = (uint32_t)block_excl_scan_u64(cnt, s, &total);
-#pragma unroll
-    for (int k = 0; k < PER; ++k)
-      if (first + k < n_all && (uint32_t)v[k] >= thr) {
-        m.key[out] = (uint32_t)v[k];
-        m.id[out] = (uint32_t)(v[k] >> 32);
-        m.fl[out] = 1;
-        ++out;
-      }
-    n = (uint32_t)total;
     __syncthreads();
-  } else {
-    // More candidates than LDS holds (K fits): select the first K at or
-    // above the floor straight from the lists (keys by radix descent, then
-    // the lowest ids among the ties), then append them to LDS.
-    auto item = [&](uint32_t i) -> uint64_t {
-      uint32_t c = 0;
-      for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
-        if (c + step < S && s.hoff[c + step] <= i) c += step;
-      return a.cands[((uint64_t)row * S + c) * kBlockCandidates + (i - s.hoff[c])];
+  };
+  auto ord = [](uint64_t c) { return c; };
+  auto weight = [&](uint64_t c) { return item_weight(c, M, inv_t); };
+  gather(0);
+  uint32_t n = s.n;
+  uint64_t bound = 0;  // the kept set's last item
+  if (n > kMergeItems) {
+    // (K fits.) The K-th item straight from the lists.
+    auto all = [&](auto f) {
+      for (uint32_t i = tid; i < n_all; i += kThreads) {
+        const uint64_t v = listed(i);
+        if ((uint32_t)v >= thr) f(token_item((uint32_t)v, (uint32_t)(v >> 32)));
+      }
     };
-    uint32_t c1 = 0;
-    for (uint32_t i = tid; i < n_all; i += kThreads) c1 += (uint32_t)item(i) >= thr;
-    const uint32_t n1 = block_sum_u32(c1, s);
-    uint32_t kap = 0, iota = kNoToken;  // keep key > kap, or key == kap and id <= iota
-    if (K < n1) {
-      uint32_t prefix = 0, pmask = 0;
-      uint64_t need = K;
-      for (int d = 3; d >= 0; --d) {
-        s.hist[tid] = 0;
-        __syncthreads();
-        for (uint32_t i = tid; i < n_all; i += kThreads) {
-          const uint32_t k = (uint32_t)item(i);
-          if (k >= thr && (k & pmask) == prefix)
-            atomicAdd((unsigned long long *)&s.hist[(k >> (8 * d)) & 255u], 1ull);
-        }
-        __syncthreads();
-        crossing_bin(s, need);
-        need -= s.sel_excl;
-        prefix |= s.sel_bin << (8 * d);
-        pmask |= 255u << (8 * d);
-        __syncthreads();
+    bound = items_crossing(all, [](uint64_t) { return true; }, ord, weight, false, K, s);
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+    gather(bound);
+    n = s.n;
+  }
+  auto each = [&](auto f) {
+    for (uint32_t i = tid; i < n; i += kThreads) f(g.items[i]);
+  };
+  if (K < n)
+    bound = items_crossing(each, [](uint64_t) { return true; }, ord, weight, false, K, s);
+  const uint32_t n2 = min(K, n);
+  if (n2 <= 64u) {
+    // One wave: the items ranked, then wave_finish.
+    if (tid == 0) s.small_n = 0;
+    __syncthreads();
+    each([&](uint64_t c) {
+      if (c >= bound) s.small[atomicAdd(&s.small_n, 1u) & 63u] = c;
+    });
+    __syncthreads();  // the items' area becomes the ranked keys'
+    if (tid < 64) {
+      const uint64_t c = lane < n2 ? s.small[lane] : 0ull;
+      uint32_t rank = 0;
+      for (uint32_t j = 0; j < n2; ++j) rank += s.small[j] > c ? 1u : 0u;
+      if (lane < n2) {
+        s.merge.key[rank] = item_key(c);
+        s.merge.id[rank] = item_id(c);
       }
-      kap = prefix;
-      // The need-th smallest id among the ties: the need-th largest of
-      // 0xffffff - id, by descent over its three bytes.
-      uint32_t ip = 0, im = 0;
-      for (int d = 2; d >= 0; --d) {
-        s.hist[tid] = 0;
-        __syncthreads();
-        for (uint32_t i = tid; i < n_all; i += kThreads) {
-          const uint64_t v = item(i);
-          if ((uint32_t)v != kap) continue;
-          const uint32_t ri = 0xffffffu - (uint32_t)(v >> 32);
-          if ((ri & im) == ip)
-            atomicAdd((unsigned long long *)&s.hist[(ri >> (8 * d)) & 255u], 1ull);
-        }
-        __syncthreads();
-        crossing_bin(s, need);
-        need -= s.sel_excl;
-        ip |= s.sel_bin << (8 * d);
-        im |= 255u << (8 * d);
-        __syncthreads();
-      }
-      iota = 0xffffffu - ip;
+      wave_lds_sync();
+      if (a.dense_q)
+        wave_finish<true>(a, rp, row, s, n2, M, u, draft);
+      else
+        wave_finish<false>(a, rp, row, s, n2, M, u, draft);
     }
-    if (tid == 0) s.u32a = 0;
+    return;
+  }
+  // Top-p (sampling.metal:615-641): in order until the running mass exceeds
+  // floor(top_p * mass).
+  if (rp.flags & kRowTopP) {
+    uint64_t m = 0;
+    each([&](uint64_t c) { m += c >= bound ? weight(c) : 0ull; });
+    const uint64_t mass2 = block_sum_u64(m, s);
+    if (mass2) {
+      const uint64_t kth = bound;
+      bound = items_crossing(each, [&](uint64_t c) { return c >= kth; }, ord, weight, true,
+                             floor_mul(mass2, rp.top_p) + 1, s);
+    }
+  }
+  uint64_t m3 = 0;
+  uint32_t k3 = 0;
+  each([&](uint64_t c) {
+    m3 += c >= bound ? weight(c) : 0ull;
+    k3 += c >= bound ? 1u : 0u;
+  });
+  const uint64_t mass3 = block_sum_u64(m3, s);
+  const uint32_t kept = (uint32_t)block_sum_u64(k3, s);
+  const double scale = (double)mass3 * 0x1p-44;
+  if (a.out_kept_ids) {
+    // The kept items in id order: grouped by id >> 9 (their counts' prefix
+    // sums), then ranked within their group.
+    for (uint32_t b = tid; b < 1024; b += kThreads) g.bins[b] = 0;
     __syncthreads();
-    for (uint32_t i = tid; i < n_all; i += kThreads) {
-      const uint64_t v = item(i);
-      const uint32_t k = (uint32_t)v, id = (uint32_t)(v >> 32);
-      if (k < thr) continue;
-      if (k > kap || (k == kap && id <= iota)) {
-        const uint32_t slot = atomicAdd(&s.u32a, 1u);
-        m.key[slot] = k;
-        m.id[slot] = id;
-        m.fl[slot] = 1;
+    each([&](uint64_t c) {
+      if (c >= bound) atomicAdd(&g.bins[item_id(c) >> 9], 1u);
+    });
+    __syncthreads();
+    const uint4 b4 = *(const uint4 *)&g.bins[4 * tid];
+    const uint32_t e0 =
+        (uint32_t)block_excl_scan_u64(b4.x + b4.y + b4.z + b4.w, s, nullptr);
+    *(uint4 *)&g.bins[4 * tid] = make_uint4(e0, e0 + b4.x, e0 + b4.x + b4.y,
+                                            e0 + b4.x + b4.y + b4.z);
+    __syncthreads();
+    each([&](uint64_t c) {
+      if (c >= bound) g.grouped[atomicAdd(&g.bins[item_id(c) >> 9], 1u)] = c;
+    });
+    __syncthreads();
+    // (Each bin now holds its group's end, the next one's start.)
+    for (uint32_t i = tid; i < kept; i += kThreads) {
+      const uint64_t c = g.grouped[i];
+      const uint32_t id = item_id(c), b = id >> 9, start = b ? g.bins[b - 1] : 0u;
+      uint32_t rank = start;
+      for (uint32_t j = start; j < g.bins[b]; ++j) rank += item_id(g.grouped[j]) < id ? 1u : 0u;
+      if (rank < a.kept_cap) {
+        a.out_kept_ids[(uint64_t)row * a.kept_cap + rank] = id;
+        a.out_kept_probs[(uint64_t)row * a.kept_cap + rank] =
+            mass3 ? (float)((double)weight_of(key_logit(item_key(c)), M, inv_t) / scale) : 0.0f;
       }
     }
+  }
+  if (mass3 == 0) {
+    if (tid == 0) write_result(a, row, kNoToken, 0.0f, kept);
+    return;
+  }
+  // The draw in id order (sampling.metal:694-829): the first item whose
+  // running weight, residual for a drafted row, passes the target.
+  const bool drafted = draft != kNoToken;
+  uint64_t total = mass3;
+  bool residual = false;
+  auto left = [&](uint64_t c) {
+    return residual_of(weight(c), mass3, draft_q(a, rp, item_id(c), s));
+  };
+  if (drafted) {
+    if (tid == 0) s.found_w = 0.0f;
     __syncthreads();
-    n = s.u32a;
-    __syncthreads();
+    uint64_t d = 0;
+    each([&](uint64_t c) {
+      if (c < bound) return;
+      d += left(c);
+      if (item_id(c) == draft) s.found_w = weight_of(key_logit(item_key(c)), M, inv_t);
+    });
+    d = block_sum_u64(d, s);
+    residual = d != 0;
+    if (residual) total = d;
   }
-  if (K <= 64u && K < n && hist_select(s, n, K, maximum)) {
-    if (tid < 64) wave_merge(a, rp, row, s, n, maximum, u, draft);
-    return;
-  }
-  if (n <= 64u) {
-    if (tid < 64) wave_merge(a, rp, row, s, n, maximum, u, draft);
-    return;
-  }
-  if (n <= (uint32_t)kThreads) {
-    small_merge(a, rp, row, s, n, maximum);
-    return;
-  }
-  if (K <= (uint32_t)kThreads && hist_select(s, n, K, maximum)) {
-    small_merge(a, rp, row, s, n, maximum);
-    return;
-  }
-  lds_sort_by_id(s, n);
-  if (K < n) lds_topk(s, n, K);
-  if (rp.flags & kRowTopP) lds_topp(s, n, maximum, rp.inv_t, rp.top_p);
-  lds_draw(a, rp, row, s, n, maximum, rp.inv_t);
+  uint64_t target = floor_mul(total, u);
+  if (target >= total) target = total - 1;
+  auto by_id = [](uint64_t c) { return c & 0x7ffffull; };  // lower ids are larger
+  auto in = [&](uint64_t c) { return c >= bound; };
+  const uint64_t hit =
+      residual ? items_crossing(each, in, by_id, left, true, target + 1, s)
+               : items_crossing(each, in, by_id, weight, true, target + 1, s);
+  if (tid == 0)
+    write_result(a, row, item_id(hit), drafted ? (float)((double)s.found_w / scale) : 0.0f, kept);
 }
 
 // Every thread's device-coherent stores complete, then one arrival; true in
@@ -1793,7 +1282,23 @@ __device__ __forceinline__ void merge_row(const SampleLaunch &a,
     }
     return;
   }
+  if (tid == 0 && cut_pass_row(rp)) a.states[row].stage = kRowDone;
   merge_sampled<DT>(a, rp, row, s);
+}
+
+// A wide row's lane: its least value among those that can carry weight (a
+// banned token's -inf, -1e4 or the like is left out): the cut passes' bins
+// then span the values the row has. A hint only.
+constexpr float kLeastLogit = -1000.0f;
+template <int N>
+__device__ __forceinline__ float lane_least(const float (&xs)[N], const SideEntries &side) {
+  float mn = __builtin_inff();
+#pragma unroll
+  for (int i = 0; i < N; ++i) mn = xs[i] > kLeastLogit ? __builtin_fminf(mn, xs[i]) : mn;
+#pragma unroll
+  for (int k = 0; k < kSideEntries; ++k)
+    mn = side.val[k] > kLeastLogit ? __builtin_fminf(mn, side.val[k]) : mn;
+  return mn;
 }
 
 // ---- the single-pass selection kernel -------------------------------------
@@ -1978,6 +1483,10 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
       s.wu[w] = wany;
       s.wu2[w] = wth;
     }
+    if (wide) {
+      const float least = -wave_max_f32(-lane_least(xs, side));
+      if (lane == 0) s.wmin[w] = least;
+    }
     if (uncut_row(rp) && tid < kWaves * 8) s.slices[tid] = 0;
     __syncthreads();
     const float bmax = __builtin_fmaxf(
@@ -2000,6 +1509,8 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
         hdr->count = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
         hdr->admitted = badm;
         hdr->overflow = 0;
+        hdr->best_value = __builtin_fminf(__builtin_fminf(s.wmin[0], s.wmin[1]),
+                                          __builtin_fminf(s.wmin[2], s.wmin[3]));
         hdr->floor_key = tk;
       }
       return;
@@ -2288,6 +1799,7 @@ struct __align__(16) FastLds {
   float wf[kWaves];
   uint32_t wu[kWaves];
   uint32_t wu2[kWaves];
+  float wmin[kWaves];
 };
 
 // LDS of the fast kernel's variant that finishes rows with no cut itself:
@@ -3099,6 +2611,10 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
     s.wu[w] = wany;
     s.wu2[w] = wth;
   }
+  if (wide) {
+    const float least = -wave_max_f32(-lane_least(xs, side));
+    if (lane == 0) s.wmin[w] = least;
+  }
   if (uncut && tid < kWaves * 8) s.slices[tid] = 0;
   __syncthreads();
   const float bmax = __builtin_fmaxf(
@@ -3129,6 +2645,9 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
     // No candidates: every lane that admits a token holds one at or above the
     // least of the lanes' maxima (the summary's count and floor).
     c = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
+    if (tid == 0)
+      hdr->best_value = __builtin_fminf(__builtin_fminf(s.wmin[0], s.wmin[1]),
+                                        __builtin_fminf(s.wmin[2], s.wmin[3]));
   } else {
     uint32_t thr = tk;
     if (flags & kRowMinP)
@@ -3292,72 +2811,6 @@ __device__ __forceinline__ int rank_select(const uint64_t (&v)[PER], uint32_t va
   }
   __syncthreads();
   return (int)need;
-}
-
-// The last steps of a row with at most 64 items left, s.merge.key/id[0, n)
-// in (key desc, id asc) order (rank_select), by one wave in registers. Rank
-// order gives the top-k cut and the walk of top-p (sampling.metal:585-650);
-// sorting the kept items by id gives the draw's order and the kept outputs
-// (sampling.metal:700-829). The results equal wave_merge's.
-__device__ __forceinline__ void wave_finish(const SampleLaunch &a, const RowParams &rp,
-                                            uint32_t row, const Lds &s, uint32_t n,
-                                            float maximum, float u, uint32_t draft) {
-  const MergeLds &m = s.merge;
-  const uint32_t lane = lane_id();
-  const uint32_t key = lane < n ? m.key[lane] : 0u;
-  const uint32_t id = lane < n ? m.id[lane] : kNoToken;
-  const uint32_t n2 = min(rp.top_k, n);
-  const bool in2 = lane < n2;
-  const float w = in2 ? weight_of(key_logit(key), maximum, rp.inv_t) : 0.0f;
-  const uint64_t wq = quantize(w);
-  uint32_t n3 = n2;
-  if (rp.flags & kRowTopP) {
-    const uint64_t incl = wave_incl_scan_u64(wq);
-    const uint64_t mass2 = readlane_u64(incl, 63);
-    if (mass2) {
-      const uint64_t nucleus = floor_mul(mass2, rp.top_p);
-      const uint64_t hm = ballot(in2 && incl - wq <= nucleus && incl > nucleus);
-      if (hm) n3 = (uint32_t)__builtin_ctzll(hm) + 1;
-    }
-  }
-  const bool kept = lane < n3;
-  const uint64_t mass3 = wave_sum_u64(kept ? wq : 0);
-  const double scale = (double)mass3 * 0x1p-44;
-  const bool drafted = draft != kNoToken;
-  uint64_t d = kept ? wq : 0;
-  if (drafted) {
-    float q = 0.0f;
-    for (int j = 15; j >= 0; --j) q = s.cids[j] == id ? s.cprobs[j] : q;
-    const uint64_t r = kept ? residual_of(wq, mass3, q) : 0;
-    if (ballot(r > 0)) d = r;
-  }
-  const uint64_t fm = ballot(drafted && kept && id == draft);
-  const float fw = u2f(readlane_u32(f2u(w), fm ? (int)__builtin_ctzll(fm) : 0));
-  // Id order of the kept items, each carrying the lane of its rank (ids are
-  // below 2^19, so id and lane share 32 bits).
-  uint32_t e = kept ? (id << 6) | lane : 0xffffffffu;
-  e = wave_sort_asc_u32(e);
-  const uint32_t src = e & 63u, iid = e >> 6;
-  const uint64_t dq = shfl_u64(d, (int)src);
-  const float wi = __shfl(w, (int)src, kWave);
-  if (a.out_kept_ids && kept && lane < a.kept_cap) {
-    a.out_kept_ids[(uint64_t)row * a.kept_cap + lane] = iid;
-    a.out_kept_probs[(uint64_t)row * a.kept_cap + lane] =
-        mass3 ? (float)((double)wi / scale) : 0.0f;
-  }
-  if (mass3 == 0) {
-    if (lane == 0) write_result(a, row, kNoToken, 0.0f, n3);
-    return;
-  }
-  const uint64_t dd = kept ? dq : 0ull;
-  const uint64_t incl = wave_incl_scan_u64(dd);
-  const uint64_t total = readlane_u64(incl, 63);
-  uint64_t target = floor_mul(total, u);
-  if (target >= total) target = total - 1;
-  const uint64_t hm = ballot(kept && incl - dd <= target && incl > target);
-  const uint32_t token = hm ? readlane_u32(iid, (int)__builtin_ctzll(hm)) : kNoToken;
-  if (lane == 0)
-    write_result(a, row, token, drafted && fm ? (float)((double)fw / scale) : 0.0f, n3);
 }
 
 // The general merge of a row for merge_small_kernel, out of line so that
@@ -3550,7 +3003,9 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
   thr = max(thr, s.row_floor);
   const uint32_t K = rp.top_k;
   const uint32_t n_all = s.hoff[S];
-  if (!s.row_overflow && thr > kLowestKey && (!s.row_long || n_all <= kSlots)) {
+  // (A top-k past a wave's worth goes straight to the general merge.)
+  const bool few = K <= 64u || (rp.flags & kRowMinP);
+  if (few && !s.row_overflow && thr > kLowestKey && (!s.row_long || n_all <= kSlots)) {
     uint32_t valid = 0;
     if (!s.row_long) {
 #pragma unroll
@@ -3789,7 +3244,7 @@ struct __align__(16) CutLds {
   uint32_t sel_chunk;
   uint64_t sel_excl;
   uint64_t u64a;
-  uint64_t bound;  // the kept set's last token, as cut_item
+  uint64_t bound;  // the kept set's last token, as token_item
 };
 
 // A (row, chunk)'s part of the candidate area during these passes, in 64-bit
@@ -3827,13 +3282,6 @@ __device__ __forceinline__ uint32_t cut_bin_at(float below, float scale) {
 __device__ __forceinline__ uint32_t cut_bin(float v, float maximum, float scale) {
   return cut_bin_at(maximum - v, scale);
 }
-// A token as one word that orders as (key, lower id first): ids are below 2^19.
-__device__ __forceinline__ uint64_t cut_item(uint32_t key, uint32_t id) {
-  return ((uint64_t)key << 19) | (0x7ffffu - id);
-}
-__device__ __forceinline__ uint32_t cut_key(uint64_t item) { return (uint32_t)(item >> 19); }
-__device__ __forceinline__ uint32_t cut_id(uint64_t item) { return 0x7ffffu - ((uint32_t)item & 0x7ffffu); }
-
 // A chunk of a row of these passes: xs[i] as load_chunk leaves it. A row with
 // no penalty requests its logits first thing (fast_load), before its record
 // has arrived; a penalized one takes load_chunk.
@@ -3907,8 +3355,13 @@ __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader
   r.none = !wave_max_u32(h.admitted) || r.maximum == __builtin_inff();
   const bool minp = (rp.flags & kRowMinP) != 0;
   r.floor = minp ? __builtin_fminf(r.maximum + rp.minp_offset, r.maximum) : -__builtin_inff();
-  // The bins' range below the maximum.
+  // The bins' range below the maximum: no further than the row's least value.
   float range = -rp.minp_offset;
+  if (!minp) {
+    const float least = -wave_max_f32(lane < S ? -h.best_value : -__builtin_inff());
+    const float d = (r.maximum - least) * 1.0001f;
+    if (d > 0.0f && d < range) range = d;
+  }
   if (!minp && (rp.flags & kRowTopK)) {
     // Each chunk's floor_key: a key that `count` of its tokens reach.
     const bool in = lane < S && h.count;
@@ -4160,7 +3613,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(
         if (v >= r.floor) {
           const uint32_t slot = atomicAdd(&s.n, 1u);
           if (slot < room)
-            list[slot] = cut_item(logit_key(v), lane_base + (i / VEC) * SLAB + (i % VEC));
+            list[slot] = token_item(logit_key(v), lane_base + (i / VEC) * SLAB + (i % VEC));
         }
       }
     }
@@ -4190,118 +3643,6 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(
 }
 #endif
 
-// Wave 0 finds the highest of s.hist's (s.hcount's) 256 bins whose suffix sum
-// reaches T (the total does): s.sel_bin, and s.sel_excl the sum above it.
-__device__ __forceinline__ void cut_crossing_bin(CutLds &s, uint64_t T, bool by_mass) {
-  if (threadIdx.x < 64) {
-    const uint32_t l = threadIdx.x;
-    uint64_t h[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) h[k] = by_mass ? s.hist[4 * l + k] : s.hcount[4 * l + k];
-    const uint64_t own = h[0] + h[1] + h[2] + h[3];
-    const uint64_t incl = wave_incl_scan_u64(own);
-    const uint64_t suf = readlane_u64(incl, 63) - (incl - own);
-    const uint64_t m = ballot(suf >= T);
-    const int L = m ? 63 - (int)__builtin_clzll(m) : 0;
-    if ((int)l == L) {
-      uint64_t acc = suf - own;
-      uint32_t k = 3;
-      while (k > 0 && acc + h[k] < T) acc += h[k--];
-      s.sel_bin = 4 * l + k;
-      s.sel_excl = acc;
-    }
-  }
-  __syncthreads();
-}
-
-// The item at which the running count (or exact mass) of the items that `in`
-// takes, largest first, reaches `target` (which it does): a radix descent by
-// up to 8 bits a pass from the highest bit in which they differ, until the
-// bin holds at most a wave's worth, which one wave ranks. `each(f)` calls
-// f(item) for every item, each thread its own.
-template <class Each, class In>
-__device__ __forceinline__ uint64_t cut_crossing(Each each, In in, bool by_mass, uint64_t target,
-                                                 float M, float inv_t, CutLds &s) {
-  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  uint64_t any1 = 0, any0 = 0;  // bits set in some item, clear in some item
-  each([&](uint64_t c) {
-    if (in(c)) {
-      any1 |= c;
-      any0 |= ~c;
-    }
-  });
-  auto wave_or = [](uint64_t v) {
-    v |= xor_u64<1>(v);
-    v |= xor_u64<2>(v);
-    v |= xor_u64<4>(v);
-    v |= xor_u64<8>(v);
-    v |= xor_u64<16>(v);
-    v |= xor_u64<32>(v);
-    return v;
-  };
-  any1 = wave_or(any1);
-  any0 = wave_or(any0);
-  __syncthreads();
-  if (lane == 0) {
-    s.wl[w] = any1;
-    s.wl2[w] = any0;
-  }
-  __syncthreads();
-  any1 = s.wl[0] | s.wl[1] | s.wl[2] | s.wl[3];
-  any0 = s.wl2[0] | s.wl2[1] | s.wl2[2] | s.wl2[3];
-  const uint64_t differ = any1 & any0;
-  const int bits = differ ? 64 - (int)__builtin_clzll(differ) : 1;  // low bits not yet fixed
-  int width = min(bits, 8), shift = bits - width;
-  uint64_t prefix = any1 >> bits;  // the bits above agree
-  for (;;) {
-    const uint32_t mask = (1u << width) - 1u;
-    s.hist[tid] = 0;
-    s.hcount[tid] = 0;
-    __syncthreads();
-    each([&](uint64_t c) {
-      if (in(c) && (c >> (shift + width)) == prefix) {
-        const uint32_t d = (uint32_t)(c >> shift) & mask;
-        atomicAdd(&s.hcount[d], 1u);
-        if (by_mass)
-          atomicAdd((unsigned long long *)&s.hist[d],
-                    (unsigned long long)quantized_weight(key_logit(cut_key(c)), M, inv_t));
-      }
-    });
-    __syncthreads();
-    cut_crossing_bin(s, target, by_mass);
-    target -= s.sel_excl;
-    prefix = (prefix << width) | s.sel_bin;
-    const uint32_t n = s.hcount[s.sel_bin];
-    if (n <= 64u || shift == 0) break;
-    width = min(shift, 8);
-    shift -= width;
-    __syncthreads();
-  }
-  __syncthreads();
-  if (tid == 0) s.small_n = 0;
-  __syncthreads();
-  each([&](uint64_t c) {
-    if (in(c) && (c >> shift) == prefix) s.small[atomicAdd(&s.small_n, 1u) & 63u] = c;
-  });
-  __syncthreads();
-  if (w == 0) {
-    const uint32_t n = min(s.small_n, 64u);
-    const uint64_t c = lane < n ? s.small[lane] : 0ull;
-    uint32_t rank = 0;
-    for (uint32_t j = 0; j < n; ++j) rank += s.small[j] > c ? 1u : 0u;
-    if (lane < n) s.sorted[rank] = c;
-    wave_lds_sync();
-    const uint64_t o = lane < n ? s.sorted[lane] : 0ull;
-    const uint64_t v = lane >= n ? 0ull
-                       : by_mass ? quantized_weight(key_logit(cut_key(o)), M, inv_t)
-                                 : 1ull;
-    const uint64_t reached = ballot(lane < n && wave_incl_scan_u64(v) >= target);
-    if ((int)lane == (reached ? (int)__builtin_ctzll(reached) : (int)n - 1)) s.u64a = o;
-  }
-  __syncthreads();
-  return s.u64a;
-}
-
 // The kept set of a row from the tokens of its boundary bins (`each`): its
 // last token into s.bound, and what those tokens add to each chunk's kept
 // mass and count (s.cmass, s.ccount: the bins before them on entry).
@@ -4309,34 +3650,36 @@ template <class Each>
 __device__ __forceinline__ void cut_resolve(const RowParams &rp, const RowState &st, Each each,
                                             bool counts, CutLds &s) {
   const float M = st.maximum, inv_t = rp.inv_t;
-  auto bin = [&](uint64_t c) { return cut_bin(key_logit(cut_key(c)), M, st.scale); };
+  auto bin = [&](uint64_t c) { return cut_bin(key_logit(item_key(c)), M, st.scale); };
+  auto ord = [](uint64_t c) { return c; };
+  auto weight = [&](uint64_t c) { return item_weight(c, M, inv_t); };
   uint64_t bound = 0, mass2 = st.total;
   if (st.need_k) {
-    bound = cut_crossing(each, [&](uint64_t c) { return bin(c) == st.bk; }, false, st.need_k, M,
-                         inv_t, s);
+    bound = items_crossing(each, [&](uint64_t c) { return bin(c) == st.bk; }, ord, weight, false,
+                           st.need_k, s);
     if (st.topp) {
       uint64_t m = 0;
       each([&](uint64_t c) {
-        if (bin(c) == st.bk && c >= bound) m += quantized_weight(key_logit(cut_key(c)), M, inv_t);
+        if (bin(c) == st.bk && c >= bound) m += quantized_weight(key_logit(item_key(c)), M, inv_t);
       });
       mass2 = st.mass_bk + block_sum_u64(m, s);
     }
   }
   if (st.topp && mass2) {
     const uint64_t kth = bound;
-    bound = cut_crossing(
+    bound = items_crossing(
         each,
         [&](uint64_t c) {
           const uint32_t b = bin(c);
           return c >= kth && b >= st.b0 && b <= st.b1;
         },
-        true, floor_mul(mass2, rp.top_p) + 1 - st.mass_b0, M, inv_t, s);
+        ord, weight, true, floor_mul(mass2, rp.top_p) + 1 - st.mass_b0, s);
   }
   each([&](uint64_t c) {
     if (c >= bound && bin(c) >= st.b0) {
-      const uint32_t k = cut_id(c) / kChunkF32;
+      const uint32_t k = item_id(c) / kChunkF32;
       atomicAdd((unsigned long long *)&s.cmass[k],
-                (unsigned long long)quantized_weight(key_logit(cut_key(c)), M, inv_t));
+                (unsigned long long)quantized_weight(key_logit(item_key(c)), M, inv_t));
       if (counts) atomicAdd(&s.ccount[k], 1u);
     }
   });
@@ -4348,10 +3691,11 @@ __device__ __forceinline__ void cut_resolve(const RowParams &rp, const RowState 
 __shared__ CutLds g_cut_lds;
 __shared__ SampleLaunch g_cut_launch;
 
-// The tokens of the row's boundary bins in half `h` of chunk `c` (loads h *
-// LOADS / 2 on), into g_cut_lds.items; returns how many.
+// The tokens of the row's boundary bins in chunk `c`, from the `skip`-th on in
+// the block's order of them, into g_cut_lds.items; returns how many the chunk
+// has (the first kCutItems past `skip` are there).
 template <int DT>
-__device__ __noinline__ uint32_t cut_collect(uint32_t row, uint32_t c, uint32_t h) {
+__device__ __noinline__ uint32_t cut_collect(uint32_t row, uint32_t c, uint32_t skip) {
   constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
   const SampleLaunch &a = g_cut_launch;
   const RowParams rp = a.params[row];
@@ -4360,23 +3704,28 @@ __device__ __noinline__ uint32_t cut_collect(uint32_t row, uint32_t c, uint32_t 
   const uint32_t thr_key = st.thr_key, b0 = st.b0, b1 = st.b1, bk = st.bk;
   float xs[TPL];
   load_chunk<DT>(a, rp, row, c, g_cut_lds, xs);
-  __syncthreads();  // the prep area becomes the items'
-  if (threadIdx.x == 0) g_cut_lds.n = 0;
-  __syncthreads();
-  const uint32_t lane_base = c * kChunkF32 + threadIdx.x * VEC;
+  uint32_t hits = 0;
 #pragma unroll
   for (int i = 0; i < TPL; ++i) {
     const float v = xs[i];
-    const uint32_t k = logit_key(v), b = cut_bin(v, M, scale);
-    if ((uint32_t)(i / (TPL / 2)) == h && v == v && k >= thr_key &&
-        ((b >= b0 && b <= b1) || b == bk))
-      g_cut_lds.items[atomicAdd(&g_cut_lds.n, 1u)] =
-          cut_item(k, lane_base + (i / VEC) * SLAB + (i % VEC));
+    const uint32_t b = cut_bin(v, M, scale);
+    if (v == v && logit_key(v) >= thr_key && ((b >= b0 && b <= b1) || b == bk)) hits |= 1u << i;
   }
+  uint64_t total;
+  // (The scan's barriers also end the prep area's use: it becomes the items'.)
+  uint32_t at = (uint32_t)block_excl_scan_u64(__popc(hits), g_cut_lds, &total) - skip;
+  const uint32_t lane_base = c * kChunkF32 + threadIdx.x * VEC;
+#pragma unroll
+  for (int i = 0; i < TPL; ++i)
+    if ((hits >> i) & 1u) {
+      if (at < kCutItems)
+        g_cut_lds.items[at] =
+            token_item(logit_key(xs[i]), lane_base + (i / VEC) * SLAB + (i % VEC));
+      ++at;
+    }
   __syncthreads();
-  return g_cut_lds.n;
+  return (uint32_t)total;
 }
-static_assert(kCutItems >= kChunkF32 / 2, "half a chunk's tokens fit the items");
 
 // cut_resolve over the row's logits, for a row whose boundary bins hold more
 // tokens than the lists: each step reads the row's chunks again. Out of line
@@ -4387,11 +3736,13 @@ __device__ __noinline__ void cut_rescan(uint32_t row) {
   const RowParams rp = g_cut_launch.params[row];
   const RowState st = g_cut_launch.states[row];
   auto each = [&](auto f) {
-    for (uint32_t p = 0; p < 2 * g_cut_launch.chunks; ++p) {
-      const uint32_t n = cut_collect<DT>(row, p >> 1, p & 1u);
-      for (uint32_t i = threadIdx.x; i < n; i += kThreads) f(g_cut_lds.items[i]);
-      __syncthreads();
-    }
+    for (uint32_t c = 0; c < g_cut_launch.chunks; ++c)
+      for (uint32_t skip = 0, n = 1; skip < n; skip += kCutItems) {
+        n = cut_collect<DT>(row, c, skip);
+        for (uint32_t i = threadIdx.x; i < min(n - skip, kCutItems) && skip < n; i += kThreads)
+          f(g_cut_lds.items[i]);
+        __syncthreads();
+      }
   };
   cut_resolve(rp, st, each, g_cut_launch.out_kept_ids != nullptr, g_cut_lds);
 }
@@ -4414,10 +3765,10 @@ __device__ __forceinline__ void cut_walk(const SampleLaunch &a, const RowParams 
   const float M = st.maximum, inv_t = rp.inv_t;
   // Kept: above the kept set's last value, or equal to it up to its last id;
   // where nothing cuts, every member.
-  const float bv = bound        ? key_logit(cut_key(bound))
+  const float bv = bound        ? key_logit(item_key(bound))
                    : st.thr_key ? key_logit(st.thr_key)
                                 : -__builtin_inff();
-  const uint32_t bid = bound ? cut_id(bound) : kNoToken;
+  const uint32_t bid = bound ? item_id(bound) : kNoToken;
   auto weight = [&](float v, uint32_t t) -> uint64_t {
     uint64_t q = 0;
     if (v > bv || (v == bv && t <= bid)) q = quantized_weight(v, M, inv_t);
@@ -4471,7 +3822,7 @@ __device__ __forceinline__ void cut_resolve_wave(const RowParams &rp, const RowS
   wave_lds_sync();
   const bool in = lane < n;
   const uint64_t c = in ? s.sorted[lane] : 0ull;
-  const float v = key_logit(cut_key(c));
+  const float v = key_logit(item_key(c));
   const uint32_t b = in ? cut_bin(v, M, st.scale) : 0u;
   const uint64_t wq = in ? quantized_weight(v, M, inv_t) : 0ull;
   uint64_t bound = 0, mass2 = st.total;
@@ -4489,7 +3840,7 @@ __device__ __forceinline__ void cut_resolve_wave(const RowParams &rp, const RowS
     if (hit) bound = readlane_u64(c, (int)__builtin_ctzll(hit));
   }
   if (in && c >= bound && b >= st.b0) {
-    const uint32_t k = cut_id(c) / kChunkF32;
+    const uint32_t k = item_id(c) / kChunkF32;
     atomicAdd((unsigned long long *)&s.cmass[k], (unsigned long long)wq);
     if (counts) atomicAdd(&s.ccount[k], 1u);
   }
@@ -4533,8 +3884,8 @@ __device__ __forceinline__ void cut_pick(const SampleLaunch &a, uint32_t row, ui
     s.sel_excl = target - excl;
     s.kept = kept;
     RowState &ns = a.states[row];
-    ns.bkey = cut_key(s.bound);
-    ns.bid = s.bound ? cut_id(s.bound) : 0u;
+    ns.bkey = item_key(s.bound);
+    ns.bid = s.bound ? item_id(s.bound) : 0u;
     ns.mass3 = mass3;
     ns.kept = kept;
     ns.stage = counts || (drafted && mass3) ? kRowEmit : kRowDone;
@@ -4586,7 +3937,7 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(
     if (lane == 0) {
       s.coff[0] = 0;
       s.bound = 0;
-      s.n = over || all > kCutItems ? 0xffffffffu : all;
+      s.n = over ? 0xffffffffu : all;
     }
     wave_lds_sync();
     if (!over && all <= 64u) {
@@ -4605,10 +3956,12 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(
       __syncthreads();
       cut_rescan<DT>(row);
     } else {
-      for (uint32_t i = tid; i < n; i += kThreads) s.items[i] = item(i);
+      // Past the items' room in LDS, the rest stays in the lists.
+      for (uint32_t i = tid; i < min(n, kCutItems); i += kThreads) s.items[i] = item(i);
       __syncthreads();
       auto each = [&](auto f) {
-        for (uint32_t i = tid; i < n; i += kThreads) f(g_cut_lds.items[i]);
+        for (uint32_t i = tid; i < n; i += kThreads)
+          f(i < kCutItems ? g_cut_lds.items[i] : item(i));
       };
       cut_resolve(rp, st, each, counts, s);
     }

@@ -946,20 +946,15 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     }
   }
   if (e != hipSuccess) return hip_fail((hipError_t)e, "select launch");
-  // The small-K merge takes launches whose cut rows keep at most 64 tokens
-  // by their top-k, or have a min-p floor (which usually leaves few: rows
-  // whose floor leaves more than 64 take its general path), and read sparse
-  // draft probabilities (or none).
-  bool small = !a->draft_q && a->uniform_offset <= 0xffffffffull &&
-               a->uniform_stride <= 0xffffffffull;
+  // merge_small_kernel takes launches that read sparse draft probabilities (or
+  // none). wide: some listed row has no min-p floor (longer lists).
+  const bool small = !a->draft_q && a->uniform_offset <= 0xffffffffull &&
+                     a->uniform_stride <= 0xffffffffull;
   bool wide = false;
-  for (uint32_t r = 0; small && r < rows; ++r) {
+  for (uint32_t r = 0; r < rows; ++r) {
     const jf::RowParams &rp = params[r];
-    if (jf::wide_row(rp.flags, rp.top_k)) continue;
-    if ((rp.flags & jf::kRowSampled) && (rp.flags & kCuts) &&
-        !((rp.flags & jf::kRowTopK) && rp.top_k <= 64u) && !(rp.flags & jf::kRowMinP))
-      small = false;
-    wide |= (rp.flags & jf::kRowSampled) && (rp.flags & kCuts) && !(rp.flags & jf::kRowMinP);
+    wide |= (rp.flags & kCuts) && !(rp.flags & jf::kRowMinP) &&
+            !jf::wide_row(rp.flags, rp.top_k);
   }
   if (need_merge) {
     e = small ? jf::launch_merge_small(L, a->dtype, wide, stream)
