@@ -1286,19 +1286,41 @@ __device__ __forceinline__ void merge_row(const SampleLaunch &a,
   merge_sampled<DT>(a, rp, row, s);
 }
 
-// A wide row's lane: its least value among those that can carry weight (a
-// banned token's -inf, -1e4 or the like is left out): the cut passes' bins
-// then span the values the row has. A hint only.
+// A wide row's chunk has no candidates, only a summary: its maximum, how many
+// lanes admit a token, a key that many of its tokens reach (the least of their
+// maxima), and its least value among those that can carry weight (a banned
+// token's -inf, -1e4 or the like is left out): hints for the cut passes' bins.
 constexpr float kLeastLogit = -1000.0f;
-template <int N>
-__device__ __forceinline__ float lane_least(const float (&xs)[N], const SideEntries &side) {
+template <int N, class L>
+__device__ __forceinline__ void wide_summary(const float (&xs)[N], const SideEntries &side,
+                                             float mx, L &s, BlockHeader *hdr) {
+  const uint32_t w = threadIdx.x >> 6;
+  const bool any = mx == mx;
   float mn = __builtin_inff();
 #pragma unroll
   for (int i = 0; i < N; ++i) mn = xs[i] > kLeastLogit ? __builtin_fminf(mn, xs[i]) : mn;
 #pragma unroll
   for (int k = 0; k < kSideEntries; ++k)
     mn = side.val[k] > kLeastLogit ? __builtin_fminf(mn, side.val[k]) : mn;
-  return mn;
+  const float wmax = wave_max_f32(mx), wmin = -wave_max_f32(-mn);
+  const uint32_t floor_key = wave_min_u32(any ? logit_key(mx) : 0xffffffffu);
+  const uint32_t lanes = (uint32_t)__popcll(ballot(any));
+  if (lane_id() == 0) {
+    s.wf[w] = wmax;
+    s.wmin[w] = wmin;
+    s.wu[w] = lanes;
+    s.wu2[w] = floor_key;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  hdr->maximum = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(s.wf[0], s.wf[1]),
+                                                 __builtin_fmaxf(s.wf[2], s.wf[3])),
+                                 -3.402823466e38f);
+  hdr->count = hdr->admitted = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
+  hdr->overflow = 0;
+  hdr->best_value = __builtin_fminf(__builtin_fminf(s.wmin[0], s.wmin[1]),
+                                    __builtin_fminf(s.wmin[2], s.wmin[3]));
+  hdr->floor_key = min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3]));
 }
 
 // ---- the single-pass selection kernel -------------------------------------
@@ -1463,6 +1485,10 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
     for (int i = 0; i < TPL; ++i) mx = __builtin_fmaxf(mx, xs[i]);
 #pragma unroll
     for (int k = 0; k < kSideEntries; ++k) mx = __builtin_fmaxf(mx, side.val[k]);
+    if (wide_row(rp.flags, rp.top_k)) {
+      wide_summary(xs, side, mx, s, hdr);
+      return;
+    }
     const bool any = mx == mx;
     // A bound for the block's top-k: each wave's ceil(k/4)-th largest lane
     // maximum has that many of the wave's tokens at or above it, so the
@@ -1470,22 +1496,14 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
     const uint32_t K = rp.top_k;
     const uint32_t kw = (K + kWaves - 1) / kWaves;
     const bool bound = (rp.flags & kRowTopK) && kw <= 64;
-    const bool wide = wide_row(rp.flags, K);
     uint32_t wth = 0;
-    if (wide)
-      wth = wave_min_u32(any ? logit_key(mx) : 0xffffffffu);
-    else if (bound)
-      wth = wave_kth_largest(any ? logit_key(mx) : 0u, kw);
+    if (bound) wth = wave_kth_largest(any ? logit_key(mx) : 0u, kw);
     const float wmax = wave_max_f32(mx);
-    const uint32_t wany = (uint32_t)__popcll(ballot(any));
+    const uint32_t wany = ballot(any) != 0 ? 1u : 0u;
     if (lane == 0) {
       s.wf[w] = wmax;
       s.wu[w] = wany;
       s.wu2[w] = wth;
-    }
-    if (wide) {
-      const float least = -wave_max_f32(-lane_least(xs, side));
-      if (lane == 0) s.wmin[w] = least;
     }
     if (uncut_row(rp) && tid < kWaves * 8) s.slices[tid] = 0;
     __syncthreads();
@@ -1500,21 +1518,7 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
       return;
     }
     const uint32_t tk =
-        bound || wide ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
-    if (wide) {
-      // No candidates: every lane that admits a token holds one at or above
-      // the least of the lanes' maxima.
-      if (tid == 0) {
-        hdr->maximum = bmax;
-        hdr->count = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
-        hdr->admitted = badm;
-        hdr->overflow = 0;
-        hdr->best_value = __builtin_fminf(__builtin_fminf(s.wmin[0], s.wmin[1]),
-                                          __builtin_fminf(s.wmin[2], s.wmin[3]));
-        hdr->floor_key = tk;
-      }
-      return;
-    }
+        bound ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
     uint32_t thr = tk;
     if (rp.flags & kRowMinP)
       thr = max(thr, logit_key(__builtin_fminf(bmax + rp.minp_offset, bmax)));
@@ -2591,29 +2595,25 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
     return;
   }
 
+  // (A launch that finishes its rows here has no wide row.)
+  if (!FUSE && !ACCEPT && wide_row(flags, rp.top_k)) {
+    wide_summary(xs, side, mx, s, hdr);
+    return;
+  }
   const bool any = mx == mx;
   // The chunk's top-k bound, as select_kernel (each wave's ceil(k/4)-th
   // largest lane maximum, rounded down to a multiple of 2^16 of its key).
   const uint32_t K = rp.top_k;
   const uint32_t kw = (K + kWaves - 1) / kWaves;
   const bool bound = (flags & kRowTopK) && kw <= 64;
-  // (A launch that finishes its rows here has no wide row.)
-  const bool wide = !FUSE && !ACCEPT && wide_row(flags, K);
   uint32_t wth = 0;
-  if (wide)
-    wth = wave_min_u32(any ? logit_key(mx) : 0xffffffffu);
-  else if (bound)
-    wth = wave_kth_bound16(any ? logit_key(mx) : 0u, kw);
+  if (bound) wth = wave_kth_bound16(any ? logit_key(mx) : 0u, kw);
   const float wmax = wave_max_f32(mx);
-  const uint32_t wany = (uint32_t)__popcll(ballot(any));
+  const uint32_t wany = ballot(any) != 0 ? 1u : 0u;
   if (lane == 0) {
     s.wf[w] = wmax;
     s.wu[w] = wany;
     s.wu2[w] = wth;
-  }
-  if (wide) {
-    const float least = -wave_max_f32(-lane_least(xs, side));
-    if (lane == 0) s.wmin[w] = least;
   }
   if (uncut && tid < kWaves * 8) s.slices[tid] = 0;
   __syncthreads();
@@ -2623,7 +2623,7 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
       -3.402823466e38f);
   const uint32_t badm = s.wu[0] | s.wu[1] | s.wu[2] | s.wu[3];
   const uint32_t tk =
-      bound || wide ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
+      bound ? min(min(s.wu2[0], s.wu2[1]), min(s.wu2[2], s.wu2[3])) : 0u;
   if (uncut) {
     // The row keeps every admitted token: the uncut kernel's chunk summary,
     // or (FUSE) the row finished here.
@@ -2640,60 +2640,50 @@ __global__ __launch_bounds__(kThreads) void select_fast_kernel(
     }
     return;
   }
-  uint32_t c;
-  if (wide) {
-    // No candidates: every lane that admits a token holds one at or above the
-    // least of the lanes' maxima (the summary's count and floor).
-    c = s.wu[0] + s.wu[1] + s.wu[2] + s.wu[3];
-    if (tid == 0)
-      hdr->best_value = __builtin_fminf(__builtin_fminf(s.wmin[0], s.wmin[1]),
-                                        __builtin_fminf(s.wmin[2], s.wmin[3]));
-  } else {
-    uint32_t thr = tk;
-    if (flags & kRowMinP)
-      thr = max(thr, logit_key(__builtin_fminf(bmax + rp.minp_offset, bmax)));
-    const float tv = thr <= kLowestKey ? -__builtin_inff() : key_logit(thr);
-    uint64_t *stage = s.stage[w];
-    uint32_t run = 0;
-    auto emit = [&](float x, uint32_t token) {
-      const bool hit = x >= tv;
-      const uint64_t m = ballot(hit);
-      if (m) {
-        // Hits past the wave's list land on its last entry: the wave's count
-        // then exceeds the list and the chunk is flagged as overflowed, so
-        // its staged list is never copied out.
-        const uint32_t slot_i = min(__builtin_amdgcn_mbcnt_hi(
-                                        (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, run)),
-                                    (uint32_t)kWaveCandidates - 1u);
-        if (hit) stage[slot_i] = (uint64_t)f2u(x) | ((uint64_t)token << 32);
-        run += (uint32_t)__popcll(m);
-      }
-    };
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j)
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) emit(xs[j * VEC + e], lane_base + j * SLAB + e);
-#pragma unroll
-    for (int k = 0; k < SPT; ++k) emit(side.val[k], side.tok[k]);
-    if (lane == 0) s.wcount[w] = run;
-    __syncthreads();
-    uint32_t off[kWaves + 1], over = 0;
-    off[0] = 0;
-#pragma unroll
-    for (int k = 0; k < kWaves; ++k) {
-      const uint32_t n = s.wcount[k];
-      over |= n > kWaveCandidates;
-      off[k + 1] = off[k] + min(n, kWaveCandidates);
+  uint32_t thr = tk;
+  if (flags & kRowMinP)
+    thr = max(thr, logit_key(__builtin_fminf(bmax + rp.minp_offset, bmax)));
+  const float tv = thr <= kLowestKey ? -__builtin_inff() : key_logit(thr);
+  uint64_t *stage = s.stage[w];
+  uint32_t run = 0;
+  auto emit = [&](float x, uint32_t token) {
+    const bool hit = x >= tv;
+    const uint64_t m = ballot(hit);
+    if (m) {
+      // Hits past the wave's list land on its last entry: the wave's count
+      // then exceeds the list and the chunk is flagged as overflowed, so
+      // its staged list is never copied out.
+      const uint32_t slot_i = min(__builtin_amdgcn_mbcnt_hi(
+                                      (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, run)),
+                                  (uint32_t)kWaveCandidates - 1u);
+      if (hit) stage[slot_i] = (uint64_t)f2u(x) | ((uint64_t)token << 32);
+      run += (uint32_t)__popcll(m);
     }
-    uint64_t *dst = a.cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
-    if (!over)
-      for (uint32_t i = tid; i < off[kWaves]; i += kThreads) {
-        const uint32_t k = (i >= off[1]) + (i >= off[2]) + (i >= off[3]);
-        const uint64_t e = s.stage[k][i - off[k]];
-        dst[i] = (uint64_t)logit_key(u2f((uint32_t)e)) | (e & 0xffffffff00000000ull);
-      }
-    c = over ? kBlockCandidates + 1 : off[kWaves];
+  };
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j)
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) emit(xs[j * VEC + e], lane_base + j * SLAB + e);
+#pragma unroll
+  for (int k = 0; k < SPT; ++k) emit(side.val[k], side.tok[k]);
+  if (lane == 0) s.wcount[w] = run;
+  __syncthreads();
+  uint32_t off[kWaves + 1], over = 0;
+  off[0] = 0;
+#pragma unroll
+  for (int k = 0; k < kWaves; ++k) {
+    const uint32_t n = s.wcount[k];
+    over |= n > kWaveCandidates;
+    off[k + 1] = off[k] + min(n, kWaveCandidates);
   }
+  uint64_t *dst = a.cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
+  if (!over)
+    for (uint32_t i = tid; i < off[kWaves]; i += kThreads) {
+      const uint32_t k = (i >= off[1]) + (i >= off[2]) + (i >= off[3]);
+      const uint64_t e = s.stage[k][i - off[k]];
+      dst[i] = (uint64_t)logit_key(u2f((uint32_t)e)) | (e & 0xffffffff00000000ull);
+    }
+  const uint32_t c = over ? kBlockCandidates + 1 : off[kWaves];
   if (tid == 0) {
     hdr->maximum = bmax;
     hdr->count = min(c, (uint32_t)kBlockCandidates);
@@ -2944,9 +2934,12 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
     }
   }
   // The uncut kernel draws it, or cut_hist_kernel and the launches after it.
-  if (uncut_row(rp) || wide_row(rp.flags, rp.top_k)) return;
-  // The general path may hand a min-p row on to cut_hist_kernel.
-  if (tid == 0 && cut_pass_row(rp)) a.states[row].stage = kRowDone;
+  if (uncut_row(rp)) return;
+  if (rp.top_k > kListTopK) {
+    if (wide_row(rp.flags, rp.top_k)) return;
+    // The general path may hand a min-p row on to cut_hist_kernel.
+    if (tid == 0 && cut_pass_row(rp)) a.states[row].stage = kRowDone;
+  }
 
   if (!(rp.flags & kRowSampled)) {
     // Greedy: the largest chunk best, the lowest id among equals.
