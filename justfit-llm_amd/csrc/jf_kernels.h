@@ -89,9 +89,8 @@ struct RowState {
 static_assert(sizeof(RowState) == 128, "row states are 128 bytes");
 enum RowStage : uint32_t {
   kRowDone = 0,
-  kRowWide = 1,    // the merge's min-p row with more candidates than its lists
-  kRowGather = 2,  // cut_list_kernel found and listed its boundary bins
-  kRowEmit = 3,    // cut_draw_kernel found its kept set; outputs or a draft's draw remain
+  kRowGather = 1,  // cut_list_kernel found and listed its boundary bins
+  kRowEmit = 2,    // cut_draw_kernel found its kept set; outputs or a draft's draw remain
 };
 
 struct StagePartial {
@@ -416,6 +415,10 @@ struct CutLaunch {
   bool all;      // every row takes them by its policy (wide_row)
   bool plain;    // no row is penalized
   bool drafted;  // some row is drafted
+  bool others;   // cut_draw_kernel finishes the listed and greedy rows too (no
+                 // merge is launched),
+  bool uncut;    // and the uncut rows (no launch_uncut follows)
+  bool small;    // its listed rows may take merge_small_row
 };
 int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *stream);
 int launch_accept_chain(const AcceptChainLaunch &a, void *stream);

@@ -633,8 +633,8 @@ __device__ __forceinline__ bool uncut_row(const RowParams &rp) {
   return (rp.flags & kRowSampled) && !(rp.flags & (kRowMinP | kRowTopK | kRowTopP));
 }
 
-// Whether cut_hist_kernel and the launches after it may have the row: always
-// (wide_row), or when the merge finds its min-p candidates past the lists.
+// Whether the cut passes may have the row: always (wide_row), or when its
+// min-p candidates are past the lists (cut_takes).
 __device__ __forceinline__ bool cut_pass_row(const RowParams &rp) {
   return wide_row(rp.flags, rp.top_k) ||
          ((rp.flags & kRowSampled) && (rp.flags & kRowMinP) &&
@@ -1002,8 +1002,8 @@ __device__ __forceinline__ void wave_finish(const SampleLaunch &a, const RowPara
 // A sampled row from its candidate lists, whatever they hold: the tokens at or
 // above its threshold as items in LDS, the top-k and top-p boundaries by
 // items_crossing, and the draw by items_crossing over the ids. A min-p row
-// with more such tokens than LDS takes (and a top-k past the lists) goes on to
-// the cut passes.
+// with a top-k past the lists whose tokens they, or LDS, cannot hold is left to
+// the cut passes (cut_takes).
 template <int DT>
 __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowParams &rp,
                               uint32_t row, Lds &s) {
@@ -1067,12 +1067,7 @@ __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowPa
   }
   __syncthreads();
   const uint32_t n_all = s.hoff[S];
-  if (K > (uint32_t)kBlockCandidates && (overflow || n_all > kMergeItems)) {
-    if (tid == 0) a.states[row].stage = kRowWide;
-    return;
-  }
-  // (A lambda's own copy of what it reads: a captured reference to LDS would
-  // go through memory.)
+  if (K > (uint32_t)kBlockCandidates && (overflow || n_all > kMergeItems)) return;  // cut_takes
   ItemsLds &g = s.general;
   auto listed = [&](uint32_t i) -> uint64_t {
     uint32_t c = 0;
@@ -1262,8 +1257,7 @@ __device__ __forceinline__ void merge_row(const SampleLaunch &a,
                                           const RowParams &rp, uint32_t row,
                                           Lds &s) {
   const uint32_t S = a.chunks, tid = threadIdx.x;
-  // The uncut kernel draws it, or cut_hist_kernel and the launches after it.
-  if (uncut_row(rp) || wide_row(rp.flags, rp.top_k)) return;
+  if (uncut_row(rp)) return;  // the uncut kernel draws it
   if (!(rp.flags & kRowSampled)) {
     if (tid < 64) {
       float bv = -__builtin_inff();
@@ -1282,7 +1276,6 @@ __device__ __forceinline__ void merge_row(const SampleLaunch &a,
     }
     return;
   }
-  if (tid == 0 && cut_pass_row(rp)) a.states[row].stage = kRowDone;
   merge_sampled<DT>(a, rp, row, s);
 }
 
@@ -2826,18 +2819,18 @@ __device__ __noinline__ void merge_small_general(uint32_t row) {
 // bit 31 of `chunks_bits` says the row's draft is addressed through its
 // record (the chunk count below it), so that no later argument is read
 // from memory at the row's start.
-#if JF_IN(2)
 // SPEC: speculatively fetched list slots a thread. 10 gives floor(2560 / S)
 // slots a chunk (134 at 19 chunks); 20 gives floor(5120 / S) (165 at 31
 // chunks), for vocabularies past 163,840 tokens whose cut rows have no
 // min-p floor (their lists average about 75 candidates and reach 130).
-template <int DT, int SPEC>
-__global__ __launch_bounds__(kThreads) void merge_small_kernel(
+// `general`: the general merge of the row, called by every thread.
+template <int DT, int SPEC, class General>
+__device__ __forceinline__ void merge_small_row(
     const BlockHeader *headers, const uint64_t *cands, const RowParams *params,
     const float *uniforms, const uint32_t *uniform_index, uint32_t chunks_bits,
-    uint32_t uniform_offset, uint32_t uniform_stride, uint32_t drafted_rows, SampleLaunch a) {
-  Lds &s = g_small_lds;
-  const uint32_t row = blockIdx.x, tid = threadIdx.x;
+    uint32_t uniform_offset, uint32_t uniform_stride, uint32_t drafted_rows,
+    const SampleLaunch &a, uint32_t row, Lds &s, General general) {
+  const uint32_t tid = threadIdx.x;
   const uint32_t S = chunks_bits & 0x7fffffffu;
   const bool row_indexed = (chunks_bits >> 31) != 0;
   // Every address of the row, computed once and held in vector registers:
@@ -2933,13 +2926,7 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
       cpr = a.cand_probs[(uint64_t)rp.cand_index * 16 + tid];
     }
   }
-  // The uncut kernel draws it, or cut_hist_kernel and the launches after it.
-  if (uncut_row(rp)) return;
-  if (rp.top_k > kListTopK) {
-    if (wide_row(rp.flags, rp.top_k)) return;
-    // The general path may hand a min-p row on to cut_hist_kernel.
-    if (tid == 0 && cut_pass_row(rp)) a.states[row].stage = kRowDone;
-  }
+  if (uncut_row(rp)) return;  // the uncut kernel's
 
   if (!(rp.flags & kRowSampled)) {
     // Greedy: the largest chunk best, the lowest id among equals.
@@ -3041,17 +3028,31 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
     }
     __syncthreads();
   }
-  // What the speculative fetch does not cover: the general merge. The
-  // launch record is copied word by word from the argument segment here
-  // (one word a thread), so no field of it stays live from the kernel's
-  // entry (the compiler otherwise kept some in private memory for this).
-  {
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(&g_small_launch);
-    for (uint32_t k = tid; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
-  }
-  __syncthreads();
-  merge_small_general<DT>(row);
+  // What the speculative fetch does not cover.
+  general();
+}
+
+#if JF_IN(2)
+template <int DT, int SPEC>
+__global__ __launch_bounds__(kThreads) void merge_small_kernel(
+    const BlockHeader *headers, const uint64_t *cands, const RowParams *params,
+    const float *uniforms, const uint32_t *uniform_index, uint32_t chunks_bits,
+    uint32_t uniform_offset, uint32_t uniform_stride, uint32_t drafted_rows, SampleLaunch a) {
+  const uint32_t row = blockIdx.x;
+  merge_small_row<DT, SPEC>(
+      headers, cands, params, uniforms, uniform_index, chunks_bits, uniform_offset,
+      uniform_stride, drafted_rows, a, row, g_small_lds, [&]() {
+        // The launch record is copied word by word from the argument segment
+        // here (one word a thread), so no field of it stays live from the
+        // kernel's entry (the compiler otherwise kept some in private memory
+        // for this).
+        const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
+        uint32_t *dst = reinterpret_cast<uint32_t *>(&g_small_launch);
+        for (uint32_t k = threadIdx.x; k < sizeof(SampleLaunch) / 4; k += kThreads)
+          dst[k] = src[k];
+        __syncthreads();
+        merge_small_general<DT>(row);
+      });
 }
 #endif
 
@@ -3170,6 +3171,119 @@ __device__ __forceinline__ uint32_t walk_chunk(const SampleLaunch &a, const RowP
   return s.hit;
 }
 
+struct __align__(16) UncutLds {
+  PrepLds prep;
+  uint64_t wj[kWaves][8];
+  uint64_t wl[kWaves];
+  uint32_t cids[16];
+  float cprobs[16];
+  float cmax[kMaxChunks];       // the row's chunk maxima
+  uint64_t cscale[kMaxChunks];  // r_c, packed s_c << 32 | R_c
+  uint64_t ctot[kMaxChunks];    // T_c
+  uint32_t ccount[kMaxChunks];  // admitted (non-NaN) tokens per chunk
+  uint64_t slices[kWaves * 8];  // one chunk's slice masses
+  float row_max;
+  uint64_t row_mass;
+  uint32_t row_admitted;
+  uint32_t row_kept;
+  float pd;                     // p(draft)
+  uint32_t residual;
+  uint32_t last;
+  uint32_t sel_bin;
+  uint64_t sel_excl;
+  uint32_t slice;
+  uint64_t slice_within;
+};
+
+// The chunk summaries of a row with no cut, by one wave (lane c < S holds chunk
+// c's): the row maximum, each chunk's rescale and rescaled mass, the row mass.
+__device__ __forceinline__ void uncut_row_sums(bool in, float hm, uint32_t hadm, uint32_t hcnt,
+                                               uint64_t hmass, float inv_t, UncutLds &s) {
+  const uint32_t lane = lane_id();
+  const float m = in ? hm : -3.402823466e38f;
+  const uint32_t adm = in ? hadm : 0u;
+  const uint32_t cnt = in ? hcnt : 0u;
+  const uint64_t mass = in ? hmass : 0ull;
+  const float M = wave_max_f32(m);
+  const uint64_t R = in ? chunk_scale(m, M, inv_t) : kZeroScale;
+  const uint64_t T = scale_by(mass, R);
+  const uint64_t W = wave_sum_u64(T);
+  const uint32_t admitted = wave_sum_u32(adm), kept = wave_sum_u32(cnt);
+  if (in) {
+    s.cmax[lane] = m;
+    s.cscale[lane] = R;
+    s.ctot[lane] = T;
+    s.ccount[lane] = cnt;
+  }
+  if (lane == 0) {
+    s.row_max = M;
+    s.row_mass = W;
+    // Nothing admitted, or a +inf maximum: the sentinel with nothing kept.
+    const bool none = admitted == 0 || M == __builtin_inff();
+    s.row_admitted = none ? 0u : 1u;
+    s.row_kept = none ? 0u : kept;
+    s.pd = 0.0f;
+  }
+}
+
+// The plain draw of an uncut row from its chunk masses (one block; block-
+// uniform): the chunk, its reload together with its slice masses (which the
+// select pass wrote), the slice, the token.
+template <int DT>
+__device__ __forceinline__ void uncut_draw(const SampleLaunch &a, const RowParams &rp,
+                                           uint32_t row, UncutLds &s, uint64_t W, float u) {
+  constexpr int TPL = Geo<DT>::TPL, VEC = Geo<DT>::VEC, LOADS = Geo<DT>::LOADS,
+                SLAB = Geo<DT>::SLAB;
+  constexpr uint32_t CHUNK = Geo<DT>::CHUNK, G = LOADS * kWaves;
+  const uint32_t S = a.chunks, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  if (w == 0) {
+    const bool in = lane < S;
+    const uint64_t T = in ? s.ctot[lane] : 0ull;
+    const uint64_t incl = wave_incl_scan_u64(T);
+    uint64_t target = floor_mul(W, u);
+    if (target >= W) target = W - 1;
+    // incl at the last lane is W > target: some lane passes it.
+    const uint32_t c = (uint32_t)__builtin_ctzll(ballot(in && incl > target));
+    const uint64_t within = target - readlane_u64(incl - T, c);
+    if (lane == 0) {
+      s.sel_bin = c;
+      // The running mass inside chunk c (against m_c) that the token's
+      // prefix must pass: floor(P * r_c) > within <=> P > this.
+      s.sel_excl = unscaled_bound(within, s.cscale[c]);
+    }
+  }
+  __syncthreads();
+  const uint32_t c = s.sel_bin;
+  uint64_t vg = 0;
+  if (w == 0 && lane < G) vg = a.partials[(uint64_t)row * S + c].v[1 + lane];
+  float xs[TPL];
+  load_chunk<DT>(a, rp, row, c, s, xs);
+  if (w == 0) {
+    uint64_t wi = s.sel_excl;
+    const uint32_t gg = pick_slice(vg, G, wi);
+    if (lane == 0) {
+      s.slice = gg;
+      s.slice_within = wi;
+    }
+  }
+  __syncthreads();
+  const uint32_t g = s.slice, jg = g / kWaves;
+  if (w == g % kWaves) {
+    const float mc = s.cmax[c];
+    uint64_t q[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      float x = 0.0f;
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) x = (uint32_t)j == jg ? xs[j * VEC + e] : x;
+      q[e] = quantized_weight(x, mc, rp.inv_t);
+    }
+    uint32_t e_hit;
+    if (lane == slice_hit<VEC>(q, s.slice_within, e_hit))
+      write_result(a, row, c * CHUNK + jg * SLAB + tid * VEC + e_hit, s.pd, s.row_kept);
+  }
+}
+
 // ---- rows whose cut the candidate lists cannot hold -------------------------
 //
 // A sampled row that keeps many tokens (no top-k, or one past kListTopK, with
@@ -3202,6 +3316,8 @@ static_assert(kCutGroups == 32 && kCutBins == 2 * kThreads);
 constexpr uint32_t kCutAll = 0x100u;    // every row takes the passes by its policy
 constexpr uint32_t kCutPlain = 0x200u;  // no row is penalized, the vocabulary holds a vector
 constexpr uint32_t kCutKept = 0x400u;   // kept outputs are asked for
+constexpr uint32_t kCutUncut = 0x800u;  // cut_draw_kernel draws the uncut rows
+constexpr uint32_t kCutSmall = 0x1000u; // listed rows may take merge_small_row
 
 struct __align__(16) CutHistLds {
   PrepLds prep;
@@ -3367,6 +3483,20 @@ __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader
   return r;
 }
 
+// Whether the passes take the row (h: its chunk summaries, one a lane in every
+// wave): by its policy, or a min-p row of whose candidate lists some overflowed
+// or which hold more than the general merge in the chunks that reach the
+// floor.
+__device__ __forceinline__ bool cut_takes(const RowParams &rp, const BlockHeader &h, uint32_t S) {
+  if (!cut_pass_row(rp)) return false;
+  if (!(rp.flags & kRowMinP)) return true;
+  const float M = wave_max_f32(h.maximum);
+  const uint32_t thr = logit_key(__builtin_fminf(M + rp.minp_offset, M));
+  const bool in = lane_id() < S;
+  return ballot(in && h.overflow != 0) != 0 ||
+         wave_sum_u32(in && logit_key(h.maximum) >= thr ? h.count : 0u) > kMergeItems;
+}
+
 // Bound by the weights' arithmetic (about 30 VALU instructions a token) and
 // the Infinity Cache's reads. LDS atomics only for the tokens inside the bins'
 // range: for top-p alone the range leaves out every token that all together
@@ -3383,10 +3513,7 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const BlockHeader h = headers[(uint64_t)row * S + min(lane, S - 1)];
   const RowParams rp = load_row_policy(params + row);
-  if (!(bits & kCutAll)) {
-    if (!cut_pass_row(rp)) return;
-    if (!wide_row(rp.flags, rp.top_k) && states[row].stage != kRowWide) return;
-  }
+  if (!(bits & kCutAll) && !cut_takes(rp, h, S)) return;
   float xs[TPL];
   cut_load<DT>(a, logits, stride, V, row, chunk, (bits & kCutPlain) != 0, rp, s, xs);
 #pragma unroll
@@ -3513,14 +3640,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(
   const BlockHeader h = headers[(uint64_t)row * S + min(lane, S - 1)];
   const ulonglong2 own = *(const ulonglong2 *)(area + 2 * tid);
   const RowParams rp = load_row_policy(params + row);
-  if (!(bits & kCutAll)) {
-    if (!cut_pass_row(rp)) return;
-    if (!wide_row(rp.flags, rp.top_k)) {
-      // (The row's first block marks it kRowGather while others still start.)
-      const uint32_t stage = states[row].stage;
-      if (stage != kRowWide && stage != kRowGather) return;
-    }
-  }
+  if (!(bits & kCutAll) && !cut_takes(rp, h, S)) return;
   const bool counts = cut_counts(rp, bits);
   uint2 own_n = make_uint2(0u, 0u);
   if (counts) own_n = ((const uint2 *)(area + kCutBinCountWord))[tid];
@@ -3681,7 +3801,15 @@ __device__ __forceinline__ void cut_resolve(const RowParams &rp, const RowState 
 }
 
 #if JF_IN(3)
-__shared__ CutLds g_cut_lds;
+// cut_draw_kernel's LDS: of the cut passes' rows, the listed ones, the uncut.
+union __align__(16) FinishLds {
+  CutLds cut;
+  Lds merge;
+  UncutLds uncut;
+  __device__ FinishLds() {}
+};
+__shared__ FinishLds g_finish_lds;
+#define g_cut_lds g_finish_lds.cut
 __shared__ SampleLaunch g_cut_launch;
 
 // The tokens of the row's boundary bins in chunk `c`, from the `skip`-th on in
@@ -3885,12 +4013,67 @@ __device__ __forceinline__ void cut_pick(const SampleLaunch &a, uint32_t row, ui
   }
 }
 
+// The general merge, out of line like the rescan.
+template <int DT>
+__device__ __noinline__ void cut_finish_general(uint32_t row) {
+  const RowParams rp = g_cut_launch.params[row];
+  merge_row<DT>(g_cut_launch, rp, row, g_finish_lds.merge);
+}
+
+__device__ __forceinline__ void cut_copy_launch(const SampleLaunch &a) {
+  const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
+  uint32_t *dst = reinterpret_cast<uint32_t *>(&g_cut_launch);
+  for (uint32_t k = threadIdx.x; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
+  __syncthreads();
+}
+
+// A row of the launch that the passes do not take: a listed or greedy row as
+// the merge finishes it, an undrafted row with no cut as uncut_kernel does.
+template <int DT>
+__device__ __forceinline__ void cut_finish_other(const SampleLaunch &a, const RowParams &rp,
+                                                 uint32_t bits, uint32_t row) {
+  const uint32_t S = bits & 0xffu, tid = threadIdx.x, lane = tid & 63;
+  if (uncut_row(rp)) {
+    if (!(bits & kCutUncut)) return;
+    UncutLds &s = g_finish_lds.uncut;
+    const float u = row_uniform(a, row);
+    const BlockHeader h = a.headers[(uint64_t)row * S + min(lane, S - 1)];
+    const uint64_t mass = a.partials[(uint64_t)row * S + min(lane, S - 1)].v[0];
+    if (tid < 64) uncut_row_sums(lane < S, h.maximum, h.admitted, h.count, mass, rp.inv_t, s);
+    __syncthreads();
+    const uint64_t W = s.row_mass;
+    if (!s.row_admitted || W == 0) {
+      if (tid == 0) write_result(a, row, kNoToken, 0.0f, s.row_kept);
+      return;
+    }
+    uncut_draw<DT>(a, rp, row, s, W, u);
+    return;
+  }
+  if (!(bits & kCutSmall)) {
+    cut_copy_launch(a);
+    cut_finish_general<DT>(row);
+    return;
+  }
+  merge_small_row<DT, 10>(
+      a.headers, a.cands, a.params, a.uniforms, a.uniform_index,
+      S | (a.row_indexed ? 0x80000000u : 0u), (uint32_t)a.uniform_offset,
+      (uint32_t)a.uniform_stride, a.draft_tokens && !a.row_indexed ? a.drafted_rows : 0u, a, row,
+      g_finish_lds.merge, [&]() {
+        cut_copy_launch(a);
+        cut_finish_general<DT>(row);
+      });
+}
+
+// OTHERS: also finishes every other row of the launch (listed, greedy,
+// undrafted uncut), so that a batch of several kinds takes no merge and no
+// uncut launch (24 rows x 100,003: 46.4 -> 34.9 us a call). A separate build,
+// since that code costs the cut passes' rows 1.5 us (9.9 against 11.4).
 // Latency-bound: a block a row. Its registers (the rescan's) cost nothing
 // here, where a chunk-parallel kernel would run two waves a SIMD for them. The
 // row's record, its boundary bins and its chunks' sums go out together from
 // preloaded arguments; up to 64 listed tokens (most rows) are resolved by one
 // wave without a barrier.
-template <int DT>
+template <int DT, bool OTHERS>
 __global__ __launch_bounds__(kThreads) void cut_draw_kernel(
     const RowParams *params, const RowState *states, const uint64_t *cands,
     const float *uniforms, const uint32_t *uniform_index, const uint32_t *draft_tokens,
@@ -3904,7 +4087,18 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(
   const uint32_t at = uniform_index ? uniform_index[row] : 0u;
   const RowParams rp = load_row_policy(params + row);
   const RowState st = load_const(states + row);
-  if (!cut_pass_row(rp) || st.stage != kRowGather) return;
+  bool taken = wide_row(rp.flags, rp.top_k);
+  if (!taken && cut_pass_row(rp)) {
+    const BlockHeader h = a.headers[(uint64_t)row * S + min(lane, S - 1)];
+    taken = cut_takes(rp, h, S);
+    // (An earlier call's mark must not reach cut_emit_kernel.)
+    if (!taken && tid == 0) a.states[row].stage = kRowDone;
+  }
+  if (!taken) {
+    if constexpr (OTHERS) cut_finish_other<DT>(a, rp, bits, row);
+    return;
+  }
+  if (st.stage != kRowGather) return;
   const float u =
       uniforms[uniform_index ? (uint64_t)at : a.uniform_offset + row * a.uniform_stride];
   const bool counts = (bits & kCutKept) != 0, listed = cut_counts(rp, bits);
@@ -3943,10 +4137,7 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(
   const uint32_t n = s.n;
   if (n > 64u) {
     if (n == 0xffffffffu) {
-      const uint32_t *src = reinterpret_cast<const uint32_t *>(&a);
-      uint32_t *dst = reinterpret_cast<uint32_t *>(&g_cut_launch);
-      for (uint32_t k = tid; k < sizeof(SampleLaunch) / 4; k += kThreads) dst[k] = src[k];
-      __syncthreads();
+      cut_copy_launch(a);
       cut_rescan<DT>(row);
     } else {
       // Past the items' room in LDS, the rest stays in the lists.
@@ -4113,30 +4304,6 @@ __global__ __launch_bounds__(kThreads) void cut_emit_kernel(
 // float weight against m_c; v[kResidualSlot] the chunk's residual mass and
 // v[kResidualSlot + 1 + g] its slices' (slice g = load g / kWaves of wave
 // g % kWaves, 64 x VEC consecutive tokens, so g runs in id order).
-struct __align__(16) UncutLds {
-  PrepLds prep;
-  uint64_t wj[kWaves][8];
-  uint64_t wl[kWaves];
-  uint32_t cids[16];
-  float cprobs[16];
-  float cmax[kMaxChunks];       // the row's chunk maxima
-  uint64_t cscale[kMaxChunks];  // r_c, packed s_c << 32 | R_c
-  uint64_t ctot[kMaxChunks];    // T_c
-  uint32_t ccount[kMaxChunks];  // admitted (non-NaN) tokens per chunk
-  uint64_t slices[kWaves * 8];  // one chunk's slice masses
-  float row_max;
-  uint64_t row_mass;
-  uint32_t row_admitted;
-  uint32_t row_kept;
-  float pd;                     // p(draft)
-  uint32_t residual;
-  uint32_t last;
-  uint32_t sel_bin;
-  uint64_t sel_excl;
-  uint32_t slice;
-  uint64_t slice_within;
-};
-
 #if JF_IN(4)
 constexpr uint32_t kDraftSlot = 40;
 constexpr uint32_t kResidualSlot = 63;
@@ -4190,64 +4357,6 @@ __device__ __forceinline__ void uncut_kept(const SampleLaunch &a, const RowParam
       }
       written += (uint32_t)total;
     }
-  }
-}
-
-// The plain draw of an uncut row from its chunk masses (one block; block-
-// uniform): the chunk, its reload together with its slice masses (which the
-// select pass wrote), the slice, the token.
-template <int DT>
-__device__ __forceinline__ void uncut_draw(const SampleLaunch &a, const RowParams &rp,
-                                           uint32_t row, UncutLds &s, uint64_t W, float u) {
-  constexpr int TPL = Geo<DT>::TPL, VEC = Geo<DT>::VEC, LOADS = Geo<DT>::LOADS,
-                SLAB = Geo<DT>::SLAB;
-  constexpr uint32_t CHUNK = Geo<DT>::CHUNK, G = LOADS * kWaves;
-  const uint32_t S = a.chunks, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  if (w == 0) {
-    const bool in = lane < S;
-    const uint64_t T = in ? s.ctot[lane] : 0ull;
-    const uint64_t incl = wave_incl_scan_u64(T);
-    uint64_t target = floor_mul(W, u);
-    if (target >= W) target = W - 1;
-    // incl at the last lane is W > target: some lane passes it.
-    const uint32_t c = (uint32_t)__builtin_ctzll(ballot(in && incl > target));
-    const uint64_t within = target - readlane_u64(incl - T, c);
-    if (lane == 0) {
-      s.sel_bin = c;
-      // The running mass inside chunk c (against m_c) that the token's
-      // prefix must pass: floor(P * r_c) > within <=> P > this.
-      s.sel_excl = unscaled_bound(within, s.cscale[c]);
-    }
-  }
-  __syncthreads();
-  const uint32_t c = s.sel_bin;
-  uint64_t vg = 0;
-  if (w == 0 && lane < G) vg = a.partials[(uint64_t)row * S + c].v[1 + lane];
-  float xs[TPL];
-  load_chunk<DT>(a, rp, row, c, s, xs);
-  if (w == 0) {
-    uint64_t wi = s.sel_excl;
-    const uint32_t gg = pick_slice(vg, G, wi);
-    if (lane == 0) {
-      s.slice = gg;
-      s.slice_within = wi;
-    }
-  }
-  __syncthreads();
-  const uint32_t g = s.slice, jg = g / kWaves;
-  if (w == g % kWaves) {
-    const float mc = s.cmax[c];
-    uint64_t q[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      float x = 0.0f;
-#pragma unroll
-      for (int j = 0; j < LOADS; ++j) x = (uint32_t)j == jg ? xs[j * VEC + e] : x;
-      q[e] = quantized_weight(x, mc, rp.inv_t);
-    }
-    uint32_t e_hit;
-    if (lane == slice_hit<VEC>(q, s.slice_within, e_hit))
-      write_result(a, row, c * CHUNK + jg * SLAB + tid * VEC + e_hit, s.pd, s.row_kept);
   }
 }
 
@@ -4702,32 +4811,7 @@ __global__ __launch_bounds__(kThreads) void uncut_kernel(SampleLaunch a, uint32_
   if (!drafted && chunk != 0) return;
   const float inv_t = rp.inv_t;
   // The row's chunk summaries.
-  if (w == 0) {
-    const float m = in ? hm : -3.402823466e38f;
-    const uint32_t adm = in ? hadm : 0u;
-    const uint32_t cnt = in ? hcnt : 0u;
-    const uint64_t mass = in ? hmass : 0ull;
-    const float M = wave_max_f32(m);
-    const uint64_t R = in ? chunk_scale(m, M, inv_t) : kZeroScale;
-    const uint64_t T = scale_by(mass, R);
-    const uint64_t W = wave_sum_u64(T);
-    const uint32_t admitted = wave_sum_u32(adm), kept = wave_sum_u32(cnt);
-    if (in) {
-      s.cmax[lane] = m;
-      s.cscale[lane] = R;
-      s.ctot[lane] = T;
-      s.ccount[lane] = cnt;
-    }
-    if (lane == 0) {
-      s.row_max = M;
-      s.row_mass = W;
-      // Nothing admitted, or a +inf maximum: the sentinel with nothing kept.
-      const bool none = admitted == 0 || M == __builtin_inff();
-      s.row_admitted = none ? 0u : 1u;
-      s.row_kept = none ? 0u : kept;
-      s.pd = 0.0f;
-    }
-  }
+  if (w == 0) uncut_row_sums(lane < S, hm, hadm, hcnt, hmass, inv_t, s);
   __syncthreads();
   const uint64_t W = s.row_mass;
   if (chunk == 0 && a.out_kept_ids && s.row_admitted && a.kept_cap)
@@ -5131,7 +5215,8 @@ int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *
   const hipStream_t st = (hipStream_t)stream;
   const uint32_t bits = a.chunks | (c.all ? kCutAll : 0u) |
                         (c.plain && a.vocabulary >= 8 ? kCutPlain : 0u) |
-                        (a.out_kept_ids ? kCutKept : 0u);
+                        (a.out_kept_ids ? kCutKept : 0u) | (c.uncut ? kCutUncut : 0u) |
+                        (c.small ? kCutSmall : 0u);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, st, a.logits, a.params,
                        (const BlockHeader *)a.headers, a.cands, a.states, a.stride, a.vocabulary,
@@ -5146,7 +5231,10 @@ int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *
   };
   hipError_t e = dtype == 0 ? go(cut_hist_kernel<0>) : go(cut_hist_kernel<1>);
   if (e == hipSuccess) e = dtype == 0 ? go(cut_list_kernel<0>) : go(cut_list_kernel<1>);
-  if (e == hipSuccess) e = dtype == 0 ? draw(cut_draw_kernel<0>) : draw(cut_draw_kernel<1>);
+  if (e == hipSuccess && c.others)
+    e = dtype == 0 ? draw(cut_draw_kernel<0, true>) : draw(cut_draw_kernel<1, true>);
+  else if (e == hipSuccess)
+    e = dtype == 0 ? draw(cut_draw_kernel<0, false>) : draw(cut_draw_kernel<1, false>);
   if (e == hipSuccess && c.drafted)
     e = dtype == 0 ? go(cut_emit_kernel<0, true>) : go(cut_emit_kernel<1, true>);
   else if (e == hipSuccess && a.out_kept_ids)

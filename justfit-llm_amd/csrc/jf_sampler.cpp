@@ -851,7 +851,7 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   bool any_uncut = false, any_cut = false, any_greedy = false, uncut_drafted = false;
   // any_listed: cut rows of the merge; passes: rows that take the cut passes,
   // or may (min-p rows whose candidates may outgrow the lists).
-  bool any_listed = false, passes = false;
+  bool any_listed = false, any_wide = false, passes = false;
   for (uint32_t r = 0; r < rows; ++r) {
     const jf::RowParams &rp = params[r];
     if (!(rp.flags & jf::kRowSampled)) {
@@ -863,6 +863,7 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
       any_cut = true;
       const bool wide = jf::wide_row(rp.flags, rp.top_k);
       any_listed |= !wide;
+      any_wide |= wide;
       passes |= wide || rp.top_k > (uint32_t)jf::kBlockCandidates;
     }
   }
@@ -874,9 +875,16 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     fuse_uncut = !(params[r].flags & jf::kRowPenalized) && !params[r].extra_count;
   // The merge finishes the cut rows with candidate lists, and the greedy rows
   // unless the launch is all greedy and fast (fused) or has uncut rows and no
-  // listed ones (then uncut_kernel takes them).
-  const bool need_merge = !fused && (any_listed || (any_greedy && !any_uncut));
-  L.finish_greedy = any_greedy && !need_merge && !fused ? 1u : 0u;
+  // listed ones (then uncut_kernel takes them). A launch with rows that take
+  // the cut passes by their policy and others ends in cut_draw_kernel, which
+  // finishes the others too: no merge, and no uncut launch unless some uncut
+  // row is drafted or kept tokens are asked for. (Min-p rows alone, which
+  // mostly fit their lists, keep the merge: 64 rows x 248,320 bf16 ran 22.6 us
+  // with it, 24.7 through cut_draw_kernel.)
+  const bool others = any_wide && (any_listed || any_greedy || any_uncut);
+  const bool need_merge = !fused && !others && (any_listed || (any_greedy && !any_uncut));
+  L.finish_greedy = any_greedy && !need_merge && !fused && !others ? 1u : 0u;
+  const bool pass_uncut = others && !kept && !uncut_drafted && !n_lean;
   if (!fast) {
     e = jf::launch_select(L, a->dtype, stream, a->select_start_event,
                           split ? nullptr : a->select_done_event);
@@ -962,7 +970,7 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     if (e != hipSuccess) return hip_fail((hipError_t)e, "merge launch");
   }
   if (passes) {
-    jf::CutLaunch c{true, true, any_drafted};
+    jf::CutLaunch c{true, true, any_drafted, others, pass_uncut, small};
     for (uint32_t r = 0; r < rows; ++r) {
       c.all &= jf::wide_row(params[r].flags, params[r].top_k);
       c.plain &= !(params[r].flags & jf::kRowPenalized);
@@ -970,7 +978,7 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     e = jf::launch_cut(L, a->dtype, c, stream);
     if (e != hipSuccess) return hip_fail((hipError_t)e, "cut pass launch");
   }
-  if (any_uncut && !fuse_uncut) {
+  if (any_uncut && !fuse_uncut && !pass_uncut) {
     // residual_kernel over the kRowLean rows, then uncut_kernel: one block
     // per row, or one per (row, chunk) when other drafted uncut rows need
     // their residual pass there. A launch with lean rows and no cut row,
