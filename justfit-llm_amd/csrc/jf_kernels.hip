@@ -999,121 +999,18 @@ __device__ __forceinline__ void wave_finish(const SampleLaunch &a, const RowPara
     write_result(a, row, token, drafted && fm ? (float)((double)fw / scale) : 0.0f, n3);
 }
 
-// A sampled row from its candidate lists, whatever they hold: the tokens at or
-// above its threshold as items in LDS, the top-k and top-p boundaries by
-// items_crossing, and the draw by items_crossing over the ids. A min-p row
-// with a top-k past the lists whose tokens they, or LDS, cannot hold is left to
-// the cut passes (cut_takes).
+// A sampled row's tokens at or above its threshold as the `n` items in
+// s.general.items (of which those below `bound` are not kept): the cuts, the
+// draw and the outputs. s.cids/s.cprobs hold a sparse draft's candidates.
 template <int DT>
-__device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowParams &rp,
-                              uint32_t row, Lds &s) {
-  const uint32_t S = a.chunks, tid = threadIdx.x, lane = tid & 63;
-  const BlockHeader *hb = a.headers + (uint64_t)row * S;
-  const uint64_t *lists = a.cands + (uint64_t)row * S * kBlockCandidates;
-  const float u = row_uniform(a, row);
-  const uint32_t draft = row_draft(a, rp);
-  const uint32_t K = rp.top_k;
-  stage_candidates(a, rp, s);
-  if (tid < 64) {
-    const bool in = lane < S;
-    const BlockHeader h = hb[min(lane, S - 1)];
-    const float mx = wave_max_f32(in ? h.maximum : -3.402823466e38f);
-    const uint32_t adm = wave_max_u32(in ? h.admitted : 0u),
-                   flr = wave_max_u32(in ? h.floor_key : 0u);
-    const uint64_t omask = ballot(in && h.overflow != 0);
-    if (in) {
-      s.hcnt[lane] = h.count;
-      s.hmax[lane] = h.maximum;
-    }
-    if (lane == 0) {
-      s.u64a = omask;
-      s.row_max = mx;
-      s.row_admitted = adm;
-      s.row_floor = flr;
-    }
-  }
-  __syncthreads();
-  const float M = s.row_max, inv_t = rp.inv_t;
-  if (s.row_admitted == 0 || M == __builtin_inff()) {
-    if (tid == 0) write_result(a, row, kNoToken, 0.0f, 0);
-    return;
-  }
-  // The K-th key of the row is at least every chunk's floor.
-  uint32_t thr =
-      (rp.flags & kRowMinP) ? logit_key(__builtin_fminf(M + rp.minp_offset, M)) : 0u;
-  if (rp.flags & kRowTopK) thr = max(thr, s.row_floor);
-  uint64_t om = s.u64a;
-  const bool overflow = om != 0;
-  if (overflow && K <= (uint32_t)kBlockCandidates) {
-    // Chunks with more candidates than their lists hold (flat or tied
-    // values): select each again.
-    while (om) {
-      const uint32_t c = (uint32_t)__builtin_ctzll(om);
-      om &= om - 1;
-      const uint32_t n = reselect_chunk<DT>(a, rp, row, c, thr, K, s);
-      if (tid == 0) s.hcnt[c] = n;
-    }
-    __syncthreads();
-  }
-  // The lists of the chunks whose maximum reaches the threshold, end to end.
-  if (tid < 64) {
-    const bool use = lane < S && logit_key(s.hmax[lane]) >= thr;
-    const uint32_t incl = wave_incl_scan_u32(use ? s.hcnt[lane] : 0u);
-    if (lane < S) s.hoff[lane + 1] = incl;
-    if (lane == 0) {
-      s.hoff[0] = 0;
-      s.n = 0;
-    }
-  }
-  __syncthreads();
-  const uint32_t n_all = s.hoff[S];
-  if (K > (uint32_t)kBlockCandidates && (overflow || n_all > kMergeItems)) return;  // cut_takes
+__device__ __forceinline__ void merge_items(const SampleLaunch &a, const RowParams &rp,
+                                            uint32_t row, uint32_t n, uint64_t bound, float M,
+                                            float u, uint32_t draft, Lds &s) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63, K = rp.top_k;
+  const float inv_t = rp.inv_t;
   ItemsLds &g = s.general;
-  auto listed = [&](uint32_t i) -> uint64_t {
-    uint32_t c = 0;
-    for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
-      if (c + step < S && s.hoff[c + step] <= i) c += step;
-    return lists[(uint64_t)c * kBlockCandidates + (i - s.hoff[c])];
-  };
-  // The items at or above `thr` whose word reaches `from`, into LDS; those
-  // past its room are counted only.
-  auto gather = [&](uint64_t from) {
-    constexpr uint32_t B = 4;
-    for (uint32_t i0 = tid; i0 < n_all; i0 += B * kThreads) {
-      uint64_t v[B];
-#pragma unroll
-      for (uint32_t k = 0; k < B; ++k)
-        v[k] = i0 + k * kThreads < n_all ? listed(i0 + k * kThreads) : 0ull;
-#pragma unroll
-      for (uint32_t k = 0; k < B; ++k) {
-        const uint64_t c = token_item((uint32_t)v[k], (uint32_t)(v[k] >> 32));
-        if (i0 + k * kThreads < n_all && (uint32_t)v[k] >= thr && c >= from) {
-          const uint32_t at = atomicAdd(&s.n, 1u);
-          if (at < kMergeItems) g.items[at] = c;
-        }
-      }
-    }
-    __syncthreads();
-  };
   auto ord = [](uint64_t c) { return c; };
   auto weight = [&](uint64_t c) { return item_weight(c, M, inv_t); };
-  gather(0);
-  uint32_t n = s.n;
-  uint64_t bound = 0;  // the kept set's last item
-  if (n > kMergeItems) {
-    // (K fits.) The K-th item straight from the lists.
-    auto all = [&](auto f) {
-      for (uint32_t i = tid; i < n_all; i += kThreads) {
-        const uint64_t v = listed(i);
-        if ((uint32_t)v >= thr) f(token_item((uint32_t)v, (uint32_t)(v >> 32)));
-      }
-    };
-    bound = items_crossing(all, [](uint64_t) { return true; }, ord, weight, false, K, s);
-    if (tid == 0) s.n = 0;
-    __syncthreads();
-    gather(bound);
-    n = s.n;
-  }
   auto each = [&](auto f) {
     for (uint32_t i = tid; i < n; i += kThreads) f(g.items[i]);
   };
@@ -1231,6 +1128,124 @@ __device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowPa
                : items_crossing(each, in, by_id, weight, true, target + 1, s);
   if (tid == 0)
     write_result(a, row, item_id(hit), drafted ? (float)((double)s.found_w / scale) : 0.0f, kept);
+}
+
+// A sampled row from its candidate lists, whatever they hold: the tokens at or
+// above its threshold as items in LDS, the top-k and top-p boundaries by
+// items_crossing, and the draw by items_crossing over the ids. A min-p row
+// with a top-k past the lists whose tokens they, or LDS, cannot hold is left to
+// the cut passes (cut_takes).
+template <int DT>
+__device__ __forceinline__ void merge_sampled(const SampleLaunch &a, const RowParams &rp,
+                              uint32_t row, Lds &s) {
+  const uint32_t S = a.chunks, tid = threadIdx.x, lane = tid & 63;
+  const BlockHeader *hb = a.headers + (uint64_t)row * S;
+  const uint64_t *lists = a.cands + (uint64_t)row * S * kBlockCandidates;
+  const float u = row_uniform(a, row);
+  const uint32_t draft = row_draft(a, rp);
+  const uint32_t K = rp.top_k;
+  stage_candidates(a, rp, s);
+  if (tid < 64) {
+    const bool in = lane < S;
+    const BlockHeader h = hb[min(lane, S - 1)];
+    const float mx = wave_max_f32(in ? h.maximum : -3.402823466e38f);
+    const uint32_t adm = wave_max_u32(in ? h.admitted : 0u),
+                   flr = wave_max_u32(in ? h.floor_key : 0u);
+    const uint64_t omask = ballot(in && h.overflow != 0);
+    if (in) {
+      s.hcnt[lane] = h.count;
+      s.hmax[lane] = h.maximum;
+    }
+    if (lane == 0) {
+      s.u64a = omask;
+      s.row_max = mx;
+      s.row_admitted = adm;
+      s.row_floor = flr;
+    }
+  }
+  __syncthreads();
+  const float M = s.row_max, inv_t = rp.inv_t;
+  if (s.row_admitted == 0 || M == __builtin_inff()) {
+    if (tid == 0) write_result(a, row, kNoToken, 0.0f, 0);
+    return;
+  }
+  // The K-th key of the row is at least every chunk's floor.
+  uint32_t thr =
+      (rp.flags & kRowMinP) ? logit_key(__builtin_fminf(M + rp.minp_offset, M)) : 0u;
+  if (rp.flags & kRowTopK) thr = max(thr, s.row_floor);
+  uint64_t om = s.u64a;
+  const bool overflow = om != 0;
+  if (overflow && K <= (uint32_t)kBlockCandidates) {
+    // Chunks with more candidates than their lists hold (flat or tied
+    // values): select each again.
+    while (om) {
+      const uint32_t c = (uint32_t)__builtin_ctzll(om);
+      om &= om - 1;
+      const uint32_t n = reselect_chunk<DT>(a, rp, row, c, thr, K, s);
+      if (tid == 0) s.hcnt[c] = n;
+    }
+    __syncthreads();
+  }
+  // The lists of the chunks whose maximum reaches the threshold, end to end.
+  if (tid < 64) {
+    const bool use = lane < S && logit_key(s.hmax[lane]) >= thr;
+    const uint32_t incl = wave_incl_scan_u32(use ? s.hcnt[lane] : 0u);
+    if (lane < S) s.hoff[lane + 1] = incl;
+    if (lane == 0) {
+      s.hoff[0] = 0;
+      s.n = 0;
+    }
+  }
+  __syncthreads();
+  const uint32_t n_all = s.hoff[S];
+  if (K > (uint32_t)kBlockCandidates && (overflow || n_all > kMergeItems)) return;  // cut_takes
+  ItemsLds &g = s.general;
+  auto listed = [&](uint32_t i) -> uint64_t {
+    uint32_t c = 0;
+    for (uint32_t step = kMaxChunks / 2; step; step >>= 1)
+      if (c + step < S && s.hoff[c + step] <= i) c += step;
+    return lists[(uint64_t)c * kBlockCandidates + (i - s.hoff[c])];
+  };
+  // The items at or above `thr` whose word reaches `from`, into LDS; those
+  // past its room are counted only.
+  auto gather = [&](uint64_t from) {
+    constexpr uint32_t B = 4;
+    for (uint32_t i0 = tid; i0 < n_all; i0 += B * kThreads) {
+      uint64_t v[B];
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k)
+        v[k] = i0 + k * kThreads < n_all ? listed(i0 + k * kThreads) : 0ull;
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k) {
+        const uint64_t c = token_item((uint32_t)v[k], (uint32_t)(v[k] >> 32));
+        if (i0 + k * kThreads < n_all && (uint32_t)v[k] >= thr && c >= from) {
+          const uint32_t at = atomicAdd(&s.n, 1u);
+          if (at < kMergeItems) g.items[at] = c;
+        }
+      }
+    }
+    __syncthreads();
+  };
+  auto ord = [](uint64_t c) { return c; };
+  auto weight = [&](uint64_t c) { return item_weight(c, M, inv_t); };
+  gather(0);
+  uint32_t n = s.n;
+  uint64_t bound = 0;  // the kept set's last item
+  if (n > kMergeItems) {
+    // (K fits.) The K-th item straight from the lists.
+    auto all = [&](auto f) {
+      for (uint32_t i = tid; i < n_all; i += kThreads) {
+        const uint64_t v = listed(i);
+        if ((uint32_t)v >= thr) f(token_item((uint32_t)v, (uint32_t)(v >> 32)));
+      }
+    };
+    bound = items_crossing(all, [](uint64_t) { return true; }, ord, weight, false, K, s);
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+    gather(bound);
+    n = s.n;
+  }
+  merge_items<DT>(a, rp, row, n, bound, M, u, draft, s);
 }
 
 // Every thread's device-coherent stores complete, then one arrival; true in
@@ -2805,10 +2820,14 @@ __device__ __forceinline__ int rank_select(const uint64_t (&v)[PER], uint32_t va
 __shared__ Lds g_small_lds;
 __shared__ SampleLaunch g_small_launch;
 template <int DT>
-__device__ __noinline__ void merge_small_general(uint32_t row) {
+__device__ __noinline__ void merge_small_general(uint32_t row, uint32_t n) {
   const SampleLaunch &a = g_small_launch;
   const RowParams rp = a.params[row];
-  merge_sampled<DT>(a, rp, row, g_small_lds);
+  if (n == kNoToken)
+    merge_sampled<DT>(a, rp, row, g_small_lds);
+  else
+    merge_items<DT>(a, rp, row, n, 0, g_small_lds.row_max, row_uniform(a, row), row_draft(a, rp),
+                    g_small_lds);
 }
 #endif
 
@@ -2823,7 +2842,8 @@ __device__ __noinline__ void merge_small_general(uint32_t row) {
 // slots a chunk (134 at 19 chunks); 20 gives floor(5120 / S) (165 at 31
 // chunks), for vocabularies past 163,840 tokens whose cut rows have no
 // min-p floor (their lists average about 75 candidates and reach 130).
-// `general`: the general merge of the row, called by every thread.
+// `general`: the general merge of the row, called by every thread: from the n
+// items in s.general.items, or (kNoToken) from the candidate lists.
 template <int DT, int SPEC, class General>
 __device__ __forceinline__ void merge_small_row(
     const BlockHeader *headers, const uint64_t *cands, const RowParams *params,
@@ -3026,10 +3046,26 @@ __device__ __forceinline__ void merge_small_row(
       if (tid < 64) wave_finish(a, rp, row, s, (uint32_t)got, maximum, u, draft);
       return;
     }
+    // More than 64 of them kept, or values that do not spread: the general
+    // merge, from the items this block already holds.
     __syncthreads();
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SPEC; ++k)
+      if ((valid >> k) & 1) {
+        const uint32_t at = atomicAdd(&s.n, 1u);
+        if (at < kMergeItems)
+          s.general.items[at] = token_item((uint32_t)sv[k], (uint32_t)(sv[k] >> 32));
+      }
+    __syncthreads();
+    if (s.n <= kMergeItems) {
+      general(s.n);
+      return;
+    }
   }
   // What the speculative fetch does not cover.
-  general();
+  general(kNoToken);
 }
 
 #if JF_IN(2)
@@ -3041,7 +3077,7 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
   const uint32_t row = blockIdx.x;
   merge_small_row<DT, SPEC>(
       headers, cands, params, uniforms, uniform_index, chunks_bits, uniform_offset,
-      uniform_stride, drafted_rows, a, row, g_small_lds, [&]() {
+      uniform_stride, drafted_rows, a, row, g_small_lds, [&](uint32_t n) {
         // The launch record is copied word by word from the argument segment
         // here (one word a thread), so no field of it stays live from the
         // kernel's entry (the compiler otherwise kept some in private memory
@@ -3051,7 +3087,7 @@ __global__ __launch_bounds__(kThreads) void merge_small_kernel(
         for (uint32_t k = threadIdx.x; k < sizeof(SampleLaunch) / 4; k += kThreads)
           dst[k] = src[k];
         __syncthreads();
-        merge_small_general<DT>(row);
+        merge_small_general<DT>(row, n);
       });
 }
 #endif
@@ -4015,9 +4051,14 @@ __device__ __forceinline__ void cut_pick(const SampleLaunch &a, uint32_t row, ui
 
 // The general merge, out of line like the rescan.
 template <int DT>
-__device__ __noinline__ void cut_finish_general(uint32_t row) {
+__device__ __noinline__ void cut_finish_general(uint32_t row, uint32_t n) {
   const RowParams rp = g_cut_launch.params[row];
-  merge_row<DT>(g_cut_launch, rp, row, g_finish_lds.merge);
+  if (n == kNoToken)
+    merge_row<DT>(g_cut_launch, rp, row, g_finish_lds.merge);
+  else
+    merge_items<DT>(g_cut_launch, rp, row, n, 0, g_finish_lds.merge.row_max,
+                    row_uniform(g_cut_launch, row), row_draft(g_cut_launch, rp),
+                    g_finish_lds.merge);
 }
 
 __device__ __forceinline__ void cut_copy_launch(const SampleLaunch &a) {
@@ -4051,16 +4092,16 @@ __device__ __forceinline__ void cut_finish_other(const SampleLaunch &a, const Ro
   }
   if (!(bits & kCutSmall)) {
     cut_copy_launch(a);
-    cut_finish_general<DT>(row);
+    cut_finish_general<DT>(row, kNoToken);
     return;
   }
   merge_small_row<DT, 10>(
       a.headers, a.cands, a.params, a.uniforms, a.uniform_index,
       S | (a.row_indexed ? 0x80000000u : 0u), (uint32_t)a.uniform_offset,
       (uint32_t)a.uniform_stride, a.draft_tokens && !a.row_indexed ? a.drafted_rows : 0u, a, row,
-      g_finish_lds.merge, [&]() {
+      g_finish_lds.merge, [&](uint32_t n) {
         cut_copy_launch(a);
-        cut_finish_general<DT>(row);
+        cut_finish_general<DT>(row, n);
       });
 }
 
