@@ -40,9 +40,9 @@ def parse():
                          "V=248320, extras and sparse drafts) plus chain acceptance")
     ap.add_argument("--mode", default="auto",
                     help="C3/C4: greedy or sampled (auto: sampled); C2: general runs "
-                         "C2's batch through the general kernels (rows one float past "
-                         "16-byte alignment, top-k 3000: select_kernel, merge_kernel "
-                         "and the multi-pass stages)")
+                         "C2's batch with rows one float past 16-byte alignment and "
+                         "top-k 3000, past the candidate lists: the unaligned select "
+                         "pass and the cut passes")
     ap.add_argument("--cpu-seconds", type=float, default=20.0,
                     help="bound of the CPU-baseline sample")
     ap.add_argument("--history", default="uniform", choices=["uniform", "zipf", "mixed"],
@@ -88,13 +88,11 @@ def build_workload(cfg, mode, history="uniform"):
         name = ("C2 sampled B=64 V=151936 fp32 T0.7 top-k 50 top-p 0.9 "
                 f"presence 0.5 frequency 0.3 over {label}")
         if mode == "general":
-            # The kernels a call takes when the fast pass and the small merge
-            # cannot: rows whose logits start one float past a 16-byte
-            # boundary (an engine's views into a padded buffer) and a top-k
-            # past the merge's lists.
+            # Rows whose logits start one float past a 16-byte boundary (an
+            # engine's views into a padded buffer) and a top-k past the
+            # candidate lists: the cut passes follow the select pass.
             pol["top_k"] = 3000
             w["unaligned"] = True
-            w["kernel"] = "jf::select_kernel<0>"
             name = name.replace("top-k 50", "top-k 3000") + ", rows 4 bytes past alignment"
         w.update(V=c["V"], logits=c["logits"], policies=[J.policy(**pol)] * B,
                  histories=hists, generated=c["generated"], mark_prompt=False,

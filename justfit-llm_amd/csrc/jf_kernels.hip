@@ -1,8 +1,8 @@
 // gfx950 kernels of JustFit's logits->token path.
 //
 // One selection is one launch of select_kernel over rows x chunks blocks
-// (plus, for rows whose candidates do not fit, the multi-pass stage_kernel
-// launches). Each block holds its chunk of a row in registers: one pass over
+// (plus, for rows whose kept set the candidate lists cannot hold, the cut
+// passes). Each block holds its chunk of a row in registers: one pass over
 // HBM with 16-byte loads, the penalties, the constraint mask and the stop
 // exclusion applied on the fly (the reference's decode_sample_penalize,
 // TargetRow::admits; sampling.metal:33-37, 928-993). A greedy row reduces its
@@ -1573,8 +1573,8 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SampleLaunch a) {
     const uint32_t c = over ? kBlockCandidates + 1 : off[kWaves];
     if (tid == 0) {
       // More candidates than the list holds: the merge selects this chunk
-      // again (with the row's own thresholds) or hands the row to the
-      // multi-pass stages.
+      // again (with the row's own thresholds) or leaves the row to the cut
+      // passes.
       hdr->maximum = bmax;
       hdr->count = min(c, (uint32_t)kBlockCandidates);
       hdr->admitted = badm;

@@ -843,8 +843,8 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   const bool fused = fast && !any_sampled;
   // Sampled rows that keep every admitted token (no min-p, top-k or top-p
   // cut): the selection writes their chunk masses and uncut_kernel draws
-  // them; the merge and the stages finish the other rows and skip these, so
-  // only the cut rows decide the merge and the stages.
+  // them; the merge and the cut passes finish the other rows and skip these,
+  // so only the cut rows decide the merge and the passes.
   constexpr uint32_t kCuts = jf::kRowMinP | jf::kRowTopK | jf::kRowTopP;
   // uncut_drafted: drafted uncut rows whose residual pass stays in
   // uncut_kernel (not kRowLean).
