@@ -3538,6 +3538,9 @@ __device__ __forceinline__ bool cut_takes(const RowParams &rp, const BlockHeader
 // range: for top-p alone the range leaves out every token that all together
 // cannot hold the boundary (minp_offset), which in a language model's row is
 // most of them; they add to the mass from registers.
+// Only those add there: summing every member as well and taking the binned ones
+// off again cost 0.6 us more (64 x 151,936 fp32, top-p 0.95: 41.4 -> 40.8 us a
+// call; 24 mixed rows x 100,003: 35.1 -> 34.5).
 #if JF_IN(3)
 template <int DT>
 __global__ __launch_bounds__(kThreads) void cut_hist_kernel(
@@ -3568,24 +3571,23 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(
   if (rp.flags & kRowMinP)  // members are the tokens at or above the floor
 #pragma unroll
     for (int i = 0; i < TPL; ++i) xs[i] = xs[i] >= r.floor ? xs[i] : kNotAdmitted;
-  uint64_t all = 0, inside = 0;  // the mass of all members, of those below the last bin
+  uint64_t outside = 0;  // the mass of the members in the last bin
   uint32_t tail_n = 0;
 #pragma unroll
   for (int i = 0; i < TPL; ++i) {
     const float d = xs[i] - M;
     const WeightYK y = weight_yk_at(d * inv_t);
     const uint64_t wq = ((uint64_t)y.Y << 32) >> y.k;
-    all += wq;
     const uint32_t b = cut_bin_at(-d, r.scale);  // (NaN, not admitted: the last bin)
     if (b < kCutBins - 1) {
-      inside += wq;
       atomicAdd((unsigned long long *)&s.mass[b], (unsigned long long)wq);
       if (counts) atomicAdd(&s.count[b], 1u);
-    } else if (counts) {
-      tail_n += d == d ? 1u : 0u;
+    } else {
+      outside += wq;
+      if (counts) tail_n += d == d ? 1u : 0u;
     }
   }
-  const uint64_t tail = wave_sum_u64(all - inside);
+  const uint64_t tail = wave_sum_u64(outside);
   if (lane == 0)
     atomicAdd((unsigned long long *)&s.mass[kCutBins - 1], (unsigned long long)tail);
   if (counts) {
