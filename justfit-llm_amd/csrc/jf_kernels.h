@@ -390,7 +390,8 @@ int launch_select_fast(const FastLaunch &f, const FastRows *fr, uint32_t rows, u
 int launch_merge(const SampleLaunch &a, uint32_t dtype, void *stream);
 // wide: some cut row of the launch has no min-p floor (longer candidate
 // lists); the merge then fetches more list slots a chunk where that helps.
-int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, void *stream);
+// hold: some listed row may keep more than 64 tokens.
+int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, bool hold, void *stream);
 // Rows with no cut (grid rows x per_row: per_row = chunks when the launch
 // has drafted uncut rows, else 1).
 int launch_uncut(const SampleLaunch &a, uint32_t dtype, uint32_t per_row, void *stream);

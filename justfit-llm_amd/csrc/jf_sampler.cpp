@@ -958,14 +958,17 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   // none). wide: some listed row has no min-p floor (longer lists).
   const bool small = !a->draft_q && a->uniform_offset <= 0xffffffffull &&
                      a->uniform_stride <= 0xffffffffull;
-  bool wide = false;
+  // hold: some listed row may keep more than 64 tokens (a min-p floor and a
+  // larger top-k, or none).
+  bool wide = false, hold = false;
   for (uint32_t r = 0; r < rows; ++r) {
     const jf::RowParams &rp = params[r];
+    hold |= (rp.flags & jf::kRowMinP) && rp.top_k > 64;
     wide |= (rp.flags & kCuts) && !(rp.flags & jf::kRowMinP) &&
             !jf::wide_row(rp.flags, rp.top_k);
   }
   if (need_merge) {
-    e = small ? jf::launch_merge_small(L, a->dtype, wide, stream)
+    e = small ? jf::launch_merge_small(L, a->dtype, wide, hold, stream)
               : jf::launch_merge(L, a->dtype, stream);
     if (e != hipSuccess) return hip_fail((hipError_t)e, "merge launch");
   }
