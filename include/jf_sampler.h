@@ -185,9 +185,11 @@ void jf_stage_sampling_cycle(uint64_t seed, uint64_t *counter,
  *   logits  + r * logits_stride   (elements of dtype)
  *   masks   + r * mask_stride     (uint32 words; constrained rows only)
  *   uniforms[uniform_index ? uniform_index[r]
- *            : uniform_offset + r * uniform_stride]   (sampled rows; a
- *   stride of 0 gives every row the same uniform, the reference's
- *   correction slot; stride 1 with offset 24 its per-row tree draws)
+ *            : uniform_offset + r * uniform_stride]   (sampled rows only:
+ *   uniform_index has an entry for every row, but a greedy row's may hold
+ *   anything, and no uniform is read for it; a stride of 0 gives every row
+ *   the same uniform, the reference's correction slot; stride 1 with offset
+ *   24 its per-row tree draws)
  *   penalty table row penalty_rows[r] and extra_tokens + r * extra_stride
  *   (extra_counts[r] tokens each counted once more: the draft tokens a
  *   verify row's context adds, Sampling.cpp:118-131, sampling.metal:978-993)

@@ -140,6 +140,10 @@ struct SampleLaunch {
                           // rows
   uint32_t row_indexed;   // drafts are addressed through RowParams'
                           // draft_index/cand_index, not the row number
+  uint32_t greedy_rows;   // some row is greedy. It has no uniform, and its
+                          // place in the uniforms or their index may hold
+                          // anything: a kernel then reads a row's uniform
+                          // only once the row is known to be sampled
   const uint2 *pen_entries;
   const uint32_t *pen_offsets;
   uint32_t pen_max_entries;
@@ -180,6 +184,14 @@ struct SampleLaunch {
   uint32_t *lean_weights;
   uint64_t lean_stride;
 };
+
+// merge_small_kernel's chunk count with two facts its first loads depend on.
+constexpr uint32_t kMergeRowIndexed = 0x80000000u;   // SampleLaunch::row_indexed
+constexpr uint32_t kMergeLateUniform = 0x40000000u;  // the uniform waits for the row's record
+inline uint32_t merge_chunks_bits(const SampleLaunch &a) {
+  return a.chunks | (a.row_indexed ? kMergeRowIndexed : 0u) |
+         (a.greedy_rows ? kMergeLateUniform : 0u);
+}
 
 // The fast selection launch: the per-row facts every block needs before its
 // first load (flags, penalty table row) travel in the kernel arguments, and
@@ -401,7 +413,8 @@ int launch_uncut(const SampleLaunch &a, uint32_t dtype, uint32_t per_row, void *
 // and a share of the rows row_of[n_lean, n_lean + n_plain) (every other row
 // of the launch: greedy ones, and sampled ones with no cut, draft, penalty
 // or extra token), so no launch_uncut follows (n_lean >= 1, n_lean +
-// n_plain <= kKernargRows).
+// n_plain <= kKernargRows). Bit 31 of row_of marks a greedy row.
+constexpr uint32_t kLeanGreedy = 0x80000000u;
 struct LeanLaunch {
   SampleLaunch a;
   uint32_t n_lean;

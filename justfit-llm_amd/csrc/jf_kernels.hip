@@ -612,6 +612,8 @@ __device__ __forceinline__ void write_result(const SampleLaunch &a,
   if (a.out_kept_counts) a.out_kept_counts[row] = kept;
 }
 
+// A sampled row's uniform. Not for a greedy row: it has none, and the index
+// its entry holds (every row has an entry) may lie anywhere.
 __device__ __forceinline__ float row_uniform(const SampleLaunch &a,
                                              uint32_t row) {
   return a.uniforms[a.uniform_index ? (uint64_t)a.uniform_index[row]
@@ -2835,9 +2837,10 @@ __device__ __noinline__ void merge_small_general(uint32_t row, uint32_t n) {
 // padding): the hardware preloads them into scalar registers at wave launch
 // (14 of its 16 user registers; the argument segment's address takes two).
 // They repeat fields of `a` (drafted_rows is 0 when there are no drafts);
-// bit 31 of `chunks_bits` says the row's draft is addressed through its
-// record (the chunk count below it), so that no later argument is read
-// from memory at the row's start.
+// `chunks_bits` is merge_chunks_bits: the row's draft is addressed through its
+// record, and its uniform is read once the record is in (a launch with greedy
+// rows, which have none), so that no later argument is read from memory at
+// the row's start.
 // SPEC: speculatively fetched list slots a thread. 10 gives floor(2560 / S)
 // slots a chunk (134 at 19 chunks); 20 gives floor(5120 / S) (165 at 31
 // chunks), for vocabularies past 163,840 tokens whose cut rows have no
@@ -2856,8 +2859,9 @@ __device__ __forceinline__ void merge_small_row(
     uint32_t uniform_offset, uint32_t uniform_stride, uint32_t drafted_rows,
     const SampleLaunch &a, uint32_t row, Lds &s, General general) {
   const uint32_t tid = threadIdx.x;
-  const uint32_t S = chunks_bits & 0x7fffffffu;
-  const bool row_indexed = (chunks_bits >> 31) != 0;
+  const uint32_t S = chunks_bits & ~(kMergeRowIndexed | kMergeLateUniform);
+  const bool row_indexed = (chunks_bits & kMergeRowIndexed) != 0;
+  const bool late_uniform = (chunks_bits & kMergeLateUniform) != 0;
   // Every address of the row, computed once and held in vector registers:
   // the general path's register pressure would otherwise have the compiler
   // reload (and wait for) kernel arguments between the loads below. A load
@@ -2872,10 +2876,13 @@ __device__ __forceinline__ void merge_small_row(
   const BlockHeader *hrow = headers + (uint64_t)row * S;
   uint64_t hbase = (uint64_t)(hrow + (tid < S ? tid : 0u));
   uint64_t cbase = (uint64_t)(cands + (uint64_t)row * S * kBlockCandidates);
-  uint64_t uaddr = has_index     ? (uint64_t)(uniform_index + row)
-                   : has_uniform ? (uint64_t)(uniforms + uniform_offset + (uint64_t)row * uniform_stride)
-                                 : (uint64_t)hrow;
-  uint64_t ubase = has_uniform ? (uint64_t)uniforms : (uint64_t)hrow;
+  const uint64_t uplace =
+      has_uniform ? (uint64_t)(uniforms + uniform_offset + (uint64_t)row * uniform_stride)
+                  : (uint64_t)hrow;
+  uint64_t uaddr = has_index      ? (uint64_t)(uniform_index + row)
+                   : late_uniform ? (uint64_t)hrow
+                                  : uplace;
+  uint64_t ubase = has_index ? (uint64_t)uniforms : uplace;
   uint64_t daddr = (uint64_t)hrow, qaddr = (uint64_t)hrow, paddr = (uint64_t)hrow;
   if (has_draft) {
     daddr = (uint64_t)(a.draft_tokens + row);
@@ -2912,9 +2919,11 @@ __device__ __forceinline__ void merge_small_row(
   const uint32_t draft_raw = *(GlobalU32 *)daddr;
   const uint32_t cid_raw = *(GlobalU32 *)qaddr;
   const float cpr_raw = *(GlobalF32 *)paddr;
-  // A uniform through an index: its second load, once the index is in.
-  if (has_index) {
-    uint64_t a2 = ubase + (uint64_t)ubits * sizeof(float);
+  // A uniform through an index: its second load, once the index is in. In a
+  // launch with greedy rows, only once the record says that the row is sampled.
+  if (has_index || late_uniform) {
+    uint64_t a2 = ubase + (has_index ? (uint64_t)ubits * sizeof(float) : 0ull);
+    if (late_uniform) a2 = (prec.flags & kRowSampled) ? a2 : (uint64_t)hrow;
     asm volatile("" : "+v"(a2));
     ubits = *(GlobalU32 *)a2;
   }
@@ -4106,9 +4115,11 @@ __device__ __forceinline__ void cut_finish_other(const SampleLaunch &a, const Ro
   }
   merge_small_row<DT, 10, true>(
       a.headers, a.cands, a.params, a.uniforms, a.uniform_index,
-      S | (a.row_indexed ? 0x80000000u : 0u), (uint32_t)a.uniform_offset,
-      (uint32_t)a.uniform_stride, a.draft_tokens && !a.row_indexed ? a.drafted_rows : 0u, a, row,
-      g_finish_lds.merge, [&](uint32_t n) {
+      S | (a.row_indexed ? kMergeRowIndexed : 0u) |
+          ((rp.flags & kRowSampled) ? 0u : kMergeLateUniform),
+      (uint32_t)a.uniform_offset, (uint32_t)a.uniform_stride,
+      a.draft_tokens && !a.row_indexed ? a.drafted_rows : 0u, a, row, g_finish_lds.merge,
+      [&](uint32_t n) {
         cut_copy_launch(a);
         cut_finish_general<DT>(row, n);
       });
@@ -4483,19 +4494,21 @@ __device__ __forceinline__ void plain_draw_wave(const SampleLaunch &a, uint32_t 
 // greedy row's argmax of the chunk bests (sampling.metal:1478-1512), or a
 // sampled row's plain draw, or the sentinel.
 template <int DT>
-__device__ __forceinline__ void plain_row_block(const SampleLaunch &a, uint32_t row, LeanLds &s) {
+__device__ __forceinline__ void plain_row_block(const SampleLaunch &a, uint32_t row, bool greedy,
+                                                LeanLds &s) {
   const uint32_t S = a.chunks, lane = lane_id();
   // Every load the row needs first, none waiting on another: the record,
-  // the uniform, the chunk summaries (lane c < S).
+  // a sampled row's uniform, the chunk summaries (lane c < S).
   const bool in = lane < S;
   const uint32_t at = in ? lane : 0u;
   const RowParams rp = a.params[row];
-  const float u = row_uniform(a, row);
+  float u = 0.0f;
+  if (!greedy) u = row_uniform(a, row);
   const BlockHeader *h = a.headers + (uint64_t)row * S + at;
   const float hm = h->maximum, hbv = h->best_value;
   const uint32_t hadm = h->admitted, hcnt = h->count, hbi = h->best_id;
   const uint64_t hmass = a.partials[(uint64_t)row * S + at].v[0];
-  if (!(rp.flags & kRowSampled)) {
+  if (greedy) {
     float hv = in ? hbv : -__builtin_inff();
     uint32_t hi = in ? hbi : kNoToken;
     wave_argmax(hv, hi);
@@ -4554,13 +4567,14 @@ __global__ __launch_bounds__(kThreads) void residual_kernel(LeanLaunch l) {
   const bool finisher = l.draw && chunk + 1 == S;
   const auto draw_plain_share = [&]() {
     for (uint32_t i = lean + (w - 1) * l.n_lean; i < l.n_plain; i += (kWaves - 1) * l.n_lean)
-      plain_row_block<DT>(a, l.row_of[l.n_lean + i], s);
+      plain_row_block<DT>(a, l.row_of[l.n_lean + i] & ~kLeanGreedy,
+                          (l.row_of[l.n_lean + i] & kLeanGreedy) != 0, s);
   };
   const RowParams rp = a.params[row];
   const uint32_t draft = row_draft(a, rp);
   if (draft == kNoToken) {
     // Drawn plainly: by uncut_kernel, or here by chunk 0's block.
-    if (l.draw && chunk == 0 && w == 0) plain_row_block<DT>(a, row, s);
+    if (l.draw && chunk == 0 && w == 0) plain_row_block<DT>(a, row, false, s);
     if (finisher && w != 0) draw_plain_share();
     return;
   }
@@ -4838,7 +4852,8 @@ __global__ __launch_bounds__(kThreads) void uncut_kernel(SampleLaunch a, uint32_
   // Requested together before anything waits: the row's record, its
   // uniform, and (wave 0) its chunk summaries, one per lane (S <= 64).
   const RowParams rp = a.params[row];
-  const float u = row_uniform(a, row);
+  float u = 0.0f;
+  if (!a.greedy_rows) u = row_uniform(a, row);
   const bool in = w == 0 && lane < S;
   const BlockHeader *hl = hb + (in ? lane : 0u);
   const float hm = hl->maximum, hbv = hl->best_value;
@@ -4856,6 +4871,7 @@ __global__ __launch_bounds__(kThreads) void uncut_kernel(SampleLaunch a, uint32_
     return;
   }
   if (!uncut_row(rp)) return;  // the merge's
+  if (a.greedy_rows) u = row_uniform(a, row);
   const uint32_t draft = row_draft(a, rp);
   const bool drafted = draft != kNoToken;
   if (!drafted && chunk != 0) return;
@@ -5244,8 +5260,7 @@ int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, bool ho
   const hipStream_t st = (hipStream_t)stream;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, st, a.headers, (const uint64_t *)a.cands,
-                       a.params, a.uniforms, a.uniform_index,
-                       a.chunks | (a.row_indexed ? 0x80000000u : 0u),
+                       a.params, a.uniforms, a.uniform_index, merge_chunks_bits(a),
                        (uint32_t)a.uniform_offset, (uint32_t)a.uniform_stride,
                        a.draft_tokens && !a.row_indexed ? a.drafted_rows : 0u, a);
   };

@@ -803,6 +803,8 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   // use it as the linear prefix unless the rows are indexed.
   L.drafted_rows = !any_drafted ? 0u : row_indexed ? rows : a->drafted_rows;
   L.row_indexed = row_indexed ? 1u : 0u;
+  for (uint32_t r = 0; r < rows && !L.greedy_rows; ++r)
+    L.greedy_rows = (params[r].flags & jf::kRowSampled) ? 0u : 1u;
   L.cand_ids = a->draft_cand_ids;
   L.cand_probs = a->draft_cand_probs;
   L.dense_q = a->draft_q;
@@ -1003,7 +1005,7 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
         if (params[r].flags & jf::kRowLean)
           lean.push_back(r);
         else if (draw)
-          plain.push_back(r);
+          plain.push_back((params[r].flags & jf::kRowSampled) ? r : r | jf::kLeanGreedy);
       }
       // Launches of at most kKernargRows rows (a share of each list, at
       // least one lean row in each: the lean rows' blocks draw the others).
