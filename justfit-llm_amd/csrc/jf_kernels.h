@@ -435,6 +435,15 @@ struct CutLaunch {
   bool small;    // its listed rows may take merge_small_row
 };
 int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *stream);
+// Its kernels of one block a (row, chunk) have their chunks in the grid's x and
+// their rows in its y, which takes at most 65,535; a sampler has up to
+// 4,194,304 rows. So they run a slice of kCutSliceRows rows at a time.
+constexpr uint32_t kCutSliceRows = 32768;
+inline uint32_t cut_slices(uint32_t rows) { return (rows + kCutSliceRows - 1) / kCutSliceRows; }
+inline uint32_t cut_slice_rows(uint32_t rows, uint32_t slice) {
+  const uint32_t left = rows - slice * kCutSliceRows;
+  return left < kCutSliceRows ? left : kCutSliceRows;
+}
 int launch_accept_chain(const AcceptChainLaunch &a, void *stream);
 int launch_accept_tree(const AcceptTreeLaunch &a, void *stream);
 // jf_draft.hip; the events, when set, bracket the top-16 kernel.

@@ -3370,6 +3370,10 @@ constexpr uint32_t kCutPlain = 0x200u;  // no row is penalized, the vocabulary h
 constexpr uint32_t kCutKept = 0x400u;   // kept outputs are asked for
 constexpr uint32_t kCutUncut = 0x800u;  // cut_draw_kernel draws the uncut rows
 constexpr uint32_t kCutSmall = 0x1000u; // listed rows may take merge_small_row
+constexpr int kCutSliceShift = 16;      // from here up: the launch's slice of the rows
+__device__ __forceinline__ uint32_t cut_row_of(uint32_t bits) {
+  return (bits >> kCutSliceShift) * kCutSliceRows + blockIdx.y;
+}
 
 struct __align__(16) CutHistLds {
   PrepLds prep;
@@ -3564,7 +3568,7 @@ __global__ __launch_bounds__(kThreads) void cut_hist_kernel(
     RowState *states, uint64_t stride, uint32_t V, uint32_t bits, SampleLaunch a) {
   constexpr int TPL = Geo<DT>::TPL;
   __shared__ CutHistLds s;
-  const uint32_t S = bits & 0xffu, row = blockIdx.y, chunk = blockIdx.x;
+  const uint32_t S = bits & 0xffu, row = cut_row_of(bits), chunk = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const BlockHeader h = headers[(uint64_t)row * S + min(lane, S - 1)];
   const RowParams rp = load_row_policy(params + row);
@@ -3687,7 +3691,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(
     RowState *states, uint64_t stride, uint32_t V, uint32_t bits, SampleLaunch a) {
   constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
   __shared__ CutListLds s;
-  const uint32_t S = bits & 0xffu, row = blockIdx.y, chunk = blockIdx.x;
+  const uint32_t S = bits & 0xffu, row = cut_row_of(bits), chunk = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   uint64_t *rows = cands + (uint64_t)row * S * kBlockCandidates;
   uint64_t *area = rows + (uint64_t)chunk * kBlockCandidates;
@@ -4235,7 +4239,7 @@ __global__ __launch_bounds__(kThreads) void cut_emit_kernel(
   constexpr uint32_t VMASK = (1u << VEC) - 1u;
   __shared__ DrawLds s;
   (void)headers;
-  const uint32_t S = bits & 0xffu, row = blockIdx.y, chunk = blockIdx.x;
+  const uint32_t S = bits & 0xffu, row = cut_row_of(bits), chunk = blockIdx.x;
   const uint32_t tid = threadIdx.x;
   uint64_t *area = cands + ((uint64_t)row * S + chunk) * kBlockCandidates;
   const RowParams rp = load_row_policy(params + row);
@@ -5280,17 +5284,21 @@ int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, bool ho
 
 #if JF_IN(3)
 int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *stream) {
-  const dim3 grid(a.chunks, a.rows), block(kThreads);
+  const dim3 block(kThreads);
   const hipStream_t st = (hipStream_t)stream;
   const uint32_t bits = a.chunks | (c.all ? kCutAll : 0u) |
                         (c.plain && a.vocabulary >= 8 ? kCutPlain : 0u) |
                         (a.out_kept_ids ? kCutKept : 0u) | (c.uncut ? kCutUncut : 0u) |
                         (c.small ? kCutSmall : 0u);
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, st, a.logits, a.params,
-                       (const BlockHeader *)a.headers, a.cands, a.states, a.stride, a.vocabulary,
-                       bits, a);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    for (uint32_t i = 0; i < cut_slices(a.rows) && e == hipSuccess; ++i) {
+      hipLaunchKernelGGL(kernel, dim3(a.chunks, cut_slice_rows(a.rows, i)), block, 0, st, a.logits,
+                         a.params, (const BlockHeader *)a.headers, a.cands, a.states, a.stride,
+                         a.vocabulary, bits | i << kCutSliceShift, a);
+      e = hipGetLastError();
+    }
+    return e;
   };
   auto draw = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(a.rows), block, 0, st, a.params, (const RowState *)a.states,

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -54,7 +55,10 @@ int launch_residual(const LeanLaunch &l, uint32_t, void *) {
   return 0;
 }
 int launch_cut(const SampleLaunch &a, uint32_t, const CutLaunch &, void *) {
-  add("cut", a);
+  std::string slices;
+  for (uint32_t i = 0; i < cut_slices(a.rows); ++i)
+    slices += (i ? ", " : "") + std::to_string(cut_slice_rows(a.rows, i));
+  add("cut", a, ", \"slices\": [" + slices + "]");
   return 0;
 }
 int launch_accept_chain(const AcceptChainLaunch &, void *) { return 0; }
@@ -74,9 +78,14 @@ namespace {
 int upload(void *, const jf::RowParams *, uint32_t, jf::RowParams *, void *) { return JF_OK; }
 
 // One letter a row: g greedy, k top-k 50, n top-p alone, u no cut, d no cut
-// and drafted (a dense q).
-void batch(const char *kinds) {
-  const uint32_t rows = (uint32_t)std::strlen(kinds), V = 20000;
+// and drafted (a dense q). "n:70000": that many rows of the letters, repeated.
+void batch(const char *spec) {
+  const char *colon = std::strchr(spec, ':');
+  const std::string letters(spec, colon ? colon - spec : std::strlen(spec));
+  std::string kinds = letters;
+  if (colon)
+    for (kinds.clear(); kinds.size() < std::strtoul(colon + 1, nullptr, 10);) kinds += letters;
+  const uint32_t rows = (uint32_t)kinds.size(), V = 20000;
   static uint64_t memory[64];  // stands for every device buffer; nothing reads it
   std::vector<jf_policy> pol(rows);
   std::vector<uint32_t> draft(rows, JF_NO_TOKEN);
@@ -116,7 +125,7 @@ void batch(const char *kinds) {
   std::vector<jf::RowParams> params(rows);
   g_out.clear();
   const int rc = jf::sample_core(V, sc, &a, params.data(), upload, nullptr, nullptr);
-  std::printf("{\"batch\": \"%s\", \"rc\": %d, \"launches\": [%s]}\n", kinds, rc, g_out.c_str());
+  std::printf("{\"batch\": \"%s\", \"rc\": %d, \"launches\": [%s]}\n", spec, rc, g_out.c_str());
 }
 }  // namespace
 

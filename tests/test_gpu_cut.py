@@ -149,3 +149,26 @@ def test_cut_masks_penalties_and_other_rows():
     plain = [J.policy(temperature=1.0)] * 18  # the self-validating words' launch, after
     check(V, plain, logits=x, uniforms=rng.random(18).astype(np.float32), sampler=s)
     s.close()
+
+
+def test_cut_rows_past_a_grid_dimension():
+    """More rows than a grid has blocks in y: the cut passes' kept outputs of
+    every 997th row and of the last ones, and every greedy row among them."""
+    import torch
+    V, rows = 128, 65600
+    rng = np.random.default_rng(31)
+    x = rng.normal(0, 2.5, (rows, V)).astype(np.float32)
+    u = rng.random(rows).astype(np.float32)
+    kinds = [J.policy(temperature=0.8, top_p=0.9), J.policy(),
+             J.policy(temperature=1.0, top_k=100, top_p=0.95)]
+    pols = [kinds[r % 3] for r in range(rows)]
+    some = sorted(set(range(0, rows, 997)) | set(range(32766, 32772)) |
+                  set(range(65533, 65540)) | set(range(rows - 4, rows)))
+    print(f"case rows={rows}", flush=True)
+    g = run_gpu(V, pols, logits=x, uniforms=u, kept_capacity=V)
+    pick = {k: v[some] for k, v in g.items()}
+    assert_same(pick, run_oracle(V, [pols[r] for r in some], logits=x[some], uniforms=u[some],
+                                 kept_capacity=V))
+    np.testing.assert_array_equal(g["tokens"][1::3], x[1::3].argmax(1))
+    assert (g["tokens"] < V).all() and (g["kept_counts"][0::3] > 0).all()
+    torch.cuda.empty_cache()

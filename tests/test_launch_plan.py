@@ -50,3 +50,14 @@ def test_sampled_launches_read_uniforms_early(batch):
         assert l["greedy_rows"] == 0
         assert l.get("late_uniform", 0) == 0
         assert all(v < LEAN_GREEDY for v in l.get("row_of", []))
+
+
+@pytest.mark.parametrize("rows", [1, 64, 32767, 32768, 32769, 65535, 65536, 65600, 300001])
+def test_cut_slices_of_any_row_count(rows):
+    """The cut passes' launches hold every row once, each in a grid a launch
+    may have (65,535 blocks in y), and the slice numbers fit their argument."""
+    (b,) = plan(f"n:{rows}")
+    (cut,) = [l for l in b["launches"] if l["launch"] == "cut"]
+    assert sum(cut["slices"]) == rows
+    assert all(n == 32768 for n in cut["slices"][:-1]) and 0 < cut["slices"][-1] <= 32768
+    assert 4194304 // 32768 <= 1 << 16
