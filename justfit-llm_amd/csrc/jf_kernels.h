@@ -20,8 +20,8 @@ struct RowParams {
   float inv_t;                // 1 / temperature
   float top_p;
   float minp_offset;          // temperature * log(min_p); without min-p, how far
-                              // below the maximum a top-p or top-k row's
-                              // boundary bins need to reach (below zero)
+                              // below the maximum the weights (with top-p
+                              // alone, its boundary) reach (below zero)
   float repetition;
   float repetition_inverse;   // min(1 / repetition, FLT_MAX)
   float presence;
@@ -84,7 +84,8 @@ struct RowState {
   uint32_t bid;
   uint32_t kept;      // its size, where kept outputs are asked for
   uint64_t mass3;     // its mass
-  uint64_t reserved[6];
+  float end;          // the row's least value on the bins' scale
+  uint32_t reserved[11];
 };
 static_assert(sizeof(RowState) == 128, "row states are 128 bytes");
 enum RowStage : uint32_t {

@@ -3356,9 +3356,10 @@ __device__ __forceinline__ void uncut_draw(const SampleLaunch &a, const RowParam
 //  - cut_emit_kernel, only for kept outputs and drafted rows: writes the kept
 //    tokens, sums the residual masses, and draws a drafted row.
 // A bin falls with the key and is the same for equal keys, so the bins only
-// bracket the boundary: every decision is made on exact counts and masses, and
-// a row whose boundary bins hold more tokens than the lists (ties, a range far
-// off) is resolved by the same steps over its logits instead (cut_rescan).
+// bracket the boundary: every decision is made on exact counts and masses. A
+// chunk with more boundary tokens than its list takes (ties, flat values, a
+// range far off) leaves a finer histogram of them in the list's place, and the
+// row is resolved from those (cut_refine).
 constexpr uint32_t kCutGroup = 16, kCutGroups = kCutBins / kCutGroup;
 static_assert(kCutGroups == 32 && kCutBins == 2 * kThreads);
 
@@ -3380,17 +3381,35 @@ struct __align__(16) CutHistLds {
   uint64_t mass[kCutBins];
   uint32_t count[kCutBins];
 };
+constexpr uint32_t kCutSubs = 64;  // sub-bins of a row's boundary bins
+struct CutSubLds {
+  uint64_t mass[kCutSubs];
+  uint32_t n[kCutSubs];
+  uint32_t key[kCutSubs];   // a token's key
+  uint32_t many[kCutSubs];  // some other token's differs:
+  uint32_t lo[kCutSubs];    // the least and the largest key
+  uint32_t hi[kCutSubs];
+};
 struct __align__(16) CutListLds {
-  PrepLds prep;
+  union {
+    PrepLds prep;
+    CutSubLds sub;
+  };
   uint64_t part[kThreads];
   uint32_t part_n[kThreads];
   uint64_t wl[kWaves];
   uint32_t n;
 };
+constexpr uint32_t kCutCells = 2048;  // cells of a sub-bin's tokens past LDS
+enum CutMode : uint32_t { kSweepCollect, kSweepCount, kSweepMass };
 struct __align__(16) CutLds {
+  PrepLds prep;
   union {
-    PrepLds prep;
     uint64_t items[kCutItems];
+    struct {
+      uint64_t cell_mass[kCutCells];
+      uint32_t cell_n[kCutCells];
+    };
   };
   uint64_t hist[256];
   uint32_t hcount[256];
@@ -3402,6 +3421,18 @@ struct __align__(16) CutLds {
   uint64_t slices[kWaves * 8];
   uint64_t wl[kWaves];
   uint64_t wl2[kWaves];
+  // cut_refine's: the row's sub-bins (with the bounds of their keys), and its
+  // passes over the chunks (cut_sweep).
+  uint64_t sub_mass[kCutSubs];
+  uint32_t sub_n[kCutSubs];
+  uint32_t sub_lo[kCutSubs];
+  uint32_t sub_hi[kCutSubs];
+  uint64_t sum_mass[kMaxChunks];
+  uint32_t sum_n[kMaxChunks];
+  uint32_t tied[kMaxChunks];  // whether (for ties: how often) a chunk holds the sub-bin
+  uint64_t from, to, top;
+  uint32_t shift, mode;
+  uint64_t wj[kWaves][8];
   uint32_t kept;
   uint32_t n;
   uint32_t small_n;
@@ -3430,6 +3461,10 @@ __device__ __forceinline__ uint32_t cut_list_word(bool counts) {
 __device__ __forceinline__ uint32_t cut_list_room(bool counts) {
   return kCutMassWord - cut_list_word(counts);
 }
+// A chunk whose boundary tokens do not fit its list leaves there, for each
+// sub-bin of the row's boundary bins, three words kCutSubs apart: their mass,
+// their count, and their least key | largest key << 32.
+static_assert(3 * kCutSubs <= kCutMassWord - (kCutGroupCountWord + kCutGroups / 2));
 
 __device__ __forceinline__ uint64_t *cut_area(const SampleLaunch &a, uint32_t row, uint32_t chunk) {
   return a.cands + ((uint64_t)row * a.chunks + chunk) * kBlockCandidates;
@@ -3446,6 +3481,52 @@ __device__ __forceinline__ uint32_t cut_bin_at(float below, float scale) {
 }
 __device__ __forceinline__ uint32_t cut_bin(float v, float maximum, float scale) {
   return cut_bin_at(maximum - v, scale);
+}
+// The boundary bins' sub-bins, in falling order of value: first those of the
+// bins that may hold the top-p boundary, then those of the top-k boundary's bin
+// (which may be the same one). Within a bin a sub-bin is a step of 1 / per of
+// it; where the bins outnumber the sub-bins, `bins1` bins share one. The open
+// last bin goes in steps down to the row's least value (as its summaries have
+// it), with one more for what lies below that, and one for -inf.
+struct CutSpan {
+  uint32_t b0, bk;  // bk: kCutBins when top-k cuts nothing
+  uint32_t n1;      // sub-bins before bk's
+  uint32_t per1, bins1, per2;
+  float end, tail;  // the least value's place on the bins' scale; steps beyond the last bin's start
+};
+__device__ __forceinline__ CutSpan cut_span(uint32_t b0, uint32_t b1, uint32_t bk,
+                                            uint32_t need_k, float end) {
+  CutSpan r;
+  r.b0 = b0;
+  r.bk = need_k ? bk : kCutBins;
+  r.n1 = !need_k ? kCutSubs : b0 == bk ? 0u : kCutSubs * 2 / 3;
+  r.per2 = kCutSubs - r.n1;
+  const uint32_t span = (need_k ? min(b1, bk - 1) : b1) - b0 + 1;  // unused with n1 == 0
+  r.per1 = r.n1 && span <= r.n1 ? r.n1 / span : 1u;
+  r.bins1 = r.n1 && span > r.n1 ? (span + r.n1 - 1) / r.n1 : 1u;
+  const float past = end - (float)(kCutBins - 1);
+  r.end = end;
+  r.tail = past > 0.0f ? 1.0f / past : 0.0f;
+  return r;
+}
+// The sub-bin of a boundary bin's member v. Falls monotonically with the key,
+// as cut_bin does (x - b is exact).
+__device__ __forceinline__ uint32_t cut_sub(const CutSpan &r, float v, float maximum, float scale,
+                                            uint32_t b) {
+  const bool k = b == r.bk;
+  const uint32_t per = k ? r.per2 : r.per1;
+  const float x = (maximum - v) * scale;
+  uint32_t in;
+  if (b < kCutBins - 1) {
+    in = min((uint32_t)((x - (float)b) * (float)per), per - 1);
+  } else {
+    const uint32_t last = max(per, 4u) - 1;
+    in = v == -__builtin_inff() ? last
+         : x > r.end            ? last - 1
+                                : min((uint32_t)((x - (float)b) * r.tail * (float)(last - 2)), last - 2);
+    in = per < 4 ? 0u : in;
+  }
+  return k ? r.n1 + in : (b - r.b0) / r.bins1 * r.per1 + in;
 }
 // A chunk of a row of these passes: xs[i] as load_chunk leaves it. A row with
 // no penalty requests its logits first thing (fast_load), before its record
@@ -3511,6 +3592,7 @@ struct CutRow {
   float maximum;
   float scale;
   float floor;  // members are at or above it (-inf without min-p)
+  float end;    // the row's least value on the bins' scale
   bool none;  // nothing admitted, or a maximum of +inf: the sentinel
 };
 __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader &h, uint32_t S) {
@@ -3520,22 +3602,32 @@ __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader
   r.none = !wave_max_u32(h.admitted) || r.maximum == __builtin_inff();
   const bool minp = (rp.flags & kRowMinP) != 0;
   r.floor = minp ? __builtin_fminf(r.maximum + rp.minp_offset, r.maximum) : -__builtin_inff();
-  // The bins' range below the maximum: no further than the row's least value.
-  float range = -rp.minp_offset;
+  // The bins' range below the maximum: no further than the row's least value,
+  // nor than the weights reach (minp_offset). With a top-k, down to the least of
+  // the chunks' floor keys where enough tokens reach those (each chunk's
+  // floor_key: a key that `count` of its tokens reach); where not, its boundary
+  // lies below them, and when the weights do not reach twice as far the range
+  // is the row's (a little more, so that its least value stays out of the open
+  // last bin).
+  float range = -rp.minp_offset, span = 0.0f;
   if (!minp) {
     const float least = -wave_max_f32(lane < S ? -h.best_value : -__builtin_inff());
-    const float d = (r.maximum - least) * 1.0001f;
-    if (d > 0.0f && d < range) range = d;
-  }
-  if (!minp && (rp.flags & kRowTopK)) {
-    // Each chunk's floor_key: a key that `count` of its tokens reach.
+    span = r.maximum - least;
+    const float d = span * 1.0001f;
     const bool in = lane < S && h.count;
-    const uint32_t floor_key = wave_min_u32(in ? h.floor_key : 0xffffffffu);
-    const uint32_t reach = wave_sum_u32(in ? h.count : 0u);
-    const float d = r.maximum - key_logit(floor_key);
-    if (rp.top_k <= reach && d < 1.0e30f) range = d;
+    float f = -1.0f;
+    if (rp.flags & kRowTopK) {
+      const uint32_t floor_key = wave_min_u32(in ? h.floor_key : 0xffffffffu);
+      f = r.maximum - key_logit(floor_key);
+      if (rp.top_k <= wave_sum_u32(in ? h.count : 0u)) {
+        if (f < 1.0e30f) range = f;
+        f = -1.0f;
+      }
+    }
+    if (d > 0.0f && d < 1.0e30f && (d < range || range < 2.0f * f)) range = d;
   }
   r.scale = __builtin_fminf((float)(kCutBins - 1) / range, 3.0e38f);
+  r.end = span * r.scale;
   return r;
 }
 
@@ -3686,7 +3778,7 @@ __device__ __forceinline__ void cut_sums(const uint64_t *area, uint32_t S, uint3
 // 12.7 us against 9.1 (64 x 151,936 fp32, top-p 0.95), and 0.3 us less where
 // every chunk holds some.
 template <int DT>
-__global__ __launch_bounds__(kThreads) void cut_list_kernel(
+__global__ __launch_bounds__(kThreads, 5) void cut_list_kernel(
     const void *logits, const RowParams *params, const BlockHeader *headers, uint64_t *cands,
     RowState *states, uint64_t stride, uint32_t V, uint32_t bits, SampleLaunch a) {
   constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
@@ -3790,6 +3882,59 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(
     }
     __syncthreads();
     listed = s.n;
+    if (listed > room) {
+      // Too many: the sub-bins, in the list's place once its stores are done.
+      const CutSpan sp = cut_span(b0, b1, bk, need_k, r.end);
+      auto member = [&](float v, auto f) {
+        const uint32_t b = cut_bin(v, r.maximum, r.scale);
+        if (boundary(b) && v >= r.floor) f(cut_sub(sp, v, r.maximum, r.scale, b));
+      };
+      if (tid < kCutSubs) {
+        s.sub.mass[tid] = 0;
+        s.sub.n[tid] = 0;
+        s.sub.many[tid] = 0;
+        s.sub.lo[tid] = 0xffffffffu;
+        s.sub.hi[tid] = 0;
+      }
+      wait_memory();
+      __syncthreads();
+      opaque(xs);
+#pragma unroll
+      for (int i = 0; i < TPL; ++i)
+        member(xs[i], [&](uint32_t g) { s.sub.key[g] = logit_key(xs[i]); });
+      __syncthreads();
+      opaque(xs);
+#pragma unroll
+      for (int i = 0; i < TPL; ++i)
+        member(xs[i], [&](uint32_t g) {
+          if (s.sub.key[g] != logit_key(xs[i])) s.sub.many[g] = 1;
+        });
+      __syncthreads();
+      opaque(xs);
+      // (Counts alone for ties, whose lanes' atomics on one word take turns.)
+#pragma unroll
+      for (int i = 0; i < TPL; ++i)
+        member(xs[i], [&](uint32_t g) {
+          atomicAdd(&s.sub.n[g], 1u);
+          if (s.sub.many[g]) {
+            atomicAdd((unsigned long long *)&s.sub.mass[g],
+                      (unsigned long long)quantized_weight(xs[i], r.maximum, rp.inv_t));
+            atomicMin(&s.sub.lo[g], logit_key(xs[i]));
+            atomicMax(&s.sub.hi[g], logit_key(xs[i]));
+          }
+        });
+      __syncthreads();
+      if (tid < kCutSubs) {
+        const uint32_t n = s.sub.n[tid], key = s.sub.key[tid];
+        const bool many = s.sub.many[tid] != 0;
+        list[tid] = many ? s.sub.mass[tid]
+                    : n  ? n * quantized_weight(key_logit(key), r.maximum, rp.inv_t)
+                         : 0ull;
+        list[kCutSubs + tid] = n;
+        list[2 * kCutSubs + tid] = many ? s.sub.lo[tid] | (uint64_t)s.sub.hi[tid] << 32
+                                        : key | (uint64_t)key << 32;
+      }
+    }
   }
   if (tid == 0) {
     area[kCutMassWord] = before;
@@ -3808,6 +3953,7 @@ __global__ __launch_bounds__(kThreads) void cut_list_kernel(
       st.mass_b0 = mass_b0;
       st.mass_bk = mass_bk;
       st.total = total;
+      st.end = r.end;
       states[row] = st;
     }
   }
@@ -3870,60 +4016,350 @@ __shared__ FinishLds g_finish_lds;
 #define g_cut_lds g_finish_lds.cut
 __shared__ SampleLaunch g_cut_launch;
 
-// The tokens of the row's boundary bins in chunk `c`, from the `skip`-th on in
-// the block's order of them, into g_cut_lds.items; returns how many the chunk
-// has (the first kCutItems past `skip` are there).
+// One pass of the row's chunk `c` over its tokens whose items lie in [s.from,
+// s.to], by s.mode: counted (and their masses added) by cells of 2^s.shift items
+// in falling order, or put into s.items (from s.small_n on), and those above
+// s.to up to s.top summed for the chunk. `next` is the chunk read after it: its
+// lines are requested meanwhile, since a block that reads chunks one after
+// another otherwise waits for memory at each. Every thread of the block calls
+// it.
 template <int DT>
-__device__ __noinline__ uint32_t cut_collect(uint32_t row, uint32_t c, uint32_t skip) {
+__device__ __noinline__ void cut_sweep(uint32_t row, uint32_t c, uint32_t next) {
   constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB;
   const SampleLaunch &a = g_cut_launch;
+  CutLds &s = g_cut_lds;
   const RowParams rp = a.params[row];
-  const RowState &st = a.states[row];
-  const float M = st.maximum, scale = st.scale;
-  const uint32_t thr_key = st.thr_key, b0 = st.b0, b1 = st.b1, bk = st.bk;
+  const float M = a.states[row].maximum, inv_t = rp.inv_t;
+  const uint32_t tid = threadIdx.x;
   float xs[TPL];
-  load_chunk<DT>(a, rp, row, c, g_cut_lds, xs);
-  uint32_t hits = 0;
+  load_chunk<DT>(a, rp, row, c, s, xs);
+  // A byte of every 128-byte line of the next chunk.
+  constexpr uint32_t kSize = DT == 0 ? 4 : 2;
+  const uint64_t ahead = min(next * kChunkF32 + tid * (128 / kSize) % kChunkF32, a.vocabulary - 1);
+  uint32_t line = *((const uint8_t *)a.logits + ((uint64_t)row * a.stride + ahead) * kSize);
+  const uint64_t from = s.from, to = s.to, top = s.top;
+  const uint32_t mode = s.mode, shift = s.shift, lane_base = c * kChunkF32 + tid * VEC;
+  const bool collect = mode == kSweepCollect;
+  const float lo = key_logit(item_key(from)), hi = key_logit(item_key(collect ? top : to));
+  uint64_t m = 0;
+  uint32_t n = 0;
 #pragma unroll
   for (int i = 0; i < TPL; ++i) {
     const float v = xs[i];
-    const uint32_t b = cut_bin(v, M, scale);
-    if (v == v && logit_key(v) >= thr_key && ((b >= b0 && b <= b1) || b == bk)) hits |= 1u << i;
-  }
-  uint64_t total;
-  // (The scan's barriers also end the prep area's use: it becomes the items'.)
-  uint32_t at = (uint32_t)block_excl_scan_u64(__popc(hits), g_cut_lds, &total) - skip;
-  const uint32_t lane_base = c * kChunkF32 + threadIdx.x * VEC;
-#pragma unroll
-  for (int i = 0; i < TPL; ++i)
-    if ((hits >> i) & 1u) {
-      if (at < kCutItems)
-        g_cut_lds.items[at] =
-            token_item(logit_key(xs[i]), lane_base + (i / VEC) * SLAB + (i % VEC));
-      ++at;
+    if (!(v >= lo && v <= hi)) continue;
+    const uint64_t item = token_item(logit_key(v), lane_base + (i / VEC) * SLAB + (i % VEC));
+    if (item < from || item > top) continue;
+    if (collect && item <= to) {
+      const uint32_t at = atomicAdd(&s.small_n, 1u);
+      if (at < kCutItems) s.items[at] = item;
+      continue;
     }
+    const uint64_t wq = mode == kSweepCount ? 0ull : quantized_weight(v, M, inv_t);
+    if (collect) {
+      m += wq;
+      ++n;
+    } else if (item <= to) {
+      const uint32_t cell = (uint32_t)((to - item) >> shift) & (kCutCells - 1);
+      atomicAdd(&s.cell_n[cell], 1u);
+      if (mode == kSweepMass)
+        atomicAdd((unsigned long long *)&s.cell_mass[cell], (unsigned long long)wq);
+    }
+  }
+  if (collect) {
+    m = block_sum_u64(m, s);
+    n = (uint32_t)block_sum_u64(n, s);
+    if (tid == 0) {
+      s.sum_mass[c] = m;
+      s.sum_n[c] = n;
+    }
+  }
+  asm volatile("" : "+v"(line));
   __syncthreads();
-  return (uint32_t)total;
 }
 
-// cut_resolve over the row's logits, for a row whose boundary bins hold more
-// tokens than the lists: each step reads the row's chunks again. Out of line
-// (with the launch record copied to LDS, since a called function cannot reach
-// the kernel's arguments), so its registers stay out of the common path.
+// cut_resolve for a row of whose chunks some left sub-bins: those of all its
+// chunks together (the other chunks' lists count into them), the boundary's
+// sub-bin by their counts or masses, and the boundary in it. When all its
+// tokens have one key, the last of the ties kept lies in the chunk where their
+// running count reaches the number kept, which is read again for its id; else
+// the chunks that hold some are read again, one after another: once to collect
+// the sub-bin's tokens in LDS, where they are ranked, after as many passes as it
+// takes to find a part of them that fits there. Every thread of the block calls
+// it.
+// Ties cost the histogram pass's atomics on one word and one more chunk: a call
+// of 64 x 151,936 equal values takes 137 us with top-p 0.95 (1 row 65; 8 x
+// 524,288 91), where rereading the row for every step of the ranking took 1717
+// (1646; 5695); sub-bins of distinct values, 64 rows with top-k 20,000 and one
+// value far above the rest, 61 against 1852. What remains slow is most of a row
+// within a few neighbouring floats, under one far higher value: 310-650 us for
+// 16 rows (1490-3950 before).
 template <int DT>
-__device__ __noinline__ void cut_rescan(uint32_t row) {
-  const RowParams rp = g_cut_launch.params[row];
-  const RowState st = g_cut_launch.states[row];
-  auto each = [&](auto f) {
-    for (uint32_t c = 0; c < g_cut_launch.chunks; ++c)
-      for (uint32_t skip = 0, n = 1; skip < n; skip += kCutItems) {
-        n = cut_collect<DT>(row, c, skip);
-        for (uint32_t i = threadIdx.x; i < min(n - skip, kCutItems) && skip < n; i += kThreads)
-          f(g_cut_lds.items[i]);
+__device__ __forceinline__ void cut_refine(uint32_t row, uint32_t bits) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
+                LOADS = Geo<DT>::LOADS;
+  const SampleLaunch &a = g_cut_launch;
+  CutLds &s = g_cut_lds;
+  const RowParams rp = a.params[row];
+  const RowState st = a.states[row];
+  const uint32_t S = a.chunks, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const float M = st.maximum, scale = st.scale, inv_t = rp.inv_t;
+  const bool counts = cut_counts(rp, bits);
+  const uint32_t room = cut_list_room(counts);
+  const uint64_t *list = cut_area(a, row, 0) + cut_list_word(counts);
+  const CutSpan sp = cut_span(st.b0, st.b1, st.bk, st.need_k, st.end);
+  auto listed = [&](uint32_t c) { return s.coff[c + 1] - s.coff[c]; };
+  auto weight = [&](uint64_t c) { return item_weight(c, M, inv_t); };
+  // f(chunk, item, sub-bin) for every token of the lists that fit: a wave a chunk.
+  static_assert(kCutMassWord - kCutBinCountWord <= 512);
+  auto fit = [&](auto f) {
+    for (uint32_t c = w; c < S; c += kWaves) {
+      const uint32_t n = listed(c);
+      if (n > room) continue;
+      uint64_t v[8];
+#pragma unroll
+      for (uint32_t k = 0; k < 8; ++k)
+        v[k] = lane + 64 * k < n ? list[(uint64_t)c * kBlockCandidates + lane + 64 * k] : 0ull;
+#pragma unroll 1
+      for (uint32_t k = 0; k < 8; ++k) {
+        if (lane + 64 * k < n) {
+          const float x = key_logit(item_key(v[0]));
+          f(c, v[0], cut_sub(sp, x, M, scale, cut_bin(x, M, scale)));
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 7; ++j) v[j] = v[j + 1];
+      }
+    }
+  };
+  if (tid < kCutSubs) {
+    s.sub_mass[tid] = 0;
+    s.sub_n[tid] = 0;
+    s.sub_lo[tid] = 0xffffffffu;
+    s.sub_hi[tid] = 0;
+  }
+  __syncthreads();
+  {
+    // A wave a quarter of the chunks, lane i sub-bin i.
+    static_assert(kCutSubs == 64);
+    uint64_t m = 0;
+    uint32_t n = 0, lo = 0xffffffffu, hi = 0;
+    constexpr uint32_t B = 4;
+    for (uint32_t c0 = w; c0 < S; c0 += kWaves * B) {
+      uint64_t mv[B], nv[B], kv[B];
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k) {
+        const uint64_t *p = list + (uint64_t)min(c0 + kWaves * k, S - 1) * kBlockCandidates + lane;
+        mv[k] = p[0];
+        nv[k] = p[kCutSubs];
+        kv[k] = p[2 * kCutSubs];
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k) {
+        if (c0 + kWaves * k >= S || listed(c0 + kWaves * k) <= room || !nv[k]) continue;
+        m += mv[k];
+        n += (uint32_t)nv[k];
+        lo = min(lo, (uint32_t)kv[k]);
+        hi = max(hi, (uint32_t)(kv[k] >> 32));
+      }
+    }
+    if (n) {
+      atomicAdd((unsigned long long *)&s.sub_mass[lane], (unsigned long long)m);
+      atomicAdd(&s.sub_n[lane], n);
+      atomicMin(&s.sub_lo[lane], lo);
+      atomicMax(&s.sub_hi[lane], hi);
+    }
+  }
+  fit([&](uint32_t, uint64_t c, uint32_t g) {
+    atomicAdd((unsigned long long *)&s.sub_mass[g], (unsigned long long)weight(c));
+    atomicAdd(&s.sub_n[g], 1u);
+    atomicMin(&s.sub_lo[g], item_key(c));
+    atomicMax(&s.sub_hi[g], item_key(c));
+  });
+  __syncthreads();
+  const uint64_t sub_mass = s.sub_mass[lane];
+  const uint32_t sub_n = s.sub_n[lane];
+  // Sub-bin g's tokens in each chunk, or (marks) whether it has some.
+  auto tied = [&](uint32_t g, bool marks) {
+    __syncthreads();
+    if (tid < S)
+      s.tied[tid] = listed(tid) > room
+                        ? (uint32_t)list[(uint64_t)tid * kBlockCandidates + kCutSubs + g]
+                        : 0u;
+    __syncthreads();
+    fit([&](uint32_t c, uint64_t, uint32_t i) {
+      if (i != g) return;
+      if (marks)
+        s.tied[c] = 1;
+      else
+        atomicAdd(&s.tied[c], 1u);
+    });
+    __syncthreads();
+  };
+  // A pass over the chunks with s.tied set.
+  auto sweep = [&](uint32_t mode, uint64_t from, uint64_t to, uint64_t top, uint32_t shift) {
+    if (tid == 0) {
+      s.mode = mode;
+      s.from = from;
+      s.to = to;
+      s.top = top;
+      s.shift = shift;
+      s.small_n = 0;
+    }
+    if (tid < kMaxChunks) {
+      s.sum_mass[tid] = 0;
+      s.sum_n[tid] = 0;
+    }
+    __syncthreads();
+    for (uint32_t c = 0, next = 0; c < S; c = next) {
+      for (next = c + 1; next < S && !s.tied[next];) ++next;
+      if (s.tied[c]) cut_sweep<DT>(row, c, next);
+    }
+  };
+  // The boundary: sub-bin g; the `ties`-th token of its one key, or (ties 0)
+  // the item `bound`. First the top-k one, then from its mass the top-p one.
+  uint32_t g = 0;
+  uint64_t ties = 0, bound = 0, mass2 = st.total;
+#pragma unroll 1
+  for (uint32_t by_mass = 0; by_mass < 2; ++by_mass) {
+    if (by_mass ? !st.topp || !mass2 : !st.need_k) continue;
+    uint64_t target = by_mass ? floor_mul(mass2, rp.top_p) + 1 - st.mass_b0 : st.need_k;
+    // The sub-bin at which the running count or mass reaches the target.
+    const uint64_t own = by_mass ? sub_mass : lane >= sp.n1 ? sub_n : 0ull;
+    const uint64_t run = wave_incl_scan_u64(own);
+    const uint64_t reached = ballot(run >= target);
+    g = reached ? (uint32_t)__builtin_ctzll(reached) : kCutSubs - 1;
+    target -= readlane_u64(run - own, (int)g);
+    const uint32_t lo = s.sub_lo[g], hi = s.sub_hi[g];
+    const uint64_t wq = quantized_weight(key_logit(lo), M, inv_t);
+    uint64_t in = 0;  // the mass of g's tokens up to the boundary
+    ties = 0;
+    if (lo == hi) {
+      ties = !by_mass ? target : wq ? (target + wq - 1) / wq : 1ull;
+      in = ties * wq;
+    } else {
+      tied(g, true);
+      const uint64_t top = ((uint64_t)hi << 19) | 0x7ffffull;
+      uint64_t from = (uint64_t)lo << 19, to = top;
+      uint32_t n = s.sub_n[g];
+      while (n > kCutItems) {
+        const int shift = max(0, 64 - (int)__builtin_clzll(to - from) - 11);
+        for (uint32_t i = tid; i < kCutCells; i += kThreads) {
+          s.cell_mass[i] = 0;
+          s.cell_n[i] = 0;
+        }
+        sweep(by_mass ? kSweepMass : kSweepCount, from, to, to, (uint32_t)shift);
+        constexpr uint32_t B = kCutCells / kThreads;
+        uint64_t sum = 0;
+        for (uint32_t k = 0; k < B; ++k)
+          sum += by_mass ? s.cell_mass[B * tid + k] : (uint64_t)s.cell_n[B * tid + k];
+        uint64_t before = block_excl_scan_u64(sum, s, nullptr);
+        if (before < target && before + sum >= target) {
+          uint32_t cell = B * tid;
+          for (uint32_t k = 0; k + 1 < B; ++k) {
+            const uint64_t v = by_mass ? s.cell_mass[cell] : (uint64_t)s.cell_n[cell];
+            if (before + v >= target) break;
+            before += v;
+            ++cell;
+          }
+          s.sel_bin = cell;
+          s.sel_excl = before;
+          s.n = s.cell_n[cell];
+        }
+        __syncthreads();
+        target -= s.sel_excl;
+        to -= (uint64_t)s.sel_bin << shift;
+        if (to - from >> shift) from = to - ((1ull << shift) - 1);
+        n = s.n;
         __syncthreads();
       }
-  };
-  cut_resolve(rp, st, each, g_cut_launch.out_kept_ids != nullptr, g_cut_lds);
+      sweep(kSweepCollect, from, to, top, 0);
+      const uint32_t held = min(s.small_n, kCutItems);
+      auto each = [&](auto f) {
+#pragma unroll 1
+        for (uint32_t i = tid; i < held; i += kThreads) f(g_cut_lds.items[i]);
+      };
+      bound = items_crossing(
+          each, [](uint64_t) { return true; }, [](uint64_t c) { return c; }, weight, by_mass != 0,
+          target, s);
+      // The tokens of g at and above it, by chunk.
+      each([&](uint64_t c) {
+        if (c < bound) return;
+        atomicAdd((unsigned long long *)&s.sum_mass[item_id(c) / kChunkF32],
+                  (unsigned long long)weight(c));
+        atomicAdd(&s.sum_n[item_id(c) / kChunkF32], 1u);
+      });
+      __syncthreads();
+      in = wave_sum_u64(s.sum_mass[lane]);
+    }
+    if (!by_mass)
+      mass2 = st.mass_bk + in +
+              wave_sum_u64(lane >= sp.n1 && lane < g ? sub_mass : 0ull);
+  }
+  // Each chunk's kept mass and count in the boundary bins: the sub-bins before
+  // g, then g's kept tokens.
+  for (uint32_t c = w; c < S; c += kWaves) {
+    if (listed(c) <= room) continue;
+    const uint64_t *p = list + (uint64_t)c * kBlockCandidates + lane;
+    const uint64_t m = wave_sum_u64(lane < g ? p[0] : 0ull);
+    const uint32_t n = wave_sum_u32(lane < g ? (uint32_t)p[kCutSubs] : 0u);
+    if (lane == 0) {
+      s.cmass[c] += m;
+      s.ccount[c] += n;
+    }
+  }
+  fit([&](uint32_t c, uint64_t v, uint32_t i) {
+    if (i < g) {
+      atomicAdd((unsigned long long *)&s.cmass[c], (unsigned long long)weight(v));
+      atomicAdd(&s.ccount[c], 1u);
+    }
+  });
+  if (!ties) {
+    __syncthreads();
+    if (tid < S) {
+      s.cmass[tid] += s.sum_mass[tid];
+      s.ccount[tid] += s.sum_n[tid];
+    }
+    if (tid == 0) s.bound = bound;
+    __syncthreads();
+    return;
+  }
+  tied(g, false);
+  const uint32_t key = s.sub_lo[g];
+  const uint64_t wq = quantized_weight(key_logit(key), M, inv_t);
+  const uint32_t t = lane < S ? s.tied[lane] : 0u;
+  const uint32_t incl = wave_incl_scan_u32(t);
+  const uint32_t last = (uint32_t)min(ties, (uint64_t)readlane_u32(incl, 63));
+  const uint32_t c = (uint32_t)__builtin_ctzll(ballot(incl >= last));
+  const uint32_t nth = last - readlane_u32(incl - t, (int)c);  // from 1
+  if (w == 0 && lane < S) {
+    const uint32_t kept = lane < c ? t : lane == c ? nth : 0u;
+    s.cmass[lane] += kept * wq;
+    s.ccount[lane] += kept;
+  }
+  // The nth tie of chunk c by id, from the chunk itself.
+  float xs[TPL];
+  load_chunk<DT>(a, rp, row, c, s, xs);
+  uint32_t cnt[LOADS], off[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    cnt[j] = 0;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float v = xs[j * VEC + e];
+      cnt[j] += v == v && logit_key(v) == key ? 1u : 0u;
+    }
+  }
+  order_offsets<LOADS>(cnt, off, s);
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    uint32_t at = off[j];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float v = xs[j * VEC + e];
+      if (v == v && logit_key(v) == key && ++at == nth)
+        s.bound = token_item(key, c * kChunkF32 + tid * VEC + j * SLAB + e);
+    }
+  }
+  __syncthreads();
 }
 
 // The draw inside chunk c of a row without a draft: the first kept token, in id
@@ -4071,7 +4507,29 @@ __device__ __forceinline__ void cut_pick(const SampleLaunch &a, uint32_t row, ui
   }
 }
 
-// The general merge, out of line like the rescan.
+// The rest of a row that cut_refine resolves. Out of line (with the launch
+// record copied to LDS, since a called function cannot reach the kernel's
+// arguments) and with nothing of the caller's left to do after it, so that its
+// registers stay out of the common path.
+template <int DT>
+__device__ __noinline__ void cut_finish_refined(uint32_t row, uint32_t bits) {
+  const SampleLaunch &a = g_cut_launch;
+  CutLds &s = g_cut_lds;
+  cut_refine<DT>(row, bits);
+  const RowParams rp = a.params[row];
+  const RowState st = a.states[row];
+  const uint32_t draft = row_draft(a, rp);
+  if (threadIdx.x < 64)
+    cut_pick(a, row, a.chunks, draft, row_uniform(a, row), (bits & kCutKept) != 0, s);
+  __syncthreads();
+  if (s.u64a == 0) {
+    if (threadIdx.x == 0) write_result(a, row, kNoToken, 0.0f, s.kept);
+  } else if (draft == kNoToken) {
+    cut_walk<DT>(a, rp, st, bits, row, s.sel_chunk, s.bound, s.sel_excl, s.kept, s);
+  }
+}
+
+// The general merge, out of line too.
 template <int DT>
 __device__ __noinline__ void cut_finish_general(uint32_t row, uint32_t n) {
   const RowParams rp = g_cut_launch.params[row];
@@ -4133,13 +4591,13 @@ __device__ __forceinline__ void cut_finish_other(const SampleLaunch &a, const Ro
 // undrafted uncut), so that a batch of several kinds takes no merge and no
 // uncut launch (24 rows x 100,003: 46.4 -> 34.9 us a call). A separate build,
 // since that code costs the cut passes' rows 1.5 us (9.9 against 11.4).
-// Latency-bound: a block a row. Its registers (the rescan's) cost nothing
+// Latency-bound: a block a row. Its registers (cut_refine's) cost nothing
 // here, where a chunk-parallel kernel would run two waves a SIMD for them. The
 // row's record, its boundary bins and its chunks' sums go out together from
 // preloaded arguments; up to 64 listed tokens (most rows) are resolved by one
 // wave without a barrier.
 template <int DT, bool OTHERS>
-__global__ __launch_bounds__(kThreads) void cut_draw_kernel(
+__global__ __launch_bounds__(kThreads, OTHERS ? 1 : 2) void cut_draw_kernel(
     const RowParams *params, const RowState *states, const uint64_t *cands,
     const float *uniforms, const uint32_t *uniform_index, const uint32_t *draft_tokens,
     uint32_t bits, SampleLaunch a) {
@@ -4200,20 +4658,20 @@ __global__ __launch_bounds__(kThreads) void cut_draw_kernel(
   }
   __syncthreads();
   const uint32_t n = s.n;
+  if (n == 0xffffffffu) {
+    cut_copy_launch(a);
+    cut_finish_refined<DT>(row, bits);
+    return;
+  }
   if (n > 64u) {
-    if (n == 0xffffffffu) {
-      cut_copy_launch(a);
-      cut_rescan<DT>(row);
-    } else {
-      // Past the items' room in LDS, the rest stays in the lists.
-      for (uint32_t i = tid; i < min(n, kCutItems); i += kThreads) s.items[i] = item(i);
-      __syncthreads();
-      auto each = [&](auto f) {
-        for (uint32_t i = tid; i < n; i += kThreads)
-          f(i < kCutItems ? g_cut_lds.items[i] : item(i));
-      };
-      cut_resolve(rp, st, each, counts, s);
-    }
+    // Past the items' room in LDS, the rest stays in the lists.
+    for (uint32_t i = tid; i < min(n, kCutItems); i += kThreads) s.items[i] = item(i);
+    __syncthreads();
+    auto each = [&](auto f) {
+      for (uint32_t i = tid; i < n; i += kThreads)
+        f(i < kCutItems ? g_cut_lds.items[i] : item(i));
+    };
+    cut_resolve(rp, st, each, counts, s);
     if (tid < 64) cut_pick(a, row, S, draft, u, counts, s);
     __syncthreads();
   }

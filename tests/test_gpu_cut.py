@@ -49,8 +49,8 @@ def test_cut_rows(V, bf16):
 @pytest.mark.parametrize("decimals", [0, 1, 2])
 def test_cut_ties(decimals):
     """Rounded values: the boundary bin holds from hundreds to tens of
-    thousands of tied tokens, past the chunk lists (1008) and the LDS list
-    (3072)."""
+    thousands of tied tokens, past the chunk lists (200 where tokens are
+    counted, 472 else), so the rows are resolved from sub-bins."""
     V = 60001
     rng = np.random.default_rng(decimals)
     pols = policies(V)
@@ -149,6 +149,148 @@ def test_cut_masks_penalties_and_other_rows():
     plain = [J.policy(temperature=1.0)] * 18  # the self-validating words' launch, after
     check(V, plain, logits=x, uniforms=rng.random(18).astype(np.float32), sampler=s)
     s.close()
+
+
+def flat_rows(V, rng):
+    """Rows whose boundary bins hold more tokens of a chunk than its list takes:
+    (name, values)."""
+    normal = rng.normal(0, 2.5, V).astype(np.float32)
+    yield "constant", np.full(V, 1.5, np.float32)
+    two = np.full(V, -4.0, np.float32)
+    two[rng.choice(V, 1000, replace=False)] = 1.0
+    yield "two values", two
+    signs = np.zeros(V, np.float32)
+    signs[::3] = -0.0
+    signs[5] = 0.25
+    yield "signed zeros under one", signs
+    yield "integers", np.round(normal)
+    yield "quarters", np.round(normal * 4) / 4
+    one = normal.copy()
+    one[V // 2] = 80.0  # bins so wide that distinct values crowd them
+    yield "one far above", one
+    low = normal.copy()
+    low[::3] = -900.0
+    low[::7] = -1e5
+    low[::11] = -np.inf
+    yield "banned by value", low
+    half = normal.copy()
+    half[:V // 2] = 0.0  # ties in some chunks, spread values in the others
+    yield "half tied", half
+    near = (np.float32(3.0) + rng.integers(0, 3, V).astype(np.float32) * np.float32(2.0 ** -22))
+    near[0] = 30.0  # neighbouring floats, a third of the row each: one sub-bin
+    yield "neighbouring floats", near.astype(np.float32)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("V", [9000, 151936, 290003])
+def test_cut_flat_rows(V, bf16):
+    """Rows resolved from sub-bins (and, where one holds more than LDS, by
+    rereading its chunks): with and without counts, at top-k boundaries inside ties, at
+    their first and last token, and top-p boundaries among them."""
+    rng = np.random.default_rng(V + bf16)
+    for name, row in flat_rows(V, rng):
+        pols = [J.policy(temperature=0.8, top_p=0.95), J.policy(temperature=5.0, top_p=0.3),
+                J.policy(temperature=0.1, top_k=V // 8), J.policy(temperature=1.0, top_k=1000),
+                J.policy(temperature=1.0, top_k=1001),
+                J.policy(temperature=0.9, top_k=2000, top_p=0.9),
+                J.policy(temperature=3.0, top_k=V // 2, top_p=0.6),
+                J.policy(temperature=1.0, top_k=V - 1), J.policy(temperature=4.0, min_p=0.0005)]
+        x = np.tile(row, (len(pols), 1))
+        u = rng.random(len(pols)).astype(np.float32)
+        kw = dict(logits_bf16=WL.to_bf16_bits(x)) if bf16 else dict(logits=x)
+        print(name, flush=True)
+        check(V, pols, uniforms=u, **kw)
+        check(V, pols, uniforms=u, kept_capacity=3000, **kw)
+
+
+@pytest.mark.parametrize("n", [199, 200, 201, 400, 471, 472, 473])
+@pytest.mark.parametrize("kept", [0, 2000])
+def test_cut_list_room(n, kept):
+    """n tied boundary tokens in each of 19 chunks: just inside and just past
+    the chunk lists' room (200 where tokens are counted, 472 else), and, from
+    400 on without counts, more of them in lists that fit than LDS takes
+    (6144)."""
+    V = 19 * 8192 - 77
+    rng = np.random.default_rng(n)
+    x = np.full(V, -30.0, np.float32)
+    for c in range(19):
+        at = c * 8192 + rng.choice(8192 - 77, n + 3, replace=False)
+        x[at] = 0.0
+        x[at[:3]] = 4.0 + rng.random(3)
+    pols = [J.policy(temperature=1.0, top_p=p) for p in (0.5, 0.9, 0.99)]
+    pols += [J.policy(temperature=1.0, top_k=k) for k in (57 + 19 * n // 2, 57 + 19 * n)]
+    pols += [J.policy(temperature=1.0, top_k=57 + 19 * n // 2, top_p=0.9)]
+    xs = np.tile(x, (len(pols), 1))
+    check(V, pols, logits=xs, uniforms=rng.random(len(pols)).astype(np.float32),
+          kept_capacity=kept)
+
+
+def test_cut_flat_rows_penalized_masked_and_drafted():
+    """Sub-bins over penalized, masked and drafted rows."""
+    V, rows = 40003, 8
+    rng = np.random.default_rng(41)
+    x = np.round(rng.normal(0, 2.0, (rows, V))).astype(np.float32)
+    x[3] = 0.0
+    # Neighbouring floats under one high value: a sub-bin past LDS.
+    x[4:6] = np.float32(3.0) + rng.integers(0, 3, (2, V)).astype(np.float32) * 2.0 ** -22
+    x[4:6, 0] = 30.0
+    allowed = rng.random((rows, V)) < 0.5
+    kinds = [dict(temperature=0.8, top_p=0.95, presence=0.4, frequency=0.2),
+             dict(temperature=1.0, top_k=1500, repetition=1.2),
+             dict(temperature=1.0, top_k=3000, top_p=0.9, constrained=True),
+             dict(temperature=1.0, top_p=0.7, constrained=True, presence=0.3)]
+    pols = [J.policy(**kinds[r % 4]) for r in range(rows)]
+    hist = [rng.integers(0, V, 900).astype(np.uint32) if r % 4 != 2 else None
+            for r in range(rows)]
+    draft = rng.integers(0, V, rows).astype(np.uint32)
+    draft[:4] = x[:4].argmax(1)
+    cid = rng.integers(0, V, (rows, 16)).astype(np.uint32)
+    cid[:, 0] = draft
+    kw = dict(logits=x, masks=WL.mask_words(allowed), histories=hist,
+              generated=[450 if h is not None else 0 for h in hist], mark_prompt=[True] * rows)
+    dr = dict(draft_tokens=draft, drafted_rows=6, cand_ids=cid,
+              cand_probs=rng.dirichlet(np.ones(16), rows).astype(np.float32))
+    for kept in (0, 5000):
+        u = rng.random(rows).astype(np.float32)
+        check(V, pols, uniforms=u, kept_capacity=kept, **kw)
+        check(V, pols, uniforms=u, kept_capacity=kept, **kw, **dr)
+
+
+def test_flat_rows_cost_a_bounded_multiple():
+    """A call of rows whose tokens all tie, or whose top-k boundary lies far below
+    the maximum at a low temperature, takes a few times what a call of spread
+    rows takes (80 and 34 us against 32 measured), not the fifty times of
+    rereading the row for every step (1660 and 1810 us). The bounds are three
+    times what was measured."""
+    import torch
+    V, rows = 151936, 16
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    normal = torch.randn((rows, V), generator=g, device="cuda") * 2.5
+
+    def us(x, pol):
+        s = J.Sampler(V, rows)
+        out = torch.zeros(rows, dtype=torch.int32, device="cuda")
+        a, keep = s.sample_args(x, [pol] * rows, out, uniforms=torch.rand(rows, device="cuda"))
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        times = []
+        for _ in range(7):
+            ev[0].record()
+            for _ in range(10):
+                s.launch(a)
+            ev[1].record()
+            torch.cuda.synchronize()
+            times.append(ev[0].elapsed_time(ev[1]) * 100)
+        del keep
+        s.close()
+        return sorted(times)[3]
+
+    topp = J.policy(temperature=0.8, top_p=0.95)
+    base = us(normal, topp)
+    flat = us(torch.zeros((rows, V), device="cuda"), topp)
+    deep = us(normal, J.policy(temperature=0.1, top_k=20000))
+    print(f"spread {base:.1f} us, constant {flat:.1f}, deep top-k {deep:.1f}", flush=True)
+    assert flat < 8 * base and deep < 4 * base
 
 
 def test_cut_rows_past_a_grid_dimension():
