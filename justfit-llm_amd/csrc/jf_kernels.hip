@@ -3019,7 +3019,10 @@ __device__ __forceinline__ void merge_small_row(
   const uint32_t n_all = s.hoff[S];
   // (A top-k past a wave's worth goes straight to the general merge.)
   const bool few = K <= 64u || (rp.flags & kRowMinP);
-  if (few && !s.row_overflow && thr > kLowestKey && (!s.row_long || n_all <= kSlots)) {
+  // (A min-p row past kMergeItems is the cut passes', cut_takes, even where the
+  // fetched slots would hold it; the general merge leaves it to them.)
+  const uint32_t fetched = K > (uint32_t)kBlockCandidates ? min(kSlots, kMergeItems) : kSlots;
+  if (few && !s.row_overflow && thr > kLowestKey && n_all <= fetched) {
     uint32_t valid = 0;
     if (!s.row_long) {
 #pragma unroll

@@ -256,6 +256,32 @@ def test_cut_flat_rows_penalized_masked_and_drafted():
         check(V, pols, uniforms=u, kept_capacity=kept, **kw, **dr)
 
 
+@pytest.mark.parametrize("n", [2560, 2561, 3072, 3073, 5120, 5121])
+@pytest.mark.parametrize("listed", [False, True])
+def test_cut_minp_rows_at_the_merge_limits(n, listed):
+    """Min-p rows whose lists hold n tokens at or above the floor, around what
+    the small merge fetches (2560 slots; 5120 beside listed rows past 20
+    chunks) and what the general merge holds (3072): each finished by the merge
+    or by the cut passes, not by both and not by neither."""
+    V = 31 * 8192 - 100
+    rng = np.random.default_rng(n)
+    rows = 4
+    x = np.full((rows, V), -50.0, np.float32)
+    for r in range(rows):
+        for c in range(31):
+            k = n // 31 + (c < n % 31)
+            at = c * 8192 + rng.choice(8192 - 100, k, replace=False)
+            x[r, at] = 9.0 + rng.random(k)
+            x[r, at[0]] = 10.5
+    pols = [J.policy(temperature=1.0, min_p=0.05), J.policy(temperature=1.0, min_p=0.04, top_p=0.8),
+            J.policy(temperature=0.9, min_p=0.05, top_k=2000, top_p=0.95),
+            J.policy(temperature=0.7, top_k=50) if listed else
+            J.policy(temperature=1.0, min_p=0.05)]
+    u = rng.random(rows).astype(np.float32)
+    check(V, pols, logits=x, uniforms=u)
+    check(V, pols, logits=x, uniforms=u, kept_capacity=3000)
+
+
 def test_flat_rows_cost_a_bounded_multiple():
     """A call of rows whose tokens all tie, or whose top-k boundary lies far below
     the maximum at a low temperature, takes a few times what a call of spread
