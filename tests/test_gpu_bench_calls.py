@@ -8,9 +8,9 @@ them, C4's selection and then its tree acceptance (retained and accepted
 counts, path rows, the accepted tokens), as two calls and as the step the
 bench times (jf_sample_accept_tree); C2 also with histories clustered
 in low ids (every row, and every fourth row), which widen the penalty
-table's fixed slots from 256 to 512 a chunk, and through the general
-kernels (rows one float past 16-byte alignment, top-k 3000: select_kernel,
-merge_kernel, the multi-pass stages); and the penalized chain-verify
+table's fixed slots from 256 to 512 a chunk, and in the general mode
+(rows one float past 16-byte alignment, top-k 3000: the unaligned select
+pass and the cut passes); and the penalized chain-verify
 step (4 lanes x 16 rows, V = 248,320: extras, sparse drafts, then chain
 acceptance)."""
 import numpy as np

@@ -5,7 +5,9 @@ that hold one token, every token, or more than the chunk lists and the LDS list
 take (ties, constant rows, a range far off); boundaries in the first and the
 last bin; vocabularies of one chunk, of one token past a chunk, and whole rows;
 temperatures that leave one weight or all weights; rows of infinities and NaN;
-masks, stops and penalties; drafts with kept and unkept tokens."""
+masks, stops and penalties; drafts with kept and unkept tokens. Also the merge's
+rows next to them: top-k up to the candidate lists' limit, and min-p rows at
+its own."""
 import numpy as np
 import pytest
 
@@ -44,6 +46,41 @@ def test_cut_rows(V, bf16):
     u[:3] = 0.0, np.float32(1.0 - 2.0 ** -24), 0.5
     kw = dict(logits_bf16=WL.to_bf16_bits(x)) if bf16 else dict(logits=x)
     check(V, pols, uniforms=u, kept_capacity=V if V < 20000 else 5000, **kw)
+    check(V, pols, uniforms=u, **kw)  # (top-p alone is not counted without kept outputs)
+
+
+@pytest.mark.parametrize("kind", ["spread", "ties", "drafted", "dense"])
+@pytest.mark.parametrize("V,bf16", [(300, False), (8193, True), (20003, False), (151936, True),
+                                    (151936, False), (290003, True)])
+def test_top_k_around_the_list_limit(V, bf16, kind):
+    """Top-k from one wave's worth to just past the candidate lists (64, 65..96,
+    97), no min-p floor: the small and the general merge of lists of up to a few
+    hundred candidates a chunk, and lists that overflow (ties), with drafts."""
+    rng = np.random.default_rng(V + bf16)
+    ks = (64, 65, 72, 80, 95, 96, 97, 96)
+    pols = [J.policy(temperature=0.8, top_k=k, **(dict(top_p=0.9) if i % 2 else {}))
+            for i, k in enumerate(ks)]
+    x = rng.normal(0, 2.5, (len(ks), V)).astype(np.float32)
+    if kind == "ties":
+        x = np.round(x)
+        x[7] = 0.0
+    kw = dict(logits_bf16=WL.to_bf16_bits(x)) if bf16 else dict(logits=x)
+    if kind in ("drafted", "dense"):
+        draft = x.argmax(1).astype(np.uint32)
+        draft[::3] = rng.integers(0, V, len(draft[::3]))
+        draft[4] = NO
+        kw["draft_tokens"] = draft
+        if kind == "dense":
+            kw["dense_q"] = rng.dirichlet(np.ones(V) * 0.05, len(ks)).astype(np.float32)
+        else:
+            cid = rng.integers(0, V, (len(ks), 16)).astype(np.uint32)
+            cid[:, 0] = draft
+            kw.update(cand_ids=cid, cand_probs=rng.dirichlet(np.ones(16), len(ks))
+                      .astype(np.float32))
+    u = rng.random(len(ks)).astype(np.float32)
+    check(V, pols[:6], uniforms=u[:6], **{k: v[:6] for k, v in kw.items()})  # lists alone
+    check(V, pols, uniforms=u, **kw)  # beside a row of the cut passes
+    check(V, pols, uniforms=u, kept_capacity=100, **kw)
 
 
 @pytest.mark.parametrize("decimals", [0, 1, 2])
@@ -280,6 +317,60 @@ def test_cut_minp_rows_at_the_merge_limits(n, listed):
     u = rng.random(rows).astype(np.float32)
     check(V, pols, logits=x, uniforms=u)
     check(V, pols, logits=x, uniforms=u, kept_capacity=3000)
+
+
+def test_cut_passes_replay_under_a_hip_graph():
+    """The cut passes of jf_sample_static captured into a graph and replayed,
+    with eager calls and synchronizations between: spread, tied and crowded
+    rows, kept outputs, beside listed and greedy ones."""
+    import torch
+    V, rows, cap = 60001, 8, 2000
+    rng = np.random.default_rng(47)
+    x = rng.normal(0, 2.5, (rows, V)).astype(np.float32)
+    x[1] = np.round(x[1])
+    x[2] = 1.0
+    x[3, 9] = 70.0
+    pols = [J.policy(temperature=0.8, top_p=0.95), J.policy(temperature=1.0, top_k=1500),
+            J.policy(temperature=0.9, top_p=0.7), J.policy(temperature=1.0, top_k=20000, top_p=0.9),
+            J.policy(temperature=2.0, min_p=0.005), J.policy(temperature=0.7, top_k=50), J.policy(),
+            J.policy(temperature=0.2, top_k=9000)]
+    u = rng.random(rows).astype(np.float32)
+    want = run_oracle(V, pols, logits=x, uniforms=u, kept_capacity=cap)
+    z = lambda *s, d=torch.int32: torch.zeros(s, dtype=d, device="cuda")  # noqa: E731
+    out, kept = z(rows), (z(rows), z(rows, cap), z(rows, cap, d=torch.float32))
+    s = J.Sampler(V, rows)
+    hold = (torch.from_numpy(x).cuda(), torch.from_numpy(u).cuda())
+    a, keep = s.sample_args(hold[0], pols, out, uniforms=hold[1], kept=kept)
+
+    def same():
+        torch.cuda.synchronize()
+        assert_same(dict(tokens=out.cpu().numpy().view(np.uint32), draft_probs=want["draft_probs"],
+                         kept_counts=kept[0].cpu().numpy().view(np.uint32),
+                         kept_ids=kept[1].cpu().numpy().view(np.uint32),
+                         kept_probs=kept[2].cpu().numpy()), want)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        J.sample_static(V, a)  # outside capture: the scratch address lookup
+    same()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        J.sample_static(V, a)
+    for _ in range(4):
+        out.fill_(-1)
+        for t in kept:
+            t.zero_()
+        s.launch(a)
+        same()
+        out.fill_(-1)
+        for t in kept:
+            t.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        same()
+    del graph, keep, hold
+    s.close()
 
 
 def test_flat_rows_cost_a_bounded_multiple():

@@ -4,7 +4,7 @@ Bar: bit-exact tokens, kept sets, kept probabilities and draft probabilities
 (the oracle restates the same fp32 weight and exact integer sums); greedy ids
 bit-exact. Full-size configs C1-C3 and C5 are compared row by row; edge cases
 cover ties, empty/NaN/inf rows, masks, stop exclusion, vocabularies that do
-not fill a chunk, the multi-pass stages (top-k disabled with top-p or
+not fill a chunk, the cut passes (top-k disabled with top-p or
 min-p, large k), the two-pass draw of rows with no cut (with plain, dense
 and sparse drafts, and mixed with cut rows in one launch), and chi-square
 tests of 10^6 draws through the merge and through the two-pass draw."""
@@ -485,7 +485,7 @@ def test_unfiltered_mass_draw(bf16, greedy, draft):
 @pytest.mark.parametrize("kind", ["small", "general", "staged", "drafted"])
 def test_mixed_cut_and_uncut_rows(kind):
     """Launches mixing rows with a cut and rows that keep every admitted
-    token: the merge (small, general, or with stages for a large k) finishes
+    token: the merge (small, or with the cut passes for a large k) finishes
     the cut rows and greedy rows, the mass-and-draw launch the uncut ones."""
     rng = np.random.default_rng(71 + len(kind))
     V = 5 * 8192 + 1234
