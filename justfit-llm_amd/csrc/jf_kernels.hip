@@ -3612,7 +3612,8 @@ __device__ __forceinline__ CutRow cut_row(const RowParams &rp, const BlockHeader
   // lies below them, and when the weights do not reach twice as far the range
   // is the row's (a little more, so that its least value stays out of the open
   // last bin).
-  float range = -rp.minp_offset, span = 0.0f;
+  // (0 - x: a min-p of 1 has an offset of 0, and 1 / range is then +inf.)
+  float range = 0.0f - rp.minp_offset, span = 0.0f;
   if (!minp) {
     const float least = -wave_max_f32(lane < S ? -h.best_value : -__builtin_inff());
     span = r.maximum - least;

@@ -231,7 +231,9 @@ def test_cut_flat_rows(V, bf16):
                 J.policy(temperature=1.0, top_k=1001),
                 J.policy(temperature=0.9, top_k=2000, top_p=0.9),
                 J.policy(temperature=3.0, top_k=V // 2, top_p=0.6),
-                J.policy(temperature=1.0, top_k=V - 1), J.policy(temperature=4.0, min_p=0.0005)]
+                J.policy(temperature=1.0, top_k=V - 1), J.policy(temperature=4.0, min_p=0.0005),
+                # The floor is the maximum itself: one value, many tokens of it.
+                J.policy(temperature=1.0, min_p=1.0), J.policy(temperature=1.0, min_p=1.0, top_p=0.4)]
         x = np.tile(row, (len(pols), 1))
         u = rng.random(len(pols)).astype(np.float32)
         kw = dict(logits_bf16=WL.to_bf16_bits(x)) if bf16 else dict(logits=x)
