@@ -4515,7 +4515,8 @@ __device__ __forceinline__ void cut_pick(const SampleLaunch &a, uint32_t row, ui
 // record copied to LDS, since a called function cannot reach the kernel's
 // arguments) and with nothing of the caller's left to do after it, so that its
 // registers stay out of the common path.
-template <int DT>
+// (OTHERS: cut_draw_kernel's, whose builds allow it different registers.)
+template <int DT, bool OTHERS>
 __device__ __noinline__ void cut_finish_refined(uint32_t row, uint32_t bits) {
   const SampleLaunch &a = g_cut_launch;
   CutLds &s = g_cut_lds;
@@ -4601,7 +4602,8 @@ __device__ __forceinline__ void cut_finish_other(const SampleLaunch &a, const Ro
 // preloaded arguments; up to 64 listed tokens (most rows) are resolved by one
 // wave without a barrier.
 template <int DT, bool OTHERS>
-__global__ __launch_bounds__(kThreads, OTHERS ? 1 : 2) void cut_draw_kernel(
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(OTHERS ? 1 : 2))) void cut_draw_kernel(
     const RowParams *params, const RowState *states, const uint64_t *cands,
     const float *uniforms, const uint32_t *uniform_index, const uint32_t *draft_tokens,
     uint32_t bits, SampleLaunch a) {
@@ -4664,7 +4666,7 @@ __global__ __launch_bounds__(kThreads, OTHERS ? 1 : 2) void cut_draw_kernel(
   const uint32_t n = s.n;
   if (n == 0xffffffffu) {
     cut_copy_launch(a);
-    cut_finish_refined<DT>(row, bits);
+    cut_finish_refined<DT, OTHERS>(row, bits);
     return;
   }
   if (n > 64u) {
