@@ -345,16 +345,6 @@ __device__ __forceinline__ uint32_t row_shr_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x110 + D, 0xF, 0xF, true);
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
-  const uint32_t lo = __shfl_xor((uint32_t)v, m, kWave);
-  const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), m, kWave);
-  return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t shfl_down_u64(uint64_t v, int d) {
-  const uint32_t lo = __shfl_down((uint32_t)v, d, kWave);
-  const uint32_t hi = __shfl_down((uint32_t)(v >> 32), d, kWave);
-  return ((uint64_t)hi << 32) | lo;
-}
 __device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int src) {
   const uint32_t lo = __shfl((uint32_t)v, src, kWave);
   const uint32_t hi = __shfl((uint32_t)(v >> 32), src, kWave);

@@ -104,14 +104,17 @@ constexpr int kWaves = 4;
 constexpr int kBlockCandidates = 1024;
 constexpr int kMergeCapacity = 2048;
 constexpr uint32_t kMergeItems = 3072;  // tokens of a row the general merge holds
-constexpr int kPenaltyWordsLds = 2048;
 // A sampled row with no min-p floor whose top-k is off or past this takes the
 // cut passes; up to it, the candidate lists and the merge. The select pass
 // bounds a chunk's K-th token by its waves' ceil(K / 4)-th largest lane maxima
 // (64 of them), so the lists grow faster than K: 64 rows x 151,936 fp32 ran
 // 33.0 us at top-k 65, 38.4 at 96, 42.0 at 112, 70 at 128 (lists that overflow)
 // through the lists, and 46.8-47.5 through the cut passes; in bf16 31.3, 37.2,
-// 46.1, 70 against 43.5-44.1.
+// 46.1, 70 against 43.5-44.1. Where the line lies for other batches, at top-k
+// 96 through the lists and 97 through the cut passes: 1 row 25.6 and 24.6, 16
+// rows 26.9 and 27.4, 256 rows 49.5 and 102.8 (fp32; bf16 26.3 and 24.3, 26.9
+// and 26.8, 41.9 and 95.4), 1 row x 248,320 bf16 with top-p 61.1 and 26.9, 64
+// rows of it 69.0 and 58.5.
 constexpr uint32_t kListTopK = 96;
 constexpr uint32_t kCutBins = 512;    // bins of a row's values below its maximum
 constexpr uint32_t kCutItems = 6144;  // boundary tokens of a row resolved in LDS
@@ -403,7 +406,7 @@ int launch_select_fast(const FastLaunch &f, const FastRows *fr, uint32_t rows, u
 int launch_merge(const SampleLaunch &a, uint32_t dtype, void *stream);
 // wide: some cut row of the launch has no min-p floor (longer candidate
 // lists); the merge then fetches more list slots a chunk where that helps.
-// hold: some listed row may keep more than 64 tokens.
+// hold: some min-p row may keep more than 64 tokens.
 int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, bool hold, void *stream);
 // Rows with no cut (grid rows x per_row: per_row = chunks when the launch
 // has drafted uncut rows, else 1).

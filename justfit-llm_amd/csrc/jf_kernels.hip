@@ -1,20 +1,22 @@
 // gfx950 kernels of JustFit's logits->token path.
 //
-// One selection is one launch of select_kernel over rows x chunks blocks
-// (plus, for rows whose kept set the candidate lists cannot hold, the cut
-// passes). Each block holds its chunk of a row in registers: one pass over
-// HBM with 16-byte loads, the penalties, the constraint mask and the stop
-// exclusion applied on the fly (the reference's decode_sample_penalize,
-// TargetRow::admits; sampling.metal:33-37, 928-993). A greedy row reduces its
-// argmax (sampling.metal:1427-1512); a sampled row writes its chunk's
-// maximum and the tokens that can still belong to its min-p/top-k/top-p
-// distribution. The last block of a row to finish (the reference's
-// split_arrive_last, split_reduce.h:14-28) merges: the global maximum, the
-// min-p floor, the exact top-k in (logit desc, id asc) order, the top-p
-// nucleus, and the inverse-CDF draw in id order with the residual of a
-// drafted row (sampling.metal:585-829). Every sum that decides a token is an
-// exact 64-bit sum of floor(w * 2^44), so the parallel order never changes
-// a result.
+// One selection is a select launch over rows x chunks blocks
+// (select_fast_kernel; select_kernel for the rows it does not take) and what
+// finishes its rows: nothing more where the row's last chunk block does (greedy
+// rows, rows with no cut), the merge of the candidate lists, the cut passes for
+// rows whose kept set the lists cannot hold, the uncut draw. Each block holds
+// its chunk of a row in registers: one pass over HBM with 16-byte loads, the
+// penalties, the constraint mask and the stop exclusion applied on the fly (the
+// reference's decode_sample_penalize, TargetRow::admits; sampling.metal:33-37,
+// 928-993). A greedy row reduces its argmax (sampling.metal:1427-1512); a
+// sampled row writes its chunk's maximum and the tokens that can still belong
+// to its min-p/top-k/top-p distribution. The merge of a row (the reference's
+// split_arrive_last, split_reduce.h:14-28, has the last group to finish do it)
+// takes the global maximum, the min-p floor, the exact top-k in (logit desc, id
+// asc) order, the top-p nucleus, and the inverse-CDF draw in id order with the
+// residual of a drafted row (sampling.metal:585-829). Every sum that decides a
+// token is an exact 64-bit sum of floor(w * 2^44), so the parallel order never
+// changes a result.
 #include <hip/hip_ext.h>
 
 #include <mutex>
@@ -102,15 +104,12 @@ struct __align__(16) Lds {
   uint32_t sel_bin;
   uint64_t sel_excl;
   uint32_t hit;
-  uint32_t found_id;
   float found_w;
   uint32_t u32a;
-  uint32_t nbound;
   float row_max;
   uint32_t row_admitted;
   uint32_t row_overflow;
   uint32_t row_floor;
-  uint32_t row_maxcount;
   uint32_t row_long;  // merge_small_kernel: a list is longer than its fetched slots
   uint64_t u64a;
 };
@@ -165,22 +164,6 @@ __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, L &s) {
   if (lane_id() == 0) s.wl[threadIdx.x >> 6] = v;
   __syncthreads();
   return s.wl[0] + s.wl[1] + s.wl[2] + s.wl[3];
-}
-template <class L>
-__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, L &s) {
-  v = wave_max_u32(v);
-  __syncthreads();
-  if (lane_id() == 0) s.wu[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return max(max(s.wu[0], s.wu[1]), max(s.wu[2], s.wu[3]));
-}
-template <class L>
-__device__ __forceinline__ uint32_t block_min_u32(uint32_t v, L &s) {
-  v = wave_min_u32(v);
-  __syncthreads();
-  if (lane_id() == 0) s.wu[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return min(min(s.wu[0], s.wu[1]), min(s.wu[2], s.wu[3]));
 }
 template <class L>
 __device__ __forceinline__ float block_max_f32(float v, L &s) {
@@ -626,11 +609,8 @@ __device__ __forceinline__ uint32_t row_draft(const SampleLaunch &a, const RowPa
                                                         : kNoToken;
 }
 
-// The draft's probability of `token` for a drafted row: its dense q, or
-// the first sparse candidate that lists it (sampling.metal:703-708); the
-// merge stages the row's 16 candidates in s.cids/s.cprobs.
 // A sampled row with no min-p, top-k or top-p cut: it keeps every admitted
-// token. The merges and stages skip such rows; uncut_kernel draws them.
+// token. The merges and cut passes skip such rows; uncut_kernel draws them.
 __device__ __forceinline__ bool uncut_row(const RowParams &rp) {
   return (rp.flags & kRowSampled) && !(rp.flags & (kRowMinP | kRowTopK | kRowTopP));
 }
@@ -643,6 +623,9 @@ __device__ __forceinline__ bool cut_pass_row(const RowParams &rp) {
           rp.top_k > (uint32_t)kBlockCandidates);
 }
 
+// The draft's probability of `token` for a drafted row: its dense q, or
+// the first sparse candidate that lists it (sampling.metal:703-708); the
+// merge stages the row's 16 candidates in s.cids/s.cprobs.
 template <class L>
 __device__ __forceinline__ float draft_q(const SampleLaunch &a, const RowParams &rp,
                                          uint32_t token, const L &s) {
@@ -2719,16 +2702,17 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(SampleLaunch a) {
 
 // ---- the small-K merge -----------------------------------------------------
 //
-// One block per row, for launches whose sampled rows all keep at most 64
-// tokens (top-k <= 64) and take their draft probabilities, if any, from the
-// sparse candidates. It computes what merge_kernel computes, built for
-// latency: every kernel argument in one round trip, then every load the row
-// needs in one batch (its policy, the chunk summaries, the first slots of
-// every chunk's candidate list, the uniform, the draft and its candidates);
-// the 1024-bin histogram that leaves the top K and the boundary bin; and a
-// finish by one wave in registers. Rows the speculative fetch does not cover
-// (an overflowed chunk, a list longer than the slots fetched, values that do
-// not spread over the bins) take merge_kernel's general path.
+// One block per row, for launches that take their draft probabilities, if any,
+// from the sparse candidates. It computes what merge_kernel computes, built for
+// the latency of rows that keep at most 64 tokens: every kernel argument in one
+// round trip, then every load the row needs in one batch (its policy, the chunk
+// summaries, the first slots of every chunk's candidate list, the uniform, the
+// draft and its candidates); the 1024-bin histogram that leaves the top K and
+// the boundary bin; and a finish by one wave in registers. The others go on to
+// the general merge (merge_items, merge_sampled): rows that keep more (a top-k
+// of 65 to kListTopK at once), and rows the fetch does not cover (an overflowed
+// chunk, a list longer than the slots fetched, values that do not spread over
+// the bins).
 
 // The exact top-K (K <= 64) of a row's candidates held in registers (v[k] =
 // key | id << 32; bit k of `valid` set for an item at or above the floor),
@@ -3370,7 +3354,7 @@ static_assert(kCutGroups == 32 && kCutBins == 2 * kThreads);
 // arguments (preloaded into scalar registers): 5 pointers, the row stride, the
 // vocabulary and `bits`: the chunks per row, and these.
 constexpr uint32_t kCutAll = 0x100u;    // every row takes the passes by its policy
-constexpr uint32_t kCutPlain = 0x200u;  // no row is penalized, the vocabulary holds a vector
+constexpr uint32_t kCutPlain = 0x200u;  // no row is penalized
 constexpr uint32_t kCutKept = 0x400u;   // kept outputs are asked for
 constexpr uint32_t kCutUncut = 0x800u;  // cut_draw_kernel draws the uncut rows
 constexpr uint32_t kCutSmall = 0x1000u; // listed rows may take merge_small_row
@@ -3533,7 +3517,10 @@ __device__ __forceinline__ uint32_t cut_sub(const CutSpan &r, float v, float max
 }
 // A chunk of a row of these passes: xs[i] as load_chunk leaves it. A row with
 // no penalty requests its logits first thing (fast_load), before its record
-// has arrived; a penalized one takes load_chunk.
+// has arrived; a penalized one takes load_chunk. (V < 8, less than fast_load's
+// one vector, never holds: these rows have more than kListTopK tokens. Without
+// the test the compiler orders the output launch's loads so that it takes 11.2
+// us in place of 10.7 at 16 rows x 151,936 with kept outputs.)
 template <int DT, class L>
 __device__ __forceinline__ void cut_load(const SampleLaunch &a, const void *logits, uint64_t stride,
                                          uint32_t V, uint32_t row, uint32_t chunk, bool plain,
@@ -5751,7 +5738,7 @@ int launch_cut(const SampleLaunch &a, uint32_t dtype, const CutLaunch &c, void *
   const dim3 block(kThreads);
   const hipStream_t st = (hipStream_t)stream;
   const uint32_t bits = a.chunks | (c.all ? kCutAll : 0u) |
-                        (c.plain && a.vocabulary >= 8 ? kCutPlain : 0u) |
+                        (c.plain ? kCutPlain : 0u) |
                         (a.out_kept_ids ? kCutKept : 0u) | (c.uncut ? kCutUncut : 0u) |
                         (c.small ? kCutSmall : 0u);
   auto go = [&](auto kernel) {

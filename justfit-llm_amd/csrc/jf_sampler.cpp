@@ -960,8 +960,8 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   // none). wide: some listed row has no min-p floor (longer lists).
   const bool small = !a->draft_q && a->uniform_offset <= 0xffffffffull &&
                      a->uniform_stride <= 0xffffffffull;
-  // hold: some listed row may keep more than 64 tokens (a min-p floor and a
-  // larger top-k, or none).
+  // hold: some min-p row may keep more than 64 tokens (a larger top-k, or none).
+  // (Rows with no floor and a top-k of 65 to 96 take the general merge's lists.)
   bool wide = false, hold = false;
   for (uint32_t r = 0; r < rows; ++r) {
     const jf::RowParams &rp = params[r];
