@@ -2702,9 +2702,9 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(SampleLaunch a) {
 
 // ---- the small-K merge -----------------------------------------------------
 //
-// One block per row, for launches that take their draft probabilities, if any,
-// from the sparse candidates. It computes what merge_kernel computes, built for
-// the latency of rows that keep at most 64 tokens: every kernel argument in one
+// One block per row. It computes what merge_kernel computes (which takes launches
+// with a dense q and a row that may keep more than 64 tokens), built for the
+// latency of rows that keep at most 64 tokens: every kernel argument in one
 // round trip, then every load the row needs in one batch (its policy, the chunk
 // summaries, the first slots of every chunk's candidate list, the uniform, the
 // draft and its candidates); the 1024-bin histogram that leaves the top K and
@@ -2836,7 +2836,9 @@ __device__ __noinline__ void merge_small_general(uint32_t row, uint32_t n) {
 // call). Their registers then stay live through the rank select, 0.2-0.4 us
 // that a launch without such rows need not pay (64 x 151,936 top-k 50: 17.7 ->
 // 17.5 us; 64 chain rows x 248,320: 27.25 -> 26.9).
-template <int DT, int SPEC, bool HOLD, class General>
+// DENSE: drafted rows read a dense q (at the row's end; a separate build, since
+// the sparse candidates' loads and the q's would share the row's start).
+template <int DT, int SPEC, bool HOLD, bool DENSE, class General>
 __device__ __forceinline__ void merge_small_row(
     const BlockHeader *headers, const uint64_t *cands, const RowParams *params,
     const float *uniforms, const uint32_t *uniform_index, uint32_t chunks_bits,
@@ -2870,8 +2872,10 @@ __device__ __forceinline__ void merge_small_row(
   uint64_t daddr = (uint64_t)hrow, qaddr = (uint64_t)hrow, paddr = (uint64_t)hrow;
   if (has_draft) {
     daddr = (uint64_t)(a.draft_tokens + row);
-    qaddr = (uint64_t)(a.cand_ids + (uint64_t)row * 16 + (tid & 15));
-    paddr = (uint64_t)(a.cand_probs + (uint64_t)row * 16 + (tid & 15));
+    if constexpr (!DENSE) {
+      qaddr = (uint64_t)(a.cand_ids + (uint64_t)row * 16 + (tid & 15));
+      paddr = (uint64_t)(a.cand_probs + (uint64_t)row * 16 + (tid & 15));
+    }
   }
   uint64_t pbase = (uint64_t)(params + row);
   asm volatile("" : "+v"(hbase), "+v"(cbase), "+v"(uaddr), "+v"(ubase), "+v"(daddr),
@@ -2939,7 +2943,7 @@ __device__ __forceinline__ void merge_small_row(
     // Drafts addressed through the row's record (a batch of verify lanes):
     // their loads wait for the policy (the launch passed drafted_rows 0).
     draft = row_draft(a, rp);
-    if (draft != kNoToken && tid < 16) {
+    if (!DENSE && draft != kNoToken && tid < 16) {
       cid = a.cand_ids[(uint64_t)rp.cand_index * 16 + tid];
       cpr = a.cand_probs[(uint64_t)rp.cand_index * 16 + tid];
     }
@@ -2986,8 +2990,8 @@ __device__ __forceinline__ void merge_small_row(
     }
   }
   if (tid < 16) {
-    s.cids[tid] = draft != kNoToken ? cid : kNoToken;
-    s.cprobs[tid] = draft != kNoToken ? cpr : 0.0f;
+    s.cids[tid] = !DENSE && draft != kNoToken ? cid : kNoToken;
+    s.cprobs[tid] = !DENSE && draft != kNoToken ? cpr : 0.0f;
   }
   __syncthreads();
   const float maximum = s.row_max;
@@ -3044,7 +3048,7 @@ __device__ __forceinline__ void merge_small_row(
     }
     const int got = rank_select(sv, valid, thr, K, maximum, s);
     if (got >= 0) {
-      if (tid < 64) wave_finish(a, rp, row, s, (uint32_t)got, maximum, u, draft);
+      if (tid < 64) wave_finish<DENSE>(a, rp, row, s, (uint32_t)got, maximum, u, draft);
       return;
     }
     // More than 64 of them kept, or values that do not spread: the general
@@ -3072,13 +3076,13 @@ __device__ __forceinline__ void merge_small_row(
 }
 
 #if JF_IN(2)
-template <int DT, int SPEC, bool HOLD>
+template <int DT, int SPEC, bool HOLD, bool DENSE>
 __global__ __launch_bounds__(kThreads) void merge_small_kernel(
     const BlockHeader *headers, const uint64_t *cands, const RowParams *params,
     const float *uniforms, const uint32_t *uniform_index, uint32_t chunks_bits,
     uint32_t uniform_offset, uint32_t uniform_stride, uint32_t drafted_rows, SampleLaunch a) {
   const uint32_t row = blockIdx.x;
-  merge_small_row<DT, SPEC, HOLD>(
+  merge_small_row<DT, SPEC, HOLD, DENSE>(
       headers, cands, params, uniforms, uniform_index, chunks_bits, uniform_offset,
       uniform_stride, drafted_rows, a, row, g_small_lds, [&](uint32_t n) {
         // The launch record is copied word by word from the argument segment
@@ -4068,6 +4072,42 @@ __device__ __noinline__ void cut_sweep(uint32_t row, uint32_t c, uint32_t next) 
   __syncthreads();
 }
 
+// The nth (from 1) of the tokens of chunk c whose key is `key`, by id, into
+// s.bound. Every thread of the block calls it.
+template <int DT>
+__device__ __noinline__ void cut_nth_tie(uint32_t row, uint32_t c, uint32_t key, uint32_t nth) {
+  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
+                LOADS = Geo<DT>::LOADS;
+  const SampleLaunch &a = g_cut_launch;
+  CutLds &s = g_cut_lds;
+  const RowParams rp = a.params[row];
+  const uint32_t tid = threadIdx.x;
+  float xs[TPL];
+  load_chunk<DT>(a, rp, row, c, s, xs);
+  uint32_t cnt[LOADS], off[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    cnt[j] = 0;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float v = xs[j * VEC + e];
+      cnt[j] += v == v && logit_key(v) == key ? 1u : 0u;
+    }
+  }
+  order_offsets<LOADS>(cnt, off, s);
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    uint32_t at = off[j];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      const float v = xs[j * VEC + e];
+      if (v == v && logit_key(v) == key && ++at == nth)
+        s.bound = token_item(key, c * kChunkF32 + tid * VEC + j * SLAB + e);
+    }
+  }
+  __syncthreads();
+}
+
 // cut_resolve for a row of whose chunks some left sub-bins: those of all its
 // chunks together (the other chunks' lists count into them), the boundary's
 // sub-bin by their counts or masses, and the boundary in it. When all its
@@ -4086,8 +4126,6 @@ __device__ __noinline__ void cut_sweep(uint32_t row, uint32_t c, uint32_t next) 
 // 16 rows (1490-3950 before).
 template <int DT>
 __device__ __forceinline__ void cut_refine(uint32_t row, uint32_t bits) {
-  constexpr int VEC = Geo<DT>::VEC, TPL = Geo<DT>::TPL, SLAB = Geo<DT>::SLAB,
-                LOADS = Geo<DT>::LOADS;
   const SampleLaunch &a = g_cut_launch;
   CutLds &s = g_cut_lds;
   const RowParams rp = a.params[row];
@@ -4326,31 +4364,7 @@ __device__ __forceinline__ void cut_refine(uint32_t row, uint32_t bits) {
     s.cmass[lane] += kept * wq;
     s.ccount[lane] += kept;
   }
-  // The nth tie of chunk c by id, from the chunk itself.
-  float xs[TPL];
-  load_chunk<DT>(a, rp, row, c, s, xs);
-  uint32_t cnt[LOADS], off[LOADS];
-#pragma unroll
-  for (int j = 0; j < LOADS; ++j) {
-    cnt[j] = 0;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float v = xs[j * VEC + e];
-      cnt[j] += v == v && logit_key(v) == key ? 1u : 0u;
-    }
-  }
-  order_offsets<LOADS>(cnt, off, s);
-#pragma unroll
-  for (int j = 0; j < LOADS; ++j) {
-    uint32_t at = off[j];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float v = xs[j * VEC + e];
-      if (v == v && logit_key(v) == key && ++at == nth)
-        s.bound = token_item(key, c * kChunkF32 + tid * VEC + j * SLAB + e);
-    }
-  }
-  __syncthreads();
+  cut_nth_tie<DT>(row, c, key, nth);
 }
 
 // The draw inside chunk c of a row without a draft: the first kept token, in id
@@ -4567,7 +4581,7 @@ __device__ __forceinline__ void cut_finish_other(const SampleLaunch &a, const Ro
     cut_finish_general<DT>(row, kNoToken);
     return;
   }
-  merge_small_row<DT, 10, true>(
+  merge_small_row<DT, 10, true, false>(
       a.headers, a.cands, a.params, a.uniforms, a.uniform_index,
       S | (a.row_indexed ? kMergeRowIndexed : 0u) |
           ((rp.flags & kRowSampled) ? 0u : kMergeLateUniform),
@@ -5723,14 +5737,20 @@ int launch_merge_small(const SampleLaunch &a, uint32_t dtype, bool wide, bool ho
   };
   // The wider fetch past 20 chunks (fewer than 128 slots a chunk otherwise).
   const bool w = wide && a.chunks > 20;
-  if (dtype == 0 && hold)
-    w ? go(merge_small_kernel<0, 20, true>) : go(merge_small_kernel<0, 10, true>);
-  else if (dtype == 0)
-    w ? go(merge_small_kernel<0, 20, false>) : go(merge_small_kernel<0, 10, false>);
-  else if (hold)
-    w ? go(merge_small_kernel<1, 20, true>) : go(merge_small_kernel<1, 10, true>);
+  auto of = [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    if (a.dense_q)
+      w ? go(merge_small_kernel<DT, 20, false, true>) : go(merge_small_kernel<DT, 10, false, true>);
+    else if (hold)
+      w ? go(merge_small_kernel<DT, 20, true, false>) : go(merge_small_kernel<DT, 10, true, false>);
+    else
+      w ? go(merge_small_kernel<DT, 20, false, false>)
+        : go(merge_small_kernel<DT, 10, false, false>);
+  };
+  if (dtype == 0)
+    of(std::integral_constant<int, 0>{});
   else
-    w ? go(merge_small_kernel<1, 20, false>) : go(merge_small_kernel<1, 10, false>);
+    of(std::integral_constant<int, 1>{});
   return (int)hipGetLastError();
 }
 #endif

@@ -956,26 +956,29 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
     }
   }
   if (e != hipSuccess) return hip_fail((hipError_t)e, "select launch");
-  // merge_small_kernel takes launches that read sparse draft probabilities (or
-  // none). wide: some listed row has no min-p floor (longer lists).
-  const bool small = !a->draft_q && a->uniform_offset <= 0xffffffffull &&
-                     a->uniform_stride <= 0xffffffffull;
-  // hold: some min-p row may keep more than 64 tokens (a larger top-k, or none).
-  // (Rows with no floor and a top-k of 65 to 96 take the general merge's lists.)
-  bool wide = false, hold = false;
+  // merge_small_kernel takes launches whose uniforms fit its 32-bit arguments;
+  // with a dense q, those whose listed rows keep at most 64 tokens by their
+  // top-k (64 rows x 151,936 fp32, top-k 50: 15.8 us a call against 21.6 through
+  // merge_kernel; top-k 80 35.1 against 32.9, min-p 0.05 33.8 against 31.3).
+  // wide: some listed row has no min-p floor (longer lists); hold: some min-p
+  // row may keep more than 64 tokens (a larger top-k, or none).
+  const bool linear = a->uniform_offset <= 0xffffffffull && a->uniform_stride <= 0xffffffffull;
+  bool wide = false, hold = false, few = true;
   for (uint32_t r = 0; r < rows; ++r) {
     const jf::RowParams &rp = params[r];
+    if (!(rp.flags & kCuts) || jf::wide_row(rp.flags, rp.top_k)) continue;
     hold |= (rp.flags & jf::kRowMinP) && rp.top_k > 64;
-    wide |= (rp.flags & kCuts) && !(rp.flags & jf::kRowMinP) &&
-            !jf::wide_row(rp.flags, rp.top_k);
+    wide |= !(rp.flags & jf::kRowMinP);
+    few &= rp.top_k <= 64;
   }
+  const bool small = linear && (!a->draft_q || few);
   if (need_merge) {
     e = small ? jf::launch_merge_small(L, a->dtype, wide, hold, stream)
               : jf::launch_merge(L, a->dtype, stream);
     if (e != hipSuccess) return hip_fail((hipError_t)e, "merge launch");
   }
   if (passes) {
-    jf::CutLaunch c{true, true, any_drafted, others, pass_uncut, small};
+    jf::CutLaunch c{true, true, any_drafted, others, pass_uncut, linear && !a->draft_q};
     for (uint32_t r = 0; r < rows; ++r) {
       c.all &= jf::wide_row(params[r].flags, params[r].top_k);
       c.plain &= !(params[r].flags & jf::kRowPenalized);
