@@ -188,6 +188,36 @@ def test_cut_masks_penalties_and_other_rows():
     s.close()
 
 
+@pytest.mark.parametrize("kind", ["spread", "ties", "greedy rows", "min-p", "uncut rows"])
+@pytest.mark.parametrize("V,bf16", [(300, False), (20003, True), (151936, False), (170001, True),
+                                    (290003, False)])
+def test_dense_drafts_with_a_small_top_k(V, bf16, kind):
+    """Dense drafts and rows that keep at most 64 tokens: the small merge's build
+    for them, below and past 20 chunks, beside rows it does not draw."""
+    rng = np.random.default_rng(V + len(kind))
+    rows = 8
+    pols = [J.policy(temperature=0.8, top_k=k, top_p=p)
+            for k, p in ((50, 1.0), (64, 0.9), (1, 1.0), (20, 0.8)) * 2]
+    if kind == "min-p":
+        pols[1::2] = [J.policy(temperature=1.0, top_k=40, min_p=0.02)] * 4
+    if kind == "greedy rows":
+        pols[2], pols[5] = J.policy(), J.policy()
+    if kind == "uncut rows":
+        pols[0], pols[7] = J.policy(temperature=1.0), J.policy(temperature=0.7)
+    x = rng.normal(0, 2.5, (rows, V)).astype(np.float32)
+    if kind == "ties":
+        x = np.round(x)
+        x[6] = -2.0
+    draft = x.argmax(1).astype(np.uint32)
+    draft[1], draft[4], draft[5] = rng.integers(0, V), NO, x[5].argmin()
+    q = rng.dirichlet(np.ones(V) * 0.05, rows).astype(np.float32)
+    q[0] = 1.0  # takes every weight off: the plain draw
+    kw = dict(logits_bf16=WL.to_bf16_bits(x)) if bf16 else dict(logits=x)
+    kw.update(uniforms=rng.random(rows).astype(np.float32), draft_tokens=draft, dense_q=q)
+    check(V, pols, drafted_rows=rows - 1, **kw)
+    check(V, pols, kept_capacity=64, **kw)
+
+
 def flat_rows(V, rng):
     """Rows whose boundary bins hold more tokens of a chunk than its list takes:
     (name, values)."""
