@@ -129,6 +129,7 @@ __host__ __device__ constexpr bool wide_row(uint32_t flags, uint32_t top_k) {
          top_k > kListTopK;
 }
 
+constexpr uint32_t kNoGreedyRows = 0xffffffffu;  // SampleLaunch::uniform_row
 struct SampleLaunch {
   const void *logits;
   uint64_t stride;
@@ -144,10 +145,12 @@ struct SampleLaunch {
                           // rows
   uint32_t row_indexed;   // drafts are addressed through RowParams'
                           // draft_index/cand_index, not the row number
-  uint32_t greedy_rows;   // some row is greedy. It has no uniform, and its
-                          // place in the uniforms or their index may hold
-                          // anything: a kernel then reads a row's uniform
-                          // only once the row is known to be sampled
+  uint32_t uniform_row;   // kNoGreedyRows, or, in a launch with greedy rows, a
+                          // sampled one (0 without any). A greedy row has no
+                          // uniform, and its place in the uniforms or their
+                          // index may hold anything: a kernel then reads a
+                          // row's uniform only once the row is known to be
+                          // sampled
   const uint2 *pen_entries;
   const uint32_t *pen_offsets;
   uint32_t pen_max_entries;
@@ -194,7 +197,7 @@ constexpr uint32_t kMergeRowIndexed = 0x80000000u;   // SampleLaunch::row_indexe
 constexpr uint32_t kMergeLateUniform = 0x40000000u;  // the uniform waits for the row's record
 inline uint32_t merge_chunks_bits(const SampleLaunch &a) {
   return a.chunks | (a.row_indexed ? kMergeRowIndexed : 0u) |
-         (a.greedy_rows ? kMergeLateUniform : 0u);
+         (a.uniform_row != kNoGreedyRows ? kMergeLateUniform : 0u);
 }
 
 // The fast selection launch: the per-row facts every block needs before its

@@ -5323,8 +5323,8 @@ __global__ __launch_bounds__(kThreads) void uncut_kernel(SampleLaunch a, uint32_
   // Requested together before anything waits: the row's record, its
   // uniform, and (wave 0) its chunk summaries, one per lane (S <= 64).
   const RowParams rp = a.params[row];
-  float u = 0.0f;
-  if (!a.greedy_rows) u = row_uniform(a, row);
+  // (In a launch with greedy rows, a sampled row's: no branch before the loads.)
+  float u = row_uniform(a, a.uniform_row == kNoGreedyRows ? row : a.uniform_row);
   const bool in = w == 0 && lane < S;
   const BlockHeader *hl = hb + (in ? lane : 0u);
   const float hm = hl->maximum, hbv = hl->best_value;
@@ -5342,7 +5342,7 @@ __global__ __launch_bounds__(kThreads) void uncut_kernel(SampleLaunch a, uint32_
     return;
   }
   if (!uncut_row(rp)) return;  // the merge's
-  if (a.greedy_rows) u = row_uniform(a, row);
+  if (a.uniform_row != kNoGreedyRows) u = row_uniform(a, row);
   const uint32_t draft = row_draft(a, rp);
   const bool drafted = draft != kNoToken;
   if (!drafted && chunk != 0) return;

@@ -803,8 +803,13 @@ int sample_core(uint32_t V, const SampleScratch &sc, const jf_sample_args *a,
   // use it as the linear prefix unless the rows are indexed.
   L.drafted_rows = !any_drafted ? 0u : row_indexed ? rows : a->drafted_rows;
   L.row_indexed = row_indexed ? 1u : 0u;
-  for (uint32_t r = 0; r < rows && !L.greedy_rows; ++r)
-    L.greedy_rows = (params[r].flags & jf::kRowSampled) ? 0u : 1u;
+  uint32_t sampled_rows = 0;
+  for (uint32_t r = rows; r-- > 0;)
+    if (params[r].flags & jf::kRowSampled) {
+      L.uniform_row = r;
+      ++sampled_rows;
+    }
+  if (sampled_rows == rows) L.uniform_row = jf::kNoGreedyRows;
   L.cand_ids = a->draft_cand_ids;
   L.cand_probs = a->draft_cand_probs;
   L.dense_q = a->draft_q;

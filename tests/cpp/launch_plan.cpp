@@ -17,8 +17,8 @@ std::string g_out;
 
 void add(const char *name, const jf::SampleLaunch &a, const std::string &more = "") {
   if (!g_out.empty()) g_out += ", ";
-  g_out += "{\"launch\": \"" + std::string(name) + "\", \"greedy_rows\": " +
-           std::to_string(a.greedy_rows) + more + "}";
+  g_out += "{\"launch\": \"" + std::string(name) + "\", \"uniform_row\": " +
+           std::to_string(a.uniform_row) + more + "}";
 }
 }  // namespace
 

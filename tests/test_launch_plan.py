@@ -34,7 +34,8 @@ def test_launches_know_of_greedy_rows(batch, launch):
     names = [l["launch"] for l in b["launches"]]
     assert launch in names, names
     for l in b["launches"]:
-        assert l["greedy_rows"] == 1
+        # A sampled row, whose uniform stands for those a greedy row lacks.
+        assert l["uniform_row"] == next(r for r, k in enumerate(batch) if k != "g")
         if l["launch"] == "merge_small":
             assert l["late_uniform"] == 1 and l["chunks"] == 3
         if l["launch"] == "residual":
@@ -47,7 +48,7 @@ def test_launches_know_of_greedy_rows(batch, launch):
 def test_sampled_launches_read_uniforms_early(batch):
     (b,) = plan(batch)
     for l in b["launches"]:
-        assert l["greedy_rows"] == 0
+        assert l["uniform_row"] == 0xffffffff
         assert l.get("late_uniform", 0) == 0
         assert all(v < LEAN_GREEDY for v in l.get("row_of", []))
 
