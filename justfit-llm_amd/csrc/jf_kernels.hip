@@ -4232,6 +4232,7 @@ __device__ __forceinline__ void cut_refine(uint32_t row, uint32_t bits) {
       s.top = top;
       s.shift = shift;
       s.small_n = 0;
+      s.n = 0;
     }
     if (tid < kMaxChunks) {
       s.sum_mass[tid] = 0;
@@ -4268,8 +4269,9 @@ __device__ __forceinline__ void cut_refine(uint32_t row, uint32_t bits) {
       tied(g, true);
       const uint64_t top = ((uint64_t)hi << 19) | 0x7ffffull;
       uint64_t from = (uint64_t)lo << 19, to = top;
+      // (Eleven bits of the items' 51 a pass: at most five, whatever is read.)
       uint32_t n = s.sub_n[g];
-      while (n > kCutItems) {
+      for (int pass = 0; n > kCutItems && pass < 5; ++pass) {
         const int shift = max(0, 64 - (int)__builtin_clzll(to - from) - 11);
         for (uint32_t i = tid; i < kCutCells; i += kThreads) {
           s.cell_mass[i] = 0;
